@@ -7,6 +7,7 @@
 // of operations of Model::trainStep (:664-707) / trainStepLoop (:709-741).
 #include "../../include/kge_hip.h"
 #include "kge_kernels.h"
+#include "kge_transfer.h"
 
 #include <algorithm>
 #include <cmath>
@@ -136,43 +137,6 @@ struct DevBuf {
 int round_up(int x, int m) { return (x + m - 1) / m * m; }
 int elem_size(int et) { return et == ET_F32 ? 4 : 2; }
 int bit_length(uint64_t x) { int b = 0; while (x) { ++b; x >>= 1; } return b; }
-
-float half_to_float(uint16_t h) {
-    const uint32_t sign = (uint32_t)(h & 0x8000) << 16;
-    uint32_t exp = (h >> 10) & 0x1f, man = h & 0x3ff, u;
-    if (exp == 0) {
-        if (man == 0) u = sign;
-        else {
-            int e = -1;
-            do { ++e; man <<= 1; } while (!(man & 0x400));
-            u = sign | ((uint32_t)(127 - 15 - e) << 23) | ((man & 0x3ff) << 13);
-        }
-    } else if (exp == 31) u = sign | 0x7f800000u | (man << 13);
-    else u = sign | ((exp + 112) << 23) | (man << 13);
-    float f;
-    std::memcpy(&f, &u, 4);
-    return f;
-}
-uint16_t float_to_half(float f) {
-    uint32_t u;
-    std::memcpy(&u, &f, 4);
-    const uint32_t sign = (u >> 16) & 0x8000;
-    uint32_t mag = u & 0x7fffffffu;
-    if (mag >= 0x7f800000u) return (uint16_t)(sign | 0x7c00 | (mag > 0x7f800000u ? 0x200 : 0));
-    if (mag >= 0x477ff000u) return (uint16_t)(sign | 0x7c00);
-    if (mag < 0x38800000u) {  // subnormal half
-        if (mag < 0x33000000u) return (uint16_t)sign;
-        const int e = (int)(mag >> 23);
-        uint32_t man = (mag & 0x7fffffu) | 0x800000u;
-        const int shift = 126 - e;  // total right shift: 13 + (113 - e)
-        const uint32_t half = 1u << (shift - 1), rem = man & ((1u << shift) - 1);
-        man >>= shift;
-        if (rem > half || (rem == half && (man & 1))) ++man;
-        return (uint16_t)(sign | man);
-    }
-    mag += 0xfffu + ((mag >> 13) & 1u);
-    return (uint16_t)(sign | ((mag - 0x38000000u) >> 13));
-}
 
 enum KernelId {
     K_PLAN = 0, K_HIDDEN, K_GATHER, K_FWD, K_LOSS, K_BWD, K_REDUCE_ENT, K_ADAM_ENT, K_REDUCE_REL, K_ADAM_REL,
@@ -313,10 +277,15 @@ struct kge_engine {
     // sits in the first two entries of the relation group
     std::vector<float> h_alpha;
     int n_part;
-    // io staging
-    DevBuf<uint64_t> io_rows;
-    DevBuf<float> io_data;
-    DevBuf<uint32_t> io_idx;
+    // Reads and writes of rows and variables pass through pinned memory that the kernels address:
+    // io_n_slots slots of io_slot bytes, and the row numbers of a read_entity / write_entity call
+    static constexpr int kIoSlots = 4;
+    size_t io_n_slots = 1;
+    char *io_slots = nullptr, *d_io_slots = nullptr;
+    uint64_t *io_rows = nullptr, *d_io_rows = nullptr;
+    size_t io_slot = 0;
+    hipEvent_t io_done[kIoSlots] = {};
+    std::unique_ptr<CopyThreads> copy_threads;
 
     // timing
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -340,6 +309,9 @@ struct kge_engine {
         for (auto& e : chunk_copied) (void)hipEventDestroy(e);
         for (auto& e : chunk_planned) (void)hipEventDestroy(e);
         if (h_idx) (void)hipHostFree(h_idx);
+        for (auto& e : io_done) if (e) (void)hipEventDestroy(e);
+        if (io_slots) (void)hipHostFree(io_slots);
+        if (io_rows) (void)hipHostFree(io_rows);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -776,11 +748,67 @@ void allocate(kge_engine& E) {
     E.loss_step.alloc(ns * S);
     E.d_alpha.alloc(ns * 9 * S);
 
-    const size_t io_n = (size_t)E.S * E.rw_batch;
-    E.io_rows.alloc(io_n);
-    E.io_idx.alloc(io_n);
-    E.io_data.alloc(io_n * (3 * E.D + E.F));
+    {   // as much pinned memory as the largest transfer can use, 4 slots of 2 MiB at most (a slot holds one row at least)
+        const size_t io_n = (size_t)E.S * E.rw_batch, row = (size_t)(3 * E.D + E.F) * 4;
+        size_t most = std::max(io_n, (size_t)E.n_rows) * row;
+        for (const Variable& v : E.variables)
+            if (v.shape.size() == 2) most = std::max(most, v.shape[0] * v.shape[1] * 4);
+        E.io_slot = std::min(most, std::max<size_t>(2 << 20, std::max<size_t>(row, (size_t)std::max(2 * E.D, E.mlp) * 4)));
+        E.io_slot = (E.io_slot + 15) / 16 * 16;
+        E.io_n_slots = most <= E.io_slot ? 1 : kge_engine::kIoSlots;
+        HIP_CHECK(hipHostMalloc((void**)&E.io_slots, E.io_n_slots * E.io_slot, hipHostMallocDefault));
+        HIP_CHECK(hipHostGetDevicePointer((void**)&E.d_io_slots, E.io_slots, 0));
+        HIP_CHECK(hipHostMalloc((void**)&E.io_rows, io_n * 8, hipHostMallocDefault));
+        HIP_CHECK(hipHostGetDevicePointer((void**)&E.d_io_rows, E.io_rows, 0));
+        for (auto& e : E.io_done) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
     HIP_CHECK(hipStreamSynchronize(st));
+}
+
+// ---- host transfers ---------------------------------------------------------------
+
+// `units` units of `unit` bytes between the caller's array and the device.  launch(first, n, slot)
+// starts the kernel that moves units [first, first + n) between the device and a pinned slot.
+// Transfers of more than one slot are pipelined, the host's copies split over the copy threads
+// (created by the first such transfer).
+template <class Launch>
+void transfer(kge_engine& E, bool to_device, void* array, size_t units, size_t unit, Launch&& launch) {
+    if (units == 0 || unit == 0) return;
+    const hipStream_t st = E.stream;
+    const size_t n_slots = E.io_n_slots;
+    const size_t per = std::min(units, E.io_slot / unit), n_chunk = (units + per - 1) / per;
+    // below this a few threads' wake-up costs more than they save
+    const bool threaded = units * unit >= (size_t)1 << 20;
+    if (threaded && !E.copy_threads) E.copy_threads.reset(new CopyThreads(7));
+    SlottedCopy copy((char*)array, E.io_slots, units * unit, per * unit, (int)n_slots, to_device,
+                     threaded ? E.copy_threads.get() : nullptr);
+    auto start = [&](size_t k) {
+        const size_t slot = k % n_slots;
+        launch(k * per, std::min(per, units - k * per), E.d_io_slots + slot * per * unit);
+        HIP_CHECK(hipGetLastError());
+        if (n_chunk > 1) HIP_CHECK(hipEventRecord(E.io_done[slot], st));
+    };
+    auto finished = [&](size_t k) {
+        if (n_chunk > 1) HIP_CHECK(hipEventSynchronize(E.io_done[k % n_slots]));
+        else HIP_CHECK(hipStreamSynchronize(st));
+    };
+    if (to_device) {
+        for (size_t k = 0; k < n_chunk; ++k) {
+            if (k >= n_slots) finished(k - n_slots);
+            copy.allow(k);
+            copy.wait(k);
+            start(k);
+        }
+        HIP_CHECK(hipStreamSynchronize(st));
+    } else {
+        size_t started = 0;
+        for (size_t k = 0; k < n_chunk; ++k) {
+            while (started < n_chunk && started < k + n_slots) start(started++);
+            finished(k);
+            copy.allow(k);
+            copy.wait(k);
+        }
+    }
 }
 
 // ---- variables: "read" / "write" (src/poplar_kge.cpp:977-991) ----------------
@@ -816,8 +844,15 @@ void run_read_write(kge_engine& E, bool write, const Items& in) {
     else if (name == "feature_projection/adam_m") { buf = &E.proj_m; row0 = net * E.Fp; }
     else if (name == "feature_projection/adam_v") { buf = &E.proj_v; row0 = net * E.Fp; }
     const size_t rows = var->shape[0], cols = var->shape[1];
-    if (rows == 0 || cols == 0) return;
-    HIP_CHECK(hipStreamSynchronize(E.stream));
+    // hipMemcpy2D moves pageable rows one by one (1387 rows of 1 KB: 9.3 ms); a kernel takes the
+    // pitch off between the device and pinned memory, and the host copies whole runs (0.2 ms)
+    auto move = [&](float* dev, size_t dpitch, float* h, size_t n) {
+        transfer(E, write, h, n, cols * 4, [&](size_t first, size_t count, char* slot) {
+            float* d = dev + first * dpitch;
+            if (write) launch_copy_rows(d, dpitch, (const float*)slot, cols, (int)cols, count, E.stream);
+            else launch_copy_rows((float*)slot, cols, d, dpitch, (int)cols, count, E.stream);
+        });
+    };
     if (name.rfind("mlp_", 0) == 0) {
         const bool is_up = name.rfind("mlp_up_projection", 0) == 0;
         const bool m = name.size() > 7 && name.compare(name.size() - 7, 7, "/adam_m") == 0;
@@ -827,25 +862,17 @@ void run_read_write(kge_engine& E, bool write, const Items& in) {
         // Up: host rows [0, D) and [D, 2 D) are device rows [0, D) and [Dp, Dp + D), pitch M;
         // Down: host [M, D] in device rows of pitch Dp
         const size_t D = E.D, Dp = E.Dp, M = E.mlp;
-        for (int half = 0; half < (is_up ? 2 : 1); ++half) {
-            float* d = dev + (is_up ? (size_t)half * Dp * M : 0);
-            float* h = host + (is_up ? (size_t)half * D * M : 0);
-            const size_t dpitch = (is_up ? M : Dp) * 4, hpitch = cols * 4, n = is_up ? D : M;
-            if (write) HIP_CHECK(hipMemcpy2D(d, dpitch, h, hpitch, cols * 4, n, hipMemcpyHostToDevice));
-            else HIP_CHECK(hipMemcpy2D(h, hpitch, d, dpitch, cols * 4, n, hipMemcpyDeviceToHost));
-        }
+        if (!is_up) { move(dev, Dp, host, M); return; }
+        move(dev, M, host, D);
+        move(dev + Dp * M, M, host + D * M, D);
         return;
     }
-    if (write)
-        HIP_CHECK(hipMemcpy2D(buf->p + row0 * E.Dp, (size_t)E.Dp * 4, host, cols * 4, cols * 4, rows, hipMemcpyHostToDevice));
-    else
-        HIP_CHECK(hipMemcpy2D(host, cols * 4, buf->p + row0 * E.Dp, (size_t)E.Dp * 4, cols * 4, rows, hipMemcpyDeviceToHost));
+    move(buf->p + row0 * E.Dp, E.Dp, host, rows);
 }
 
 // ---- entity rows: "write_entity", "read_entity" (:857-871) --------------------
 
-void upload_row_ids(kge_engine& E, const uint32_t* idx, size_t per_shard, std::vector<uint64_t>& rows) {
-    rows.resize((size_t)E.S * per_shard);
+void put_row_ids(kge_engine& E, const uint32_t* idx, size_t per_shard) {
     for (int s = 0; s < E.S; ++s)
         for (size_t i = 0; i < per_shard; ++i) {
             const uint32_t v = idx[s * per_shard + i];
@@ -854,54 +881,54 @@ void upload_row_ids(kge_engine& E, const uint32_t* idx, size_t per_shard, std::v
                 msg << "entity index " << v << " out of range [0, " << E.n_entity << ")";
                 throw std::invalid_argument(msg.str());
             }
-            rows[s * per_shard + i] = (E.shared_table ? 0 : (uint64_t)s * E.n_entity) + v;
+            E.io_rows[s * per_shard + i] = (E.shared_table ? 0 : (uint64_t)s * E.n_entity) + v;
         }
-    HIP_CHECK(hipMemcpyAsync(E.io_rows.p, rows.data(), rows.size() * 8, hipMemcpyHostToDevice, E.stream));
 }
 
 void run_write_entity(kge_engine& E, const Items& in, bool raw) {
     const size_t S = E.S, rw = E.rw_batch, W = raw ? 3 * E.D + E.F : E.F;
     const uint32_t* idx = (const uint32_t*)in.array("write_indices", KGE_U32, {S, rw});
     const int kind = raw ? KGE_F32 : E.stream_kind;
-    const void* data = in.array(raw ? "write_data" : "write_features", kind, {S, rw, W});
-    std::vector<uint64_t> rows;
-    upload_row_ids(E, idx, rw, rows);
-    std::vector<float> conv;
-    const float* src = (const float*)data;
-    if (kind == KGE_F16) {
-        conv.resize(S * rw * W);
-        const uint16_t* h = (const uint16_t*)data;
-        for (size_t i = 0; i < conv.size(); ++i) conv[i] = half_to_float(h[i]);
-        src = conv.data();
+    void* data = in.array(raw ? "write_data" : "write_features", kind, {S, rw, W});
+    put_row_ids(E, idx, rw);
+    const float sigma = E.init_scale / (float)E.D;  // of the random-normal embedding (:865-866)
+    const int f16 = kind == KGE_F16;
+    if (!raw && W == 0) {
+        launch_init_rows(E.L, E.table.p, E.d_io_rows, (int64_t)(S * rw), nullptr, 0, sigma, E.seed, E.stream);
+        HIP_CHECK(hipGetLastError());
+        HIP_CHECK(hipStreamSynchronize(E.stream));
+        return;
     }
-    if (W) HIP_CHECK(hipMemcpyAsync(E.io_data.p, src, S * rw * W * 4, hipMemcpyHostToDevice, E.stream));
-    if (raw)
-        launch_rows_from_logical(E.L, E.table.p, E.io_rows.p, (int64_t)(S * rw), E.io_data.p, E.stream);
-    else  // random-normal embedding with sigma = init_scale / D (:865-866)
-        launch_init_rows(E.L, E.table.p, E.io_rows.p, (int64_t)(S * rw), E.io_data.p,
-                         E.init_scale / (float)E.D, E.seed, E.stream);
-    HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipStreamSynchronize(E.stream));
+    transfer(E, true, data, S * rw, W * (f16 ? 2 : 4), [&](size_t first, size_t n, char* slot) {
+        if (raw)
+            launch_rows_from_logical(E.L, E.table.p, E.d_io_rows + first, n, (const float*)slot, E.stream);
+        else
+            launch_init_rows(E.L, E.table.p, E.d_io_rows + first, n, slot, f16, sigma, E.seed, E.stream);
+    });
 }
 
 void run_read_entity(kge_engine& E, const Items& in) {
     const size_t S = E.S, rw = E.rw_batch, W = 3 * E.D + E.F;
     const uint32_t* idx = (const uint32_t*)in.array("read_indices", KGE_U32, {S, rw});
     void* out = in.array("read_data", E.stream_kind, {S, rw, W});
-    std::vector<uint64_t> rows;
-    upload_row_ids(E, idx, rw, rows);
-    launch_rows_to_logical(E.L, E.table.p, E.io_rows.p, (int64_t)(S * rw), E.io_data.p, E.stream);
-    HIP_CHECK(hipGetLastError());
-    if (E.stream_kind == KGE_F32) {
-        HIP_CHECK(hipMemcpyAsync(out, E.io_data.p, S * rw * W * 4, hipMemcpyDeviceToHost, E.stream));
-        HIP_CHECK(hipStreamSynchronize(E.stream));
-    } else {
-        std::vector<float> tmp(S * rw * W);
-        HIP_CHECK(hipMemcpyAsync(tmp.data(), E.io_data.p, tmp.size() * 4, hipMemcpyDeviceToHost, E.stream));
-        HIP_CHECK(hipStreamSynchronize(E.stream));
-        uint16_t* h = (uint16_t*)out;
-        for (size_t i = 0; i < tmp.size(); ++i) h[i] = float_to_half(tmp[i]);
-    }
+    put_row_ids(E, idx, rw);
+    const int f16 = E.stream_kind == KGE_F16;
+    transfer(E, false, out, S * rw, W * (f16 ? 2 : 4), [&](size_t first, size_t n, char* slot) {
+        launch_rows_to_logical(E.L, E.table.p, E.d_io_rows + first, 0, n, slot, f16, E.stream);
+    });
+}
+
+// additive: "read_entity_all": read_data [S, n_entity, 3D+F], every shard's rows in order
+void run_read_entity_all(kge_engine& E, const Items& in) {
+    const size_t S = E.S, N = E.n_entity, W = 3 * E.D + E.F;
+    const int f16 = E.stream_kind == KGE_F16;
+    const size_t unit = W * (f16 ? 2 : 4);
+    char* out = (char*)in.array("read_data", E.stream_kind, {S, N, W});
+    // private tables lie one behind the other as the array's do; a shared one is every shard's
+    for (size_t s = 0; s < (E.shared_table ? S : 1); ++s)
+        transfer(E, false, out + s * N * unit, E.n_rows, unit, [&](size_t first, size_t n, char* slot) {
+            launch_rows_to_logical(E.L, E.table.p, nullptr, first, n, slot, f16, E.stream);
+        });
 }
 
 // ---- training ------------------------------------------------------------------
@@ -2079,6 +2106,7 @@ int kge_engine_run(kge_engine* engine, const char* command, kge_item* items, siz
         const std::string cmd = command;
         if (cmd == "train_step_loop") run_train_step_loop(E, in);
         else if (cmd == "read_entity") run_read_entity(E, in);
+        else if (cmd == "read_entity_all") run_read_entity_all(E, in);
         else if (cmd == "write_entity") run_write_entity(E, in, false);
         else if (cmd == "write_entity_raw") run_write_entity(E, in, true);
         else if (cmd == "read") run_read_write(E, false, in);

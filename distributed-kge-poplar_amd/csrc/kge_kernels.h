@@ -417,15 +417,20 @@ struct RowLayout {
     int emb_etype, mom_etype, feat_etype;
     int64_t off_m, off_s, off_f, pitch;  // bytes; embedding at offset 0
 };
-// logical float32 rows [n, 3D+F] <-> physical rows at base + idx[i]*pitch
-void launch_rows_to_logical(const RowLayout& L, const char* base, const uint64_t* rows, int64_t n,
-                            float* out, hipStream_t stream);
+// logical rows [n, 3D+F] <-> physical rows at base + row * pitch.  The logical side may be host
+// memory that the device addresses.  rows: null for the rows row0, row0 + 1, ...; out_f16: float16
+// rows (else float32)
+void launch_rows_to_logical(const RowLayout& L, const char* base, const uint64_t* rows, uint64_t row0, int64_t n,
+                            void* out, int out_f16, hipStream_t stream);
 void launch_rows_from_logical(const RowLayout& L, char* base, const uint64_t* rows, int64_t n,
                               const float* in, hipStream_t stream);
+// rows of `cols` floats from pitch to pitch (floats); either side may be device-visible host memory
+void launch_copy_rows(float* dst, int64_t dpitch, const float* src, int64_t spitch, int cols, int64_t rows,
+                      hipStream_t stream);
 // write_entity: embedding ~ N(0, sigma) from a counter-based generator keyed by
-// (seed, row, column); zero moments; features from `features` [n, F] float32.
+// (seed, row, column); zero moments; features from `features` [n, F], float32 or float16.
 void launch_init_rows(const RowLayout& L, char* base, const uint64_t* rows, int64_t n,
-                      const float* features, float sigma, uint32_t seed, hipStream_t stream);
+                      const void* features, int features_f16, float sigma, uint32_t seed, hipStream_t stream);
 
 // ---- standalone ops --------------------------------------------------------
 void launch_distance(int dist_fn, const float* a, const float* b, float* out, int M, int N, int D,

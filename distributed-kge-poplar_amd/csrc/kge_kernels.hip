@@ -2398,26 +2398,36 @@ DEVINL void locate(const RowLayout& L, int c, int64_t& off, int& k, int& et) {
     else { off = L.off_f; k = c - 3 * L.D; et = L.feat_etype; }
 }
 
+// Rows of a read or write stream, [n, 3D+F] of `OT` (float, or __half for the float16 streams), in
+// host memory that the device addresses: a wave stores (loads) four elements per lane, so that an
+// access crosses PCIe as one run of 512 or 1024 bytes.  QUAD: D and F are multiples of four, every
+// four elements lie in one section.  rows: null for the consecutive rows from row0 on.
+template <class OT>
+DEVINL void store4_as(OT* out, float4 v) {
+    if constexpr (sizeof(OT) == 4) *reinterpret_cast<float4*>(out) = v;
+    else store4(reinterpret_cast<char*>(out), 0, ET_F16, v);
+}
+template <class OT, bool QUAD>
 __global__ __launch_bounds__(256) void k_rows_to_logical(RowLayout L, const char* __restrict__ base,
-                                                         const uint64_t* __restrict__ rows, int64_t n,
-                                                         float* __restrict__ out) {
+                                                         const uint64_t* __restrict__ rows, uint64_t row0,
+                                                         OT* __restrict__ out) {
     const int W = 3 * L.D + L.F;
     const int64_t i = blockIdx.x;
-    if (i >= n) return;
-    const char* row = base + (int64_t)rows[i] * L.pitch;
-    for (int c = threadIdx.x; c < W; c += 256) {
+    const char* row = base + (int64_t)(rows ? rows[i] : row0 + i) * L.pitch;
+    for (int c = threadIdx.x * (QUAD ? 4 : 1); c < W; c += 256 * (QUAD ? 4 : 1)) {
         int64_t off; int k, et;
         locate(L, c, off, k, et);
-        out[i * W + c] = load1(row + off, k, et);
+        if constexpr (QUAD) store4_as(out + i * W + c, load4(row + off, k, et));
+        else if constexpr (sizeof(OT) == 4) out[i * W + c] = load1(row + off, k, et);
+        else out[i * W + c] = __float2half_rn(load1(row + off, k, et));
     }
 }
 
 __global__ __launch_bounds__(256) void k_rows_from_logical(RowLayout L, char* __restrict__ base,
                                                            const uint64_t* __restrict__ rows,
-                                                           int64_t n, const float* __restrict__ in) {
+                                                           const float* __restrict__ in) {
     const int W = 3 * L.D + L.F;
     const int64_t i = blockIdx.x;
-    if (i >= n) return;
     char* row = base + (int64_t)rows[i] * L.pitch;
     for (int c = threadIdx.x; c < W; c += 256) {
         int64_t off; int k, et;
@@ -2426,15 +2436,37 @@ __global__ __launch_bounds__(256) void k_rows_from_logical(RowLayout L, char* __
     }
 }
 
-void launch_rows_to_logical(const RowLayout& L, const char* base, const uint64_t* rows, int64_t n,
-                            float* out, hipStream_t stream) {
+void launch_rows_to_logical(const RowLayout& L, const char* base, const uint64_t* rows, uint64_t row0, int64_t n,
+                            void* out, int out_f16, hipStream_t stream) {
     if (n == 0) return;
-    hipLaunchKernelGGL(k_rows_to_logical, dim3((unsigned)n), dim3(256), 0, stream, L, base, rows, n, out);
+    const bool quad = L.D % 4 == 0 && L.F % 4 == 0;
+#define KGE_ROWS(T_, Q_)                                                                                     \
+    hipLaunchKernelGGL((k_rows_to_logical<T_, Q_>), dim3((unsigned)n), dim3(256), 0, stream, L, base, rows, row0, (T_*)out)
+    if (out_f16) { if (quad) KGE_ROWS(__half, true); else KGE_ROWS(__half, false); }
+    else         { if (quad) KGE_ROWS(float, true); else KGE_ROWS(float, false); }
+#undef KGE_ROWS
 }
 void launch_rows_from_logical(const RowLayout& L, char* base, const uint64_t* rows, int64_t n,
                               const float* in, hipStream_t stream) {
     if (n == 0) return;
-    hipLaunchKernelGGL(k_rows_from_logical, dim3((unsigned)n), dim3(256), 0, stream, L, base, rows, n, in);
+    hipLaunchKernelGGL(k_rows_from_logical, dim3((unsigned)n), dim3(256), 0, stream, L, base, rows, in);
+}
+
+// rows of `cols` floats between two pitches (floats)
+__global__ __launch_bounds__(256) void k_copy_rows(float* __restrict__ dst, int64_t dpitch, const float* __restrict__ src,
+                                                   int64_t spitch, int cols) {
+    const float* s = src + (int64_t)blockIdx.x * spitch;
+    float* d = dst + (int64_t)blockIdx.x * dpitch;
+    if (((dpitch | spitch | cols) & 3) == 0) {
+        for (int c = threadIdx.x * 4; c < cols; c += 1024) *reinterpret_cast<float4*>(d + c) = *reinterpret_cast<const float4*>(s + c);
+    } else {
+        for (int c = threadIdx.x; c < cols; c += 256) d[c] = s[c];
+    }
+}
+void launch_copy_rows(float* dst, int64_t dpitch, const float* src, int64_t spitch, int cols, int64_t rows,
+                      hipStream_t stream) {
+    if (rows == 0 || cols == 0) return;
+    hipLaunchKernelGGL(k_copy_rows, dim3((unsigned)rows), dim3(256), 0, stream, dst, dpitch, src, spitch, cols);
 }
 
 // counter-based normal generator: two rounds of a 64-bit mix, then Box-Muller
@@ -2453,28 +2485,40 @@ DEVINL float normal_at(uint32_t seed, uint64_t row, uint32_t col) {
 
 // Model::writeEntity (src/poplar_kge.cpp:864-871): emb ~ N(0, sigma), zero
 // moments, host features; padding columns are zero.
+template <class FT, bool QUAD>  // FT: element type of the features as the caller has them; QUAD: F % 4 == 0
 __global__ __launch_bounds__(256) void k_init_rows(RowLayout L, char* __restrict__ base,
-                                                   const uint64_t* __restrict__ rows, int64_t n,
-                                                   const float* __restrict__ features, float sigma,
+                                                   const uint64_t* __restrict__ rows,
+                                                   const FT* __restrict__ features, float sigma,
                                                    uint32_t seed) {
     const int64_t i = blockIdx.x;
-    if (i >= n) return;
     const uint64_t r = rows[i];
     char* row = base + (int64_t)r * L.pitch;
+    const char* feat = reinterpret_cast<const char*>(features + i * L.F);
+    constexpr int kFt = sizeof(FT) == 4 ? ET_F32 : ET_F16;
+    // the features first: they come across PCIe, and the generator's arithmetic covers the way
+    if constexpr (QUAD) {
+        for (int f = threadIdx.x * 4; f < L.Fp; f += 1024)
+            store4(row + L.off_f, f, L.feat_etype, f < L.F ? load4(feat, f, kFt) : make_float4(0.f, 0.f, 0.f, 0.f));
+    } else {
+        for (int f = threadIdx.x; f < L.Fp; f += 256)
+            store1(row + L.off_f, f, L.feat_etype, f < L.F ? load1(feat, f, kFt) : 0.f);
+    }
     for (int k = threadIdx.x; k < L.Dp; k += 256) {
         store1(row, k, L.emb_etype, k < L.D ? sigma * normal_at(seed, r, k) : 0.f);
         store1(row + L.off_m, k, L.mom_etype, 0.f);
         store1(row + L.off_s, k, L.mom_etype, 0.f);
     }
-    for (int f = threadIdx.x; f < L.Fp; f += 256)
-        store1(row + L.off_f, f, L.feat_etype, f < L.F ? features[i * L.F + f] : 0.f);
 }
 
 void launch_init_rows(const RowLayout& L, char* base, const uint64_t* rows, int64_t n,
-                      const float* features, float sigma, uint32_t seed, hipStream_t stream) {
+                      const void* features, int features_f16, float sigma, uint32_t seed, hipStream_t stream) {
     if (n == 0) return;
-    hipLaunchKernelGGL(k_init_rows, dim3((unsigned)n), dim3(256), 0, stream, L, base, rows, n,
-                       features, sigma, seed);
+#define KGE_INIT(T_, Q_)                                                                                  \
+    hipLaunchKernelGGL((k_init_rows<T_, Q_>), dim3((unsigned)n), dim3(256), 0, stream, L, base, rows,     \
+                       (const T_*)features, sigma, seed)
+    if (features_f16) { if (L.F % 4 == 0) KGE_INIT(__half, true); else KGE_INIT(__half, false); }
+    else              { if (L.F % 4 == 0) KGE_INIT(float, true); else KGE_INIT(float, false); }
+#undef KGE_INIT
 }
 
 // --------------------------------------------------------------------------

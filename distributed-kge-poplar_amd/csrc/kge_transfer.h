@@ -1,0 +1,137 @@
+// Bulk transfers between the caller's host arrays and the device, through pinned memory.
+//
+// The caller's arrays are pageable, so their bytes pass through pinned slots that the kernels
+// address directly (a kernel gathers table rows and stores them to the slot across PCIe: no
+// device-side staging buffer, no separate copy).  What bounds a large transfer then is the host's
+// own memcpy between slot and array, most of all the first touch of a fresh array's pages, so it
+// is split over a few threads and runs beside the next slot's kernel.
+#pragma once
+
+#include <algorithm>
+#include <atomic>
+#include <condition_variable>
+#include <cstddef>
+#include <cstring>
+#include <functional>
+#include <memory>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+namespace kge {
+
+// A handful of threads that all run one function at a time, woken once per transfer.  Created by
+// the first large transfer of its owner, joined with it.
+class CopyThreads {
+   public:
+    explicit CopyThreads(int n) {
+        for (int i = 0; i < n; ++i) threads_.emplace_back([this, i] { loop(i); });
+    }
+    ~CopyThreads() {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            quit_ = true;
+        }
+        wake_.notify_all();
+        for (auto& t : threads_) t.join();
+    }
+    CopyThreads(const CopyThreads&) = delete;
+    CopyThreads& operator=(const CopyThreads&) = delete;
+    int size() const { return (int)threads_.size(); }
+    void start(std::function<void(int)> fn) {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            fn_ = std::move(fn);
+            running_ = (int)threads_.size();
+            ++job_;
+        }
+        wake_.notify_all();
+    }
+    void wait() {
+        std::unique_lock<std::mutex> lock(mu_);
+        done_.wait(lock, [this] { return running_ == 0; });
+    }
+
+   private:
+    void loop(int i) {
+        long seen = 0;
+        for (;;) {
+            {
+                std::unique_lock<std::mutex> lock(mu_);
+                wake_.wait(lock, [&] { return quit_ || job_ != seen; });
+                if (quit_) return;
+                seen = job_;
+            }
+            fn_(i);
+            std::lock_guard<std::mutex> lock(mu_);
+            if (--running_ == 0) done_.notify_all();
+        }
+    }
+    std::mutex mu_;
+    std::condition_variable wake_, done_;
+    std::function<void(int)> fn_;
+    std::vector<std::thread> threads_;
+    long job_ = 0;
+    int running_ = 0;
+    bool quit_ = false;
+};
+
+// The copies of one transfer: chunk k of `n_chunks` is bytes [k * chunk, ...) of the caller's array
+// and lies in slot k % n_slots.  allow(k) lets the threads work on chunk k, wait(k) returns when it
+// is copied; the calling thread takes a share of every chunk inside wait().
+class SlottedCopy {
+   public:
+    // to_slot: array -> slots, else slots -> array.  threads: null for a copy by the calling thread alone
+    SlottedCopy(char* array, char* slots, size_t total, size_t chunk, int n_slots, bool to_slot, CopyThreads* threads)
+        : array_(array), slots_(slots), total_(total), chunk_(chunk), n_slots_(n_slots), to_slot_(to_slot),
+          threads_(threads), parts_(threads ? threads->size() + 1 : 1),
+          left_(new std::atomic<int>[n_chunks()]) {
+        for (size_t k = 0; k < n_chunks(); ++k) left_[k].store(parts_ - 1, std::memory_order_relaxed);
+        if (threads_) threads_->start([this](int i) {
+            for (size_t k = 0; k < n_chunks(); ++k) {
+                while (allowed_.load(std::memory_order_acquire) <= k) {
+                    if (stop_.load(std::memory_order_relaxed)) return;
+                    std::this_thread::yield();
+                }
+                copy_part(k, i + 1);
+                left_[k].fetch_sub(1, std::memory_order_release);
+            }
+        });
+    }
+    ~SlottedCopy() {
+        stop_.store(true);
+        if (threads_) threads_->wait();
+    }
+    SlottedCopy(const SlottedCopy&) = delete;
+    SlottedCopy& operator=(const SlottedCopy&) = delete;
+    size_t n_chunks() const { return (total_ + chunk_ - 1) / chunk_; }
+    void allow(size_t k) { allowed_.store(k + 1, std::memory_order_release); }
+    void wait(size_t k) {
+        copy_part(k, 0);
+        while (left_[k].load(std::memory_order_acquire)) std::this_thread::yield();
+    }
+
+   private:
+    void copy_part(size_t k, int part) {
+        const size_t n = std::min(chunk_, total_ - k * chunk_);
+        // parts end on whole pages of the array, so that no two threads touch the same new page
+        auto cut = [&](int q) { return q == parts_ ? n : std::min(n, (n * q / parts_) & ~(size_t)4095); };
+        const size_t a = cut(part), b = cut(part + 1);
+        if (a >= b) return;
+        char* arr = array_ + k * chunk_ + a;
+        char* slot = slots_ + (k % n_slots_) * chunk_ + a;
+        if (to_slot_) std::memcpy(slot, arr, b - a);
+        else std::memcpy(arr, slot, b - a);
+    }
+    char *array_, *slots_;
+    size_t total_, chunk_;
+    int n_slots_;
+    bool to_slot_;
+    CopyThreads* threads_;
+    int parts_;
+    std::unique_ptr<std::atomic<int>[]> left_;
+    std::atomic<size_t> allowed_{0};
+    std::atomic<bool> stop_{false};
+};
+
+}  // namespace kge

@@ -327,8 +327,7 @@ class Engine:
         self.uninitialized_variables.discard(name)
 
     def read_variable(self, name: str) -> np.ndarray:
-        dtype = self.variable_to_dtype[name]
-        value = np.full(self.variable_to_shape[name], np.nan if dtype.kind == "f" else 0, dtype=dtype)
+        value = np.empty(self.variable_to_shape[name], dtype=self.variable_to_dtype[name])  # written whole
         self.engine.run("read", dict(name=name, value=value))
         return value
 
@@ -362,15 +361,16 @@ class Engine:
 
     def read_entity(self, offset: int) -> np.ndarray:
         idx = self._rw_indices(offset)
-        out = np.zeros(self.settings.entity_data_r_shape, dtype=self.settings.execution.dtype)
+        out = np.empty(self.settings.entity_data_r_shape, dtype=self.settings.execution.dtype)  # written whole
         self.engine.run("read_entity", dict(read_indices=idx, read_data=self._int16_if_float16(out)))
         return out[:, :self.settings.model.n_entity - offset, :]
 
     def read_entity_all(self) -> np.ndarray:
         """The whole table on the host -- only sensible for small models."""
-        step = self.settings.execution.rw_batch_size
-        return np.concatenate(
-            [self.read_entity(o) for o in range(0, self.settings.model.n_entity, step)], axis=1)
+        m = self.settings.model
+        out = np.empty((m.n_shard, m.n_entity, self.settings.entity_data_r_size), dtype=self.settings.execution.dtype)
+        self.engine.run("read_entity_all", dict(read_data=self._int16_if_float16(out)))
+        return out
 
     # ---- seeded helpers ------------------------------------------------------
     def random_normal(self, shape: Shape, dtype: Union[str, np.dtype] = "float32") -> np.ndarray:

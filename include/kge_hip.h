@@ -89,7 +89,8 @@ int kge_engine_create(const kge_item* settings, size_t n_settings, const char* g
  *   "variables"        served by the two functions below, because its result is
  *                      a list and not an array                      (:993-998)
  * Additive commands, not in the reference: "write_entity_raw" (full rows from
- * the host), "stage_batch" + "train_step_loop" with {"staged": true} (keeps the
+ * the host), "read_entity_all" (read_data [S, n_entity, 3D+F]: every shard's rows in
+ * order), "stage_batch" + "train_step_loop" with {"staged": true} (keeps the
  * index arrays resident in HBM), "gather_benchmark", "timing", "plan_dump" (the
  * distinct rows, segments and sorted items the device derived for one step). */
 int kge_engine_run(kge_engine* engine, const char* command, kge_item* items, size_t n_items,
