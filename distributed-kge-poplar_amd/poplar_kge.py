@@ -509,13 +509,17 @@ class Engine:
         they are merged to the overall n_best here, best first."""
         ex, S = self.settings.execution, self.settings.model.n_shard
         Hb, n_best = ex.predict_hr_batch_size, ex.predict_n_best
-        scores = np.full((S, S, Hb, n_best), np.nan, np.float32)  # [query shard, tail shard, query, rank]
-        rows = np.zeros(scores.shape, np.uint32)
+        scores = np.empty((S, S, Hb, n_best), np.float32)  # [query shard, tail shard, query, rank], written whole
+        rows = np.empty(scores.shape, np.uint32)
         self.engine.run("predict", dict(
             predict_head=np.ascontiguousarray(idx_relation[:, :, 0], np.uint32),
             predict_relation=np.ascontiguousarray(idx_relation[:, :, 1], np.uint32),
             predict_entity_count=np.ascontiguousarray(self.shard_to_entity_count, np.uint32),
             predict_scores=scores, predict_indices=rows))
+        if S == 1:  # one list per query, best first already
+            shard_idx = np.zeros((1, Hb, n_best, 2), np.uint32)
+            shard_idx[..., 1] = rows[0]
+            return Predictions(shard_idx=shard_idx, score=scores[0])
         tail_shard = np.broadcast_to(np.arange(S, dtype=np.uint32)[None, :, None, None], rows.shape)
         shard_idx = np.stack([tail_shard, rows], axis=-1)          # [S, S, Hb, n_best, 2]
         pooled = Predictions(shard_idx=shard_idx.transpose(0, 2, 1, 3, 4).reshape(S, Hb, S * n_best, 2),
