@@ -672,6 +672,9 @@ __global__ __launch_bounds__(NW * 64) void k_score_fwd_mfma(FwdParams p) {
     float* const dist_blk = p.dist ? p.dist + (size_t)d * B * T : nullptr;
     const float nb = DIST == DIST_L2 ? nb_s[n_loc] : 0.f;
     const float mult = (OM == 0 && sh.tmult && n < T) ? sh.tmult[(size_t)d * T + n] : 1.f;
+    // columns behind a block's distinct tails repeat its first row, the most popular one more often
+    // than not: no pair of theirs is worth a second look
+    const bool col_counts = !sh.tcount || n < (int)sh.tcount[d];
 #pragma unroll
     for (int t = 0; t < AT; ++t) {
         // phase 1 (straight-line): squared distances and which of them cancelled
@@ -680,7 +683,7 @@ __global__ __launch_bounds__(NW * 64) void k_score_fwd_mfma(FwdParams p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int m_loc = wm + 32 * t + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            const bool live = ALIGNED || (m0 + m_loc < B && n < T);
+            const bool live = col_counts && (ALIGNED || (m0 + m_loc < B && n < T));
             val[r] = acc[t][r];
             if (DIST == DIST_L2) {
                 const float na = na_s[m_loc];
@@ -689,32 +692,63 @@ __global__ __launch_bounds__(NW * 64) void k_score_fwd_mfma(FwdParams p) {
                 if (live && val[r] < kNearRatio * (na + nb)) near |= 1u << r;
             }
         }
-        // phase 2 (rare): the wave recomputes the cancelled pairs directly
+        // phase 2 (rare): the wave recomputes the cancelled pairs directly, four at a time: two pairs
+        // of each of two lanes, sixteen lanes to a pair.  (Pairs come in runs: a popular row among
+        // the heads against its own column puts them all on two lanes.  One pair at a time, each a
+        // round trip to memory, such a tile ran on alone for tens of us.)
         if (DIST == DIST_L2 && __ballot(cancel != 0u)) {
             near = 0u;
+            uint32_t left = cancel;
+            uint64_t owners;
+            while ((owners = __ballot(left != 0u)) != 0) {
+                const int l0 = __ffsll((long long)owners) - 1;
+                const uint64_t rest = owners & (owners - 1);
+                const int l1 = rest ? __ffsll((long long)rest) - 1 : l0;
+                const int src = lane & 32 ? l1 : l0;
+                const uint32_t bits = __shfl(left, src, 64), upper = bits & (bits - 1);
+                const int fr = __ffs((int)((lane & 16) && upper ? upper : bits)) - 1;
+                const int fm = m0 + wm + 32 * t + 8 * (fr >> 2) + 4 * (src >> 5) + (fr & 3), fn = n0 + wn + (src & 31);
+                const char* ar = row_ptr(p.ent_a, p.a_c0 + d * B + fm);
+                const float* rr = p.a_rel_mode ? p.rel + (size_t)p.crel[d * B + fm] * Dp : nullptr;
+                const char* br = row_ptr(p.ent_b, p.b_c0 + d * T + fn);
+                float part = 0.f;
+                for (int k0 = 0; k0 < Dp; k0 += 256) {
+                    float4 a[4], b[4];
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) {
+                        const int k = k0 + 64 * x + (lane & 15) * 4;
+                        a[x] = b[x] = make_float4(0, 0, 0, 0);
+                        if (k < Dp) {
+                            a[x] = combine_rel(load4(ar, k, p.ent_a), rr, k, p.a_rel_mode);
+                            b[x] = load4(br, k, p.ent_b);
+                        }
+                    }
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) {
+                        const float dx = a[x].x - b[x].x, dy = a[x].y - b[x].y, dz = a[x].z - b[x].z, dw = a[x].w - b[x].w;
+                        part += dx * dx + dy * dy + dz * dz + dw * dw;
+                    }
+                }
+#pragma unroll
+                for (int off = 8; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
+                // the four sums to their lanes: pair 2 h + x belongs to lane l_h, its x-th set bit
+                const int base = (lane == l0) ? 0 : 32;
+                const float v0 = __shfl(part, base, 64), v1 = __shfl(part, base + 16, 64);
+                if (lane == l0 || lane == l1) {
+                    const uint32_t mine = left, up = mine & (mine - 1);
+                    const uint32_t b0 = mine ^ up, b1 = up & (0u - up);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        if ((b0 >> r) & 1u) val[r] = v0;
+                        if ((b1 >> r) & 1u) val[r] = v1;
+                    }
+                    left = up & (up - 1);
+                }
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m_loc = wm + 32 * t + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                const int m = m0 + m_loc;
-                uint64_t todo = __ballot((cancel >> r) & 1u);
-                while (todo) {
-                    const int src = __ffsll((long long)todo) - 1;
-                    todo &= todo - 1;
-                    const int fm = __shfl(m, src, 64), fn = __shfl(n, src, 64);
-                    const char* ar = row_ptr(p.ent_a, p.a_c0 + d * B + fm);
-                    const float* rr = p.a_rel_mode ? p.rel + (size_t)p.crel[d * B + fm] * Dp : nullptr;
-                    const char* br = row_ptr(p.ent_b, p.b_c0 + d * T + fn);
-                    float part = 0.f;
-                    for (int k = lane * 4; k < Dp; k += 256) {
-                        const float4 a = combine_rel(load4(ar, k, p.ent_a), rr, k, p.a_rel_mode);
-                        const float4 b = load4(br, k, p.ent_b);
-                        const float dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z, dw = a.w - b.w;
-                        part += dx * dx + dy * dy + dz * dz + dw * dw;
-                    }
-                    part = wave_sum(part);
-                    if (lane == src) val[r] = part;
-                }
-                const bool live = ALIGNED || (m < B && n < T);
+                const bool live = col_counts && (ALIGNED || (m0 + m_loc < B && n < T));
                 if (live && val[r] < kNearRatio * (na_s[m_loc] + nb)) near |= 1u << r;
             }
         }
