@@ -1294,7 +1294,7 @@ void run_step(kge_engine& E, int i) {
         ra.D = E.D; ra.Dp = E.Dp;
         for (int q = 0; q < 3; ++q) { ra.power[q] = E.reg_p[q]; ra.weight[q] = E.reg_w[q]; }
         ra.loss_scale = E.loss_scale;
-        ra.add_val = E.reg_val.p; ra.add_fh = E.reg_fh.p; ra.loss_row = E.reg_loss_row.p;
+        ra.add_val = E.reg_w[0] > 0 || E.reg_w[2] > 0 ? E.reg_val.p : nullptr; ra.add_fh = E.reg_fh.p; ra.loss_row = E.reg_loss_row.p;
         ra.uses = 2.f; ra.accumulate = 0;
         if (roles) {  // the two entityHidden calls see different rows: one launch for each
             ra.uses = 1.f;
@@ -1384,7 +1384,9 @@ void run_step(kge_engine& E, int i) {
     ae.partial = E.partial.p;
     // (with dropout the feature part's gradient is formed per role by launch_role_sums)
     ae.grad_out = (E.F && !roles) ? E.gsum.p : nullptr;
-    if (E.reg_on) { ae.grad_add = E.reg_val.p; ae.grad_out_add = E.reg_fh.p; }
+    // (no gradient for the embedding from a regulariser of the feature part alone)
+    float* const reg_val = E.reg_on && (E.reg_w[0] > 0 || E.reg_w[2] > 0) ? E.reg_val.p : nullptr;
+    if (E.reg_on) { ae.grad_add = reg_val; ae.grad_out_add = E.reg_fh.p; }
     ae.p_base = E.table.p; ae.m_base = E.table.p + E.L.off_m; ae.v_base = E.table.p + E.L.off_s;
     ae.pitch = E.L.pitch; ae.p_etype = E.L.emb_etype; ae.m_etype = E.L.mom_etype; ae.v_is_sqrt = 1;
     ae.alpha = alpha;
@@ -1409,7 +1411,7 @@ void run_step(kge_engine& E, int i) {
         }
         for (int net = 0; net < nets; ++net)  // what reaches the embedding adds up over the networks
             launch_mlp_bwd_rows(ma[net], E.gsum.p + net * rows_n,
-                                net ? E.mlp_gval.p : (E.reg_on ? E.reg_val.p : nullptr),
+                                net ? E.mlp_gval.p : reg_val,
                                 E.mlp_gpre.p + (size_t)net * R * E.mlp, E.mlp_gval.p, E.mlp_gfp.p + net * rows_n, st);
         AdamArgs upd = ae;
         upd.grad_out = nullptr; upd.grad_out_add = nullptr; upd.grad_add = E.mlp_gval.p;
@@ -1454,20 +1456,15 @@ void run_step(kge_engine& E, int i) {
         launch_adam_rows2(ar, ae, st);
     }
 
-    // dense Adam on rows [0, rows) of a parameter of row pitch `width`; shard s owns rows
-    // [s*rows/S, (s+1)*rows/S) and its step size (group `group` of this step's step sizes)
+    // dense Adam on rows [0, last_row) of a parameter of row pitch `width`; shard s owns rows
+    // [s*rows/S, (s+1)*rows/S) (the last one also the padding rows behind them) and its step size
+    // (group `group` of this step's step sizes)
     auto dense_adam = [&](float* p, float* m, float* v, const float* g, int rows, int last_row, int64_t width,
                           int group) {
+        AdamArgs af = aa;
+        af.alpha = alpha + (size_t)group * E.S;
         const int n_slices = E.shared_table ? 1 : E.S;
-        for (int s = 0; s < n_slices; ++s) {
-            const int r0 = E.shared_table ? 0 : s * (rows / E.S);
-            const int r1 = (E.shared_table || s == E.S - 1) ? last_row : (s + 1) * (rows / E.S);
-            if (r1 <= r0) continue;
-            const size_t o = (size_t)r0 * width;
-            launch_adam_flat(p + o, m + o, v + o, g + o, (int64_t)(r1 - r0) * width,
-                             E.h_alpha[((size_t)i * 9 + group) * E.S + s], E.beta_m, E.beta_v, E.epsilon,
-                             E.weight_decay, 0, st);
-        }
+        launch_adam_slices(p, m, v, g, last_row * width, std::max(1, rows / n_slices) * width, n_slices, af, st);
     };
     for (int net = 0; net < nets && E.F; ++net) {
         const float* g_rows = E.gsum.p + net * rows_n;  // d loss / d (feature part) per distinct row

@@ -362,7 +362,7 @@ struct RegArgs {
     int D, Dp;
     float power[3], weight[3];  // embedding, feature product, hidden
     float loss_scale;
-    float* add_val;             // [rows, Dp] gradient for the embedding
+    float* add_val;             // [rows, Dp] gradient for the embedding (or null)
     float* add_fh;              // [rows, Dp] gradient for the feature product (or null)
     float* loss_row;            // [rows] the row's share of the loss
     float uses;                 // entityHidden calls this launch stands for: 2 (heads' and tails' calls
@@ -440,6 +440,9 @@ void launch_distance_grad(int dist_fn, const float* a, const float* b, const flo
 void launch_adam_flat(float* p, float* m, float* v, const float* g, int64_t n, float alpha,
                       float beta_m, float beta_v, float epsilon, float weight_decay, int v_is_sqrt,
                       hipStream_t stream);
+// Adam on n elements of which slices of `slice` have step sizes of their own (a.alpha); n, slice % 4 == 0
+void launch_adam_slices(float* p, float* m, float* v, const float* g, int64_t n, int64_t slice, int n_slices,
+                        const AdamArgs& a, hipStream_t stream);
 void launch_fill_u32(uint32_t* p, uint32_t value, int64_t n, hipStream_t stream);
 void launch_iota_keys(const uint32_t* idx, uint32_t* keys, uint32_t* vals, int64_t n, int64_t rows,
                       hipStream_t stream);

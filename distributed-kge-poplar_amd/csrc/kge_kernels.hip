@@ -2125,68 +2125,122 @@ void launch_loss_finalize(const float* loss_part, int n_step, int S, int n_part,
 // norm regularisers: one wave per distinct row, two passes over the row (sums, then gradients)
 
 // |x^p| and its share of the gradient |x^p| / x (0 at x = 0: the reference's pow backward
-// divides by x + (x == 0), src/pag/pag.cpp:483-503)
-DEVINL float abs_pow(float x, float p) { return fabsf(powf(x, p)); }
+// divides by x + (x == 0), src/pag/pag.cpp:483-503).  KIND: 3 and 2 for those powers (products,
+// where powf is some forty instructions), 0 for any other.
+template <int KIND>
+DEVINL float abs_pow(float x, float p) {
+    return KIND == 3 ? fabsf(x * x * x) : KIND == 2 ? x * x : fabsf(powf(x, p));
+}
+template <int KIND>
+DEVINL float abs_pow_over(float x, float p) {
+    return KIND == 3 ? x * fabsf(x) : KIND == 2 ? x : x != 0.f ? fabsf(powf(x, p)) / x : 0.f;
+}
+DEVINL float sum_pow4(float4 x, float p) {
+    const float v[4] = {x.x, x.y, x.z, x.w};
+    float s = 0.f;
+    if (p == 3.f) { for (int i = 0; i < 4; ++i) s += abs_pow<3>(v[i], p); }
+    else if (p == 2.f) { for (int i = 0; i < 4; ++i) s += abs_pow<2>(v[i], p); }
+    else { for (int i = 0; i < 4; ++i) s += abs_pow<0>(v[i], p); }
+    return s;
+}
+DEVINL float4 pow_over4(float4 x, float p, float c) {
+    if (p == 3.f)
+        return make_float4(c * abs_pow_over<3>(x.x, p), c * abs_pow_over<3>(x.y, p), c * abs_pow_over<3>(x.z, p), c * abs_pow_over<3>(x.w, p));
+    if (p == 2.f) return make_float4(c * x.x, c * x.y, c * x.z, c * x.w);
+    return make_float4(c * abs_pow_over<0>(x.x, p), c * abs_pow_over<0>(x.y, p), c * abs_pow_over<0>(x.z, p), c * abs_pow_over<0>(x.w, p));
+}
+DEVINL float4 f4sub(float4 a, float4 b) { return make_float4(a.x - b.x, a.y - b.y, a.z - b.z, a.w - b.w); }
 
+// Rows of at most 256 columns are held in registers between the passes.  (Padding columns hold
+// zeros in both rows: they add nothing and get zero gradient.)
 __global__ __launch_bounds__(256) void k_reg_rows(RegArgs a) {
     const int lane = threadIdx.x & 63;
     const int u = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int uc = min(u, a.max_rows - 1);  // plan entries past the count are stale but inside the arrays
+    const uint32_t key = a.uniq_key[uc], s0 = a.seg_start[uc], s1 = a.seg_start[uc + 1], real = a.seg_real[uc];
     if (u >= (int)a.counts[0]) return;
-    const uint32_t key = a.uniq_key[u];
-    const float mult = (float)((a.seg_start[u + 1] - a.seg_start[u]) - a.seg_real[u]);
+    const float mult = (float)((s1 - s0) - real);
     const char* erow = a.emb_base + (int64_t)key * a.pitch;
     const float* hrow = a.hidden ? a.hidden + (size_t)u * a.Dp : nullptr;
     float sum[3] = {0.f, 0.f, 0.f};
-    for (int k = lane; k < a.D; k += 64) {
-        const float v = load1(erow, k, a.emb_etype), h = hrow ? hrow[k] : v;
-        if (a.weight[0] > 0.f) sum[0] += abs_pow(v, a.power[0]);
-        if (a.weight[1] > 0.f) sum[1] += abs_pow(h - v, a.power[1]);
-        if (a.weight[2] > 0.f) sum[2] += abs_pow(h, a.power[2]);
+    float4 v0 = make_float4(0, 0, 0, 0), h0 = v0;
+    for (int k = lane * 4; k < a.Dp; k += 256) {
+        const float4 v = load4(erow, k, a.emb_etype), h = hrow ? *reinterpret_cast<const float4*>(hrow + k) : v;
+        if (k < 256) { v0 = v; h0 = h; }
+        if (a.weight[0] > 0.f) sum[0] += sum_pow4(v, a.power[0]);
+        if (a.weight[1] > 0.f) sum[1] += sum_pow4(f4sub(h, v), a.power[1]);
+        if (a.weight[2] > 0.f) sum[2] += sum_pow4(h, a.power[2]);
     }
     float norm[3], coef[3], loss = 0.f;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-        sum[q] = wave_sum(sum[q]);
+        sum[q] = a.weight[q] > 0.f ? wave_sum(sum[q]) : 0.f;
         norm[q] = a.weight[q] > 0.f ? powf(sum[q], 1.f / a.power[q]) : 0.f;
         // d loss / d x_k = seed * (norm / sum) * |x_k^p| / x_k, seed = uses * mult * weight * loss_scale
         coef[q] = sum[q] != 0.f ? a.uses * mult * a.weight[q] * a.loss_scale * norm[q] / sum[q] : 0.f;
         loss += a.uses * mult * a.weight[q] * norm[q];
     }
     if (lane == 0) a.loss_row[u] = a.accumulate ? a.loss_row[u] + loss : loss;
-    for (int k = lane; k < a.Dp; k += 64) {
-        float gv = 0.f, gf = 0.f;
-        if (k < a.D) {
-            const float v = load1(erow, k, a.emb_etype), h = hrow ? hrow[k] : v, f = h - v;
-            if (a.weight[0] > 0.f && v != 0.f) gv += coef[0] * abs_pow(v, a.power[0]) / v;
-            if (a.weight[1] > 0.f && f != 0.f) gf += coef[1] * abs_pow(f, a.power[1]) / f;
-            if (a.weight[2] > 0.f && h != 0.f) {
-                const float gh = coef[2] * abs_pow(h, a.power[2]) / h;
-                gv += gh; gf += gh;
-            }
+    for (int k = lane * 4; k < a.Dp; k += 256) {
+        float4 v = v0, h = h0;
+        if (k >= 256) {
+            v = load4(erow, k, a.emb_etype);
+            h = hrow ? *reinterpret_cast<const float4*>(hrow + k) : v;
         }
-        a.add_val[(size_t)u * a.Dp + k] = a.accumulate ? a.add_val[(size_t)u * a.Dp + k] + gv : gv;
-        if (a.add_fh) a.add_fh[(size_t)u * a.Dp + k] = gf;
+        float4 gv = make_float4(0, 0, 0, 0), gf = gv;
+        if (a.weight[0] > 0.f) gv = pow_over4(v, a.power[0], coef[0]);
+        if (a.weight[1] > 0.f) gf = pow_over4(f4sub(h, v), a.power[1], coef[1]);
+        if (a.weight[2] > 0.f) {
+            const float4 gh = pow_over4(h, a.power[2], coef[2]);
+            gv = f4add(gv, gh); gf = f4add(gf, gh);
+        }
+        const size_t o = (size_t)u * a.Dp + k;
+        if (a.add_val)
+            *reinterpret_cast<float4*>(a.add_val + o) = a.accumulate ? f4add(*reinterpret_cast<const float4*>(a.add_val + o), gv) : gv;
+        if (a.add_fh) *reinterpret_cast<float4*>(a.add_fh + o) = gf;
     }
 }
 void launch_reg_rows(const RegArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL(k_reg_rows, dim3((a.max_rows + 3) / 4), dim3(256), 0, stream, a);
 }
 
-__global__ __launch_bounds__(64) void k_reg_loss(const uint32_t* __restrict__ uniq_key,
-                                                 const uint32_t* __restrict__ counts,
-                                                 const float* __restrict__ loss_row, uint32_t rows_per_shard,
-                                                 float* __restrict__ out) {
-    const int s = blockIdx.x, lane = threadIdx.x;
+// One workgroup per shard.  The distinct rows ascend, so a shard's are one run of them: the first
+// wave finds its ends 64 probes at a time, and thread t adds the run's entries t, t + 1024, ...
+// (16 shards of 1500 rows: 105 us when every workgroup walked all rows with one wave, now 9.)
+__global__ __launch_bounds__(1024) void k_reg_loss(const uint32_t* __restrict__ uniq_key,
+                                                   const uint32_t* __restrict__ counts,
+                                                   const float* __restrict__ loss_row, uint32_t rows_per_shard,
+                                                   float* __restrict__ out) {
+    __shared__ int ends[2];
+    __shared__ float red[16];
+    const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int U = (int)counts[0];
+    if (wave < 2) {  // the first row whose key is at least (s + wave) * rows_per_shard
+        const uint64_t bound = (uint64_t)(s + wave) * rows_per_shard;
+        int lo = 0, hi = U;  // the answer lies in [lo, hi]
+        while (lo < hi) {
+            const int step = (hi - lo + 63) / 64, at = lo + lane * step;
+            const int below = __popcll(__ballot(at < hi && (uint64_t)uniq_key[min(at, hi - 1)] < bound));
+            if (below == 0) { hi = lo; break; }
+            hi = min(hi, lo + below * step);  // (the probe behind the last one below, or the end)
+            lo = lo + (below - 1) * step + 1;
+        }
+        if (lane == 0) ends[wave] = lo;
+    }
+    __syncthreads();
     float part = 0.f;
-    for (int u = lane; u < U; u += 64)
-        if (uniq_key[u] / rows_per_shard == (uint32_t)s) part += loss_row[u];
+    for (int u = ends[0] + tid; u < ends[1]; u += 1024) part += loss_row[u];
     part = wave_sum(part);
-    if (lane == 0) out[s] = part;
+    if (lane == 0) red[wave] = part;
+    __syncthreads();
+    if (wave == 0) {
+        part = wave_sum(lane < 16 ? red[lane] : 0.f);
+        if (lane == 0) out[s] = part;
+    }
 }
 void launch_reg_loss(const uint32_t* uniq_key, const uint32_t* counts, const float* loss_row,
                      uint32_t rows_per_shard, int S, float* out, hipStream_t stream) {
-    hipLaunchKernelGGL(k_reg_loss, dim3(S), dim3(64), 0, stream, uniq_key, counts, loss_row, rows_per_shard, out);
+    hipLaunchKernelGGL(k_reg_loss, dim3(S), dim3(1024), 0, stream, uniq_key, counts, loss_row, rows_per_shard, out);
 }
 
 // --------------------------------------------------------------------------
@@ -2605,6 +2659,29 @@ void launch_adam_flat(float* p, float* m, float* v, const float* g, int64_t n, f
     a.epsilon = epsilon; a.weight_decay = weight_decay; a.v_is_sqrt = v_is_sqrt;
     hipLaunchKernelGGL(k_adam_flat, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, p, m, v,
                        g, n, a, alpha);
+}
+
+// The same on a parameter whose slices of `slice` elements have step sizes of their own (alpha[0],
+// alpha[1], ..; the last one's also for what lies behind it): one launch for all of a parameter's
+// shards (16 launches took 39 us for a 768 x 256 parameter, this one 5).  n, slice % 4 == 0.
+__global__ __launch_bounds__(256) void k_adam_slices(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
+                                                     const float* __restrict__ g, uint32_t n, uint32_t slice,
+                                                     uint32_t n_slices, AdamArgs a) {
+    const uint32_t i = (blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= n) return;
+    const float alpha = a.alpha[min(i / slice, n_slices - 1)];
+    float4 p4 = *reinterpret_cast<const float4*>(p + i), m4 = *reinterpret_cast<const float4*>(m + i);
+    float4 v4 = *reinterpret_cast<const float4*>(v + i);
+    adam4(p4, m4, v4, *reinterpret_cast<const float4*>(g + i), a, alpha);
+    *reinterpret_cast<float4*>(p + i) = p4;
+    *reinterpret_cast<float4*>(m + i) = m4;
+    *reinterpret_cast<float4*>(v + i) = v4;
+}
+void launch_adam_slices(float* p, float* m, float* v, const float* g, int64_t n, int64_t slice, int n_slices,
+                        const AdamArgs& a, hipStream_t stream) {
+    if (n == 0) return;
+    hipLaunchKernelGGL(k_adam_slices, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, stream, p, m, v, g,
+                       (uint32_t)n, (uint32_t)slice, (uint32_t)n_slices, a);
 }
 
 __global__ __launch_bounds__(256) void k_fill_u32(uint32_t* p, uint32_t value, int64_t n) {
