@@ -271,6 +271,7 @@ struct kge_engine {
     DevBuf<float> up, up_m, up_v, down, down_m, down_v, g_up, g_down;
     DevBuf<float> mlp_fproj, mlp_concat, mlp_pre, mlp_gpre, mlp_gfp, mlp_gval, p_fproj, p_concat, p_pre;
     DevBuf<float> opnd_n, cmat, dcm, transh_mm, relgrad;  // TransH: [n | tails], c, d loss / d c, its products, relation contributions
+    DevBuf<float> bwd_pieces;  // split sums of the scoring backward
     DevBuf<float> coef, dist, grad, opnd, partial, rel_partial, rel_gsum, hidden, gsum, gproj, featd, gproj_part, gemm_part, projR, loss_part, loss_step, d_alpha;
     // [n_step][entity, relation, normal, then per feature network projection, mlp up, mlp down][S]; the relation update indexes its two
     // groups as one array (key / rows_per_alpha), a shared table's [relation, normal] pair
@@ -732,7 +733,9 @@ void allocate(kge_engine& E) {
     }
     ScoreShape sh = {};
     sh.S = E.S; sh.B = E.B; sh.T = E.T;
+    sh.Dp = E.Dp;
     sh.score_fn = E.score_fn; sh.dist_fn = E.dist_fn; sh.use_mfma = E.use_mfma;
+    if (E.score_fn != SCORE_TRANSH) E.bwd_pieces.alloc(score_bwd_pieces(sh));
     E.n_part = fused ? score_fwd_parts(sh) : E.B;
     if (E.use_mfma && E.dist_fn == DIST_L2) {
         E.nearflag.alloc(nearflag_words(sh));
@@ -1271,7 +1274,7 @@ void run_step(kge_engine& E, int i) {
             launch_mul_rows(E.dcm.p, E.coef.p, (int64_t)SB * E.T, st);
         }
         { KernelTimer t(E, K_BWD);
-          launch_score_bwd(dot, dense_n, E.rel.p, crel, E.dcm.p, nullptr, E.transh_mm.p, st);
+          launch_score_bwd(dot, dense_n, E.rel.p, crel, E.dcm.p, nullptr, E.transh_mm.p, nullptr, st);
           TranshBwd tb;
           tb.pt = E.opnd.p; tb.nt = E.opnd_n.p; tb.coef = E.coef.p; tb.cmat = E.cmat.p;
           tb.mm = E.transh_mm.p; tb.grad = E.grad.p; tb.S = E.S; tb.B = E.B; tb.T = E.T; tb.Dp = E.Dp;
@@ -1281,7 +1284,7 @@ void run_step(kge_engine& E, int i) {
         { KernelTimer t(E, K_FWD);
           launch_score_fwd(sh, dense, E.rel.p, crel, clabel, E.coef.p, E.dist.p, E.nearflag.p, loss_part, fused, st); }
         if (!fused) { KernelTimer t(E, K_LOSS); launch_loss_rows(sh, clabel, E.coef.p, E.dist.p, loss_part, nullptr, st); }
-        { KernelTimer t(E, K_BWD); launch_score_bwd(sh, dense, E.rel.p, crel, E.coef.p, E.nearflag.p, E.grad.p, st); }
+        { KernelTimer t(E, K_BWD); launch_score_bwd(sh, dense, E.rel.p, crel, E.coef.p, E.nearflag.p, E.grad.p, E.bwd_pieces.p, st); }
     }
 
     if (E.reg_on) {

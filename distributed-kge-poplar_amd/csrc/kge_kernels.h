@@ -262,7 +262,9 @@ void launch_log_softmax(const float* x, const float* dy, float* out, int64_t row
 // contributions, from the coefficient matrix.
 void launch_score_bwd(const ScoreShape& sh, const RowSource& ent, const float* rel,
                       const uint32_t* crel, const float* coef, const uint32_t* nearflag, float* grad,
-                      hipStream_t stream);
+                      float* pieces, hipStream_t stream);
+// floats of scratch (`pieces`) the launch above wants for sums that it splits (without it: null)
+size_t score_bwd_pieces(const ScoreShape& sh);
 
 // Where gradient contributions come from.  transform: 0 none; 1 multiply head
 // rows (c < n_head) by rel[crel[c]] (DistMult, entity plan); 2 multiply by the

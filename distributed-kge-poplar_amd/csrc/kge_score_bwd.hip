@@ -792,12 +792,12 @@ void launch_bwd(const BwdParams& p, int dist_fn, hipStream_t stream) {
 
 
 // --------------------------------------------------------------------------
-// L1 backward, both sides in one pass over the pairs.  c * signum(a - b) has no
+// L1 backward, both sides in one pass over the pairs, at any shape.  c * signum(a - b) has no
 // contraction form, so this is vector-ALU work; computing the term once and
 // adding it to the head's sum and (negated) to the tail's sum halves it.
-// One workgroup of 16 waves per (block, 64-column slice); a lane owns one
-// column.  Wave w keeps tails [w*tw, (w+1)*tw) and their gradient sums in
-// registers and walks over all heads; a head's sum over one wave's tails is a
+// One workgroup of 16 waves per (block, 64-column slice, group of heads, group of at most 512
+// tails: l1_pair_split); a lane owns one column.  Wave w keeps tails [w*tw, (w+1)*tw) of the
+// group and their gradient sums in registers and walks over the group's heads; a head's sum over one wave's tails is a
 // partial, the 16 partials of a head meet in LDS and are added in wave order
 // (deterministic).  The coefficients of a (head, tail range) are the same for
 // every lane: the workgroup stages the coefficient rows of eight heads at a time
@@ -810,7 +810,18 @@ void launch_bwd(const BwdParams& p, int dist_fn, hipStream_t stream) {
 constexpr int L1P_CB = 8;      // heads per chunk
 constexpr int L1P_WAVES = 16;
 
-constexpr int L1P_MAX_T = 512;  // tails per block at most (32 per wave)
+constexpr int L1P_MAX_T = 512;  // tails per workgroup at most (32 per wave)
+
+// One workgroup's share of a block: its heads, its tails, its 64 columns.
+struct L1Pair {
+    const float* a_rows;  // the first head's value in this lane's column
+    const float* b_rows;  // the first tail's
+    const float* coef;    // coefficient of the first head and the first tail; rows `ldc` apart
+    float* grad_a;        // where the first head's gradient in this lane's column goes
+    float* grad_b;
+    int n_head, n_tail, ldc, Dp;
+    bool col;             // this lane has a column
+};
 
 // the work of one wave with exactly TW tails (TW even): straight-line code over
 // its tails, their values and sums in registers.
@@ -827,22 +838,35 @@ constexpr int L1P_MAX_T = 512;  // tails per block at most (32 per wave)
 //           columns, before the 16 waves' values are added.
 // The column and row-part sums of a chunk come from the coefficient rows staged in LDS, by waves
 // 8 .. 15 while waves 0 .. 7 add the head partials of the chunk before.
-template <int TW>
-DEVINL void l1_pair_wave(const float* __restrict__ a_rows, const float* __restrict__ b_rows,
-                         const float* __restrict__ cblk, float* __restrict__ grad_a, float* __restrict__ grad_b,
-                         int B, int T, int Dp, int t_live, int w, int lane,
+// FULL: whole chunks of heads, 16-byte coefficient loads, readable zero coefficients up to the next
+// multiple of 32 tails and a column in every lane: no bounds checks.
+template <int TW, bool FULL>
+DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane,
                          float (*part)[L1P_WAVES][L1P_CB][64], float (*cs)[L1P_CB][L1P_MAX_T],
                          float (*col_half)[L1P_MAX_T], float (*row_part)[L1P_CB][L1P_WAVES]) {
     // In LDS a wave's TW columns start at a multiple of four (TWS apart): its reads stay 16-byte
     // ones when TW is not a multiple of four.  Column c lies at lds_col(c).
     constexpr int TWS = (TW + 3) & ~3;
+    constexpr int TL = TW * L1P_WAVES, T4 = TL / 4;  // tails of the workgroup, filled up
     auto lds_col = [](int c) { return (c / TW) * TWS + c % TW; };
-    const int tid = threadIdx.x, t4 = t_live / 4, l0 = w * TWS;
+    const int tid = threadIdx.x, l0 = w * TWS, Dp = q.Dp, n_head = q.n_head;
     // staging: thread -> (head, four columns) of a chunk's coefficient rows, stored as two pairs
     // (TW is even, so a pair never straddles two waves' columns)
-    const bool stager = tid < L1P_CB * t4;
-    const int s_head = tid / t4, s_col = (tid - s_head * t4) * 4;
+    const bool stager = tid < L1P_CB * T4;
+    const int s_head = tid / T4, s_col = (tid - s_head * T4) * 4;
     const int s_lo = lds_col(s_col), s_hi = lds_col(s_col + 2);
+    auto fetch = [&](int b0) __attribute__((always_inline)) {
+        const float* src = q.coef + (size_t)(b0 + s_head) * q.ldc + s_col;
+        if constexpr (FULL) return *reinterpret_cast<const float4*>(src);
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (b0 + s_head < n_head) {
+            if (s_col + 0 < q.n_tail) v.x = src[0];
+            if (s_col + 1 < q.n_tail) v.y = src[1];
+            if (s_col + 2 < q.n_tail) v.z = src[2];
+            if (s_col + 3 < q.n_tail) v.w = src[3];
+        }
+        return v;
+    };
     auto stage = [&](int buf, float4 v) __attribute__((always_inline)) {
         *reinterpret_cast<float2*>(&cs[buf][s_head][s_lo]) = make_float2(v.x, v.y);
         *reinterpret_cast<float2*>(&cs[buf][s_head][s_hi]) = make_float2(v.z, v.w);
@@ -851,23 +875,25 @@ DEVINL void l1_pair_wave(const float* __restrict__ a_rows, const float* __restri
     const int u = tid - 512, u_lds = u >= 0 ? lds_col(u) : 0;
     float4 c_next = make_float4(0.f, 0.f, 0.f, 0.f);
     if (stager) {
-        c_next = *reinterpret_cast<const float4*>(cblk + (size_t)s_head * T + s_col);
+        c_next = fetch(0);
         stage(0, c_next);
     }
     float bt[TW], gt[TW];
 #pragma unroll
     for (int j = 0; j < TW; ++j) {
-        bt[j] = b_rows[(size_t)j * Dp];
+        const int t = w * TW + j;
+        bt[j] = q.b_rows[(size_t)(FULL ? t : min(t, q.n_tail - 1)) * Dp];
         gt[j] = 0.f;
     }
     // the heads' values, asked for two heads ahead of their use (one ahead leaves the load's
     // latency showing at the end of every head: 170 -> 161 us on the 22.8M-row L1 workload;
     // three ahead measures the same as two)
-    float a_q0 = a_rows[0], a_q1 = a_rows[(size_t)min(1, B - 1) * Dp];
+    float a_q0 = q.a_rows[0], a_q1 = q.a_rows[(size_t)min(1, n_head - 1) * Dp];
     __syncthreads();
-    for (int b0 = 0, buf = 0; b0 < B; b0 += L1P_CB, buf ^= 1) {
-        const bool more = b0 + L1P_CB < B;
-        if (stager && more) c_next = *reinterpret_cast<const float4*>(cblk + (size_t)(b0 + L1P_CB + s_head) * T + s_col);
+    int buf = 0;
+    for (int b0 = 0; b0 < n_head; b0 += L1P_CB, buf ^= 1) {
+        const bool more = b0 + L1P_CB < n_head;
+        if (stager && more) c_next = fetch(b0 + L1P_CB);
         if (b0 > 0) {
 #pragma unroll
             for (int j4 = 0; j4 < TW; j4 += 4) {
@@ -879,7 +905,7 @@ DEVINL void l1_pair_wave(const float* __restrict__ a_rows, const float* __restri
             }
         }
         if (u >= 0) {
-            if (u < t_live) {
+            if (u < TL) {
                 float sum = 0.f;
 #pragma unroll
                 for (int h = 0; h < L1P_CB; ++h) sum += cs[buf][h][u_lds];
@@ -897,7 +923,7 @@ DEVINL void l1_pair_wave(const float* __restrict__ a_rows, const float* __restri
         for (int bi = 0; bi < L1P_CB; ++bi) {
             const float a = a_q0;
             a_q0 = a_q1;
-            a_q1 = a_rows[(size_t)min(b0 + bi + 2, B - 1) * Dp];
+            a_q1 = q.a_rows[(size_t)min(b0 + bi + 2, n_head - 1) * Dp];
             const float* c = &cs[buf][bi][l0];
             float gp = 0.f;
 #pragma unroll
@@ -917,23 +943,50 @@ DEVINL void l1_pair_wave(const float* __restrict__ a_rows, const float* __restri
         if (stager && more) stage(buf ^ 1, c_next);
         __syncthreads();
         // waves 0 .. 7 add the 16 partials of head b0 + w
-        if (w < L1P_CB) {
+        if (w < L1P_CB && (FULL || (b0 + w < n_head && q.col))) {
             float sum = 0.f;
 #pragma unroll
             for (int v = 0; v < L1P_WAVES; ++v) sum += fmaf(2.f, part[buf][v][w][lane], -row_part[buf][w][v]);
-            grad_a[(size_t)(b0 + w) * Dp] = sum;
+            q.grad_a[(size_t)(b0 + w) * Dp] = sum;
         }
     }
-    const int last = ((B / L1P_CB) - 1) & 1;
+    const int last = buf ^ 1;
 #pragma unroll
-    for (int j = 0; j < TW; ++j) grad_b[(size_t)j * Dp] = -2.f * (gt[j] - col_half[last][l0 + j]);
+    for (int j = 0; j < TW; ++j) {
+        const int t = w * TW + j;
+        if (FULL || (t < q.n_tail && q.col)) q.grad_b[(size_t)t * Dp] = -2.f * (gt[j] - col_half[last][l0 + j]);
+    }
 }
 
+// How a block's pairs are divided: `heads` x `tails` groups, every group a workgroup per 64 columns.
+// A group holds at most 512 tails.  A split leaves the other side's sums in pieces, which
+// k_l1_pair_sum adds up: heads' gradients in `tails` pieces [tails][S * B][Dp], then the tails' in
+// `heads` pieces [heads][S * T][Dp].
+struct L1Split { int heads, tails; };
+static L1Split l1_pair_split(const ScoreShape& sh) {
+    // A workgroup of sixteen waves fills a CU.  Tails first (a group of 64 still gives every wave
+    // four), then heads, as long as the chip has CUs without work; more groups than CUs only add
+    // pieces.  16 blocks of 512 x 1536 with D = 256: 4 groups of 384 tails, 256 workgroups.
+    const int base = sh.S * ((sh.Dp + 63) / 64);
+    L1Split k = {1, (sh.T + L1P_MAX_T - 1) / L1P_MAX_T};
+    if (k.tails == 3 && base * 4 <= 256) k.tails = 4;
+    while (base * k.tails * 2 <= 256 && sh.T >= 128 * k.tails) k.tails *= 2;
+    while (base * k.tails * k.heads * 2 <= 256 && sh.B >= 64 * k.heads) k.heads *= 2;
+    return k;
+}
+size_t score_bwd_pieces(const ScoreShape& sh) {
+    if (sh.dist_fn != DIST_L1 || sh.score_fn == SCORE_DISTMULT || !sh.use_mfma) return 0;
+    const L1Split k = l1_pair_split(sh);
+    return ((k.tails > 1 ? (size_t)k.tails * sh.S * sh.B : 0) + (k.heads > 1 ? (size_t)k.heads * sh.S * sh.T : 0)) * sh.Dp;
+}
+
+template <bool FULL>
 __global__ __launch_bounds__(1024) void k_score_bwd_l1_pair(const float* __restrict__ operands,
                                                             const float* __restrict__ coef,
-                                                            float* __restrict__ grad, int B, int T,
-                                                            int Dp, int a_c0, int b_c0,
-                                                            const uint32_t* __restrict__ tcount, int tpad) {
+                                                            float* __restrict__ grad_heads, float* __restrict__ grad_tails,
+                                                            int S, int B, int T, int Dp, int a_c0, int b_c0,
+                                                            int h_groups, int t_groups, int h_size,
+                                                            const uint32_t* __restrict__ tcount) {
     // the coefficient rows first: their reads in the inner loop then carry the whole address
     // offset in the instruction
     __shared__ __attribute__((aligned(16))) struct {
@@ -942,42 +995,93 @@ __global__ __launch_bounds__(1024) void k_score_bwd_l1_pair(const float* __restr
         float row_part[2][L1P_CB][L1P_WAVES];
         float part[2][L1P_WAVES][L1P_CB][64];
     } lds;
-    const TileId tile = xcd_tile(Dp / 64, 1, (int)gridDim.x / (Dp / 64));
+    const TileId tile = xcd_tile((Dp + 63) / 64, h_groups * t_groups, S);
     const int d = tile.z, lane = threadIdx.x & 63, k = tile.x * 64 + lane;
+    const int hg = tile.y / t_groups, tg = tile.y - hg * t_groups;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // merged tails: the block's distinct tails in whole groups of 32 (two per wave), split evenly
-    // over the waves.  The columns between that and the forward pass's limit (whole groups of
-    // `tpad`) stand for no tail position: their coefficients are zero and nothing reads their
-    // gradient rows.  331 instead of 343 columns per block on average on the 22.8M-row workload,
-    // and the launch's time follows that average (158.6 -> 155 us), not its largest block.
-    const int t_fwd = tail_limit(tcount, d, T, tpad);
-    const int t_live = __builtin_amdgcn_readfirstlane(tcount ? min(t_fwd, ((int)tcount[d] + 31) & ~31) : t_fwd);
-    const int tw = t_live / L1P_WAVES, t0 = w * tw;
-    const float* a_rows = operands + (size_t)(a_c0 + d * B) * Dp + k;
-    const float* b_rows = operands + (size_t)(b_c0 + d * T + t0) * Dp + k;
-    const float* cblk = coef + (size_t)d * B * T;
-    float* grad_a = grad + (size_t)(a_c0 + d * B) * Dp + k;
-    float* grad_b = grad + (size_t)(b_c0 + d * T + t0) * Dp + k;
+    // merged tails: the block's distinct tails alone.  The columns between them and the forward
+    // pass's limit stand for no tail position: their coefficients are zero and nothing reads
+    // their gradient rows.  The groups share the live tails evenly, in steps of 32 (an even number
+    // per wave: 331 instead of 343 columns per block on average on the 22.8M-row workload, and
+    // the launch's time follows that average (158.6 -> 155 us), not its largest block).
+    const int live = tcount ? min(T, (int)tcount[d]) : T;
+    const int t_size = ((live + t_groups - 1) / t_groups + 31) & ~31;
+    const int t0 = tg * t_size, h0 = hg * h_size;
+    L1Pair q;
+    q.n_tail = __builtin_amdgcn_readfirstlane(min(t_size, live - t0));
+    q.n_head = __builtin_amdgcn_readfirstlane(min(h_size, B - h0));
+    q.col = FULL || k < Dp;
+    const int kc = FULL ? k : min(k, Dp - 1);
+    q.Dp = Dp; q.ldc = T;
+    q.grad_a = grad_heads + ((size_t)(t_groups > 1 ? tg : 0) * S * B + (size_t)d * B + h0) * Dp + kc;
+    q.grad_b = grad_tails + ((size_t)(h_groups > 1 ? hg : 0) * S * T + (size_t)d * T + t0) * Dp + kc;
+    if (q.n_head <= 0 || q.n_tail <= 0) {  // rounding left this group empty: its pieces of the sums are zero
+        if (q.col) {
+            for (int b = w; b < q.n_head; b += L1P_WAVES) q.grad_a[(size_t)b * Dp] = 0.f;
+            for (int t = w; t < q.n_tail; t += L1P_WAVES) q.grad_b[(size_t)t * Dp] = 0.f;
+        }
+        return;
+    }
+    q.a_rows = operands + (size_t)(a_c0 + d * B + h0) * Dp + kc;
+    q.b_rows = operands + (size_t)(b_c0 + d * T + t0) * Dp + kc;
+    q.coef = coef + ((size_t)d * B + h0) * T + t0;
+    const int tw = ((q.n_tail + 31) & ~31) / L1P_WAVES;
 #define KGE_L1P(TW_) \
-    case TW_: l1_pair_wave<TW_>(a_rows, b_rows, cblk, grad_a, grad_b, B, T, Dp, t_live, w, lane, lds.part, lds.cs, lds.col_half, lds.row_part); break;
-    switch (tw) {  // one of sixteen copies of the loop, chosen per block
+    case TW_: l1_pair_wave<TW_, FULL>(q, w, lane, lds.part, lds.cs, lds.col_half, lds.row_part); break;
+    switch (tw) {  // one of sixteen copies of the loop, chosen per group
         KGE_L1P(2) KGE_L1P(4) KGE_L1P(6) KGE_L1P(8) KGE_L1P(10) KGE_L1P(12) KGE_L1P(14) KGE_L1P(16)
         KGE_L1P(18) KGE_L1P(20) KGE_L1P(22) KGE_L1P(24) KGE_L1P(26) KGE_L1P(28) KGE_L1P(30) KGE_L1P(32)
     }
 #undef KGE_L1P
 }
 
-// shapes the paired L1 kernel takes: tails split evenly over 16 waves, whole
-// chunks of heads, whole 64-column slices, and enough workgroups for the chip
-static bool l1_pair_ok(const ScoreShape& sh) {
-    // (T % 64 == 0: every live count is a multiple of 32, 2 tails per wave at least)
-    return sh.T % 64 == 0 && sh.T >= 128 && sh.T <= L1P_MAX_T && sh.B % L1P_CB == 0 &&
-           sh.Dp % 64 == 0 && sh.S * (sh.Dp / 64) >= 128 && (!sh.tcount || sh.tpad == 64);
+// The pieces of the split sides added up, in group order: one wave per row of 256 columns.
+__global__ __launch_bounds__(256) void k_l1_pair_sum(const float* __restrict__ head_pieces, int n_head_pieces,
+                                                     const float* __restrict__ tail_pieces, int n_tail_pieces,
+                                                     float* __restrict__ grad, int n_head, int n_tail, int T, int Dp,
+                                                     const uint32_t* __restrict__ tcount) {
+    const int slabs = (Dp + 255) / 256;
+    const int g = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int row0 = g / slabs, k = (g - row0 * slabs) * 256 + (threadIdx.x & 63) * 4;
+    const int first = n_head_pieces > 1 ? 0 : n_head;  // rows of `grad` that come in pieces: [first, ..)
+    const int r = first + row0;
+    if (r >= n_head + (n_tail_pieces > 1 ? n_tail : 0) || k >= Dp) return;
+    const bool tail = r >= n_head;
+    const int q = tail ? r - n_head : r;
+    if (tail && tcount && q % T >= (int)tcount[q / T]) return;  // never written, never read
+    const float* src = (tail ? tail_pieces : head_pieces) + (size_t)q * Dp + k;
+    const int n = tail ? n_tail_pieces : n_head_pieces;
+    const size_t pitch = (size_t)(tail ? n_tail : n_head) * Dp;
+    float4 sum = *reinterpret_cast<const float4*>(src);
+    for (int i = 1; i < n; ++i) sum = f4add(sum, *reinterpret_cast<const float4*>(src + i * pitch));
+    *reinterpret_cast<float4*>(grad + (size_t)r * Dp + k) = sum;
+}
+
+static void launch_l1_pair(const ScoreShape& sh, const float* ops, const float* coef, float* grad, float* pieces,
+                           hipStream_t stream) {
+    const L1Split k = l1_pair_split(sh);
+    const int S = sh.S, B = sh.B, T = sh.T, Dp = sh.Dp, n_head = S * B, n_tail = S * T;
+    float* const heads = k.tails > 1 ? pieces : grad;
+    float* const tail_pieces = pieces + (k.tails > 1 ? (size_t)k.tails * n_head * Dp : 0);
+    float* const tails = k.heads > 1 ? tail_pieces : grad + (size_t)n_head * Dp;
+    const int h_size = ((B + k.heads - 1) / k.heads + L1P_CB - 1) / L1P_CB * L1P_CB;
+    const dim3 grid = tile_grid((Dp + 63) / 64, k.heads * k.tails, S);
+    const bool full = T % 32 == 0 && B % L1P_CB == 0 && Dp % 64 == 0;
+    if (full)
+        hipLaunchKernelGGL(k_score_bwd_l1_pair<true>, grid, dim3(1024), 0, stream, ops, coef, heads, tails, S, B, T, Dp, 0,
+                           n_head, k.heads, k.tails, h_size, sh.tcount);
+    else
+        hipLaunchKernelGGL(k_score_bwd_l1_pair<false>, grid, dim3(1024), 0, stream, ops, coef, heads, tails, S, B, T, Dp, 0,
+                           n_head, k.heads, k.tails, h_size, sh.tcount);
+    if (k.heads == 1 && k.tails == 1) return;
+    const int rows = (k.tails > 1 ? n_head : 0) + (k.heads > 1 ? n_tail : 0), slabs = (Dp + 255) / 256;
+    hipLaunchKernelGGL(k_l1_pair_sum, dim3((rows * slabs + 3) / 4), dim3(256), 0, stream, heads, k.tails, tails, k.heads,
+                       grad, n_head, n_tail, T, Dp, sh.tcount);
 }
 
 void launch_score_bwd(const ScoreShape& sh, const RowSource& ent, const float* rel,
                       const uint32_t* crel, const float* coef, const uint32_t* nearflag, float* grad,
-                      hipStream_t stream) {
+                      float* pieces, hipStream_t stream) {
     BwdParams p;
     p.ent_a = ent; p.ent_b = ent; p.rel = rel; p.crel = crel; p.coef = coef; p.grad = grad;
     p.coef_div = nullptr; p.add_base = nullptr;
@@ -1008,11 +1112,8 @@ void launch_score_bwd(const ScoreShape& sh, const RowSource& ent, const float* r
             hipLaunchKernelGGL((k_score_bwd_mfma_both<DIST_DOT, 32, true, 8>), grid, dim3(512), 0, stream, p);
         return;
     }
-    if (dist_fn == DIST_L1 && sh.use_mfma && sh.operands_dense && plain && ent.pitch == (int64_t)sh.Dp * 4 && l1_pair_ok(sh)) {
-        const float* ops = reinterpret_cast<const float*>(ent.base);
-        const dim3 grid = tile_grid(sh.Dp / 64, 1, sh.S);
-        hipLaunchKernelGGL(k_score_bwd_l1_pair, grid, dim3(1024), 0, stream, ops, coef, grad, sh.B, sh.T, sh.Dp, p.a_c0,
-                           p.b_c0, sh.tcount, sh.tpad);
+    if (dist_fn == DIST_L1 && sh.use_mfma && sh.operands_dense && plain && ent.pitch == (int64_t)sh.Dp * 4 && (pieces || !score_bwd_pieces(sh))) {
+        launch_l1_pair(sh, reinterpret_cast<const float*>(ent.base), coef, grad, pieces, stream);
         return;
     }
     p.side_b = 0; p.grad_c0 = p.a_c0;
