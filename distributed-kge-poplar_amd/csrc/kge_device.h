@@ -85,6 +85,32 @@ DEVINL float4 combine_rel(float4 e, const float* relrow, int k, int rel_mode) {
     return rel_mode == 1 ? f4add(e, r) : f4mul(e, r);
 }
 
+// The predicted tail's columns k .. k+3 of the modes that mix columns: `v` the head row's own, `row`
+// the whole head row, `rrow` the relation's.
+//   3  complex product on the halves: column kk pairs with kk +- half (src/poplar_kge.cpp:501-510)
+//   4  rotation by the relation's phases (src/poplar_kge.cpp:516-530): phase, sine and cosine in
+//      float16, the rotation itself in float32
+DEVINL float4 relation_xf(float4 v, const char* row, int etype, const float* rrow, int k, int half, int rel_mode) {
+    float* vv = &v.x;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        const int kk = k + x;
+        if (kk >= 2 * half) { vv[x] = 0.f; continue; }
+        const int kq = kk < half ? kk : kk - half, pp = kk < half ? kk + half : kk - half;
+        const float e2 = load1(row, pp, etype);
+        if (rel_mode == 3) {
+            vv[x] = kk < half ? vv[x] * rrow[kk] - e2 * rrow[pp]    // re = h_re r_re - h_im r_im
+                              : e2 * rrow[kk] + vv[x] * rrow[pp];   // im = h_re r_im + h_im r_re
+        } else {
+            const float th = (float)(_Float16)rrow[kq];
+            const float sn = (float)(_Float16)sinf(th), cs = (float)(_Float16)cosf(th);
+            vv[x] = kk < half ? vv[x] * cs - e2 * sn     // re = h_re cos - h_im sin
+                              : vv[x] * cs + e2 * sn;    // im = h_im cos + h_re sin
+        }
+    }
+    return v;
+}
+
 DEVINL float wave_sum(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

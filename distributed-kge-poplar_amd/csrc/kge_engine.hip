@@ -271,6 +271,11 @@ struct kge_engine {
     DevBuf<float> up, up_m, up_v, down, down_m, down_v, g_up, g_down;
     DevBuf<float> mlp_fproj, mlp_concat, mlp_pre, mlp_gpre, mlp_gfp, mlp_gval, p_fproj, p_concat, p_pre;
     DevBuf<float> opnd_n, cmat, dcm, transh_mm, relgrad;  // TransH: [n | tails], c, d loss / d c, its products, relation contributions
+    // L2 and dot scoring on three-piece operands (kge_split.hip)
+    bool split = false;
+    int Kp = 0, Bp = 0, Tp = 0;
+    DevBuf<char> rowsp, coefp;
+    DevBuf<float> row_norm, rowpart, colpart;
     DevBuf<float> bwd_pieces;  // split sums of the scoring backward
     DevBuf<float> coef, dist, grad, opnd, partial, rel_partial, rel_gsum, hidden, gsum, gproj, featd, gproj_part, gemm_part, projR, loss_part, loss_step, d_alpha;
     // [n_step][entity, relation, normal, then per feature network projection, mlp up, mlp down][S]; the relation update indexes its two
@@ -673,6 +678,10 @@ void allocate(kge_engine& E) {
     E.r_crow.alloc(ns * E.r_cstride);
     E.r_hot_count.alloc(ns * 2);
 
+    ScoreShape sh = {};
+    sh.S = E.S; sh.B = E.B; sh.T = E.T; sh.Dp = E.Dp;
+    sh.score_fn = E.score_fn; sh.dist_fn = E.dist_fn; sh.use_mfma = E.use_mfma;
+    E.split = !E.score_bf16 && split_scoring(sh);
     E.coef.alloc(SB * E.T);
     const bool fused = E.loss_fn == LOSS_LOGSIGMOID && E.neg_adv <= 0.f && !E.score_bf16;
     if (!fused && E.dist_fn == DIST_L2) E.dist.alloc(SB * E.T);
@@ -685,7 +694,17 @@ void allocate(kge_engine& E) {
         E.gemm_part.alloc(std::max(p_head, p_tail));
     }
     E.grad.alloc(R * E.Dp);
-    E.opnd.alloc(R * E.Dp);
+    if (E.split) {
+        E.Kp = round_up(E.Dp, 32); E.Bp = round_up(E.B, 32); E.Tp = round_up(E.T, 32);
+        // rows and columns that no kernel writes are read and dropped or multiplied by zero: finite
+        E.rowsp.alloc(split_bytes(R, E.Kp));
+        E.rowsp.zero(st);
+        E.coefp.alloc(split_bytes(S * E.Bp, E.Tp));
+        E.coefp.zero(st);
+        E.row_norm.alloc(R + kSplitSpareRows);
+        E.rowpart.alloc(S * E.Bp * (E.Tp / 32));
+        E.colpart.alloc(S * (E.Bp / 32) * E.Tp);
+    } else E.opnd.alloc(R * E.Dp);
     if (E.merge_tails) {
         // columns past a block's distinct tails are never written; the kernels that read whole
         // tiles of them (and drop the results) must find finite values there
@@ -731,12 +750,8 @@ void allocate(kge_engine& E) {
             E.mlp_gfp.zero(st);
         }
     }
-    ScoreShape sh = {};
-    sh.S = E.S; sh.B = E.B; sh.T = E.T;
-    sh.Dp = E.Dp;
-    sh.score_fn = E.score_fn; sh.dist_fn = E.dist_fn; sh.use_mfma = E.use_mfma;
     if (E.score_fn != SCORE_TRANSH) E.bwd_pieces.alloc(score_bwd_pieces(sh));
-    E.n_part = fused ? score_fwd_parts(sh) : E.B;
+    E.n_part = !fused ? E.B : E.split ? split_fwd_parts(sh) : score_fwd_parts(sh);
     if (E.use_mfma && E.dist_fn == DIST_L2) {
         E.nearflag.alloc(nearflag_words(sh));
         E.nearflag.zero(st);
@@ -1199,6 +1214,10 @@ void run_step(kge_engine& E, int i) {
     // dense operands: every contribution's row, float32, relation applied to the heads
     { KernelTimer t(E, K_GATHER);
       TailCols tc = {sh.tcount, E.T, E.tpad};
+      if (E.split)
+          launch_gather_pieces(ent, E.rel.p, crel, rel_mode_of(E), E.D / 2, (int)SB, (int)R, E.Dp, E.Kp, E.rowsp.p,
+                               E.row_norm.p, st, &tc);
+      else
       launch_gather_operands(ent, E.rel.p, crel, rel_mode_of(E), E.D / 2, (int)SB, (int)R, E.Dp,
                              E.opnd.p, E.score_bf16 ? E.opnd16.p : nullptr, st, &tc); }
     RowSource dense;
@@ -1280,6 +1299,25 @@ void run_step(kge_engine& E, int i) {
           tb.mm = E.transh_mm.p; tb.grad = E.grad.p; tb.S = E.S; tb.B = E.B; tb.T = E.T; tb.Dp = E.Dp;
           launch_transh_bwd(tb, st);
           launch_transh_back(ent, E.rel.p, crel, E.n_rel, (int)SB, E.Dp, E.grad.p, E.transh_mm.p, E.relgrad.p, st); }
+    } else if (E.split) {
+        const SplitCoef sc = {E.coefp.p, E.rowpart.p, E.colpart.p, E.Bp, E.Tp};
+        { KernelTimer t(E, K_FWD);
+          SplitFwd f = {};
+          f.sh = sh; f.a = f.b = E.rowsp.p; f.norm_a = f.norm_b = E.row_norm.p;
+          f.a_c0 = 0; f.b_c0 = (int)SB; f.Kp = E.Kp; f.clabel = clabel;
+          f.coef = E.coef.p; f.dist = fused ? nullptr : E.dist.p; f.loss_part = loss_part; f.nearflag = E.nearflag.p;
+          f.out = sc;
+          launch_split_fwd(f, fused, st); }
+        if (!fused) {
+            KernelTimer t(E, K_LOSS);
+            launch_loss_rows(sh, clabel, E.coef.p, E.dist.p, loss_part, nullptr, st);
+            launch_coef_pieces(sh, E.coef.p, E.nearflag.p, sc, st);
+        }
+        { KernelTimer t(E, K_BWD);
+          SplitBwd b = {};
+          b.rows = E.rowsp.p; b.Kp = E.Kp; b.b_c0 = (int)SB; b.in = sc; b.coef = E.coef.p; b.nearflag = E.nearflag.p;
+          b.grad = E.grad.p; b.S = E.S; b.B = E.B; b.T = E.T; b.Dp = E.Dp; b.tcount = sh.tcount; b.tpad = sh.tpad;
+          launch_split_bwd(b, E.dist_fn == DIST_L2 && E.score_fn != SCORE_DISTMULT, st); }
     } else {
         { KernelTimer t(E, K_FWD);
           launch_score_fwd(sh, dense, E.rel.p, crel, clabel, E.coef.p, E.dist.p, E.nearflag.p, loss_part, fused, st); }

@@ -241,6 +241,49 @@ inline size_t nearflag_words(const ScoreShape& sh) {
 }
 int score_fwd_parts(const ScoreShape& sh);
 
+// ---- scoring on three-piece operands (kge_split.hip; L2 and dot, any shape) ----
+// Piece matrices hold every float32 value as three bfloat16 pieces, rows of 6 * Kp bytes (columns
+// filled up to a multiple of 32 with zeros).  The product kernels read whole tiles: kSplitSpareRows
+// rows behind a matrix's last must be readable and finite.
+constexpr int kSplitSpareRows = 128;
+inline size_t split_bytes(size_t rows, size_t cols) {
+    return (rows + kSplitSpareRows) * ((cols + 31) / 32 * 32) * 6 + 128 * 6;
+}
+void launch_gather_pieces(const RowSource& ent, const float* rel, const uint32_t* crel, int rel_mode, int half,
+                          int n_head, int n_rows, int Dp, int Kp, void* out, float* norm, hipStream_t stream,
+                          const TailCols* tail_cols);
+// The coefficient matrices [S][Bp][Tp] (B and T filled up to multiples of 32) as pieces, and their
+// sums over the 32 x 32 sub-blocks: rowpart [S][Bp][Tp / 32], colpart [S][Bp / 32][Tp] (L2 only)
+struct SplitCoef { char* coefp; float* rowpart; float* colpart; int Bp, Tp; };
+struct SplitFwd {
+    ScoreShape sh;
+    const char* a; const char* b;          // piece matrices of the rows; block d's from a_c0 + d B and b_c0 + d T
+    const float* norm_a; const float* norm_b;  // their squared norms
+    int a_c0, b_c0, Kp;
+    const uint32_t* clabel;
+    float* coef;        // [S, B, T] scores (without fused loss); the flagged sub-blocks' coefficients
+    float* dist;        // or null
+    float* loss_part;   // split_fwd_parts per block
+    uint32_t* nearflag; // [S, Bp / 32, Tp / 32]
+    SplitCoef out;      // written with the fused loss
+};
+bool split_scoring(const ScoreShape& sh);  // whether a step's scoring takes this form
+int split_fwd_parts(const ScoreShape& sh);
+void launch_split_fwd(const SplitFwd& p, bool fused_loss, hipStream_t stream);
+// `coef` as launch_loss_rows leaves it -> pieces and sums
+void launch_coef_pieces(const ScoreShape& sh, const float* coef, const uint32_t* nearflag, const SplitCoef& out,
+                        hipStream_t stream);
+struct SplitBwd {
+    const char* rows; int Kp, b_c0;  // heads from row 0, tails from row b_c0
+    SplitCoef in;
+    const float* coef;               // float32 coefficients of the flagged sub-blocks
+    const uint32_t* nearflag;
+    float* grad;                     // [R, Dp]
+    int S, B, T, Dp;
+    const uint32_t* tcount; int tpad;
+};
+void launch_split_bwd(const SplitBwd& p, bool l2, hipStream_t stream);
+
 // Row-wise losses (softmax; logsigmoid with adversarial weighting): converts
 // the raw scores in `coef` to backward coefficients in place; loss_part gets
 // S * B partial sums.  `coef16` (may be null): a bfloat16 copy of the coefficients; with

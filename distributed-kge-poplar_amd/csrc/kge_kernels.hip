@@ -10,6 +10,7 @@
 //   reduce_chunks + adam_rows   multiUpdateAdd + fr::nn::adam + Buffer::write
 //                  (src/fructose/frnn.cpp:61-90, src/poplar_kge.cpp:695-704)
 #include "kge_device.h"
+#include "kge_loss.h"
 
 #include <algorithm>
 #include <cstdint>
@@ -38,33 +39,8 @@ __global__ __launch_bounds__(256) void k_gather_operands(RowSource ent, const fl
     const float* rrow = (c < n_head && rel_mode) ? rel + (size_t)crel[c] * Dp : nullptr;
     for (int k = lane * 4; k < Dp; k += 256) {
         float4 v = load4(row, k, ent);
-        if (XF && rrow && rel_mode == 3) {
-            // complex product: column kk pairs with kk +- half (src/poplar_kge.cpp:501-510)
-            float* vv = &v.x;
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                const int kk = k + x;
-                if (kk >= 2 * half) { vv[x] = 0.f; continue; }
-                const int pp = kk < half ? kk + half : kk - half;
-                const float e2 = load1(row, pp, ent.etype);
-                vv[x] = kk < half ? vv[x] * rrow[kk] - e2 * rrow[pp]    // re = h_re r_re - h_im r_im
-                                  : e2 * rrow[kk] + vv[x] * rrow[pp];   // im = h_re r_im + h_im r_re
-            }
-        } else if (XF && rrow && rel_mode == 4) {
-            // rotation by the relation's phases (src/poplar_kge.cpp:516-530): phase, sine and
-            // cosine in float16, the rotation itself in float32
-            float* vv = &v.x;
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                const int kk = k + x;
-                if (kk >= 2 * half) { vv[x] = 0.f; continue; }
-                const int kq = kk < half ? kk : kk - half, pp = kk < half ? kk + half : kk - half;
-                const float th = (float)(_Float16)rrow[kq];
-                const float sn = (float)(_Float16)sinf(th), cs = (float)(_Float16)cosf(th);
-                const float e2 = load1(row, pp, ent.etype);
-                vv[x] = kk < half ? vv[x] * cs - e2 * sn     // re = h_re cos - h_im sin
-                                  : vv[x] * cs + e2 * sn;    // im = h_im cos + h_re sin
-            }
+        if (XF && rrow && rel_mode >= 3) {
+            v = relation_xf(v, row, ent.etype, rrow, k, half, rel_mode);
         } else if (rrow) v = combine_rel(v, rrow, k, rel_mode);
         // + 0 turns a -0 into +0, so that a difference of stored operands is never -0
         // (the paired L1 backward reads the sign off the difference's bit pattern)
@@ -159,57 +135,6 @@ void launch_gather_operands(const RowSource& ent, const float* rel, const uint32
 
 // --------------------------------------------------------------------------
 // scoring: forward
-
-// logSigmoid and its derivative exactly as src/pag/pag.cpp:894-903
-DEVINL float log_sigmoid(float z) { return z > -11.f ? -log1pf(expf(-z)) : z; }
-DEVINL float log_sigmoid_grad(float z) { return 1.f / (1.f + expf(fminf(z, 11.f))); }
-
-// The same two functions from ONE hardware exponential (the scoring epilogues
-// evaluate them once per score): with u = exp(-|z|) in (0, 1],
-//   z >= 0:        logsig = -log1p(u),     dlogsig = u' / (1 + u'),  u' = max(u, e^-11)  (the +11 clamp;
-//                  u / (1 + u) grows with u, so the clamp can move to the quotient)
-//   -11 < z < 0:   logsig = z - log1p(u),  dlogsig = 1 / (1 + u)
-//   z <= -11:      logsig = z              (the reference drops the log1p term there)
-// log1p(u) = log(w) - ((w - 1) - u) / w with w = 1 + u keeps the low bits of u.
-DEVINL void log_sigmoid_both(float z, float& value, float& grad) {
-    // single hardware instructions: exp2, rcp and log2 (about 1 ulp each; w is in [1, 2], so
-    // none of the range fix-ups of the library forms is needed)
-    const float u = __builtin_amdgcn_exp2f(-1.44269504089f * fabsf(z));
-    const float w = 1.f + u;
-    const float rw = __builtin_amdgcn_rcpf(w);
-    const float l1p = 0.69314718056f * __builtin_amdgcn_logf(w) - ((w - 1.f) - u) * rw;
-    // straight-line selects (lanes of a wave mix both signs of z):
-    //   value = min(z, 0) - log1p(u), without the log1p term for z <= -11
-    //   grad  = u / (1 + u) clamped below at its value for u = e^-11 (z >= 0), 1 / (1 + u) (z < 0)
-    value = fminf(z, 0.f) - (z > -11.f ? l1p : 0.f);
-    const float g_pos = fmaxf(u * rw, 1.670142184e-5f);  // e^-11 / (1 + e^-11)
-    grad = z >= 0.f ? g_pos : rw;
-}
-
-// The same for both signs of one score: exp(-|z|) serves z = s and z = -s alike.
-DEVINL void log_sigmoid_pair(float s, float& v_pos, float& g_pos, float& v_neg, float& g_neg) {
-    const float u = __builtin_amdgcn_exp2f(-1.44269504089f * fabsf(s));
-    const float w = 1.f + u;
-    const float rw = __builtin_amdgcn_rcpf(w);
-    const float l1p = 0.69314718056f * __builtin_amdgcn_logf(w) - ((w - 1.f) - u) * rw;
-    const float g_big = fmaxf(u * rw, 1.670142184e-5f);  // e^-11 / (1 + e^-11)
-    v_pos = fminf(s, 0.f) - (s > -11.f ? l1p : 0.f);
-    v_neg = fminf(-s, 0.f) - (s < 11.f ? l1p : 0.f);
-    g_pos = s >= 0.f ? g_big : rw;
-    g_neg = s <= 0.f ? g_big : rw;
-}
-
-// The logsigmoid loss of one score column that stands for `mult` tail positions, one of them the
-// positive's label if `pos` (src/poplar_kge.cpp:615-636 summed over the positions that share the
-// row): returns the loss term (before the normalisation) and sets d loss / d score (times grad_scale).
-DEVINL float logsigmoid_column(float score, bool pos, float mult, float w_pos, float w_neg, float grad_scale,
-                               float& dscore) {
-    float v_pos, g_pos, v_neg, g_neg;
-    log_sigmoid_pair(score, v_pos, g_pos, v_neg, g_neg);
-    const float wp = pos ? w_pos : 0.f, wn = (mult - (pos ? 1.f : 0.f)) * w_neg;
-    dscore = (wn * g_neg - wp * g_pos) * grad_scale;
-    return -(wp * v_pos + wn * v_neg);
-}
 
 struct FwdParams {
     ScoreShape sh;
@@ -385,12 +310,6 @@ __global__ __launch_bounds__(256) void k_score_fwd(FwdParams p) {
 
 
 constexpr int FM_TM = 128, FM_TN = 64;
-constexpr float kCancelRatio = 0.125f;  // recompute when d^2 < ratio * (|a|^2 + |b|^2)
-// Below this ratio the backward's product form self*sum(c) - sum(c*other) would
-// lose accuracy against the reference's c*(self-other); such 32x32 sub-blocks
-// are flagged for the backward kernel, which handles them in the direct form.
-constexpr float kNearRatio = 1.f / 4096.f;
-
 // BKT = embedding columns staged per iteration: with 128 a whole D = 256 row
 // takes two iterations, the loads of the second in flight under the first's
 // matrix work (99 KB of LDS).  NW = waves per workgroup: 8 (two per SIMD, each

@@ -1,0 +1,703 @@
+// gfx950 scoring kernels on three-piece operands (L2 and dot): the operand gather, the forward
+// scores with the fused loss, and both sides of the backward.
+//
+// Every float32 value is the exact sum of three bfloat16 pieces, and a float32 product is six
+// products of pieces (split4_bf16, mfma_split6's order).  Splitting while staging, as a kernel
+// that reads float32 operands must, costs more vector instructions than the products cost matrix
+// instructions, and every tile that reads a row splits it again.  Here every value is split once,
+// by the kernel that makes it: the gather writes the operand rows as pieces, the forward writes the
+// backward's coefficients as pieces, and the product kernels copy tiles straight from memory into
+// LDS (global_load_lds, no registers, no vector instructions), so that their waves do little else
+// than read fragments and multiply.
+//
+// Piece matrix: row r, column k, piece q at  r * pitch + (k / 32) * 192 + q * 64 + (k % 32) * 2  bytes:
+// the three pieces of 32 columns lie together, and a slab of a row is 192 consecutive bytes.  Columns
+// are filled with zeros to a multiple of 32.
+#include "kge_device.h"
+#include "kge_loss.h"
+
+#include <algorithm>
+#include <cstdint>
+
+namespace kge {
+
+// --------------------------------------------------------------------------
+// global memory -> LDS copies and their waits
+
+// 64 lanes x 16 bytes: lane l's bytes at base + off go to LDS byte lds + 16 l (base, lds: wave-uniform)
+DEVINL void lds_copy16(const char* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+// until at most N of this wave's memory operations are under way, then for the workgroup's other waves
+template <int N>
+DEVINL void wait_copies_and_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+DEVINL uint32_t lds_address(const void* p) {
+    return (uint32_t)(size_t)(const __attribute__((address_space(3))) char*)p;
+}
+
+// neighbouring lanes' values (lane ^ 1)
+DEVINL float swap1(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));
+}
+DEVINL float swap2(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));
+}
+
+// four columns of a piece-matrix row, k % 4 == 0
+DEVINL float4 load_pieces4(const char* row, int k) {
+    const char* p = row + (size_t)(k >> 5) * 192 + (k & 31) * 2;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const uint2 raw = *reinterpret_cast<const uint2*>(p + 64 * q);
+        v.x += bf16_lo_f32(raw.x); v.y += bf16_hi_f32(raw.x);
+        v.z += bf16_lo_f32(raw.y); v.w += bf16_hi_f32(raw.y);
+    }
+    return v;
+}
+DEVINL float load_piece1(const char* row, int k) {
+    const char* p = row + (size_t)(k >> 5) * 192 + (k & 31) * 2;
+    float v = 0.f;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) v += bf16_to_f32(*reinterpret_cast<const uint16_t*>(p + 64 * q));
+    return v;
+}
+DEVINL void store_pieces4(char* row, int k, float4 v) {
+    uint2 piece[3];
+    split4_bf16(as_x4(v), piece);
+    char* p = row + (size_t)(k >> 5) * 192 + (k & 31) * 2;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2*>(p + 64 * q) = piece[q];
+}
+// two neighbouring values -> three words of two pieces each
+DEVINL void split2(float a, float b, uint32_t w[3]) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        w[q] = pack_bf16(a, b);
+        if (q < 2) { a -= bf16_lo_f32(w[q]); b -= bf16_hi_f32(w[q]); }
+    }
+}
+
+// --------------------------------------------------------------------------
+// operand gather: RPW contributions per wave, their entity (or hidden) rows with the relation
+// applied for the heads, as pieces; and the rows' squared norms.
+template <int RPW, bool XF>  // XF: the complex product and the rotation compiled in
+__global__ __launch_bounds__(256) void k_gather_pieces(RowSource ent, const float* __restrict__ rel,
+                                                       const uint32_t* __restrict__ crel, int rel_mode, int half,
+                                                       int n_head, int n_rows, int Dp, int Kp, char* __restrict__ out,
+                                                       float* __restrict__ norm, TailCols tc) {
+    const int lane = threadIdx.x & 63;
+    const int c0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW;
+    if (c0 >= n_rows) return;
+    // the row numbers are asked for together with the block's tail count (rows past it are
+    // never used, but their slots hold valid numbers): one round trip instead of two
+    uint32_t key[RPW], rkey[RPW];
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) {
+        const int c = min(c0 + r, n_rows - 1);  // a row past the end repeats the last one
+        key[r] = ent.index ? ent.index[c] : (uint32_t)c;
+        rkey[r] = (c < n_head && rel_mode) ? crel[c] : 0u;
+    }
+    bool live[RPW], any = false;
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) {
+        live[r] = c0 + r < n_rows && tc.live(c0 + r - n_head);
+        any = any || live[r];
+    }
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) asm volatile("" : "+v"(key[r]), "+v"(rkey[r]));
+    if (!any) return;
+    const char* row[RPW];
+    const float* rrow[RPW];
+    float sq[RPW];
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) {
+        row[r] = ent.base + (int64_t)key[r] * ent.pitch;
+        rrow[r] = (c0 + r < n_head && rel_mode) ? rel + (size_t)rkey[r] * Dp : nullptr;
+        sq[r] = 0.f;
+    }
+    for (int k = lane * 4; k < Kp; k += 256) {
+        float4 v[RPW], w[RPW];
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {  // all loads first
+            v[r] = w[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (k < Dp) {
+                v[r] = load4(row[r], k, ent);
+                if (rrow[r] && rel_mode <= 2) w[r] = *reinterpret_cast<const float4*>(rrow[r] + k);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {
+            if (rrow[r] && k < Dp) {
+                if (XF && rel_mode >= 3) v[r] = relation_xf(v[r], row[r], ent.etype, rrow[r], k, half, rel_mode);
+                else v[r] = rel_mode == 1 ? f4add(v[r], w[r]) : f4mul(v[r], w[r]);
+            }
+            sq[r] += v[r].x * v[r].x + v[r].y * v[r].y + v[r].z * v[r].z + v[r].w * v[r].w;
+            if (live[r]) store_pieces4(out + (size_t)(c0 + r) * Kp * 6, k, v[r]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) {
+        const float s = wave_sum(sq[r]);
+        if (lane == 0 && live[r]) norm[c0 + r] = s;
+    }
+}
+
+void launch_gather_pieces(const RowSource& ent, const float* rel, const uint32_t* crel, int rel_mode, int half,
+                          int n_head, int n_rows, int Dp, int Kp, void* out, float* norm, hipStream_t stream,
+                          const TailCols* tail_cols) {
+    TailCols tc = {};
+    if (tail_cols) tc = *tail_cols;
+    // two rows per wave where that leaves enough waves: the kernel is resident waves over the
+    // latency of the chain row number -> row -> store, and a wave may as well keep two chains going
+#define KGE_GATHER(N_, X_)                                                                                            \
+    hipLaunchKernelGGL((k_gather_pieces<N_, X_>), dim3((n_rows + 4 * N_ - 1) / (4 * N_)), dim3(256), 0, stream, ent, rel, \
+                       crel, rel_mode, half, n_head, n_rows, Dp, Kp, (char*)out, norm, tc)
+    if (rel_mode >= 3) KGE_GATHER(1, true);
+    else if (n_rows >= 8192) KGE_GATHER(2, false);
+    else KGE_GATHER(1, false);
+#undef KGE_GATHER
+}
+
+// --------------------------------------------------------------------------
+// tiles in LDS
+
+// Contraction-innermost operand: R rows x 32 columns of a piece matrix as [piece][row][32], a row's
+// four 16-byte chunks at position chunk ^ ((row / 4) % 4): sixteen rows' reads of one chunk fall on
+// all banks.  One copy instruction moves sixteen rows of one piece.
+template <int R>
+struct RowTile {
+    static constexpr int kBytes = 3 * R * 64, kCopies = 3 * R / 16;
+    // offset of copy x's bytes for this lane, from the tile's first row and slab
+    static DEVINL uint32_t source(int x, int lane, int pitch) {
+        const int piece = x / (R / 16), row = (x % (R / 16)) * 16 + (lane >> 2);
+        const int chunk = (lane & 3) ^ ((row >> 2) & 3);
+        return (uint32_t)(row * pitch + piece * 64 + chunk * 16);
+    }
+    // the 16-column step `ks`'s fragment of rows row0 .. row0 + 31 (this lane: row row0 + lane % 32)
+    static DEVINL floatx4 fragment(const char* tile, int piece, int row0, int ks, int lane) {
+        const int row = row0 + (lane & 31), chunk = (2 * ks + (lane >> 5)) ^ ((row >> 2) & 3);
+        return *reinterpret_cast<const floatx4*>(tile + piece * (R * 64) + row * 64 + chunk * 16);
+    }
+};
+
+// Contraction-outermost operand: 32 rows (contraction) x C columns of a piece matrix as
+// [piece][row][C], read back transposed (ds_read_b64_tr_b16: sixteen lanes read a 4 x 16 block and
+// each receives one column of it).  A row's 32-byte units sit at position unit ^ 2 (row % 4): the four
+// rows that a read instruction's half takes fall on different banks.  One copy instruction moves
+// 512 / C rows of one piece.
+template <int C>
+struct ColTile {
+    static constexpr int kBytes = 3 * 32 * C * 2, kCopies = 3 * C / 16;
+    static constexpr int kKey = C >= 128 ? 3 : 1;  // (a row of 64 columns has four units)
+    static DEVINL uint32_t source(int x, int lane, int pitch) {
+        constexpr int chunks = C / 8, rows = 64 / chunks;
+        const int piece = x / (C / 16), row = (x % (C / 16)) * rows + lane / chunks, pos = lane % chunks;
+        const int chunk = pos ^ ((row & kKey) << 2);  // 16-byte chunks: two to a unit
+        const int col = chunk * 8;
+        return (uint32_t)(row * pitch + (col >> 5) * 192 + piece * 64 + (col & 31) * 2);
+    }
+    // columns col0 .. col0 + 31 over the sixteen rows of step `ks` (this lane: column
+    // col0 + lane % 32, rows 8 (lane / 32) .. + 7)
+    static DEVINL floatx4 fragment(const char* tile, int piece, int col0, int ks, int lane) {
+        typedef short s16x4 __attribute__((ext_vector_type(4)));
+        typedef const __attribute__((address_space(3))) s16x4* lds_ptr;
+        const int g = lane >> 4, r4 = (lane & 15) >> 2;
+        const int unit = ((col0 >> 4) + (g & 1)) ^ ((r4 & kKey) << 1);
+        const char* p = tile + piece * (64 * C) + (16 * ks + 8 * (g >> 1) + r4) * (2 * C) + unit * 32 + (lane & 3) * 8;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(lds_ptr)p);
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(lds_ptr)(p + 4 * 2 * C));
+        typedef short s16x8 __attribute__((ext_vector_type(8)));
+        return __builtin_bit_cast(floatx4, s16x8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w});
+    }
+};
+
+// The product loop of a TM x TN tile: n_slab slabs of 32 contraction steps, two tile copies in LDS
+// (one fills while the other is multiplied, one barrier per slab).  TA, TB: RowTile / ColTile;
+// a_step, b_step: bytes from slab to slab.  Waves as WM x WN, each (TM/WM) x (TN/WN) in 32 x 32
+// accumulators.
+template <class TA, class TB, int TM, int TN, int WM, int WN>
+struct SplitProduct {
+    static constexpr int NW = WM * WN, AM = TM / WM / 32, AN = TN / WN / 32;
+    static constexpr int kStage = TA::kBytes + TB::kBytes, kLds = 2 * kStage;
+    static constexpr int kCopies = TA::kCopies + TB::kCopies, kEach = kCopies / NW;
+    static_assert(kCopies % NW == 0, "every wave issues the same number of copies");
+
+    // meanwhile(): what the caller has to fetch for itself, under the first slab's way from memory
+    template <class Meanwhile>
+    static DEVINL void run(char* smem, const char* a, int a_pitch, size_t a_step, const char* b, int b_pitch, size_t b_step,
+                           int n_slab, floatx16 (&acc)[AM][AN], int lane, int wave, Meanwhile&& meanwhile) {
+        uint32_t off[kEach];
+#pragma unroll
+        for (int i = 0; i < kEach; ++i) {
+            const int x = wave + NW * i;
+            off[i] = x < TA::kCopies ? TA::source(x, lane, a_pitch) : TB::source(x - TA::kCopies, lane, b_pitch);
+        }
+        const uint32_t lds0 = lds_address(smem);
+        auto fill = [&](int slab) __attribute__((always_inline)) {
+            const char* as = a + slab * a_step;
+            const char* bs = b + slab * b_step;
+            const uint32_t to = lds0 + (slab & 1) * kStage;
+#pragma unroll
+            for (int i = 0; i < kEach; ++i) {
+                const int x = wave + NW * i;
+                lds_copy16(x < TA::kCopies ? as : bs, off[i], to + x * 1024);
+            }
+        };
+        fill(0);
+        meanwhile();
+        const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
+        for (int slab = 0; slab < n_slab; ++slab) {
+            wait_copies_and_barrier<0>();
+            if (slab + 1 < n_slab) fill(slab + 1);
+            const char* ta = smem + (slab & 1) * kStage;
+            const char* tb = ta + TA::kBytes;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                floatx4 fa[AM][3], fb[AN][3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+#pragma unroll
+                    for (int m = 0; m < AM; ++m) fa[m][q] = TA::fragment(ta, q, wm + 32 * m, ks, lane);
+#pragma unroll
+                    for (int n = 0; n < AN; ++n) fb[n][q] = TB::fragment(tb, q, wn + 32 * n, ks, lane);
+                }
+                // six products, smallest first; the accumulators in turn, so that an instruction
+                // does not wait for the one before it
+                constexpr int qa[6] = {0, 2, 1, 0, 1, 0}, qb[6] = {2, 0, 1, 1, 0, 0};
+#pragma unroll
+                for (int x = 0; x < 6; ++x)
+#pragma unroll
+                    for (int m = 0; m < AM; ++m)
+#pragma unroll
+                        for (int n = 0; n < AN; ++n)
+                            acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                                __builtin_bit_cast(bf16x8, fa[m][qa[x]]), __builtin_bit_cast(bf16x8, fb[n][qb[x]]),
+                                acc[m][n], 0, 0, 0);
+            }
+        }
+    }
+};
+
+// --------------------------------------------------------------------------
+// the coefficient matrix as pieces
+
+// A 32 x 32 block of coefficients in accumulator layout (register r of lane l: row
+// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32) to its place in the piece matrix, block corner
+// (m0, n0) of block d.  Neighbouring lanes swap values so that a lane stores two columns of one row as
+// one word.  For L2 also the block's row sums and column sums.
+template <int DIST>
+DEVINL void store_coef_block(const float (&c)[16], const SplitCoef& p, int d, int m0, int n0, int lane) {
+    const int Bp = p.Bp, Tp = p.Tp;
+    if (m0 >= Bp || n0 >= Tp) return;
+    const int cl = lane & 31, hl = lane >> 5;
+    const bool odd = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
+    char* const base = p.coefp + ((size_t)d * Bp + m0) * Tp * 6 + (size_t)(n0 >> 5) * 192 + (cl & ~1) * 2;
+    float s[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float got = swap1(odd ? c[2 * i] : c[2 * i + 1]);
+        const float x = odd ? got : c[2 * i], y = odd ? c[2 * i + 1] : got;  // row 2 i + odd of this lane's half
+        s[i] = x + y;
+        uint32_t w[3];
+        split2(x, y, w);
+        char* const q = base + (size_t)(8 * (i >> 1) + 4 * hl + 2 * (i & 1) + odd) * Tp * 6;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<uint32_t*>(q + 64 * k) = w[k];
+    }
+    if (DIST != DIST_L2) return;
+    // row sums: at each step a lane keeps half of its rows and hands the other half's sums over
+    float t[4], u[2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) t[i] = (b1 ? s[2 * i + 1] : s[2 * i]) + swap2(b1 ? s[2 * i] : s[2 * i + 1]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) u[i] = (b2 ? t[2 * i + 1] : t[2 * i]) + __shfl_xor(b2 ? t[2 * i] : t[2 * i + 1], 4, 64);
+    float v = (b3 ? u[1] : u[0]) + __shfl_xor(b3 ? u[0] : u[1], 8, 64);
+    v += __shfl_xor(v, 16, 64);
+    const int r = lane & 15;
+    if (!(lane & 16))
+        p.rowpart[((size_t)d * Bp + m0 + 8 * (r >> 2) + 4 * hl + (r & 3)) * (Tp >> 5) + (n0 >> 5)] = v;
+    float col = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) col += c[k];
+    col += __shfl_xor(col, 32, 64);
+    if (lane < 32) p.colpart[((size_t)d * (Bp >> 5) + (m0 >> 5)) * Tp + n0 + lane] = col;
+}
+
+// The same from float32 coefficients in memory (the losses that are formed row by row): one wave
+// per 32 x 32 block.
+template <int DIST>
+__global__ __launch_bounds__(256) void k_coef_pieces(ScoreShape sh, const float* __restrict__ coef,
+                                                     const uint32_t* __restrict__ nearflag, SplitCoef p) {
+    const int lane = threadIdx.x & 63, MT = p.Bp >> 5, NT = p.Tp >> 5;
+    const int g = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int d = g / (MT * NT), mt = (g - d * MT * NT) / NT, nt = g % NT;
+    if (d >= sh.S || 32 * nt >= tail_limit(sh.tcount, d, sh.T, sh.tpad)) return;
+    const float* src = coef + (size_t)d * sh.B * sh.T;
+    const bool skip = DIST == DIST_L2 && nearflag[((size_t)d * MT + mt) * NT + nt] != 0u;  // direct form
+    const int n = 32 * nt + (lane & 31);
+    float c[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int m = 32 * mt + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        c[r] = (!skip && m < sh.B && n < sh.T) ? src[(size_t)m * sh.T + n] : 0.f;
+    }
+    store_coef_block<DIST>(c, p, d, 32 * mt, 32 * nt, lane);
+}
+
+// --------------------------------------------------------------------------
+// forward
+
+// (kCancelRatio, kNearRatio: kge_loss.h)
+template <int DIST, int OM, int TM, int TN, int WM, int WN>
+__global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_fwd(SplitFwd p) {
+    using P = SplitProduct<RowTile<TM>, RowTile<TN>, TM, TN, WM, WN>;
+    __shared__ __attribute__((aligned(16))) char smem[P::kLds];
+    __shared__ float na_s[TM], nb_s[TN], red[WM * WN];
+    __shared__ uint32_t label_s[TM];
+    const ScoreShape& sh = p.sh;
+    const int B = sh.B, T = sh.T, Kp = p.Kp;
+    const TileId tile = xcd_tile((T + TN - 1) / TN, (B + TM - 1) / TM, sh.S);
+    const int d = tile.z, m0 = tile.y * TM, n0 = tile.x * TN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t_live = tail_limit(sh.tcount, d, T, sh.tpad);
+    if (n0 >= t_live) {  // merged tails: the block has no such column
+        if (OM == 0 && tid == 0) p.loss_part[(size_t)d * (tile.gx * tile.gy) + tile.y * tile.gx + tile.x] = 0.f;
+        return;
+    }
+    const int a_row = p.a_c0 + d * B, b_row = p.b_c0 + d * T;
+    const int pitch = Kp * 6;
+    const char* a = p.a + (int64_t)(a_row + m0) * pitch;
+    const char* b = p.b + (int64_t)(b_row + n0) * pitch;
+    floatx16 acc[P::AM][P::AN];
+#pragma unroll
+    for (int m = 0; m < P::AM; ++m)
+#pragma unroll
+        for (int n = 0; n < P::AN; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
+    P::run(smem, a, pitch, 192, b, pitch, 192, Kp / 32, acc, lane, wave, [&]() __attribute__((always_inline)) {
+        for (int i = tid; i < TM; i += WM * WN * 64) {
+            if (DIST == DIST_L2) na_s[i] = p.norm_a[a_row + m0 + i];
+            if (OM == 0) label_s[i] = m0 + i < B ? p.clabel[d * B + m0 + i] : 0u;
+        }
+        if (DIST == DIST_L2)
+            for (int i = tid; i < TN; i += WM * WN * 64) nb_s[i] = p.norm_b[b_row + n0 + i];
+    });
+
+    // epilogue.  Register r of lane l holds row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
+    const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
+    const int cl = lane & 31, hl = lane >> 5;
+    const float Tn = (float)T;
+    const float w_pos = uniform_f32(0.5f * Tn), w_neg = uniform_f32((0.5f * Tn) / (float)(T - 1));
+    const float inv_norm = uniform_f32(1.f / ((float)sh.S * (float)B * Tn));
+    const float grad_scale = uniform_f32(inv_norm * sh.loss_scale);
+    const int Bp = p.out.Bp, Tp = p.out.Tp, MT = Bp >> 5, NT = Tp >> 5;
+    float loss_acc = 0.f;
+#pragma unroll
+    for (int mi = 0; mi < P::AM; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < P::AN; ++ni) {
+            const int mb = wm + 32 * mi, nbk = wn + 32 * ni;  // the sub-block's corner in the tile
+            const int n = n0 + nbk + cl;
+            // columns behind a block's distinct tails repeat its first row, the most popular one more
+            // often than not: no pair of theirs is worth a second look
+            const bool col_counts = n < (sh.tcount ? (int)sh.tcount[d] : T);
+            float val[16];
+            uint32_t cancel = 0u, near = 0u;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                val[r] = acc[mi][ni][r];
+                if (DIST == DIST_L2) {
+                    const int m_loc = mb + 8 * (r >> 2) + 4 * hl + (r & 3);
+                    const float ns = na_s[m_loc] + nb_s[nbk + cl];
+                    val[r] = ns - 2.f * val[r];
+                    const bool live = col_counts && m0 + m_loc < B;
+                    if (live && val[r] < kCancelRatio * ns) cancel |= 1u << r;
+                    if (live && val[r] < kNearRatio * ns) near |= 1u << r;
+                }
+            }
+            // rare: the wave recomputes the cancelled pairs directly, two pairs of each of two lanes at
+            // a time, sixteen lanes to a pair
+            if (DIST == DIST_L2 && __ballot(cancel != 0u)) {
+                near = 0u;
+                uint32_t left = cancel;
+                uint64_t owners;
+                while ((owners = __ballot(left != 0u)) != 0) {
+                    const int l0 = __ffsll((long long)owners) - 1;
+                    const uint64_t rest = owners & (owners - 1);
+                    const int l1 = rest ? __ffsll((long long)rest) - 1 : l0;
+                    const int src = lane & 32 ? l1 : l0;
+                    const uint32_t bits = __shfl(left, src, 64), upper = bits & (bits - 1);
+                    const int fr = __ffs((int)((lane & 16) && upper ? upper : bits)) - 1;
+                    const char* ar = a + (int64_t)(mb + 8 * (fr >> 2) + 4 * (src >> 5) + (fr & 3)) * pitch;
+                    const char* br = b + (int64_t)(nbk + (src & 31)) * pitch;
+                    float part = 0.f;
+                    for (int k = (lane & 15) * 4; k < Kp; k += 64) {
+                        const float4 x = load_pieces4(ar, k), y = load_pieces4(br, k);
+                        const float dx = x.x - y.x, dy = x.y - y.y, dz = x.z - y.z, dw = x.w - y.w;
+                        part += dx * dx + dy * dy + dz * dz + dw * dw;
+                    }
+#pragma unroll
+                    for (int o = 8; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
+                    const int at = (lane == l0) ? 0 : 32;
+                    const float v0 = __shfl(part, at, 64), v1 = __shfl(part, at + 16, 64);
+                    if (lane == l0 || lane == l1) {
+                        const uint32_t up = left & (left - 1);
+                        const uint32_t b0 = left ^ up, b1 = up & (0u - up);
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            if ((b0 >> r) & 1u) val[r] = v0;
+                            if ((b1 >> r) & 1u) val[r] = v1;
+                        }
+                        left = up & (up - 1);
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m_loc = mb + 8 * (r >> 2) + 4 * hl + (r & 3);
+                    if (col_counts && m0 + m_loc < B && val[r] < kNearRatio * (na_s[m_loc] + nb_s[nbk + cl])) near |= 1u << r;
+                }
+            }
+            const bool flagged = DIST == DIST_L2 && __ballot(near != 0u) != 0;
+            if (DIST == DIST_L2 && p.nearflag && lane == 0 && m0 + mb < Bp && n0 + nbk < Tp)
+                p.nearflag[((size_t)d * MT + ((m0 + mb) >> 5)) * NT + ((n0 + nbk) >> 5)] = flagged ? 1u : 0u;
+            if (OM != 0) {  // raw scores (and distances)
+                float* const out = p.coef + (size_t)d * B * T;
+                float* const out_d = (DIST == DIST_L2 && p.dist) ? p.dist + (size_t)d * B * T : nullptr;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m0 + mb + 8 * (r >> 2) + 4 * hl + (r & 3);
+                    const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(fmaxf(val[r], 0.f)) : val[r];
+                    if (m < B && n < T) {
+                        out[(size_t)m * T + n] = score_is_distance_value(sh.score_fn) ? dist : sh.gamma - dist;
+                        if (out_d) out_d[(size_t)m * T + n] = dist;
+                    }
+                }
+                continue;
+            }
+            const float mult = n < T ? (sh.tmult ? sh.tmult[(size_t)d * T + n] : 1.f) : 0.f;
+            float c[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m_loc = mb + 8 * (r >> 2) + 4 * hl + (r & 3);
+                const bool live = m0 + m_loc < B && n < T;
+                const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(fmaxf(val[r], 0.f)) : val[r];
+                const float score = score_is_distance_value(sh.score_fn) ? dist : sh.gamma - dist;
+                float ds;
+                const float term = logsigmoid_column(score, (uint32_t)n == label_s[m_loc], mult, w_pos, w_neg, grad_scale, ds);
+                if (live) loss_acc += term;
+                float v = score_is_distance_value(sh.score_fn) ? ds : -ds;
+                if (DIST == DIST_L2) v = dist != 0.f ? v * __builtin_amdgcn_rcpf(dist) : 0.f;
+                c[r] = live ? v : 0.f;
+            }
+            if (flagged) {  // the backward takes this block in the direct form, from the coefficients as they are
+                float* const out = p.coef + (size_t)d * B * T;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m0 + mb + 8 * (r >> 2) + 4 * hl + (r & 3);
+                    if (m < B && n < T) out[(size_t)m * T + n] = c[r];
+                    c[r] = 0.f;
+                }
+            }
+            store_coef_block<DIST>(c, p.out, d, m0 + mb, n0 + nbk, lane);
+        }
+    if (OM == 0) {
+        loss_acc = wave_sum(loss_acc);
+        if (lane == 0) red[wave] = loss_acc;
+        __syncthreads();
+        if (tid == 0) {
+            float tot = 0.f;
+#pragma unroll
+            for (int w = 0; w < WM * WN; ++w) tot += red[w];
+            p.loss_part[(size_t)d * (tile.gx * tile.gy) + tile.y * tile.gx + tile.x] = tot * inv_norm;
+        }
+    }
+}
+
+// --------------------------------------------------------------------------
+// backward.  out[i, k] = sum_j c[i, j] phi(self[i, k], other[j, k]), phi = other (dot) or self - other
+// (L2: self[i, k] sum_j c[i, j] - the product).  Head side: i = heads, the coefficient rows lie along
+// the contraction.  Tail side: i = tails, they lie across it.  `other` always lies across it.
+
+template <int DIST, bool SIDE_B, int TM, int TN, int WM, int WN>
+DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, char* smem, float* csum_s) {
+    using TA = std::conditional_t<SIDE_B, ColTile<TM>, RowTile<TM>>;
+    using P = SplitProduct<TA, ColTile<TN>, TM, TN, WM, WN>;
+    const int i0 = tile_y * TM, kt0 = tile_x * TN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int B = p.B, T = p.T, Bp = p.in.Bp, Tp = p.in.Tp, MT = Bp >> 5, NT = Tp >> 5, pitch = p.Kp * 6;
+    const int t_live = tail_limit(p.tcount, d, T, p.tpad);  // merged tails: the block's live columns
+    const int n_self = SIDE_B ? t_live : B, n_slab = ((SIDE_B ? B : t_live) + 31) >> 5;
+    if (i0 >= n_self) return;
+    const int head0 = d * B, tail0 = p.b_c0 + d * T, self0 = SIDE_B ? tail0 : head0, other0 = SIDE_B ? head0 : tail0;
+    const char* const coef = p.in.coefp + (size_t)d * Bp * Tp * 6;
+    const char* const a = SIDE_B ? coef + (size_t)(i0 >> 5) * 192 : coef + (size_t)i0 * Tp * 6;
+    const char* const other = p.rows + (int64_t)other0 * pitch;
+    const char* const b = other + (size_t)(kt0 >> 5) * 192;
+    const uint32_t* const nflag = DIST == DIST_L2 ? p.nearflag + (size_t)d * MT * NT : nullptr;
+    floatx16 acc[P::AM][P::AN];
+#pragma unroll
+    for (int m = 0; m < P::AM; ++m)
+#pragma unroll
+        for (int n = 0; n < P::AN; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
+    uint32_t seen = 0u;  // flagged blocks among the tile's
+    P::run(smem, a, Tp * 6, SIDE_B ? (size_t)32 * Tp * 6 : 192, b, pitch, (size_t)32 * pitch, n_slab, acc, lane, wave,
+           [&]() __attribute__((always_inline)) {
+               if (DIST != DIST_L2) return;
+               // the self rows' coefficient sums, from the sub-blocks' in a fixed order
+               for (int i = tid; i < TM; i += WM * WN * 64) {
+                   float s = 0.f;
+                   if (SIDE_B) {
+                       if (i0 + i < Tp)
+                           for (int q = 0; q < MT; ++q) s += p.in.colpart[((size_t)d * MT + q) * Tp + i0 + i];
+                   } else if (i0 + i < Bp) {
+                       for (int q = 0; q < n_slab; ++q) s += p.in.rowpart[((size_t)d * Bp + i0 + i) * NT + q];
+                   }
+                   csum_s[i] = s;
+               }
+               for (int x = tid; x < TM / 32 * n_slab; x += WM * WN * 64) {
+                   const int st = (i0 >> 5) + x / n_slab, ot = x % n_slab;
+                   if (SIDE_B ? st < NT : st < MT) seen |= SIDE_B ? nflag[(size_t)ot * NT + st] : nflag[(size_t)st * NT + ot];
+               }
+           });
+    const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
+    const int cl = lane & 31, hl = lane >> 5;
+    const char* const self = p.rows + (int64_t)(self0 + i0) * pitch;
+    if (DIST == DIST_L2 && __syncthreads_or(seen != 0u)) {
+        // slabs in which some pair of a sub-block is nearly identical: c (self - other) directly, as
+        // the reference codelet does (their coefficients went into the product as zeros; acc holds
+        // the negated sum)
+        const float* const cf = p.coef + (size_t)d * B * T;
+#pragma unroll
+        for (int mi = 0; mi < P::AM; ++mi)
+            for (int ot = 0; ot < n_slab; ++ot) {
+                const int st = (i0 + wm + 32 * mi) >> 5;
+                if (st >= (SIDE_B ? NT : MT)) continue;
+                if ((SIDE_B ? nflag[(size_t)ot * NT + st] : nflag[(size_t)st * NT + ot]) == 0u) continue;
+#pragma unroll
+                for (int ni = 0; ni < P::AN; ++ni) {
+                    const int k = kt0 + wn + 32 * ni + cl;
+                    if (kt0 + wn + 32 * ni >= p.Kp) continue;
+                    float sv[16];
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        sv[r] = load_piece1(self + (int64_t)(wm + 32 * mi + 8 * (r >> 2) + 4 * hl + (r & 3)) * pitch, k);
+                    for (int j = 32 * ot; j < min(32 * ot + 32, SIDE_B ? B : t_live); ++j) {
+                        const float o = load_piece1(other + (int64_t)j * pitch, k);
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            const int i = i0 + wm + 32 * mi + 8 * (r >> 2) + 4 * hl + (r & 3);
+                            const float c = i < n_self ? (SIDE_B ? cf[(size_t)j * T + i] : cf[(size_t)i * T + j]) : 0.f;
+                            acc[mi][ni][r] = fmaf(-c, sv[r] - o, acc[mi][ni][r]);
+                        }
+                    }
+                }
+            }
+    }
+    // neighbouring lanes swap values: a lane stores two columns of one row
+    const bool odd = lane & 1;
+    float* const out = p.grad + (size_t)(self0 + i0) * p.Dp;
+#pragma unroll
+    for (int mi = 0; mi < P::AM; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < P::AN; ++ni) {
+            const int k = kt0 + wn + 32 * ni + (cl & ~1);
+            if (k >= p.Dp) continue;
+            const char* const sp = self + (size_t)(k >> 5) * 192 + (k & 31) * 2;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float got = swap1(odd ? acc[mi][ni][2 * i] : acc[mi][ni][2 * i + 1]);
+                float x = odd ? got : acc[mi][ni][2 * i], y = odd ? acc[mi][ni][2 * i + 1] : got;
+                const int row = wm + 32 * mi + 8 * (i >> 1) + 4 * hl + 2 * (i & 1) + odd;
+                if (i0 + row >= n_self) continue;
+                if (DIST == DIST_L2) {
+                    float sx = 0.f, sy = 0.f;
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) {
+                        const uint32_t w = *reinterpret_cast<const uint32_t*>(sp + (int64_t)row * pitch + 64 * q);
+                        sx += bf16_lo_f32(w); sy += bf16_hi_f32(w);
+                    }
+                    x = sx * csum_s[row] - x;
+                    y = sy * csum_s[row] - y;
+                }
+                *reinterpret_cast<float2*>(out + (size_t)row * p.Dp + k) = make_float2(x, y);
+            }
+        }
+}
+
+// Both sides in one launch: the side whose tiles loop over more rows comes first, for every block, so
+// that the long tiles do not start last.  A block's tiles of one side stay together on one XCD.
+template <int DIST, int TM, int TN, int WM, int WN>
+__global__ __launch_bounds__(WM * WN * 64) void k_split_bwd(SplitBwd p) {
+    using PA = SplitProduct<RowTile<TM>, ColTile<TN>, TM, TN, WM, WN>;
+    __shared__ __attribute__((aligned(16))) char smem[PA::kLds];
+    __shared__ float csum_s[TM];
+    const int gx = (p.Dp + TN - 1) / TN, ga = (p.B + TM - 1) / TM, gb = (p.T + TM - 1) / TM;
+    const bool heads_first = p.T >= p.B;
+    const int n_first = gx * (heads_first ? ga : gb) * p.S;
+    const int L = blockIdx.x;
+    if ((L < n_first) == heads_first) {
+        const TileId tile = xcd_tile(gx, ga, p.S, heads_first ? L : L - n_first);
+        split_bwd_tile<DIST, false, TM, TN, WM, WN>(p, tile.z, tile.x, tile.y, smem, csum_s);
+    } else {
+        const TileId tile = xcd_tile(gx, gb, p.S, heads_first ? L - n_first : L);
+        split_bwd_tile<DIST, true, TM, TN, WM, WN>(p, tile.z, tile.x, tile.y, smem, csum_s);
+    }
+}
+
+// --------------------------------------------------------------------------
+// launches
+
+// Tiles of 64 x 64, four waves, three workgroups to a CU: at these sizes a launch is bound by the
+// latency of its slabs and by how many workgroups there are, not by the matrix cores.
+constexpr int kTile = 64;
+
+int split_fwd_parts(const ScoreShape& sh) {
+    return ((sh.T + kTile - 1) / kTile) * ((sh.B + kTile - 1) / kTile);
+}
+
+void launch_split_fwd(const SplitFwd& p, bool fused_loss, hipStream_t stream) {
+    const ScoreShape& sh = p.sh;
+    const dim3 grid = tile_grid((sh.T + kTile - 1) / kTile, (sh.B + kTile - 1) / kTile, sh.S);
+    const bool l2 = sh.dist_fn == DIST_L2 && sh.score_fn != SCORE_DISTMULT;
+#define KGE_FWD(D_, OM_) hipLaunchKernelGGL((k_split_fwd<D_, OM_, kTile, kTile, 2, 2>), grid, dim3(256), 0, stream, p)
+    if (l2) { if (fused_loss) KGE_FWD(DIST_L2, 0); else KGE_FWD(DIST_L2, 1); }
+    else    { if (fused_loss) KGE_FWD(DIST_DOT, 0); else KGE_FWD(DIST_DOT, 1); }
+#undef KGE_FWD
+}
+
+void launch_coef_pieces(const ScoreShape& sh, const float* coef, const uint32_t* nearflag, const SplitCoef& out,
+                        hipStream_t stream) {
+    const int n = sh.S * (out.Bp / 32) * (out.Tp / 32);
+    const bool l2 = sh.dist_fn == DIST_L2 && sh.score_fn != SCORE_DISTMULT;
+    if (l2) hipLaunchKernelGGL(k_coef_pieces<DIST_L2>, dim3((n + 3) / 4), dim3(256), 0, stream, sh, coef, nearflag, out);
+    else hipLaunchKernelGGL(k_coef_pieces<DIST_DOT>, dim3((n + 3) / 4), dim3(256), 0, stream, sh, coef, nearflag, out);
+}
+
+void launch_split_bwd(const SplitBwd& p, bool l2, hipStream_t stream) {
+    const dim3 grid(((p.Dp + kTile - 1) / kTile) * ((p.B + kTile - 1) / kTile + (p.T + kTile - 1) / kTile) * p.S);
+    if (l2) hipLaunchKernelGGL((k_split_bwd<DIST_L2, kTile, kTile, 2, 2>), grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((k_split_bwd<DIST_DOT, kTile, kTile, 2, 2>), grid, dim3(256), 0, stream, p);
+}
+
+// Where these kernels are taken.  At whole 128-row tiles and enough of them the kernels that split
+// float32 operands while staging are as fast or faster (22.8M-row workload, 64 blocks of 256 x 512:
+// forward 40 against 42 us, backward 57 against 67, and the gather writes a third less): the
+// piece matrices cost half as much memory traffic again, and with that many tiles the
+// staging's vector work hides behind other workgroups' matrix work.  Elsewhere - ragged sizes, which
+// those kernels take with bounds checks and float32 matrix instructions, and few tiles - these
+// are the faster ones: one block of 256 x 64, D = 64: forward 11.2 -> 10.5 us, backward 37 -> 12;
+// four of 200 x 268, D = 100: 17.4 -> 7.8 and 49 -> 10.6.
+bool split_scoring(const ScoreShape& sh) {
+    if (sh.use_mfma != 2 || sh.score_fn == SCORE_TRANSH) return false;
+    if (sh.dist_fn == DIST_L1 && sh.score_fn != SCORE_DISTMULT) return false;
+    const bool whole = sh.B % 128 == 0 && sh.T % 128 == 0 && sh.Dp % 64 == 0;
+    return !whole || (int64_t)sh.S * (sh.B / 128) * (sh.T / 64) < 128;
+}
+
+}  // namespace kge

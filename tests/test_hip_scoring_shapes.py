@@ -24,3 +24,20 @@ pytestmark = pytest.mark.gpu
 def test_l1_shapes(oracle64, S, B, A, D, merge):
     run_case(oracle64, dict(distance_fn="L1", n_shard=S, batch=B, a2a=A, dim=D, feature=0, n_entity=4000,
                             n_relation=16, gamma=4.0), n_step=2, **{"execution.merge_tails": merge})
+
+
+# L2 and dot on three-piece operands: tiles of 64 x 64 over slabs of 32, matrices filled up to 32
+@pytest.mark.parametrize("merge", [True, False])
+@pytest.mark.parametrize("score_fn,distance_fn", [("TransE", "L2"), ("DistMult", "MatMul"), ("ComplEx", "L2")])
+@pytest.mark.parametrize("loss_fn", ["logsigmoid", "softmax"])
+@pytest.mark.parametrize("S,B,A,D", [
+    (1, 1, 2, 2),         # one pair of rows and two columns
+    (1, 31, 33, 30),      # around one 32 x 32 sub-block
+    (2, 64, 32, 32),      # exactly a tile, exactly a slab
+    (1, 65, 97, 66),      # one over a tile, a sub-block and two slabs
+    (3, 130, 43, 100),    # several tiles, none of them whole
+    (2, 128, 64, 64),     # whole tiles, few of them
+])
+def test_l2_and_dot_shapes(oracle64, score_fn, distance_fn, loss_fn, S, B, A, D, merge):
+    run_case(oracle64, dict(score_fn=score_fn, distance_fn=distance_fn, loss_fn=loss_fn, n_shard=S, batch=B, a2a=A, dim=D,
+                            feature=0, n_entity=1500, n_relation=6, gamma=4.0), n_step=2, **{"execution.merge_tails": merge})
