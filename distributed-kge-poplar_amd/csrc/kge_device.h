@@ -154,7 +154,7 @@ DEVINL TileId xcd_tile(int gx, int gy, int gz, int L) {
     return id;
 }
 DEVINL TileId xcd_tile(int gx, int gy, int gz) { return xcd_tile(gx, gy, gz, (int)blockIdx.x); }
-static dim3 tile_grid(int gx, int gy, int gz) { return dim3((unsigned)(gx * gy * gz)); }
+static inline dim3 tile_grid(int gx, int gy, int gz) { return dim3((unsigned)(gx * gy * gz)); }
 
 
 // f(integral_constant<0>) ... f(integral_constant<N-1>): a loop whose index is a compile-time constant

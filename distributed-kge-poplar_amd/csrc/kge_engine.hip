@@ -276,6 +276,11 @@ struct kge_engine {
     int Kp = 0, Bp = 0, Tp = 0;
     DevBuf<char> rowsp, coefp;
     DevBuf<float> row_norm, rowpart, colpart;
+    // feature products on pieces (kge_feature.hip): W of every network as a piece matrix, kept by
+    // the update and formed afresh after a write from outside
+    bool split_feat = false, proj_pieces_fresh = false;
+    size_t proj_pieces_bytes = 0;  // of one network's
+    DevBuf<char> projp;
     DevBuf<float> bwd_pieces;  // split sums of the scoring backward
     DevBuf<float> coef, dist, grad, opnd, partial, rel_partial, rel_gsum, hidden, gsum, gproj, featd, gproj_part, gemm_part, projR, loss_part, loss_step, d_alpha;
     // [n_step][entity, relation, normal, then per feature network projection, mlp up, mlp down][S]; the relation update indexes its two
@@ -729,8 +734,13 @@ void allocate(kge_engine& E) {
         if (roles) E.role_idx.alloc(R);
         E.gsum.alloc(E.nets * R * E.Dp);
         E.gsum.zero(E.stream);  // rows past a step's distinct count are read (times zero): keep them finite
-        E.featd.alloc(R * E.Fp);
-        E.gproj_part.alloc((size_t)16 * E.Fp * E.Dp);
+        E.split_feat = E.use_mfma == 2 && !E.score_bf16;
+        if (E.split_feat) {
+            E.proj_pieces_bytes = split_bytes(round_up(E.Fp, 32), E.Dp);
+            E.projp.alloc(E.nets * E.proj_pieces_bytes);
+            E.projp.zero(st);  // rows behind the last feature meet zeros
+        } else E.featd.alloc(R * E.Fp);
+        E.gproj_part.alloc((size_t)(E.split_feat ? feature_grad_parts((int)R, E.Fp, E.Dp) : 16) * E.Fp * E.Dp);
         if (E.score_bf16) {
             E.feat16.alloc(R * E.Fp);
             E.projR.alloc((size_t)E.Fp * E.Dp);
@@ -885,6 +895,7 @@ void run_read_write(kge_engine& E, bool write, const Items& in) {
         move(dev + Dp * M, M, host + D * M, D);
         return;
     }
+    if (write && buf == &E.proj) E.proj_pieces_fresh = false;
     move(buf->p + row0 * E.Dp, E.Dp, host, rows);
 }
 
@@ -1115,6 +1126,15 @@ void run_plan(kge_engine& E, int s0, int sn, hipStream_t st) {
     HIP_CHECK(hipGetLastError());
 }
 
+// W as pieces, unless they are what the last update left
+static void refresh_proj_pieces(kge_engine& E, hipStream_t st) {
+    if (!E.split_feat || E.proj_pieces_fresh) return;
+    for (int net = 0; net < E.nets; ++net)
+        launch_split_matrix(E.proj.p + (size_t)net * E.Fp * E.Dp, E.Fp, E.Dp, round_up(E.Dp, 32),
+                            E.projp.p + net * E.proj_pieces_bytes, st);
+    E.proj_pieces_fresh = true;
+}
+
 // how the gather combines a head row with its relation row (launch_gather_operands)
 static int rel_mode_of(const kge_engine& E) {
     if (E.score_fn == SCORE_TRANSH) return 0;  // launch_transh_predict turns the copied head rows into p
@@ -1175,6 +1195,7 @@ void run_step(kge_engine& E, int i) {
             f.featd = E.featd.p; f.gproj_part = E.gproj_part.p; f.use_mfma = E.use_mfma;
             f.round_bf16 = E.score_bf16 ? 1 : 0; f.projR = E.projR.p;
             f.feat16 = E.feat16.p;
+            f.wp = E.split_feat ? E.projp.p + net * E.proj_pieces_bytes : nullptr;
             FeatureArgs fp = f;  // the feature part alone, without the embedding
             fp.emb_base = nullptr;
             float* hid = E.hidden.p + net * rows_n;          // value + feature part
@@ -1501,11 +1522,12 @@ void run_step(kge_engine& E, int i) {
     // [s*rows/S, (s+1)*rows/S) (the last one also the padding rows behind them) and its step size
     // (group `group` of this step's step sizes)
     auto dense_adam = [&](float* p, float* m, float* v, const float* g, int rows, int last_row, int64_t width,
-                          int group) {
+                          int group, int n_part = 1, void* pieces = nullptr) {
         AdamArgs af = aa;
         af.alpha = alpha + (size_t)group * E.S;
         const int n_slices = E.shared_table ? 1 : E.S;
-        launch_adam_slices(p, m, v, g, last_row * width, std::max(1, rows / n_slices) * width, n_slices, af, st);
+        launch_adam_slices(p, m, v, g, n_part, last_row * width, std::max(1, rows / n_slices) * width, n_slices, af, pieces,
+                           (int)width, st);
     };
     for (int net = 0; net < nets && E.F; ++net) {
         const float* g_rows = E.gsum.p + net * rows_n;  // d loss / d (feature part) per distinct row
@@ -1537,10 +1559,14 @@ void run_step(kge_engine& E, int i) {
             g_rows = E.mlp_gfp.p + net * rows_n;  // the projected features' gradient
         }
         const size_t proj_o = (size_t)net * E.Fp * E.Dp;
-        { KernelTimer t(E, K_PROJ_GRAD); launch_proj_grad(fa[net], g_rows, E.gproj.p + proj_o, st); }
+        const int n_part = E.split_feat ? feature_grad_parts((int)R, E.Fp, E.Dp) : 1;
+        { KernelTimer t(E, K_PROJ_GRAD);
+          if (E.split_feat) launch_feature_grad(fa[net], g_rows, E.gproj_part.p, n_part, st);
+          else launch_proj_grad(fa[net], g_rows, E.gproj.p + proj_o, st); }
         KernelTimer t(E, K_ADAM_PROJ);
-        dense_adam(E.proj.p + proj_o, E.proj_m.p + proj_o, E.proj_v.p + proj_o, E.gproj.p + proj_o, E.F, E.Fp, E.Dp,
-                   3 + 3 * net);
+        dense_adam(E.proj.p + proj_o, E.proj_m.p + proj_o, E.proj_v.p + proj_o,
+                   E.split_feat ? E.gproj_part.p : E.gproj.p + proj_o, E.F, E.Fp, E.Dp, 3 + 3 * net, n_part,
+                   E.split_feat ? E.projp.p + net * E.proj_pieces_bytes : nullptr);
     }
     HIP_CHECK(hipGetLastError());
 }
@@ -1592,6 +1618,7 @@ void run_train_step_loop(kge_engine& E, const Items& in) {
     std::memcpy(E.h_alpha_pin, E.h_alpha.data(), E.h_alpha.size() * 4);
     HIP_CHECK(hipMemcpyAsync(E.d_alpha.p, E.h_alpha_pin, E.h_alpha.size() * 4, hipMemcpyHostToDevice, st));
     HIP_CHECK(hipEventRecord(E.ev[1], st));
+    refresh_proj_pieces(E, st);
     E.step_of_first = (int)E.step - s0;  // step i of the batch is optimiser step E.step + (i - s0)
     // the per-step counts (distinct rows, chunks, rows with chunks, biggest row) size the launches of
     // calls long enough to pay for the wait; the segment kernel writes them into pinned host memory
@@ -1903,7 +1930,7 @@ void run_predict(kge_engine& E, const Items& in) {
         E.p_best_i.alloc((size_t)Q * nb);
         if (E.F) {
             E.p_hidden.alloc((size_t)std::max(Qp, chunk) * Dp);
-            E.p_featd.alloc((size_t)std::max(Qp, chunk) * E.Fp);
+            if (!E.split_feat) E.p_featd.alloc((size_t)std::max(Qp, chunk) * E.Fp);
             if (E.mlp) {
                 E.p_fproj.alloc((size_t)std::max(Qp, chunk) * Dp);
                 E.p_concat.alloc((size_t)std::max(Qp, chunk) * 2 * Dp);
@@ -1931,6 +1958,7 @@ void run_predict(kge_engine& E, const Items& in) {
         const uint32_t counts[2] = {(uint32_t)Qp, (uint32_t)chunk};
         HIP_CHECK(hipMemcpy(E.p_count.p, counts, sizeof(counts), hipMemcpyHostToDevice));
     }
+    refresh_proj_pieces(E, st);
     // rows `idx[0..n)` of the table as a row source: the embeddings, or hidden = emb + feature . W
     // (`net`: the head's feature network for the queries, the tail's for the candidates)
     auto rows_of = [&](const uint32_t* idx, int n, int net) {
@@ -1946,6 +1974,7 @@ void run_predict(kge_engine& E, const Items& in) {
             fa.emb_etype = E.L.emb_etype; fa.feat_etype = E.L.feat_etype;
             fa.Dp = Dp; fa.Fp = E.Fp; fa.proj = E.proj.p + (size_t)net * E.Fp * Dp;
             fa.featd = E.p_featd.p; fa.use_mfma = E.use_mfma;
+            fa.wp = E.split_feat ? E.projp.p + net * E.proj_pieces_bytes : nullptr;
             if (E.mlp) {
                 FeatureArgs fp = fa;
                 fp.emb_base = nullptr;

@@ -1,0 +1,357 @@
+// gfx950 kernels of the feature projection (src/poplar_kge.cpp:451-462): hidden = embedding + feature . W
+// for the distinct rows, and dW = feature^T . gradient.
+//
+// Both are float32 products formed from bfloat16 matrix instructions.  A feature stored in 16 bits is
+// exactly two bfloat16 pieces (float16: 8 + 3 significant bits) or one (bfloat16), W and the
+// gradient are three; the products of pieces below 2^-24 of the result are left out: five, three or
+// (float32 features) six instructions per sixteen contraction steps.  The features are read where they
+// lie, in the table, and split while they are staged: no dense copy of them is made.
+#include "kge_split.h"
+
+#include <algorithm>
+#include <cstdint>
+
+namespace kge {
+
+template <int FT> struct Pieces { static constexpr int n = FT == ET_F16 ? 2 : FT == ET_BF16 ? 1 : 3; };
+
+// eight consecutive features, as they lie
+template <int FT> struct Raw8 { uint4 v[FT == ET_F32 ? 2 : 1]; };
+template <int FT>
+DEVINL void load_raw8(Raw8<FT>& r, const char* row, int f, int Fp) {  // features f .. f + 7, zero from Fp on (Fp % 4 == 0, 16-bit: % 8)
+    constexpr int half = FT == ET_F32 ? 4 : 8;
+#pragma unroll
+    for (int h = 0; h < 8 / half; ++h)
+        r.v[h] = f + half * h < Fp ? *reinterpret_cast<const uint4*>(row + (size_t)(f + half * h) * (FT == ET_F32 ? 4 : 2))
+                                   : make_uint4(0u, 0u, 0u, 0u);
+}
+// -> piece q of the eight, for every piece
+template <int FT>
+DEVINL void split_raw8(const Raw8<FT>& r, uint4 (&piece)[Pieces<FT>::n]) {
+    if constexpr (FT == ET_BF16) {
+        piece[0] = r.v[0];
+    } else {
+        float x[8];
+        if constexpr (FT == ET_F32) {
+            const uint32_t w[8] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w, r.v[1].x, r.v[1].y, r.v[1].z, r.v[1].w};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[i] = __uint_as_float(w[i]);
+        } else {
+            const uint32_t w[4] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&w[i]));
+                x[2 * i] = f.x; x[2 * i + 1] = f.y;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < Pieces<FT>::n; ++q) {
+            uint32_t w[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                w[i] = pack_bf16(x[2 * i], x[2 * i + 1]);
+                if (q + 1 < Pieces<FT>::n) { x[2 * i] -= bf16_lo_f32(w[i]); x[2 * i + 1] -= bf16_hi_f32(w[i]); }
+            }
+            piece[q] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    }
+}
+
+// the products of one sixteen-step: AM accumulators, one fragment column of the other operand,
+// smallest terms first
+template <int PA, int AM>
+DEVINL void feature_products(const floatx4 (&fa)[AM][PA], const floatx4 (&fb)[3], floatx16 (&acc)[AM]) {
+    constexpr int n = PA == 3 ? 6 : PA == 2 ? 5 : 3;
+    constexpr int qa[6] = {PA == 3 ? 0 : PA == 2 ? 1 : 0, PA == 3 ? 2 : 0, PA == 3 ? 1 : PA == 2 ? 1 : 0, 0, PA == 3 ? 1 : 0, 0};
+    constexpr int qb[6] = {PA == 3 ? 2 : PA == 2 ? 1 : 2, PA == 3 ? 0 : PA == 2 ? 2 : 1, PA == 3 ? 1 : 0, 1, 0, 0};
+#pragma unroll
+    for (int x = 0; x < n; ++x)
+#pragma unroll
+        for (int m = 0; m < AM; ++m)
+            acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[m][qa[x]]),
+                                                             __builtin_bit_cast(bf16x8, fb[qb[x]]), acc[m], 0, 0, 0);
+}
+
+// hidden.  A workgroup of NW waves takes 32 AM rows x 32 NW columns, every wave all of the rows and 32 of
+// the columns: with D <= 256 a row's features come from memory once.  W lies as a piece matrix
+// (launch_split_matrix) and goes straight into LDS.
+template <int FT, int AM, int NW>
+__global__ __launch_bounds__(NW * 64) void k_feature_fwd(FeatureArgs a, const char* __restrict__ wp, int w_pitch,
+                                                         float* __restrict__ hidden) {
+    constexpr int PA = Pieces<FT>::n, TM = 32 * AM, TN = 32 * NW, NT = NW * 64;
+    constexpr int NC = (TM * 4 + NT - 1) / NT;  // 16-byte chunks of a slab per thread
+    // Slabs whose features are asked for together: a row of the table is a round trip of microseconds
+    // (and its loads hold up the copies behind them: they return in order), so it is paid once for
+    // 768 16-bit features, not once per slab (94 us for 24k rows of 768 features and 256 columns).
+    constexpr int KS = (FT == ET_F32 ? 12 : 24) / NC;
+    using TA = RowTile<TM>;
+    using TB = ColTile<TN>;
+    constexpr int kA = PA * TM * 64, kStage = kA + TB::kBytes, kEach = TB::kCopies / NW;
+    __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
+    __shared__ uint32_t key_s[TM];
+    const int gx = (a.Dp + TN - 1) / TN;
+    const int u0 = (int)blockIdx.x / gx * TM, n0 = (int)blockIdx.x % gx * TN;
+    const int U = (int)a.counts[0];
+    if (u0 >= U) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (int i = tid; i < TM; i += NT) key_s[i] = a.uniq_key[min(u0 + i, U - 1)];
+    __syncthreads();
+    const char* src[NC];
+    int dst[NC], kc[NC];
+    bool on[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int c = tid + NT * i, row = min(c >> 2, TM - 1);
+        on[i] = TM * 4 % NT == 0 || c < TM * 4;
+        kc[i] = (c & 3) * 8;
+        src[i] = a.feat_base + (int64_t)key_s[row] * a.pitch;
+        dst[i] = row * 64 + ((c & 3) ^ ((row >> 2) & 3)) * 16;
+    }
+    uint32_t off[kEach];
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) off[i] = TB::source(wave + NW * i, lane, w_pitch);
+    const char* const w0 = wp + (size_t)(n0 >> 5) * 192;
+    const uint32_t lds0 = lds_address(smem) + kA;
+    auto fill = [&](int slab) __attribute__((always_inline)) {
+        const char* from = w0 + (size_t)slab * 32 * w_pitch;
+#pragma unroll
+        for (int i = 0; i < kEach; ++i) lds_copy16(from, off[i], lds0 + (slab & 1) * kStage + (wave + NW * i) * 1024);
+    };
+    const int n_slab = (a.Fp + 31) / 32;
+    fill(0);
+    // the embeddings are what the accumulators start from: fetched after the loop, a chain of two round
+    // trips at a time, they took as long as the product (24k rows: 99 us, 55 without them)
+    const int k = n0 + 32 * wave + (lane & 31);
+    floatx16 acc[AM];
+    const bool add = a.emb_base && k < a.Dp, wide = a.emb_etype == ET_F32;
+    const char* const col = a.emb_base + (add ? k : 0) * (wide ? 4 : 2);
+#pragma unroll
+    for (int m = 0; m < AM; ++m)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {  // as they lie: a conversion here would wait for each load
+            const char* at = col + (int64_t)key_s[32 * m + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)] * a.pitch;
+            acc[m][r] = !add ? 0.f : wide ? *reinterpret_cast<const float*>(at) : __uint_as_float(*reinterpret_cast<const uint16_t*>(at));
+        }
+    if (!wide)
+#pragma unroll
+        for (int m = 0; m < AM; ++m)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint16_t raw = (uint16_t)__float_as_uint(acc[m][r]);
+                acc[m][r] = load1(reinterpret_cast<const char*>(&raw), 0, a.emb_etype);
+            }
+    for (int s0 = 0; s0 < n_slab; s0 += KS) {
+        Raw8<FT> raw[KS][NC];
+#pragma unroll
+        for (int x = 0; x < KS; ++x)
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+                if (on[i]) load_raw8<FT>(raw[x][i], src[i], 32 * (s0 + x) + kc[i], a.Fp);
+        static_for<KS>([&](auto xc) __attribute__((always_inline)) {
+            constexpr int x = decltype(xc)::value;
+            const int slab = s0 + x;
+            if (slab >= n_slab) return;
+            // (a tile copy was last read two slabs ago, before the barrier of the slab in between)
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+                if (on[i]) {
+                    uint4 piece[PA];
+                    split_raw8<FT>(raw[x][i], piece);
+#pragma unroll
+                    for (int q = 0; q < PA; ++q)
+                        *reinterpret_cast<uint4*>(smem + (slab & 1) * kStage + q * (TM * 64) + dst[i]) = piece[q];
+                }
+            wait_copies_and_barrier<0>();
+            if (slab + 1 < n_slab) fill(slab + 1);
+            const char* ta = smem + (slab & 1) * kStage;
+            const char* tb = ta + kA;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                floatx4 fa[AM][PA], fb[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) fb[q] = TB::fragment(tb, q, 32 * wave, ks, lane);
+#pragma unroll
+                for (int m = 0; m < AM; ++m)
+#pragma unroll
+                    for (int q = 0; q < PA; ++q) fa[m][q] = TA::fragment(ta, q, 32 * m, ks, lane);
+                feature_products<PA, AM>(fa, fb, acc);
+            }
+        });
+    }
+    if (k >= a.Dp) return;
+#pragma unroll
+    for (int m = 0; m < AM; ++m)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int u = u0 + 32 * m + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            if (u < U) hidden[(size_t)u * a.Dp + k] = acc[m][r];
+        }
+}
+
+// dW.  A workgroup takes 32 AM features x 32 NW columns over its share of the rows (the output has
+// few tiles: the contraction is split, the parts are added up by the update's kernel).  Both
+// operands lie across the contraction and are split while staged.
+template <int FT, int AM, int NW>
+__global__ __launch_bounds__(NW * 64) void k_feature_grad(FeatureArgs a, const float* __restrict__ grad, int n_split,
+                                                          float* __restrict__ part) {
+    constexpr int PA = Pieces<FT>::n, TM = 32 * AM, TN = 32 * NW, NT = NW * 64;
+    static_assert(TM == 128 || TM == 64, "ColTile");
+    constexpr int NA = (32 * TM / 8 + NT - 1) / NT, NB = 32 * TN / 4 / NT;
+    using TA = ColTile<TM>;
+    using TB = ColTile<TN>;
+    constexpr int kA = PA * 32 * TM * 2, kStage = kA + TB::kBytes;
+    __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
+    const int gx = (a.Dp + TN - 1) / TN, gy = (a.Fp + TM - 1) / TM;
+    const int split = (int)blockIdx.x / (gx * gy), t = (int)blockIdx.x % (gx * gy), f0 = t / gx * TM, n0 = t % gx * TN;
+    const int U = (int)a.counts[0];
+    const int share = ((U + n_split - 1) / n_split + 31) & ~31;
+    const int ub = split * share, ue = min(U, ub + share), n_slab = ue > ub ? (ue - ub + 31) / 32 : 0;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    floatx16 acc[AM];
+#pragma unroll
+    for (int m = 0; m < AM; ++m)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[m][r] = 0.f;
+    uint32_t key[NA];       // the next slab's rows
+    Raw8<FT> raw[NA];
+    float4 g[NB];
+    auto row_a = [&](int i) { return (tid + NT * i) / (TM / 8); };
+    auto keys = [&](int slab) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) key[i] = a.uniq_key[min(ub + 32 * slab + row_a(i), ue - 1)];
+    };
+    auto load = [&](int slab) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+            load_raw8<FT>(raw[i], a.feat_base + (int64_t)key[i] * a.pitch, f0 + (tid + NT * i) % (TM / 8) * 8,
+                          ub + 32 * slab + row_a(i) < ue ? a.Fp : 0);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int x = tid + NT * i, u = ub + 32 * slab + x / (TN / 4), k = n0 + x % (TN / 4) * 4;
+            g[i] = k < a.Dp ? *reinterpret_cast<const float4*>(grad + (size_t)min(u, ue - 1) * a.Dp + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    auto stage = [&](int slab) __attribute__((always_inline)) {
+        char* const to = smem + (slab & 1) * kStage;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const int row = row_a(i), chunk = (tid + NT * i) % (TM / 8);
+            if (NT * NA != 32 * TM / 8 && row >= 32) continue;
+            uint4 piece[PA];
+            split_raw8<FT>(raw[i], piece);
+#pragma unroll
+            for (int q = 0; q < PA; ++q)
+                *reinterpret_cast<uint4*>(to + q * (32 * TM * 2) + row * (2 * TM) + (chunk ^ ((row & TA::kKey) << 2)) * 16) = piece[q];
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int x = tid + NT * i, row = x / (TN / 4), c4 = x % (TN / 4);
+            uint2 piece[3];
+            split4_bf16(as_x4(g[i]), piece);
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                *reinterpret_cast<uint2*>(to + kA + q * (32 * TN * 2) + row * (2 * TN) + ((c4 >> 1) ^ ((row & TB::kKey) << 2)) * 16 +
+                                          (c4 & 1) * 8) = piece[q];
+        }
+    };
+    if (n_slab > 0) {
+        keys(0);
+        load(0);
+        keys(1);
+        stage(0);
+        load(min(1, n_slab - 1));
+        keys(2);
+    }
+    for (int slab = 0; slab < n_slab; ++slab) {
+        __syncthreads();
+        if (slab + 1 < n_slab) {
+            stage(slab + 1);
+            load(slab + 2);  // (past the end: the last row again, its features as zeros)
+            keys(slab + 3);
+        }
+        const char* ta = smem + (slab & 1) * kStage;
+        const char* tb = ta + kA;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            floatx4 fa[AM][PA], fb[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) fb[q] = TB::fragment(tb, q, 32 * wave, ks, lane);
+#pragma unroll
+            for (int m = 0; m < AM; ++m)
+#pragma unroll
+                for (int q = 0; q < PA; ++q) fa[m][q] = TA::fragment(ta, q, 32 * m, ks, lane);
+            feature_products<PA, AM>(fa, fb, acc);
+        }
+    }
+    const int k = n0 + 32 * wave + (lane & 31);
+    if (k >= a.Dp) return;
+    float* const out = part + (size_t)split * a.Fp * a.Dp;
+#pragma unroll
+    for (int m = 0; m < AM; ++m)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int f = f0 + 32 * m + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            if (f < a.Fp) out[(size_t)f * a.Dp + k] = acc[m][r];
+        }
+}
+
+// float32 rows -> piece matrix
+__global__ __launch_bounds__(256) void k_split_matrix(const float* __restrict__ in, int rows, int Dp, int Kp, char* __restrict__ out) {
+    const int per_row = Kp / 4, i = blockIdx.x * 256 + threadIdx.x, row = i / per_row, k = (i - row * per_row) * 4;
+    if (row >= rows) return;
+    store_pieces4(out + (size_t)row * Kp * 6, k, k < Dp ? *reinterpret_cast<const float4*>(in + (size_t)row * Dp + k) : make_float4(0.f, 0.f, 0.f, 0.f));
+}
+void launch_split_matrix(const float* in, int rows, int Dp, int Kp, void* out, hipStream_t stream) {
+    if (rows == 0) return;
+    hipLaunchKernelGGL(k_split_matrix, dim3((unsigned)(((int64_t)rows * (Kp / 4) + 255) / 256)), dim3(256), 0, stream, in, rows, Dp, Kp, (char*)out);
+}
+
+// columns per workgroup: the whole width up to 256
+static int feature_waves(int Dp) { return Dp > 128 ? 8 : Dp > 64 ? 4 : 2; }
+
+void launch_feature_fwd(const FeatureArgs& a, float* hidden, hipStream_t stream) {
+    const int nw = feature_waves(a.Dp), gx = (a.Dp + 32 * nw - 1) / (32 * nw), w_pitch = (a.Dp + 31) / 32 * 192;
+    // rows per workgroup: a workgroup of eight waves fills a CU, so the tile height is the one with the
+    // fewest rows per CU over all rounds (24k rows: 96, one round of 250)
+    int am = 1;
+    int64_t best = INT64_MAX;
+    const int slots = 256 * (8 / nw);
+    for (int t = 1; t <= 4; ++t) {
+        const int64_t tiles = (int64_t)((a.max_rows + 32 * t - 1) / (32 * t)) * gx;
+        const int64_t cost = (tiles + slots - 1) / slots * (2 + 3 * t);  // (a tile's W slabs cost as much as some rows)
+        if (cost < best) { best = cost; am = t; }
+    }
+    const dim3 grid((unsigned)(((a.max_rows + 32 * am - 1) / (32 * am)) * gx));
+#define KGE_FF(F_, A_, W_) hipLaunchKernelGGL((k_feature_fwd<F_, A_, W_>), grid, dim3(W_ * 64), 0, stream, a, (const char*)a.wp, w_pitch, hidden)
+#define KGE_FF_A(F_, W_)                                                                             \
+    do {                                                                                             \
+        if (am == 1) KGE_FF(F_, 1, W_); else if (am == 2) KGE_FF(F_, 2, W_);                         \
+        else if (am == 3) KGE_FF(F_, 3, W_); else KGE_FF(F_, 4, W_);                                 \
+    } while (0)
+#define KGE_FF_W(F_) do { if (nw == 8) KGE_FF_A(F_, 8); else if (nw == 4) KGE_FF_A(F_, 4); else KGE_FF_A(F_, 2); } while (0)
+    if (a.feat_etype == ET_F16) KGE_FF_W(ET_F16);
+    else if (a.feat_etype == ET_BF16) KGE_FF_W(ET_BF16);
+    else KGE_FF_W(ET_F32);
+#undef KGE_FF
+#undef KGE_FF_A
+#undef KGE_FF_W
+}
+
+// parts of the split contraction: as many as give every CU a workgroup, none with less than four slabs
+int feature_grad_parts(int max_rows, int Fp, int Dp) {
+    const int nw = feature_waves(Dp), tiles = ((Fp + 127) / 128) * ((Dp + 32 * nw - 1) / (32 * nw));
+    return std::max(1, std::min({256 * (8 / nw) / tiles, max_rows / 128, kFeatureGradParts}));
+}
+void launch_feature_grad(const FeatureArgs& a, const float* grad_rows, float* part, int n_part, hipStream_t stream) {
+    const int nw = feature_waves(a.Dp);
+    const dim3 grid((unsigned)(((a.Fp + 127) / 128) * ((a.Dp + 32 * nw - 1) / (32 * nw)) * n_part));
+#define KGE_FG(F_, W_) hipLaunchKernelGGL((k_feature_grad<F_, 4, W_>), grid, dim3(W_ * 64), 0, stream, a, grad_rows, n_part, part)
+#define KGE_FG_W(F_) do { if (nw == 8) KGE_FG(F_, 8); else if (nw == 4) KGE_FG(F_, 4); else KGE_FG(F_, 2); } while (0)
+    if (a.feat_etype == ET_F16) KGE_FG_W(ET_F16);
+    else if (a.feat_etype == ET_BF16) KGE_FG_W(ET_BF16);
+    else KGE_FG_W(ET_F32);
+#undef KGE_FG
+#undef KGE_FG_W
+}
+
+}  // namespace kge

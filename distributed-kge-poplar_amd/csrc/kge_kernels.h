@@ -438,7 +438,16 @@ struct FeatureArgs {
     uint16_t* feat16;
     int round_bf16;         // features and W enter their products rounded to bfloat16
     float* projR;           // scratch [Fp, Dp]: W rounded, for the float32 kernels
+    const void* wp;         // W as a piece matrix (launch_split_matrix), or null: the kernels below without it
 };
+// float32 rows [rows, Dp] -> piece matrix of Kp columns
+void launch_split_matrix(const float* in, int rows, int Dp, int Kp, void* out, hipStream_t stream);
+// the two feature products on pieces (kge_feature.hip; a.wp): the second one's contraction comes in
+// `n_part` parts [n_part][Fp, Dp] to be added up (feature_grad_parts, at most kFeatureGradParts)
+constexpr int kFeatureGradParts = 64;
+int feature_grad_parts(int max_rows, int Fp, int Dp);
+void launch_feature_fwd(const FeatureArgs& a, float* hidden, hipStream_t stream);
+void launch_feature_grad(const FeatureArgs& a, const float* grad_rows, float* part, int n_part, hipStream_t stream);
 void launch_hidden_fwd(const FeatureArgs& a, float* hidden, hipStream_t stream);
 // gproj[f, :] = sum_u feature[u, f] * grad_rows[u, :]
 void launch_proj_grad(const FeatureArgs& a, const float* grad_rows, float* gproj,
@@ -485,9 +494,11 @@ void launch_distance_grad(int dist_fn, const float* a, const float* b, const flo
 void launch_adam_flat(float* p, float* m, float* v, const float* g, int64_t n, float alpha,
                       float beta_m, float beta_v, float epsilon, float weight_decay, int v_is_sqrt,
                       hipStream_t stream);
-// Adam on n elements of which slices of `slice` have step sizes of their own (a.alpha); n, slice % 4 == 0
-void launch_adam_slices(float* p, float* m, float* v, const float* g, int64_t n, int64_t slice, int n_slices,
-                        const AdamArgs& a, hipStream_t stream);
+// Adam on n elements of which slices of `slice` have step sizes of their own (a.alpha); n, slice % 4 == 0.
+// The gradient is the sum of n_part arrays of n.  pieces (or null): the updated parameter, rows of
+// `width`, once more as a piece matrix.
+void launch_adam_slices(float* p, float* m, float* v, const float* g, int n_part, int64_t n, int64_t slice, int n_slices,
+                        const AdamArgs& a, void* pieces, int width, hipStream_t stream);
 void launch_fill_u32(uint32_t* p, uint32_t value, int64_t n, hipStream_t stream);
 void launch_iota_keys(const uint32_t* idx, uint32_t* keys, uint32_t* vals, int64_t n, int64_t rows,
                       hipStream_t stream);

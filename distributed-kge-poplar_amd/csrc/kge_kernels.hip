@@ -11,6 +11,7 @@
 //                  (src/fructose/frnn.cpp:61-90, src/poplar_kge.cpp:695-704)
 #include "kge_device.h"
 #include "kge_loss.h"
+#include "kge_split.h"
 
 #include <algorithm>
 #include <cstdint>
@@ -2240,6 +2241,7 @@ static RowSource dense_rows(const float* base, int cols) {
 // product on the matrix cores (the scoring backward's dot kernel: coefficient
 // matrix = dense features, other rows = W), the embedding added in its epilogue.
 void launch_hidden_fwd(const FeatureArgs& a, float* hidden, hipStream_t stream) {
+    if (a.wp) { launch_feature_fwd(a, hidden, stream); return; }
     if (feature_bf16_ok(a)) {
         // hidden [U, Dp] = features [U, Fp] . W [Fp, Dp] + embedding: A = features, Bt = W^T
         hipLaunchKernelGGL(k_gather_features, dim3((a.max_rows + 3) / 4), dim3(256), 0, stream, a,
@@ -2582,25 +2584,41 @@ void launch_adam_flat(float* p, float* m, float* v, const float* g, int64_t n, f
 
 // The same on a parameter whose slices of `slice` elements have step sizes of their own (alpha[0],
 // alpha[1], ..; the last one's also for what lies behind it): one launch for all of a parameter's
-// shards (16 launches took 39 us for a 768 x 256 parameter, this one 5).  n, slice % 4 == 0.
+// shards (16 launches took 39 us for a 768 x 256 parameter, this one 5).  n, slice % 4 == 0.  The parts
+// of the gradient are added up here, in order, and the new values leave as pieces for the next
+// step's product too.
 __global__ __launch_bounds__(256) void k_adam_slices(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
-                                                     const float* __restrict__ g, uint32_t n, uint32_t slice,
-                                                     uint32_t n_slices, AdamArgs a) {
+                                                     const float* __restrict__ g, int n_part, uint32_t n, uint32_t slice,
+                                                     uint32_t n_slices, AdamArgs a, char* __restrict__ pieces, uint32_t width) {
     const uint32_t i = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= n) return;
     const float alpha = a.alpha[min(i / slice, n_slices - 1)];
     float4 p4 = *reinterpret_cast<const float4*>(p + i), m4 = *reinterpret_cast<const float4*>(m + i);
     float4 v4 = *reinterpret_cast<const float4*>(v + i);
-    adam4(p4, m4, v4, *reinterpret_cast<const float4*>(g + i), a, alpha);
+    float4 g4 = *reinterpret_cast<const float4*>(g + i);
+    int q = 1;
+    for (; q + 8 <= n_part; q += 8) {  // eight loads under way
+        float4 t[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) t[x] = *reinterpret_cast<const float4*>(g + (size_t)(q + x) * n + i);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) g4 = f4add(g4, t[x]);
+    }
+    for (; q < n_part; ++q) g4 = f4add(g4, *reinterpret_cast<const float4*>(g + (size_t)q * n + i));
+    adam4(p4, m4, v4, g4, a, alpha);
     *reinterpret_cast<float4*>(p + i) = p4;
     *reinterpret_cast<float4*>(m + i) = m4;
     *reinterpret_cast<float4*>(v + i) = v4;
+    if (pieces) {
+        const uint32_t row = i / width;
+        store_pieces4(pieces + (size_t)row * ((width + 31) / 32 * 192), (int)(i - row * width), p4);
+    }
 }
-void launch_adam_slices(float* p, float* m, float* v, const float* g, int64_t n, int64_t slice, int n_slices,
-                        const AdamArgs& a, hipStream_t stream) {
+void launch_adam_slices(float* p, float* m, float* v, const float* g, int n_part, int64_t n, int64_t slice, int n_slices,
+                        const AdamArgs& a, void* pieces, int width, hipStream_t stream) {
     if (n == 0) return;
-    hipLaunchKernelGGL(k_adam_slices, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, stream, p, m, v, g,
-                       (uint32_t)n, (uint32_t)slice, (uint32_t)n_slices, a);
+    hipLaunchKernelGGL(k_adam_slices, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, stream, p, m, v, g, n_part,
+                       (uint32_t)n, (uint32_t)slice, (uint32_t)n_slices, a, (char*)pieces, (uint32_t)width);
 }
 
 __global__ __launch_bounds__(256) void k_fill_u32(uint32_t* p, uint32_t value, int64_t n) {
