@@ -282,7 +282,7 @@ struct kge_engine {
     size_t proj_pieces_bytes = 0;  // of one network's
     DevBuf<char> projp;
     DevBuf<float> bwd_pieces;  // split sums of the scoring backward
-    DevBuf<float> coef, dist, grad, opnd, partial, rel_partial, rel_gsum, hidden, gsum, gproj, featd, gproj_part, gemm_part, projR, loss_part, loss_step, d_alpha;
+    DevBuf<float> coef, dist, grad, opnd, partial, rel_partial, hidden, gsum, gproj, featd, gproj_part, gemm_part, projR, loss_part, loss_step, d_alpha;
     // [n_step][entity, relation, normal, then per feature network projection, mlp up, mlp down][S]; the relation update indexes its two
     // groups as one array (key / rows_per_alpha), a shared table's [relation, normal] pair
     // sits in the first two entries of the relation group
@@ -351,9 +351,9 @@ bool feature_modifier(kge_engine& E, const std::string& key, float value) {
     return true;
 }
 
-// DistMult, ComplEx and RotatE form a row's gradient contributions from rows of the other
-// table when they are summed (TransE's and TransH's are materialised before that)
-bool contributions_read_tables(const kge_engine& E) {
+// DistMult's, ComplEx's and RotatE's head gradients are formed from rows of both tables
+// (launch_head_back) before they are summed
+bool head_back_needed(const kge_engine& E) {
     return E.score_fn == SCORE_DISTMULT || E.score_fn == SCORE_COMPLEX || E.score_fn == SCORE_ROTATE;
 }
 
@@ -548,7 +548,7 @@ void parse_settings(kge_engine& E, const Items& s) {
     // regularisers (they count a row's members that carry no gradient as its gathered slots),
     // and for tail lists that fit one workgroup's sort.
     E.keep_gradients = s.find("execution.keep_gradients") ? s.boolean("execution.keep_gradients") : false;
-    if (E.keep_gradients && (E.F || contributions_read_tables(E)))
+    if (E.keep_gradients && (E.F || head_back_needed(E)))
         throw std::invalid_argument("'execution.keep_gradients' is implemented for score functions whose gradient "
                                     "contributions are used as stored (TransE, TransH) without entity features");
     E.merge_tails = s.find("execution.merge_tails") ? s.boolean("execution.merge_tails") : true;
@@ -719,7 +719,7 @@ void allocate(kge_engine& E) {
     }
     E.partial.alloc((size_t)E.e_cstride * E.Dp);
     E.rel_partial.alloc((size_t)E.r_cstride * E.Dp);
-    if (contributions_read_tables(E)) E.rel_gsum.alloc((size_t)E.n_rel * E.Dp);
+    if (head_back_needed(E)) E.relgrad.alloc(SB * E.Dp);
     if (E.score_fn == SCORE_TRANSH) {
         E.opnd_n.alloc(R * E.Dp);
         E.transh_mm.alloc(R * E.Dp);
@@ -1379,18 +1379,18 @@ void run_step(kge_engine& E, int i) {
     aa.one_minus_beta_m = 1.f - E.beta_m; aa.one_minus_beta_v = 1.f - E.beta_v;
     aa.epsilon = E.epsilon; aa.weight_decay = E.weight_decay;
 
-    // both reductions read pre-update rows (DistMult and ComplEx multiply by them), so they
-    // come before both updates
+    if (head_back_needed(E)) {
+        KernelTimer t(E, K_REDUCE_REL);
+        launch_head_back(E.score_fn, ent, E.rel.p, crel, E.D / 2, (int)SB, E.Dp, E.grad.p, E.relgrad.p, st);
+    }
     ContribSrc rsrc = {};
     rsrc.sorted_item = E.r_sorted_vals + (size_t)i * E.n_rel_items;
-    rsrc.grad = transh ? E.relgrad.p : E.grad.p;  // TransH: rows [0, SB) embedding, [SB, 2 SB) normal contributions
-    rsrc.transform = E.score_fn == SCORE_DISTMULT ? 2 : E.score_fn == SCORE_COMPLEX ? 4 : E.score_fn == SCORE_ROTATE ? 6 : 0;
-    rsrc.n_head = (int)SB; rsrc.half = E.D / 2;
-    rsrc.rel = E.rel.p; rsrc.crel = crel; rsrc.ent = ent;
+    // TransH: rows [0, SB) embedding, [SB, 2 SB) normal contributions
+    rsrc.grad = transh || head_back_needed(E) ? E.relgrad.p : E.grad.p;
+    rsrc.n_head = (int)SB;
     ContribSrc esrc = rsrc;
     esrc.sorted_item = E.e_sorted_vals + (size_t)i * 2 * R;
     esrc.grad = E.grad.p;
-    esrc.transform = E.score_fn == SCORE_DISTMULT ? 1 : E.score_fn == SCORE_COMPLEX ? 3 : E.score_fn == SCORE_ROTATE ? 5 : 0;
 
     ReduceArgs rr = {};
     rr.src = rsrc;
@@ -1407,21 +1407,17 @@ void run_step(kge_engine& E, int i) {
     re.counts = e_counts; re.max_chunks = E.e_cstride; re.chunk = E.chunk;
     if (E.counts_known) re.max_chunks = (int)E.h_e_counts[4 * (size_t)i + 1];
     re.partial = E.partial.p; re.Dp = E.Dp;
-    // Contributions used as stored, nothing between the sums and the updates, and no row with
+    // Nothing between the sums and the updates, and no row with
     // more contributions than a handful of workgroups sum in the time the other rows take (known
     // from the plan's read-back): the rows with chunks are summed and updated by workgroups of
     // their own inside the update's launch, and the first-level reduction (a launch whose time
     // is all latency) is not needed.  A row of 5 600 contributions (the 22.8M-row workload's
     // hottest) takes its eight workgroups longer than the whole update takes otherwise; one of
     // 2 200 (the 1M-row workload's) fits under it.
-    const bool hot_in_update = !contributions_read_tables(E) && !E.mlp && !roles && E.counts_known &&
+    const bool hot_in_update = !E.mlp && !roles && E.counts_known &&
                                std::max(E.h_e_counts[4 * (size_t)i + 3], E.h_r_counts[4 * (size_t)i + 3]) <= kHotInUpdateMax;
     if (!hot_in_update) { KernelTimer t(E, K_REDUCE_ENT); launch_reduce_chunks2(re, rr, st); }
 
-    // With DistMult / ComplEx the relation rows' direct contributions read entity rows and
-    // the entity rows' read relation rows, so neither table may be updated before
-    // the other's gradient is complete: materialise the relation gradient first.
-    // (TransE contributions do not depend on either table.)
     AdamArgs ar = aa;
     ar.src = rsrc;
     ar.uniq_key = E.r_uniq.p + (size_t)i * E.r_ustride;
@@ -1479,25 +1475,7 @@ void run_step(kge_engine& E, int i) {
         upd.grad_out = nullptr; upd.grad_out_add = nullptr; upd.grad_add = E.mlp_gval.p;
         launch_adam_rows(upd, st);
     };
-    if (contributions_read_tables(E)) {
-        // entity update first (reads pre-update relation rows), writing its summed
-        // gradient is not needed; then the relation update reads POST-update entity
-        // rows unless its gradient was materialised: do that with a zero-step pass
-        ar.grad_out = E.rel_gsum.p;
-        ar.no_update = 1;
-        if (E.F && !E.mlp && !roles) {
-            // with entity features the relation rows' contributions read the hidden rows formed
-            // at the start of the step, not the table: their sum can share the entity update's launch
-            KernelTimer t(E, K_ADAM_ENT);
-            launch_adam_rows2(ar, ae, st);
-        } else {
-            { KernelTimer t(E, K_ADAM_REL); launch_adam_rows(ar, st); }
-            entity_update();
-        }
-        ar.grad_out = nullptr; ar.no_update = 0;
-        ar.grad_direct = E.rel_gsum.p;
-        { KernelTimer t(E, K_ADAM_REL); launch_adam_rows(ar, st); }
-    } else if (E.mlp || roles) {
+    if (E.mlp || roles) {
         entity_update();
         KernelTimer t(E, K_ADAM_REL);
         launch_adam_rows(ar, st);
@@ -2351,7 +2329,7 @@ int kge_scatter_add(float* grad_t, int64_t rows, int64_t cols, const uint32_t* i
     sp.seg_real = u32(L.off_real); sp.hot_rows = nullptr; sp.hot_count = nullptr; sp.host_counts = nullptr;
     launch_find_segments2(job, nullptr, 1, u32(L.off_scratch), st);
     ReduceArgs ra = {};
-    ra.src.sorted_item = sv; ra.src.grad = grad_out; ra.src.transform = 0;
+    ra.src.sorted_item = sv; ra.src.grad = grad_out;
     ra.chunk_pos = sp.chunk_pos; ra.chunk_len = sp.chunk_len; ra.counts = sp.counts;
     ra.max_chunks = (int)L.cmax; ra.chunk = 32; ra.partial = (float*)(w + L.off_partial);
     ra.Dp = (int)cols;

@@ -309,18 +309,16 @@ void launch_score_bwd(const ScoreShape& sh, const RowSource& ent, const float* r
 // floats of scratch (`pieces`) the launch above wants for sums that it splits (without it: null)
 size_t score_bwd_pieces(const ScoreShape& sh);
 
-// Where gradient contributions come from.  transform: 0 none; 1 multiply head
-// rows (c < n_head) by rel[crel[c]] (DistMult, entity plan); 2 multiply by the
-// head entity row (DistMult, relation plan); 3 / 4 the same two for ComplEx: the
-// product with the complex conjugate on the halves [0, half) | [half, 2 half); 5 / 6 for
-// RotatE: the rotation back (entity plan), the phases' gradient in float16 (relation plan).
+// DistMult, ComplEx, RotatE: the head contributions' rows of `grad` (d loss / d predicted tail) turned
+// into the head rows' gradients in place, and the relation rows' contributions into relgrad [n_head, Dp]
+void launch_head_back(int score_fn, const RowSource& ent, const float* rel, const uint32_t* crel, int half, int n_head,
+                      int Dp, float* grad, float* relgrad, hipStream_t stream);
+
+// Where gradient contributions come from: contribution c is row c of `grad`.
 struct ContribSrc {
     const uint32_t* sorted_item;  // this step's sorted values
     const float* grad;            // [R, Dp]
-    int transform, n_head, half;
-    const float* rel;
-    const uint32_t* crel;
-    RowSource ent;
+    int n_head;                   // contributions before this are heads'
 };
 
 // Deterministic segmented reduction, first level (rows with many
@@ -351,7 +349,6 @@ struct AdamArgs {
     const uint32_t* counts;
     int max_rows;
     const float* partial;      // [chunks, Dp]
-    const float* grad_direct;  // [rows, Dp] used instead of the contributions when non-null
     float* grad_out;           // [rows, Dp] or null
     char* p_base;              // parameter rows: p_base + key * pitch
     char* m_base;
@@ -373,8 +370,8 @@ void launch_adam_rows(const AdamArgs& a, hipStream_t stream);
 void launch_adam_rows2(const AdamArgs& a0, const AdamArgs& a1, hipStream_t stream);  // one launch
 // The same two updates without the first-level reduction (launch_reduce_chunks) before them:
 // a row with chunks ("hot", SegPlan::hot_rows) is summed and updated by workgroups of its own,
-// one per 32 columns, the other rows by one wave each as in launch_adam_rows.  Contributions
-// as stored (ContribSrc::transform 0) only.  max_hot: upper bound of *hot_count.
+// one per 32 columns, the other rows by one wave each as in launch_adam_rows.
+// max_hot: upper bound of *hot_count.
 struct HotRows {
     const uint32_t* hot_rows;
     const uint32_t* hot_count;

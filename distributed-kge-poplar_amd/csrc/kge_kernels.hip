@@ -1525,77 +1525,80 @@ void launch_row_range(uint32_t base, int n_live, int n, uint32_t* out, hipStream
 // --------------------------------------------------------------------------
 // segmented reduction + Adam
 
-// One gradient contribution (row c of the contribution-gradient matrix), four
-// columns from k, with the DistMult product rule applied on load.
-template <bool XF>  // XF: the ComplEx / RotatE transforms (3 .. 6) are compiled in
-DEVINL float4 load_contrib(const ContribSrc& cs, uint32_t c, int k, int Dp) {
-    float4 g = *reinterpret_cast<const float4*>(cs.grad + (size_t)c * Dp + k);
-    if (XF && cs.transform >= 5) {
-        // RotatE: the predicted tail is (h_re, h_im) rotated by the phases.  Entity plan: the
-        // gradient rotated back.  Relation plan: the phases' gradient, formed in float16 as the
-        // reference's float16 sine / cosine backward ops form it (src/pag/pag.cpp:552-637),
-        // in columns [0, half); zero above.
-        if (c < (uint32_t)cs.n_head) {
-            const float* gr = cs.grad + (size_t)c * Dp;
-            const float* rr = cs.rel + (size_t)cs.crel[c] * Dp;
-            const char* er = row_ptr(cs.ent, c);
-            float* gg = &g.x;
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                const int kk = k + x;
-                if (kk >= 2 * cs.half) { gg[x] = 0.f; continue; }
-                const int kq = kk < cs.half ? kk : kk - cs.half;
-                const float th = (float)(_Float16)rr[kq];
-                const _Float16 sn = (_Float16)sinf(th), cs16 = (_Float16)cosf(th);
-                const float g_re = gr[kq], g_im = gr[kq + cs.half];
-                if (cs.transform == 5) {
-                    gg[x] = kk < cs.half ? g_re * (float)cs16 + g_im * (float)sn
-                                         : g_im * (float)cs16 - g_re * (float)sn;
-                } else if (kk < cs.half) {
-                    const float h_re = load1(er, kq, cs.ent.etype), h_im = load1(er, kq + cs.half, cs.ent.etype);
-                    const _Float16 g_sin = (_Float16)(-g_re * h_im + g_im * h_re);
-                    const _Float16 g_cos = (_Float16)(g_re * h_re + g_im * h_im);
-                    const _Float16 from_cos = -g_cos * sn, from_sin = g_sin * cs16;
-                    gg[x] = (float)(_Float16)(from_cos + from_sin);
-                } else {
-                    gg[x] = 0.f;
-                }
-            }
+// The heads' gradients of the score functions whose predicted tail is no plain sum of head and
+// relation, one wave per positive: from d loss / d (predicted tail), row c of `grad`, to the head
+// row's gradient in the same place and the relation row's in row c of `relgrad`.  Formed here once,
+// both are summed by the same kernels as TransE's; formed where they are summed (every
+// contribution a chain of loads from three tables, sines and cosines included, and the relations'
+// sum apart from the entities' update) they took 132 us of the 16-shard RotatE workload's step.
+template <int SCORE>
+__global__ __launch_bounds__(256) void k_head_back(RowSource ent, const float* __restrict__ rel,
+                                                   const uint32_t* __restrict__ crel, int half, int n_head, int Dp,
+                                                   float* __restrict__ grad, float* __restrict__ relgrad) {
+    const int lane = threadIdx.x & 63;
+    const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (c >= n_head) return;
+    const char* er = row_ptr(ent, c);
+    const float* rr = rel + (size_t)crel[c] * Dp;
+    float* gr = grad + (size_t)c * Dp;
+    float* rg = relgrad + (size_t)c * Dp;
+    if constexpr (SCORE == SCORE_DISTMULT) {  // h * r: the product rule
+        for (int k = lane * 4; k < Dp; k += 256) {
+            const float4 g = *reinterpret_cast<const float4*>(gr + k), h = load4(er, k, ent);
+            const float4 r = *reinterpret_cast<const float4*>(rr + k);
+            *reinterpret_cast<float4*>(gr + k) = f4mul(g, r);
+            *reinterpret_cast<float4*>(rg + k) = f4mul(g, h);
         }
-    } else if (XF && cs.transform >= 3) {
-        // ComplEx: the predicted tail is the complex product h r, so the head's gradient is
-        // g conj(r) and the relation's g conj(h) (column kk pairs with kk +- half):
-        //   re: g_re o_re + g_im o_im      im: g_im o_re - g_re o_im      (o = r or h)
-        if (c < (uint32_t)cs.n_head) {
-            const float* gr = cs.grad + (size_t)c * Dp;
-            const float* rr = cs.rel + (size_t)cs.crel[c] * Dp;
-            const char* er = row_ptr(cs.ent, c);
-            float* gg = &g.x;
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                const int kk = k + x;
-                if (kk >= 2 * cs.half) { gg[x] = 0.f; continue; }
-                const int pp = kk < cs.half ? kk + cs.half : kk - cs.half;
-                const float o_k = cs.transform == 3 ? rr[kk] : load1(er, kk, cs.ent.etype);
-                const float o_p = cs.transform == 3 ? rr[pp] : load1(er, pp, cs.ent.etype);
-                const float g_p = gr[pp];
-                gg[x] = kk < cs.half ? gg[x] * o_k + g_p * o_p : gg[x] * o_p - g_p * o_k;
-            }
-        }
-    } else if (cs.transform == 1) {
-        if (c < (uint32_t)cs.n_head)
-            g = f4mul(g, *reinterpret_cast<const float4*>(cs.rel + (size_t)cs.crel[c] * Dp + k));
-    } else if (cs.transform == 2) {
-        g = f4mul(g, load4(row_ptr(cs.ent, c), k, cs.ent));
+        return;
     }
-    return g;
+    for (int k = lane; k < half; k += 64) {
+        const float g_re = gr[k], g_im = gr[k + half];
+        const float h_re = load1(er, k, ent.etype), h_im = load1(er, k + half, ent.etype);
+        if constexpr (SCORE == SCORE_COMPLEX) {
+            // the complex product h r: the head's gradient is g conj(r), the relation's g conj(h)
+            const float r_re = rr[k], r_im = rr[k + half];
+            gr[k] = g_re * r_re + g_im * r_im;
+            gr[k + half] = g_im * r_re - g_re * r_im;
+            rg[k] = g_re * h_re + g_im * h_im;
+            rg[k + half] = g_im * h_re - g_re * h_im;
+        } else {
+            // (h_re, h_im) rotated by the phases: the gradient rotated back; the phases' gradient formed
+            // in float16 as the reference's float16 sine / cosine backward ops form it
+            // (src/pag/pag.cpp:552-637), in columns [0, half), zero above
+            const float th = (float)(_Float16)rr[k];
+            const _Float16 sn = (_Float16)sinf(th), cs = (_Float16)cosf(th);
+            gr[k] = g_re * (float)cs + g_im * (float)sn;
+            gr[k + half] = g_im * (float)cs - g_re * (float)sn;
+            const _Float16 g_sin = (_Float16)(-g_re * h_im + g_im * h_re);
+            const _Float16 g_cos = (_Float16)(g_re * h_re + g_im * h_im);
+            const _Float16 from_cos = -g_cos * sn, from_sin = g_sin * cs;
+            rg[k] = (float)(_Float16)(from_cos + from_sin);
+            rg[k + half] = 0.f;
+        }
+    }
+    for (int k = 2 * half + lane; k < Dp; k += 64) gr[k] = rg[k] = 0.f;  // padding columns
+}
+void launch_head_back(int score_fn, const RowSource& ent, const float* rel, const uint32_t* crel, int half, int n_head,
+                      int Dp, float* grad, float* relgrad, hipStream_t stream) {
+#define KGE_HB(S_)                                                                                              \
+    hipLaunchKernelGGL(k_head_back<S_>, dim3((n_head + 3) / 4), dim3(256), 0, stream, ent, rel, crel, half, n_head, \
+                       Dp, grad, relgrad)
+    if (score_fn == SCORE_DISTMULT) KGE_HB(SCORE_DISTMULT);
+    else if (score_fn == SCORE_COMPLEX) KGE_HB(SCORE_COMPLEX);
+    else KGE_HB(SCORE_ROTATE);
+#undef KGE_HB
+}
+
+// One gradient contribution, four columns from k.
+DEVINL float4 load_contrib(const ContribSrc& cs, uint32_t c, int k, int Dp) {
+    return *reinterpret_cast<const float4*>(cs.grad + (size_t)c * Dp + k);
 }
 
 // Ordered sum of the contributions at sorted positions [pos, pos + n), columns
 // k..k+3: eight independent row loads in flight, added in position order.
 // Must be called by every lane of the wave (the item indices travel by
 // shuffle); lanes with `active` false load nothing and return zero.
-template <int NB, bool XF>
+template <int NB>
 DEVINL float4 sum_contribs(const ContribSrc& cs, uint32_t pos, uint32_t n, int k, int Dp, int lane,
                            bool active) {
     float4 acc = make_float4(0, 0, 0, 0);
@@ -1605,7 +1608,7 @@ DEVINL float4 sum_contribs(const ContribSrc& cs, uint32_t pos, uint32_t n, int k
 #pragma unroll
         for (int x = 0; x < NB; ++x) {
             const uint32_t c = __shfl(mine, x, 64);
-            v[x] = (active && j + x < n) ? load_contrib<XF>(cs, c, k, Dp) : make_float4(0, 0, 0, 0);
+            v[x] = (active && j + x < n) ? load_contrib(cs, c, k, Dp) : make_float4(0, 0, 0, 0);
         }
 #pragma unroll
         for (int x = 0; x < NB; ++x) acc = f4add(acc, v[x]);
@@ -1618,7 +1621,7 @@ DEVINL float4 sum_contribs(const ContribSrc& cs, uint32_t pos, uint32_t n, int k
 // NW = 16 serves chunks of up to 256 contributions with the same two rounds of
 // eight loads per wave that NW = 4 needs for 64: four times fewer partials for
 // the second level to walk through.
-template <int NW, bool XF>
+template <int NW>
 __global__ __launch_bounds__(NW * 64) void k_reduce_chunks(ReduceArgs a0, ReduceArgs a1) {
     __shared__ __attribute__((aligned(16))) float part[NW - 1][256];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1650,7 +1653,7 @@ __global__ __launch_bounds__(NW * 64) void k_reduce_chunks(ReduceArgs a0, Reduce
     const int k = slab * 256 + lane * 4;
     // sixteen loads in flight: a wave's share of a 64-item chunk in one round (same order of
     // additions as any other round size)
-    float4 acc = sum_contribs<16, XF>(a.src, pos + w0, w1 - w0, k, Dp, lane, k < Dp);
+    float4 acc = sum_contribs<16>(a.src, pos + w0, w1 - w0, k, Dp, lane, k < Dp);
     if (wave > 0) *reinterpret_cast<float4*>(&part[wave - 1][lane * 4]) = acc;
     __syncthreads();
     if (wave == 0 && k < Dp) {
@@ -1663,14 +1666,10 @@ __global__ __launch_bounds__(NW * 64) void k_reduce_chunks(ReduceArgs a0, Reduce
 static void launch_reduce_kernel(const ReduceArgs& a0, const ReduceArgs& a1, hipStream_t stream) {
     const int n = (a0.max_chunks + a1.max_chunks) * ((std::max(a0.Dp, a1.Dp) + 255) / 256);
     if (n == 0) return;
-    const bool xf = (a0.max_chunks && a0.src.transform >= 3) || (a1.max_chunks && a1.src.transform >= 3);
-    if (std::max(a0.chunk, a1.chunk) > 64) {
-        if (xf) hipLaunchKernelGGL((k_reduce_chunks<16, true>), dim3(n), dim3(1024), 0, stream, a0, a1);
-        else hipLaunchKernelGGL((k_reduce_chunks<16, false>), dim3(n), dim3(1024), 0, stream, a0, a1);
-    } else {
-        if (xf) hipLaunchKernelGGL((k_reduce_chunks<4, true>), dim3(n), dim3(256), 0, stream, a0, a1);
-        else hipLaunchKernelGGL((k_reduce_chunks<4, false>), dim3(n), dim3(256), 0, stream, a0, a1);
-    }
+    if (std::max(a0.chunk, a1.chunk) > 64)
+        hipLaunchKernelGGL(k_reduce_chunks<16>, dim3(n), dim3(1024), 0, stream, a0, a1);
+    else
+        hipLaunchKernelGGL(k_reduce_chunks<4>, dim3(n), dim3(256), 0, stream, a0, a1);
 }
 void launch_reduce_chunks(const ReduceArgs& a, hipStream_t stream) {
     ReduceArgs none = a;
@@ -1703,7 +1702,7 @@ DEVINL void adam4(float4& p, float4& m, float4& v, float4 g, const AdamArgs& a, 
 // row itself, stores): what the kernel gets through is the number of resident waves over that
 // chain's length, so the plain form is compiled for eight waves per SIMD (four contribution
 // loads in flight instead of eight buy the registers).
-template <bool MF32, bool XF>
+template <bool MF32>
 DEVINL void adam_rows_body(const AdamArgs& a0, const AdamArgs& a1) {
     const int lane = threadIdx.x & 63;
     // two tables share the launch: blocks [0, ceil(a0.max_rows * slabs / 4)) serve the first; a
@@ -1718,11 +1717,8 @@ DEVINL void adam_rows_body(const AdamArgs& a0, const AdamArgs& a1) {
     // but inside the arrays): one round trip less in front of every row
     const int uc = min(u, a.max_rows - 1);
     const uint32_t key = a.uniq_key[uc];
-    uint32_t q0 = 0, q1 = 0, pos = 0, n_real = 0;
-    if (!a.grad_direct) {
-        q0 = a.chunk_off[uc]; q1 = a.chunk_off[uc + 1];
-        pos = a.seg_start[uc]; n_real = a.seg_real[uc];
-    }
+    const uint32_t q0 = a.chunk_off[uc], q1 = a.chunk_off[uc + 1];
+    const uint32_t pos = a.seg_start[uc], n_real = a.seg_real[uc];
     if (u >= (int)a.counts[0]) return;
     const float alpha = a.alpha[a.rows_per_alpha ? key / a.rows_per_alpha : 0u];
     const int Dp = a.Dp;
@@ -1733,8 +1729,8 @@ DEVINL void adam_rows_body(const AdamArgs& a0, const AdamArgs& a1) {
         const int k = slab * 256 + lane * 4;
         const bool active = k < Dp;
         float4 g = make_float4(0, 0, 0, 0);
-        if (!a.grad_direct && q1 == q0 && n_real)  // wave-uniform: all lanes take part in the shuffles
-            g = sum_contribs<XF ? 8 : 4, XF>(a.src, pos, n_real, k, Dp, lane, active);
+        if (q1 == q0 && n_real)  // wave-uniform: all lanes take part in the shuffles
+            g = sum_contribs<4>(a.src, pos, n_real, k, Dp, lane, active);
         if (!active) return;
         float4 p = load4(prow, k, a.p_etype);
         float4 m, v;
@@ -1745,10 +1741,8 @@ DEVINL void adam_rows_body(const AdamArgs& a0, const AdamArgs& a1) {
             m = load4(mrow, k, a.m_etype);
             v = load4(vrow, k, a.m_etype);
         }
-        if (a.grad_direct) {
-            g = *reinterpret_cast<const float4*>(a.grad_direct + (size_t)u * Dp + k);
-        } else if (q1 > q0) {
-            constexpr int NP = XF ? 8 : 4;  // partial sums in flight
+        if (q1 > q0) {
+            constexpr int NP = 4;  // partial sums in flight
             for (uint32_t q = q0; q < q1; q += NP) {
                 float4 t[NP];
 #pragma unroll
@@ -1780,11 +1774,7 @@ DEVINL void adam_rows_body(const AdamArgs& a0, const AdamArgs& a1) {
 
 template <bool MF32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_adam_rows(AdamArgs a0, AdamArgs a1) {
-    adam_rows_body<MF32, false>(a0, a1);
-}
-template <bool MF32>  // with the ComplEx / RotatE transforms of the contributions compiled in
-__global__ __launch_bounds__(256) void k_adam_rows_xf(AdamArgs a0, AdamArgs a1) {
-    adam_rows_body<MF32, true>(a0, a1);
+    adam_rows_body<MF32>(a0, a1);
 }
 
 // One launch for both tables without a first-level reduction before it.
@@ -1922,7 +1912,7 @@ __global__ __launch_bounds__(kHotWaves * 64) __attribute__((amdgpu_waves_per_eu(
         const bool active = k < Dp;
         float4 g = make_float4(0, 0, 0, 0);
         if (n_real)  // wave-uniform: all lanes take part in the shuffles
-            g = sum_contribs<4, false>(a.src, pos, n_real, k, Dp, lane, active);
+            g = sum_contribs<4>(a.src, pos, n_real, k, Dp, lane, active);
         if (!active) return;
         float4 p = load4(prow, k, a.p_etype);
         float4 m, v;
@@ -1978,11 +1968,8 @@ static void launch_adam_kernel(const AdamArgs& a0, const AdamArgs& a1, hipStream
     const dim3 grid((a0.max_rows * slabs + 3) / 4 + (a1.max_rows * slabs + 3) / 4);
     if (grid.x == 0) return;
     const bool f32 = (a0.max_rows == 0 || a0.m_etype == ET_F32) && (a1.max_rows == 0 || a1.m_etype == ET_F32);
-    const bool xf = (a0.max_rows && a0.src.transform >= 3) || (a1.max_rows && a1.src.transform >= 3);
-    if (f32 && !xf) hipLaunchKernelGGL((k_adam_rows<true>), grid, dim3(256), 0, stream, a0, a1);
-    else if (f32) hipLaunchKernelGGL((k_adam_rows_xf<true>), grid, dim3(256), 0, stream, a0, a1);
-    else if (!xf) hipLaunchKernelGGL((k_adam_rows<false>), grid, dim3(256), 0, stream, a0, a1);
-    else hipLaunchKernelGGL((k_adam_rows_xf<false>), grid, dim3(256), 0, stream, a0, a1);
+    if (f32) hipLaunchKernelGGL((k_adam_rows<true>), grid, dim3(256), 0, stream, a0, a1);
+    else hipLaunchKernelGGL((k_adam_rows<false>), grid, dim3(256), 0, stream, a0, a1);
 }
 void launch_adam_rows(const AdamArgs& a, hipStream_t stream) {
     AdamArgs none = a;
@@ -3203,7 +3190,7 @@ __global__ __launch_bounds__(256) void k_role_sums(DropoutArgs a, ContribSrc cs,
         float4 gh = make_float4(0, 0, 0, 0), gt = gh;
         for (uint32_t j = 0; j < n; ++j) {
             const uint32_t c = cs.sorted_item[pos + j];
-            const float4 v = load_contrib<true>(cs, c, k, a.Dp);
+            const float4 v = load_contrib(cs, c, k, a.Dp);
             if (c < (uint32_t)cs.n_head) gh = f4add(gh, v); else gt = f4add(gt, v);
         }
         if (add_head) {  // the regularisers' share (of the tensors after dropout)

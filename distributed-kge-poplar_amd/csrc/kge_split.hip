@@ -244,7 +244,7 @@ template <int DIST, int OM, int TM, int TN, int WM, int WN>
 __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_fwd(SplitFwd p) {
     using P = SplitProduct<RowTile<TM>, RowTile<TN>, TM, TN, WM, WN>;
     __shared__ __attribute__((aligned(16))) char smem[P::kLds];
-    __shared__ float na_s[TM], nb_s[TN], red[WM * WN];
+    __shared__ float na_s[TM], nb_s[TN], mult_s[TN], red[WM * WN];
     __shared__ uint32_t label_s[TM];
     const ScoreShape& sh = p.sh;
     const int B = sh.B, T = sh.T, Kp = p.Kp;
@@ -256,6 +256,7 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
         if (OM == 0 && tid == 0) p.loss_part[(size_t)d * (tile.gx * tile.gy) + tile.y * tile.gx + tile.x] = 0.f;
         return;
     }
+    const int n_live = sh.tcount ? (int)sh.tcount[d] : T;
     const int a_row = p.a_c0 + d * B, b_row = p.b_c0 + d * T;
     const int pitch = Kp * 6;
     const char* a = p.a + (int64_t)(a_row + m0) * pitch;
@@ -274,6 +275,9 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
         }
         if (DIST == DIST_L2)
             for (int i = tid; i < TN; i += WM * WN * 64) nb_s[i] = p.norm_b[b_row + n0 + i];
+        if (OM == 0)
+            for (int i = tid; i < TN; i += WM * WN * 64)
+                mult_s[i] = n0 + i < T ? (sh.tmult ? sh.tmult[(size_t)d * T + n0 + i] : 1.f) : 0.f;
     });
 
     // epilogue.  Register r of lane l holds row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
@@ -293,7 +297,7 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
             const int n = n0 + nbk + cl;
             // columns behind a block's distinct tails repeat its first row, the most popular one more
             // often than not: no pair of theirs is worth a second look
-            const bool col_counts = n < (sh.tcount ? (int)sh.tcount[d] : T);
+            const bool col_counts = n < n_live;
             float val[16];
             uint32_t cancel = 0u, near = 0u;
 #pragma unroll
@@ -367,7 +371,7 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
                 }
                 continue;
             }
-            const float mult = n < T ? (sh.tmult ? sh.tmult[(size_t)d * T + n] : 1.f) : 0.f;
+            const float mult = mult_s[nbk + cl];
             float c[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -498,23 +502,27 @@ DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, cha
             const int k = kt0 + wn + 32 * ni + (cl & ~1);
             if (k >= p.Dp) continue;
             const char* const sp = self + (size_t)(k >> 5) * 192 + (k & 31) * 2;
+            uint32_t w[DIST == DIST_L2 ? 8 : 1][3];
+            if (DIST == DIST_L2)
+#pragma unroll
+                for (int i = 0; i < 8; ++i)  // all loads before any use, rows past the last among them
+#pragma unroll
+                    for (int q = 0; q < 3; ++q)
+                        w[i][q] = *reinterpret_cast<const uint32_t*>(
+                            sp + (int64_t)(wm + 32 * mi + 8 * (i >> 1) + 4 * hl + 2 * (i & 1) + odd) * pitch + 64 * q);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const float got = swap1(odd ? acc[mi][ni][2 * i] : acc[mi][ni][2 * i + 1]);
                 float x = odd ? got : acc[mi][ni][2 * i], y = odd ? acc[mi][ni][2 * i + 1] : got;
                 const int row = wm + 32 * mi + 8 * (i >> 1) + 4 * hl + 2 * (i & 1) + odd;
-                if (i0 + row >= n_self) continue;
                 if (DIST == DIST_L2) {
                     float sx = 0.f, sy = 0.f;
 #pragma unroll
-                    for (int q = 0; q < 3; ++q) {
-                        const uint32_t w = *reinterpret_cast<const uint32_t*>(sp + (int64_t)row * pitch + 64 * q);
-                        sx += bf16_lo_f32(w); sy += bf16_hi_f32(w);
-                    }
+                    for (int q = 0; q < 3; ++q) { sx += bf16_lo_f32(w[i][q]); sy += bf16_hi_f32(w[i][q]); }
                     x = sx * csum_s[row] - x;
                     y = sy * csum_s[row] - y;
                 }
-                *reinterpret_cast<float2*>(out + (size_t)row * p.Dp + k) = make_float2(x, y);
+                if (i0 + row < n_self) *reinterpret_cast<float2*>(out + (size_t)row * p.Dp + k) = make_float2(x, y);
             }
         }
 }
