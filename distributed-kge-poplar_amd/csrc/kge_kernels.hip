@@ -1362,8 +1362,8 @@ void launch_log_softmax(const float* x, const float* dy, float* out, int64_t row
 // predict: running top-k over a stream of score chunks
 // (TopKCollector, src/poplar_kge.cpp:743-809).  One workgroup per query keeps
 // its n_best (score, index) pairs sorted by (score descending, index
-// ascending).  New scores are compared with the current n_best-th score 16384
-// at a time (64 per thread, all loads in flight together); the few that beat it
+// ascending).  New scores are compared with the current n_best-th score 32768
+// at a time (32 per thread, all loads in flight together); the few that beat it
 // are collected in LDS (in any order) and merged by rank: every element of
 // (current best, candidates) counts the candidates that come before it, a
 // candidate also finds its place among the sorted best by binary search, and
@@ -1373,13 +1373,17 @@ void launch_log_softmax(const float* x, const float* dy, float* out, int64_t row
 // A pass with more than 1024 candidates is redone 1024 scores at a time.
 
 constexpr int TK_BLOCK = 1024;  // most n_best, and the candidate list's capacity
-constexpr int TK_SPAN = 16384;
+// Sixteen waves per query: a sweep's merges follow one another, and with four waves (a 64 KB pass in
+// flight per query) a chunk of 262144 scores took 135 us, as long as its scoring; the sweep of
+// 1M rows for 128 queries then waited for the merges (0.79 ms).
+constexpr int TK_THREADS = 1024;
+constexpr int TK_SPAN = 32768;
 
 DEVINL bool topk_before(float sa, uint32_t ia, float sb, uint32_t ib) {
     return sa > sb || (sa == sb && ia < ib);
 }
 
-__global__ __launch_bounds__(256) void k_topk_merge(const float* __restrict__ scores, int64_t ld,
+__global__ __launch_bounds__(TK_THREADS) void k_topk_merge(const float* __restrict__ scores, int64_t ld,
                                                     int n_valid, uint32_t first_index, int n_best,
                                                     float* __restrict__ best_score,
                                                     uint32_t* __restrict__ best_index) {
@@ -1394,7 +1398,7 @@ __global__ __launch_bounds__(256) void k_topk_merge(const float* __restrict__ sc
     const float* row = scores + (size_t)q * ld;
     float* bs = best_score + (size_t)q * n_best;
     uint32_t* bi = best_index + (size_t)q * n_best;
-    for (int i = tid; i < n_best; i += 256) {
+    for (int i = tid; i < n_best; i += TK_THREADS) {
         cur_s[i] = bs[i];
         cur_i[i] = bi[i];
     }
@@ -1413,11 +1417,11 @@ __global__ __launch_bounds__(256) void k_topk_merge(const float* __restrict__ sc
             int* counter = &n_cand[pass % 3];
             if (tid == 0) n_cand[(pass + 1) % 3] = 0;
             ++pass;
-            constexpr int NV = TK_SPAN / 1024;
+            constexpr int NV = TK_SPAN / (4 * TK_THREADS);
             float4 v[NV];
 #pragma unroll
             for (int j = 0; j < NV; ++j) {  // rows are 16-byte aligned and hold a multiple of 4 scores
-                const int i = base + 1024 * j + tid * 4;
+                const int i = base + 4 * TK_THREADS * j + tid * 4;
                 v[j] = i < end ? *reinterpret_cast<const float4*>(row + i) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
             }
 #pragma unroll
@@ -1425,7 +1429,7 @@ __global__ __launch_bounds__(256) void k_topk_merge(const float* __restrict__ sc
                 const float* vv = &v[j].x;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int i = base + 1024 * j + tid * 4 + e;
+                    const int i = base + 4 * TK_THREADS * j + tid * 4 + e;
                     if (i < end && vv[e] > kth) {  // false for NaN
                         const int slot = atomicAdd(counter, 1);
                         if (slot < TK_BLOCK) {
@@ -1446,19 +1450,19 @@ __global__ __launch_bounds__(256) void k_topk_merge(const float* __restrict__ sc
             if (c == 0) continue;
             changed = true;
             // candidates padded to whole groups of four with entries that come before nothing
-            for (int x = c + tid; x < ((c + 3) & ~3); x += 256) {
+            for (int x = c + tid; x < ((c + 3) & ~3); x += TK_THREADS) {
                 cand_s[x] = -INFINITY;
                 cand_i[x] = 0xffffffffu;
             }
             __syncthreads();
-            // a thread's elements: candidates tid + 256 m (m < 4), current best tid + 256 (m - 4)
-            constexpr int PER = TK_BLOCK / 256;
+            // a thread's elements: candidates tid + TK_THREADS m (m < PER), then the current best
+            constexpr int PER = TK_BLOCK / TK_THREADS;
             float es[2 * PER];
             uint32_t ei[2 * PER];
             int r[2 * PER];
 #pragma unroll
             for (int m = 0; m < PER; ++m) {
-                const int e = tid + 256 * m;
+                const int e = tid + TK_THREADS * m;
                 es[m] = e < c ? cand_s[e] : -INFINITY;
                 ei[m] = e < c ? cand_i[e] : 0xffffffffu;
                 int lo = 0, hi = e < c ? n_best : 0;
@@ -1479,7 +1483,7 @@ __global__ __launch_bounds__(256) void k_topk_merge(const float* __restrict__ sc
                 const uint4 i4 = *reinterpret_cast<const uint4*>(&cand_i[x]);
 #pragma unroll
                 for (int m = 0; m < 2 * PER; ++m) {
-                    const bool live = m < PER ? 256 * m < c : 256 * (m - PER) < n_best;  // uniform
+                    const bool live = m < PER ? TK_THREADS * m < c : TK_THREADS * (m - PER) < n_best;  // uniform
                     if (!live) continue;
                     r[m] += (topk_before(s4.x, i4.x, es[m], ei[m]) ? 1 : 0) + (topk_before(s4.y, i4.y, es[m], ei[m]) ? 1 : 0) +
                             (topk_before(s4.z, i4.z, es[m], ei[m]) ? 1 : 0) + (topk_before(s4.w, i4.w, es[m], ei[m]) ? 1 : 0);
@@ -1492,7 +1496,7 @@ __global__ __launch_bounds__(256) void k_topk_merge(const float* __restrict__ sc
                     next_i[r[m]] = ei[m];
                 }
             __syncthreads();
-            for (int i = tid; i < n_best; i += 256) {
+            for (int i = tid; i < n_best; i += TK_THREADS) {
                 cur_s[i] = next_s[i];
                 cur_i[i] = next_i[i];
             }
@@ -1500,7 +1504,7 @@ __global__ __launch_bounds__(256) void k_topk_merge(const float* __restrict__ sc
         }
     }
     if (changed)
-        for (int i = tid; i < n_best; i += 256) {
+        for (int i = tid; i < n_best; i += TK_THREADS) {
             bs[i] = cur_s[i];
             bi[i] = cur_i[i];
         }
@@ -1509,7 +1513,7 @@ __global__ __launch_bounds__(256) void k_topk_merge(const float* __restrict__ sc
 void launch_topk_merge(const float* scores, int64_t ld, int n_queries, int n_valid, uint32_t first_index,
                        int n_best, float* best_score, uint32_t* best_index, hipStream_t stream) {
     if ((ld & 3) || n_valid > ld || ((uintptr_t)scores & 15)) throw std::invalid_argument("top-k merge: score rows must be 16-byte aligned");
-    hipLaunchKernelGGL(k_topk_merge, dim3(n_queries), dim3(256), 0, stream, scores, ld, n_valid, first_index,
+    hipLaunchKernelGGL(k_topk_merge, dim3(n_queries), dim3(TK_THREADS), 0, stream, scores, ld, n_valid, first_index,
                        n_best, best_score, best_index);
 }
 
