@@ -1989,6 +1989,7 @@ void run_predict(kge_engine& E, const Items& in) {
     dense.index = nullptr; dense.count = Dp; dense.vec = 1;
     RowSource dense_n = dense;
     dense_n.base = (const char*)E.p_opnd_n.p;
+    const bool sweep = predict_scores_takes(sh);
     ScoreShape dot = sh;
     dot.score_fn = SCORE_DISTMULT; dot.dist_fn = DIST_DOT;
 
@@ -2024,22 +2025,28 @@ void run_predict(kge_engine& E, const Items& in) {
             // matrix-core kernels (their fast staging path takes float32 rows, and converting while
             // copying costs less than the slower path does).
             const int live_tiles = round_up(live, 64);
-            const bool in_place = !E.F && !transh &&
+            const bool in_place = !E.F && !transh && !sweep &&
                                   (E.L.emb_etype == ET_F32 || !E.use_mfma || (E.dist_fn == DIST_L1 && E.score_fn != SCORE_DISTMULT));
-            const int n_tail = in_place ? live_tiles : chunk;  // rows the scoring launch covers = the scores' row pitch
+            // The sweep's own kernel takes exactly the live rows, of any type, where they lie (hidden rows
+            // where the projection wrote them).
+            const int n_tail = in_place || sweep ? live_tiles : chunk;  // rows the scoring launch covers = the scores' row pitch
             RowSource tails;
-            if (!E.F && (in_place || live == chunk)) {
+            if (!E.F && (in_place || sweep || live == chunk)) {
                 tails.base = E.table.p + (table_off + r0) * E.L.pitch; tails.pitch = E.L.pitch;
                 tails.etype = E.L.emb_etype; tails.index = nullptr; tails.count = Dp; tails.vec = 1;
             } else {
                 launch_row_range((uint32_t)(table_off + r0), live, chunk, tail_idx, st);
                 tails = rows_of(tail_idx, chunk, E.nets - 1);
             }
-            if (!in_place)
+            if (!in_place && !sweep)
                 launch_gather_operands(tails, E.rel.p, nullptr, 0, 0, 0, chunk, Dp, E.p_opnd.p + (size_t)Qp * Dp, nullptr, st);
             // this buffer's previous scores must have been merged
             if (n_chunk >= kge_engine::kScoreBuffers) HIP_CHECK(hipStreamWaitEvent(st, E.merged[buf], 0));
-            if (in_place) {
+            if (sweep) {
+                ScoreShape shq = sh;  // (the merge looks at the queries' rows alone)
+                shq.B = Q;
+                launch_predict_scores(shq, E.p_opnd.p, tails, live, scores, n_tail, st);
+            } else if (in_place) {
                 ScoreShape shp = sh;
                 shp.T = n_tail;
                 launch_score_fwd_rows(shp, dense, tails, scores, st);

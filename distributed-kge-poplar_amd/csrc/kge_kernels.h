@@ -235,6 +235,11 @@ void launch_score_fwd(const ScoreShape& sh, const RowSource& ent, const float* r
 // raw scores of rows `a` against rows `b` of a second source (no relation, no loss): out [S, B, T]
 void launch_score_fwd_rows(const ScoreShape& sh, const RowSource& a, const RowSource& b, float* scores,
                            hipStream_t stream);
+// The same for a prediction sweep, where it applies (kge_predict.hip): scores [sh.B, ldc], rows 0 .. n_row - 1
+// of `b`, of any element type.
+bool predict_scores_takes(const ScoreShape& sh);
+void launch_predict_scores(const ScoreShape& sh, const float* a, const RowSource& b, int n_row, float* scores, int ldc,
+                           hipStream_t stream);
 // words of the near-identical-pair flag matrix the L2 matrix-core path needs
 inline size_t nearflag_words(const ScoreShape& sh) {
     return (size_t)sh.S * ((sh.B + 31) / 32) * ((sh.T + 31) / 32);

@@ -1,0 +1,258 @@
+// gfx950 kernel of the prediction sweep's scores (L2 and dot): a few queries against very many table
+// rows (src/poplar_kge.cpp:743-808).
+//
+// Every table row is read once, where it lies and in its own type, and split once into its three bfloat16
+// pieces; up to 128 queries meet it, whose pieces stay in registers for the whole launch.  Four waves hold
+// 32 queries each (192 registers at 256 columns) and multiply a tile of 32 rows (six instructions per
+// sixteen columns: mfma_split6's order); four more fetch, four tiles ahead, and split the next tile
+// into the other LDS copy.  Waves that do both, one to a SIMD, paid for every instruction's latency
+// alone and left the merge kernel beside them no issue slots: 1M float32 rows of 256 columns for 128 queries
+// 0.90 ms.  With one tile ahead instead of four a launch of 262144 rows takes 174 us, not 130.
+// The training forward's kernel, which this replaces for sweeps, splits the 128 queries again for
+// every 64 rows, needs 16-bit rows copied to float32 first and takes widths that are no multiple of 64 on
+// float32 instructions.  Per pass, before and now, 128 queries: 1M x 256 float32 758 -> 701 us; 500k x 256
+// float16 659 -> 503; 300k x 100 float32 459 -> 429; four shards of 100k x 130, 512 queries, 5193 -> 4427;
+// 500k x 128, 16 queries, dot: 282 -> 239.
+// What bounds it: a launch of 262144 rows takes 130 us alone on 192 CUs (155 beside a merge), its products 55 at
+// the nominal rate of these CUs and its bytes 50; two accumulators in turn instead of one and score rows of
+// another length than a power of two did not change that, so it is a single multiplying wave
+// per SIMD, whose fragment reads, products and epilogue follow one another.
+//
+#include "kge_loss.h"
+#include "kge_split.h"
+
+#include <algorithm>
+#include <cstdint>
+
+namespace kge {
+
+struct PredictArgs {
+    const float* a;        // queries' predicted tails [n_query, Dp]
+    RowSource b;           // rows (no index)
+    float* scores;         // [n_query, ldc]
+    int n_query, n_row, ldc, Dp;
+    int distance_value;    // score = the distance (or the product) itself, else gamma - it
+    float gamma;
+};
+
+constexpr int PT_ROWS = 32, PT_WAVES = 4;
+
+// four columns of a row, as they lie
+template <int ET> struct Raw4 { uint2 v[ET == ET_F32 ? 2 : 1]; };
+template <int ET>
+DEVINL float4 raw4_f32(const Raw4<ET>& r) {
+    if constexpr (ET == ET_F32)
+        return make_float4(__uint_as_float(r.v[0].x), __uint_as_float(r.v[0].y), __uint_as_float(r.v[1].x), __uint_as_float(r.v[1].y));
+    else
+        return load4(reinterpret_cast<const char*>(r.v), 0, ET);
+}
+
+template <int DIST, int ET, int NS>  // ET: the rows' element type, NS: slabs of 32 columns
+__global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(PredictArgs p) {
+    using Tile = RowTile<PT_ROWS>;
+    constexpr int PF = 4, kL = NS == 8 ? 12 : 0;  // kL: steps whose queries' third piece waits in LDS (registers: 256)
+    constexpr int kBuf = NS * Tile::kBytes;
+    __shared__ __attribute__((aligned(16))) char smem[2 * kBuf];
+    __shared__ float na_s[32 * PT_WAVES], nb_s[2][PT_ROWS];
+    __shared__ __attribute__((aligned(16))) floatx4 fa2_s[PT_WAVES][kL ? kL : 1][64];
+    // tid: within the four waves of this role
+    const int tid = threadIdx.x & (PT_WAVES * 64 - 1), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int Dp = p.Dp, n_tile = (p.n_row + PT_ROWS - 1) / PT_ROWS;
+    const int step = gridDim.x;
+    int tile = blockIdx.x;
+    if (tile >= n_tile) return;
+
+    if (threadIdx.x >= PT_WAVES * 64) {
+        // waves 4 .. 7: rows into pieces.  Thread -> row, four columns of every slab.
+        const int s_row = tid >> 3, c4 = tid & 7;
+        char* const s_at = smem + s_row * 64 + ((c4 >> 1) ^ ((s_row >> 2) & 3)) * 16 + (c4 & 1) * 8;
+        Raw4<ET> raw[PF][NS];
+        auto fetch = [&](Raw4<ET> (&raw)[NS], int t) __attribute__((always_inline)) {  // past the last row or tile: the last again
+            const char* const row = p.b.base + (int64_t)min(t * PT_ROWS + s_row, p.n_row - 1) * p.b.pitch;
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                int k = 32 * s + 4 * c4;
+                if (s >= NS - 2) k = min(k, Dp - 4);  // only the last two slabs may reach past Dp (zeros when staged)
+                const char* at = row + (size_t)k * (ET == ET_F32 ? 4 : 2);
+                if constexpr (ET == ET_F32) {
+                    const uint4 t4 = *reinterpret_cast<const uint4*>(at);
+                    raw[s].v[0] = make_uint2(t4.x, t4.y); raw[s].v[1] = make_uint2(t4.z, t4.w);
+                } else {
+                    raw[s].v[0] = *reinterpret_cast<const uint2*>(at);
+                }
+            }
+        };
+        static_for<PF>([&](auto x) __attribute__((always_inline)) { fetch(raw[x.value], min(tile + x.value * step, n_tile - 1)); });
+        while (tile < n_tile)
+            static_for<PF>([&](auto x) __attribute__((always_inline)) {
+                if (tile >= n_tile) return;
+                constexpr int buf = x.value & 1;
+                float sq = 0.f;
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    float4 v = raw4_f32<ET>(raw[x.value][s]);
+                    if (s >= NS - 2 && 32 * s + 4 * c4 >= Dp) v = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (DIST == DIST_L2) sq += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+                    uint2 piece[3];
+                    split4_bf16(as_x4(v), piece);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q)
+                        *reinterpret_cast<uint2*>(s_at + buf * kBuf + s * Tile::kBytes + q * (PT_ROWS * 64)) = piece[q];
+                }
+                fetch(raw[x.value], min(tile + PF * step, n_tile - 1));
+                if (DIST == DIST_L2) {
+                    sq += __shfl_xor(sq, 1, 64); sq += __shfl_xor(sq, 2, 64); sq += __shfl_xor(sq, 4, 64);
+                    if (c4 == 0) nb_s[buf][s_row] = sq;
+                }
+                // barrier i: tile i is in LDS; the other waves then multiply it while tile i + 1 is staged into
+                // the copy that they left before barrier i
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                tile += step;
+            });
+        return;
+    }
+
+    // waves 0 .. 3: 32 queries each (a wave without any keeps the barriers).  Lane's query q0 + lane % 32,
+    // columns 16 ks + 8 (lane / 32) .. + 7 of step ks.
+    const int q0 = blockIdx.y * (32 * PT_WAVES) + 32 * wave;
+    const bool active = q0 < p.n_query;
+    floatx4 fa[2 * NS][3];
+    float na = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 2 * NS; ++ks) {
+        const float* row = p.a + (size_t)min(q0 + (lane & 31), p.n_query - 1) * Dp;
+        uint2 piece[2][3];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int k = 16 * ks + 8 * (lane >> 5) + 4 * h;
+            float4 v = *reinterpret_cast<const float4*>(row + min(k, Dp - 4));
+            if (k >= Dp) v = make_float4(0.f, 0.f, 0.f, 0.f);
+            na += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+            split4_bf16(as_x4(v), piece[h]);
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+            fa[ks][q] = __builtin_bit_cast(floatx4, uint4{piece[0][q].x, piece[0][q].y, piece[1][q].x, piece[1][q].y});
+        if (ks < kL) fa2_s[wave][ks][lane] = fa[ks][2];
+    }
+    if (DIST == DIST_L2) {
+        na += __shfl_xor(na, 32, 64);
+        if (lane < 32) na_s[32 * wave + lane] = na;  // (read by this wave alone)
+    }
+    for (int buf = 0; tile < n_tile; tile += step, buf ^= 1) {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (!active) continue;
+        const char* const cur = smem + buf * kBuf;
+        floatx16 acc[2];  // in turn: an instruction does not wait for the one before it
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.f;
+        floatx4 fb[2][3], f2[2];  // this step's and the next one's
+#pragma unroll
+        for (int q = 0; q < 3; ++q) fb[0][q] = Tile::fragment(cur, q, 0, 0, lane);
+        if (kL) f2[0] = fa2_s[wave][0][lane];
+#pragma unroll
+        for (int ks = 0; ks < 2 * NS; ++ks) {
+            if (ks + 1 < 2 * NS)
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    fb[(ks + 1) & 1][q] = Tile::fragment(cur + (ks + 1) / 2 * Tile::kBytes, q, 0, (ks + 1) & 1, lane);
+            if (ks + 1 < kL) f2[(ks + 1) & 1] = fa2_s[wave][ks + 1][lane];
+            const floatx4 f[3] = {fa[ks][0], fa[ks][1], ks < kL ? f2[ks & 1] : fa[ks][2]};
+            constexpr int qa[6] = {0, 2, 1, 0, 1, 0}, qb[6] = {2, 0, 1, 1, 0, 0};  // smallest first
+#pragma unroll
+            for (int x = 0; x < 6; ++x)
+                acc[x & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, f[qa[x]]),
+                                                                     __builtin_bit_cast(bf16x8, fb[ks & 1][qb[x]]),
+                                                                     acc[x & 1], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);  // the reads stay a step ahead of their use
+        }
+
+        // register r of lane l: query 8 (r / 4) + 4 (l / 32) + r % 4, row l % 32
+        const int n = tile * PT_ROWS + (lane & 31), hl = lane >> 5;
+        const float nb = DIST == DIST_L2 ? nb_s[buf][lane & 31] : 0.f;
+        float val[16];
+        uint32_t cancel = 0u;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = 8 * (r >> 2) + 4 * hl + (r & 3);
+            val[r] = acc[0][r] + acc[1][r];
+            if (DIST == DIST_L2) {
+                const float ns = na_s[32 * wave + m] + nb;
+                val[r] = ns - 2.f * val[r];
+                if (n < p.n_row && q0 + m < p.n_query && val[r] < kCancelRatio * ns) cancel |= 1u << r;
+            }
+        }
+        // rare: the wave recomputes the cancelled pairs directly, two pairs at a time, 32 lanes to a pair
+        if (DIST == DIST_L2) {
+            uint64_t owners;
+            while ((owners = __ballot(cancel != 0u)) != 0) {
+                const int l0 = __ffsll((long long)owners) - 1;
+                const uint64_t rest = owners & (owners - 1);
+                const int l1 = rest ? __ffsll((long long)rest) - 1 : l0;
+                const int src = hl ? l1 : l0;
+                const int fr = __ffs((int)__shfl(cancel, src, 64)) - 1;
+                const float* ar = p.a + (size_t)(q0 + 8 * (fr >> 2) + 4 * (src >> 5) + (fr & 3)) * Dp;
+                const char* br = p.b.base + (int64_t)(tile * PT_ROWS + (src & 31)) * p.b.pitch;
+                float part = 0.f;
+                for (int k = (lane & 31) * 4; k < Dp; k += 128) {
+                    const float4 x = *reinterpret_cast<const float4*>(ar + k), y = load4(br, k, ET);
+                    const float dx = x.x - y.x, dy = x.y - y.y, dz = x.z - y.z, dw = x.w - y.w;
+                    part += dx * dx + dy * dy + dz * dz + dw * dw;
+                }
+#pragma unroll
+                for (int o = 16; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
+                const float v0 = __shfl(part, 0, 64), v1 = __shfl(part, 32, 64);
+                if (lane == l0 || lane == l1) {
+                    const uint32_t bit = cancel & (0u - cancel);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if ((bit >> r) & 1u) val[r] = lane == l0 ? v0 : v1;
+                    cancel ^= bit;
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = q0 + 8 * (r >> 2) + 4 * hl + (r & 3);
+            const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(fmaxf(val[r], 0.f)) : val[r];
+            if (m < p.n_query && n < p.n_row) p.scores[(size_t)m * p.ldc + n] = p.distance_value ? dist : p.gamma - dist;
+        }
+    }
+}
+
+// Whether launch_predict_scores takes a sweep.  Up to 256 columns, as many as the registers hold the
+// queries of; L2 and dot only (L1 has no product form), by bfloat16 pieces only.
+bool predict_scores_takes(const ScoreShape& sh) {
+    if (sh.use_mfma != 2 || sh.score_fn == SCORE_TRANSH || sh.Dp > 256) return false;
+    return sh.score_fn == SCORE_DISTMULT || sh.dist_fn != DIST_L1;
+}
+
+// scores[q * ldc + r] of queries a [sh.B, Dp] against rows 0 .. n_row - 1 of `b` (16-byte aligned sections)
+void launch_predict_scores(const ScoreShape& sh, const float* a, const RowSource& b, int n_row, float* scores, int ldc,
+                           hipStream_t stream) {
+    PredictArgs p = {a, b, scores, sh.B, n_row, ldc, sh.Dp, score_is_distance_value(sh.score_fn) ? 1 : 0, sh.gamma};
+    const bool l2 = sh.score_fn != SCORE_DISTMULT && sh.dist_fn == DIST_L2;
+    // A workgroup fills its CU and stays for the launch, so the merge of the chunk before (a workgroup per
+    // query, two to a CU) needs CUs of its own beside it: 1M rows for 128 queries on all 256 CUs 0.90 ms,
+    // on 192 0.73.  What is left is divided among the groups of 128 queries, whose workgroups walk the
+    // same tiles at the same time.
+    const int groups = (sh.B + 32 * PT_WAVES - 1) / (32 * PT_WAVES), cus = 256 - std::min(64, (sh.B + 1) / 2);
+    const dim3 grid((unsigned)std::min(std::max(1, cus / groups), (n_row + PT_ROWS - 1) / PT_ROWS), (unsigned)groups);
+#define KGE_PS(D_, E_, N_) hipLaunchKernelGGL((k_predict_scores<D_, E_, N_>), grid, dim3(2 * PT_WAVES * 64), 0, stream, p)
+#define KGE_PS_N(D_, E_)                                                                    \
+    do {                                                                                    \
+        if (sh.Dp <= 64) KGE_PS(D_, E_, 2); else if (sh.Dp <= 128) KGE_PS(D_, E_, 4);       \
+        else if (sh.Dp <= 192) KGE_PS(D_, E_, 6); else KGE_PS(D_, E_, 8);                   \
+    } while (0)
+#define KGE_PS_E(D_)                                                                        \
+    do {                                                                                    \
+        if (b.etype == ET_F32) KGE_PS_N(D_, ET_F32);                                        \
+        else if (b.etype == ET_BF16) KGE_PS_N(D_, ET_BF16); else KGE_PS_N(D_, ET_F16);      \
+    } while (0)
+    if (l2) KGE_PS_E(DIST_L2); else KGE_PS_E(DIST_DOT);
+#undef KGE_PS
+#undef KGE_PS_N
+#undef KGE_PS_E
+}
+
+}  // namespace kge

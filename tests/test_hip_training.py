@@ -242,6 +242,42 @@ def test_predict_vs_brute_force(variant):
     assert agree.mean() > 0.99
 
 
+@pytest.mark.parametrize("score_fn", ["TransE", "DistMult"])
+@pytest.mark.parametrize("dim,dtype,n_query,n_entity", [
+    (4, "float32", 1, 6), (62, "float32", 33, 34), (64, "float16", 32, 33), (66, "float32", 130, 1000),
+    (128, "bfloat16", 3, 65), (130, "float16", 129, 97), (192, "float32", 40, 8225), (250, "float16", 5, 500),
+    (256, "float32", 257, 6000), (256, "bfloat16", 128, 9000), (260, "float32", 7, 300)])
+def test_predict_sweep_edges(score_fn, dim, dtype, n_query, n_entity):
+    """The sweep kernel at the edges of its tiles (32 rows, groups of 32 and of 128 queries), of its
+    column slabs (64 at a time up to 256; 260 takes the general kernels) and for every row type."""
+    import poplar_kge as kge
+    from oracle.kge_oracle import predict_reference
+
+    settings = kge.Settings.create_demo()
+    settings.seed = 7
+    m, ex = settings.model, settings.execution
+    m.score_fn, m.distance_fn = score_fn, "L2" if score_fn == "TransE" else "MatMul"
+    m.n_shard, m.n_entity, m.embedding_size, m.entity_feature_size = 1, n_entity, dim, 0
+    settings.data.batch_size, settings.data.a2a_size, ex.rw_batch_size = 2, 2, 4096
+    ex.predict_hr_batch_size, ex.predict_n_best, ex.predict_chunk_rows = n_query, 4, 4096
+    if dtype == "float16":
+        ex.dtype = "float16"
+    elif dtype == "bfloat16":
+        ex.embedding_dtype = "bfloat16"
+    settings.prepare()
+    counts = np.array([n_entity - 1])
+    engine = kge.Engine(settings, counts)
+    engine.initialise_all(np.zeros((1, n_entity, 0), np.float16))
+    state = _oracle_state(engine.read_all())
+    queries = _random_queries(engine, n_query)
+    found = engine.predict(queries)
+    want_idx, want_score = predict_reference(_oracle_cfg(settings), state, queries, counts, 4)
+    np.testing.assert_allclose(found.score, want_score, rtol=1e-5, atol=1e-5)
+    agree = np.all(found.shard_idx == want_idx, axis=-1)
+    close = np.abs(found.score - want_score) <= 1e-5 * np.maximum(1.0, np.abs(want_score))
+    assert np.all(agree | close)
+
+
 @pytest.mark.parametrize("chunk_rows", [None, 4096])
 def test_predict_ties_go_to_the_lower_row(chunk_rows):
     """All embeddings zero: every tail scores the same, so each tail shard's n_best are its
