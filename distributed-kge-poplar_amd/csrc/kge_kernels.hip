@@ -1140,59 +1140,63 @@ __global__ __launch_bounds__(256) void k_loss_rows(ScoreShape sh, const uint32_t
     const float* mu = sh.tmult ? sh.tmult + (size_t)blk * T : nullptr;
     float loss = 0.f;
     if (sh.loss_fn == LOSS_SOFTMAX && (T & 3) == 0 && T <= 2048) {
-        // the row stays in registers (up to eight float4 per lane): one read, one write
+        // The row stays in registers (up to eight float4 per lane): one read, one write, one exponential
+        // per column.  All loads are asked for before any is used (in the loop that used them, each was a
+        // round trip of its own), and the label's column, which every lane knows, has a load and the
+        // two exponentials of its position to itself instead of a branch per column.  8192 rows of about 1040
+        // live columns with bfloat16 coefficients: 22.4 -> 17.2 us.
         const float corr = sh.softmax_correction;
         constexpr int NV = 8;
         floatx4 z[NV], m[NV];
-        float mx = -INFINITY;
+        const bool has_label = label < (uint32_t)TL;  // (the stand-alone loss takes labels as they come)
+        const float z_label = has_label ? s[label] : -INFINITY;
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const int t = 4 * lane + 256 * i;
-            if (t < TL) {
+            const int t = min(4 * lane + 256 * i, T - 4);  // (past the end: the row's last columns, masked below)
+            z[i] = m[i] = floatx4{1.f, 1.f, 1.f, 1.f};
+            if (256 * i < TL) {
                 z[i] = *reinterpret_cast<const floatx4*>(s + t);
-                m[i] = mu ? *reinterpret_cast<const floatx4*>(mu + t) : floatx4{1.f, 1.f, 1.f, 1.f};
-#pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    const bool pos = (uint32_t)(t + x) == label;
-                    if (m[i][x] == 0.f) z[i][x] = -INFINITY;  // no position holds this column
-                    if (!pos || m[i][x] > 1.f) mx = fmaxf(mx, z[i][x] + corr);
-                    if (pos) mx = fmaxf(mx, z[i][x]);
-                }
+                if (mu) m[i] = *reinterpret_cast<const floatx4*>(mu + t);
             }
         }
+        float mx = z_label;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            if (256 * i < TL) {
+                const int t = 4 * lane + 256 * i;
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    // m becomes the column's negatives: all its positions, or all but the label's
+                    m[i][x] = t < TL ? m[i][x] - ((uint32_t)(t + x) == label ? 1.f : 0.f) : 0.f;
+                    if (m[i][x] > 0.f) mx = fmaxf(mx, z[i][x] + corr);
+                }
+            }
         mx = wave_max(mx);
         float sum = 0.f;
 #pragma unroll
         for (int i = 0; i < NV; ++i)
-            if (4 * lane + 256 * i < TL)
+            if (256 * i < TL)
 #pragma unroll
                 for (int x = 0; x < 4; ++x) {
-                    const bool pos = (uint32_t)(4 * lane + 256 * i + x) == label;
-                    const float neg = m[i][x] - (pos ? 1.f : 0.f);
-                    if (neg > 0.f) sum += neg * __expf(z[i][x] + corr - mx);
-                    if (pos) sum += __expf(z[i][x] - mx);
+                    z[i][x] = m[i][x] > 0.f ? m[i][x] * __expf(z[i][x] + corr - mx) : 0.f;
+                    sum += z[i][x];
                 }
-        sum = wave_sum(sum);
-        const float lse = mx + logf(sum);
+        const float e_label = __expf(z_label - mx);
+        sum = wave_sum(sum) + e_label;
+        const float inv_sum = 1.f / sum, lse = mx + logf(sum);
         const float inv_norm = 1.f / ((float)sh.S * (float)sh.B);
         const float gs = inv_norm * sh.loss_scale;
         const float sgn = score_is_distance_value(sh.score_fn) ? 1.f : -1.f;
+        const float g_label = e_label * inv_sum - 1.f;
+        if (lane == 0 && has_label) loss = -(z_label - lse) * inv_norm;
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int t = 4 * lane + 256 * i;
             if (t < TL) {
                 floatx4 c;
 #pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    const bool pos = (uint32_t)(t + x) == label;
-                    const float neg = m[i][x] - (pos ? 1.f : 0.f);
-                    float g = neg > 0.f ? neg * __expf(z[i][x] + corr - lse) : 0.f;
-                    if (pos) {
-                        loss = -(z[i][x] - lse) * inv_norm;
-                        g += __expf(z[i][x] - lse) - 1.f;
-                    }
-                    c[x] = sgn * g * gs;
-                }
+                for (int x = 0; x < 4; ++x)
+                    c[x] = sgn * (z[i][x] * inv_sum + ((uint32_t)(t + x) == label ? g_label : 0.f)) * gs;
                 if (dr) {
                     const floatx4 dv = *reinterpret_cast<const floatx4*>(dr + t);
 #pragma unroll
