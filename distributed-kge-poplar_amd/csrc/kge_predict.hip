@@ -50,7 +50,8 @@ DEVINL float4 raw4_f32(const Raw4<ET>& r) {
 template <int DIST, int ET, int NS>  // ET: the rows' element type, NS: slabs of 32 columns
 __global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(PredictArgs p) {
     using Tile = RowTile<PT_ROWS>;
-    constexpr int PF = 4, kL = NS == 8 ? 12 : 0;  // kL: steps whose queries' third piece waits in LDS (registers: 256)
+    constexpr int PF = 4;                    // tiles asked for ahead (even: a register set stays with its LDS copy)
+    constexpr int kL = NS == 8 ? 12 : 0;     // steps whose queries' third piece waits in LDS: 256 registers are not enough
     constexpr int kBuf = NS * Tile::kBytes;
     __shared__ __attribute__((aligned(16))) char smem[2 * kBuf];
     __shared__ float na_s[32 * PT_WAVES], nb_s[2][PT_ROWS];
