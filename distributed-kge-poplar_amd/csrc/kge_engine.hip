@@ -701,7 +701,8 @@ void allocate(kge_engine& E) {
     E.grad.alloc(R * E.Dp);
     if (E.split) {
         E.Kp = round_up(E.Dp, 32); E.Bp = round_up(E.B, 32); E.Tp = round_up(E.T, 32);
-        // rows and columns that no kernel writes are read and dropped or multiplied by zero: finite
+        // rows and columns that no kernel writes are read and dropped, or (columns filled up to whole
+        // slabs) multiplied by each other: zeros
         E.rowsp.alloc(split_bytes(R, E.Kp));
         E.rowsp.zero(st);
         E.coefp.alloc(split_bytes(S * E.Bp, E.Tp));

@@ -100,12 +100,13 @@ template <int C>
 struct ColTile {
     static constexpr int kBytes = 3 * 32 * C * 2, kCopies = 3 * C / 16;
     static constexpr int kKey = C >= 128 ? 3 : 1;  // (a row of 64 columns has four units)
-    static DEVINL uint32_t source(int x, int lane, int pitch) {
+    // (rows past `last` repeat it)
+    static DEVINL uint32_t source(int x, int lane, int pitch, int last = 31) {
         constexpr int chunks = C / 8, rows = 64 / chunks;
         const int piece = x / (C / 16), row = (x % (C / 16)) * rows + lane / chunks, pos = lane % chunks;
         const int chunk = pos ^ ((row & kKey) << 2);  // 16-byte chunks: two to a unit
         const int col = chunk * 8;
-        return (uint32_t)(row * pitch + (col >> 5) * 192 + piece * 64 + (col & 31) * 2);
+        return (uint32_t)(min(row, last) * pitch + (col >> 5) * 192 + piece * 64 + (col & 31) * 2);
     }
     // columns col0 .. col0 + 31 over the sixteen rows of step `ks` (this lane: column
     // col0 + lane % 32, rows 8 (lane / 32) .. + 7)

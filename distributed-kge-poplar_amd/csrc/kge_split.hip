@@ -107,6 +107,9 @@ void launch_gather_pieces(const RowSource& ent, const float* rel, const uint32_t
 // (one fills while the other is multiplied, one barrier per slab).  TA, TB: RowTile / ColTile;
 // a_step, b_step: bytes from slab to slab.  Waves as WM x WN, each (TM/WM) x (TN/WN) in 32 x 32
 // accumulators.
+// b_rows: rows of `b` along the contraction where it lies across it (ColTile).  The last slab's rows past them
+// repeat the last one: their coefficients are zero, but what lies behind a block's rows are other
+// blocks', and zero times a neighbour's infinity or NaN would be this block's NaN.
 template <class TA, class TB, int TM, int TN, int WM, int WN>
 struct SplitProduct {
     static constexpr int NW = WM * WN, AM = TM / WM / 32, AN = TN / WN / 32;
@@ -117,7 +120,7 @@ struct SplitProduct {
     // meanwhile(): what the caller has to fetch for itself, under the first slab's way from memory
     template <class Meanwhile>
     static DEVINL void run(char* smem, const char* a, int a_pitch, size_t a_step, const char* b, int b_pitch, size_t b_step,
-                           int n_slab, floatx16 (&acc)[AM][AN], int lane, int wave, Meanwhile&& meanwhile) {
+                           int n_slab, int b_rows, floatx16 (&acc)[AM][AN], int lane, int wave, Meanwhile&& meanwhile) {
         uint32_t off[kEach];
 #pragma unroll
         for (int i = 0; i < kEach; ++i) {
@@ -129,6 +132,15 @@ struct SplitProduct {
             const char* as = a + slab * a_step;
             const char* bs = b + slab * b_step;
             const uint32_t to = lds0 + (slab & 1) * kStage;
+            if constexpr (!std::is_same_v<TB, RowTile<TN>>) {
+                const int last = b_rows - 32 * slab - 1;
+                if (last < 31)  // the last slab's offsets take the others' place
+#pragma unroll
+                    for (int i = 0; i < kEach; ++i) {
+                        const int x = wave + NW * i;
+                        if (x >= TA::kCopies) off[i] = TB::source(x - TA::kCopies, lane, b_pitch, last);
+                    }
+            }
 #pragma unroll
             for (int i = 0; i < kEach; ++i) {
                 const int x = wave + NW * i;
@@ -268,7 +280,7 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
         for (int n = 0; n < P::AN; ++n)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
-    P::run(smem, a, pitch, 192, b, pitch, 192, Kp / 32, acc, lane, wave, [&]() __attribute__((always_inline)) {
+    P::run(smem, a, pitch, 192, b, pitch, 192, Kp / 32, 0, acc, lane, wave, [&]() __attribute__((always_inline)) {
         for (int i = tid; i < TM; i += WM * WN * 64) {
             if (DIST == DIST_L2) na_s[i] = p.norm_a[a_row + m0 + i];
             if (OM == 0) label_s[i] = m0 + i < B ? p.clabel[d * B + m0 + i] : 0u;
@@ -423,7 +435,7 @@ DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, cha
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int B = p.B, T = p.T, Bp = p.in.Bp, Tp = p.in.Tp, MT = Bp >> 5, NT = Tp >> 5, pitch = p.Kp * 6;
     const int t_live = tail_limit(p.tcount, d, T, p.tpad);  // merged tails: the block's live columns
-    const int n_self = SIDE_B ? t_live : B, n_slab = ((SIDE_B ? B : t_live) + 31) >> 5;
+    const int n_self = SIDE_B ? t_live : B, n_other = SIDE_B ? B : t_live, n_slab = (n_other + 31) >> 5;
     if (i0 >= n_self) return;
     const int head0 = d * B, tail0 = p.b_c0 + d * T, self0 = SIDE_B ? tail0 : head0, other0 = SIDE_B ? head0 : tail0;
     const char* const coef = p.in.coefp + (size_t)d * Bp * Tp * 6;
@@ -439,7 +451,7 @@ DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, cha
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
     uint32_t seen = 0u;  // flagged blocks among the tile's
-    P::run(smem, a, Tp * 6, SIDE_B ? (size_t)32 * Tp * 6 : 192, b, pitch, (size_t)32 * pitch, n_slab, acc, lane, wave,
+    P::run(smem, a, Tp * 6, SIDE_B ? (size_t)32 * Tp * 6 : 192, b, pitch, (size_t)32 * pitch, n_slab, n_other, acc, lane, wave,
            [&]() __attribute__((always_inline)) {
                if (DIST != DIST_L2) return;
                // the self rows' coefficient sums, from the sub-blocks' in a fixed order
@@ -480,7 +492,7 @@ DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, cha
 #pragma unroll
                     for (int r = 0; r < 16; ++r)
                         sv[r] = load_piece1(self + (int64_t)(wm + 32 * mi + 8 * (r >> 2) + 4 * hl + (r & 3)) * pitch, k);
-                    for (int j = 32 * ot; j < min(32 * ot + 32, SIDE_B ? B : t_live); ++j) {
+                    for (int j = 32 * ot; j < min(32 * ot + 32, n_other); ++j) {
                         const float o = load_piece1(other + (int64_t)j * pitch, k);
 #pragma unroll
                         for (int r = 0; r < 16; ++r) {

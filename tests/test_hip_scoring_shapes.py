@@ -1,6 +1,9 @@
 """The scoring kernels away from whole tiles, against the float64 oracle through the training step:
 sizes around the edges of tiles and groups, one row, splits of a side over several workgroups."""
 
+import hip_harness as H
+import kge_cases as K
+import numpy as np
 import pytest
 
 from test_hip_step import run_case
@@ -41,3 +44,45 @@ def test_l1_shapes(oracle64, S, B, A, D, merge):
 def test_l2_and_dot_shapes(oracle64, score_fn, distance_fn, loss_fn, S, B, A, D, merge):
     run_case(oracle64, dict(score_fn=score_fn, distance_fn=distance_fn, loss_fn=loss_fn, n_shard=S, batch=B, a2a=A, dim=D,
                             feature=0, n_entity=1500, n_relation=6, gamma=4.0), n_step=2, **{"execution.merge_tails": merge})
+
+
+def _two_disjoint_blocks(kind, loss_fn, B, A, D, bad, merge):
+    """One step of two blocks that share no row (entity or relation); `bad`: (role, value) of block 1's
+    first head or tail, or None.  Returns the losses and block 0's rows afterwards."""
+    import libpoplar_kge
+
+    c = K.cfg_dict(score_fn="TransE" if kind != "MatMul" else "DistMult", distance_fn=kind, loss_fn=loss_fn, shared_table=True,
+                   n_shard=2, batch=B, a2a=A, dim=D, feature=0, n_entity=2 * (B + 2 * A) + 1, n_relation=2 * B, gamma=4.0)
+    rng = np.random.default_rng(3)
+    state = K.make_state(c, rng)
+    N = B + 2 * A
+    remote = (1 + np.arange(2 * N, dtype=np.uint32)).reshape(2, 1, N)
+    a2a = np.broadcast_to((B + np.arange(2 * A, dtype=np.uint32)).reshape(2, A), (2, 1, 2, A))
+    batch = dict(remote=remote, a2a=a2a, head=np.broadcast_to(np.arange(B, dtype=np.uint32), (2, 1, B)),
+                 relation=np.arange(2 * B, dtype=np.uint32).reshape(2, 1, B),
+                 tail=rng.integers(0, 2 * A, (2, 1, B)).astype(np.uint32))
+    if bad:
+        state["entity_data"][remote[1, 0, 0] if bad[0] == "head" else remote[0, 0, B + A], min(3, D - 1)] = bad[1]
+    engine = libpoplar_kge.Engine(H.engine_settings(c, 1, **{"execution.merge_tails": merge}), "")
+    H.load_state(engine, c, state)
+    loss = H.train(engine, c, 0.1, batch)
+    after = H.read_state(engine, c)
+    rows = np.concatenate([remote[0, 0, :B], remote[0, 0, B:B + A], remote[1, 0, B:B + A]])  # block 0's heads, its tails
+    return loss, after["entity_data"][rows], after["relation_embedding"][:B]
+
+
+# A block's last slab of 32 rows may reach into the next block's: nothing of that block may enter.
+# (33, 42): both sides ragged, the head slab of block 0 reads block 1's heads, its tail slab block 1's tails
+# (64, 42), (33, 64): one side whole
+@pytest.mark.parametrize("kind", ["L2", "MatMul", "L1"])
+@pytest.mark.parametrize("loss_fn,merge", [("logsigmoid", True), ("softmax", True), ("logsigmoid", False)])
+@pytest.mark.parametrize("B,A,D", [(33, 21, 30), (64, 21, 64), (33, 32, 64), (1, 1, 2)])
+def test_nonfinite_row_stays_in_its_block(kind, loss_fn, merge, B, A, D):
+    clean = _two_disjoint_blocks(kind, loss_fn, B, A, D, None, merge)
+    assert all(np.isfinite(x).all() for x in clean)
+    for role in ("head", "tail"):
+        for value in (np.inf, -np.inf, np.nan):
+            got = _two_disjoint_blocks(kind, loss_fn, B, A, D, (role, value), merge)
+            assert got[0][0] == clean[0][0]
+            np.testing.assert_array_equal(got[1], clean[1])
+            np.testing.assert_array_equal(got[2], clean[2])
