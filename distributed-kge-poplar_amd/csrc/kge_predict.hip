@@ -177,14 +177,18 @@ __global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(Predict
         for (int r = 0; r < 16; ++r) {
             const int m = 8 * (r >> 2) + 4 * hl + (r & 3);
             val[r] = acc[0][r] + acc[1][r];
+            bool good = fabsf(val[r]) < INFINITY;  // (dot)
             if (DIST == DIST_L2) {
                 const float ns = na_s[32 * wave + m] + nb;
                 val[r] = ns - 2.f * val[r];
-                if (n < p.n_row && q0 + m < p.n_query && val[r] < kCancelRatio * ns) cancel |= 1u << r;
+                good = val[r] >= kCancelRatio * ns;
             }
+            if (!good && n < p.n_row && q0 + m < p.n_query) cancel |= 1u << r;
         }
-        // rare: the wave recomputes the cancelled pairs directly, two pairs at a time, 32 lanes to a pair
-        if (DIST == DIST_L2) {
+        // rare: the wave recomputes pairs directly, two at a time, 32 lanes to a pair: those that
+        // cancelled, and those that are not finite (an infinity's pieces are infinity and NaN; from the
+        // values themselves its distance is infinite and its row comes last, not, as NaN clamped to 0, first)
+        {
             uint64_t owners;
             while ((owners = __ballot(cancel != 0u)) != 0) {
                 const int l0 = __ffsll((long long)owners) - 1;
@@ -197,8 +201,12 @@ __global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(Predict
                 float part = 0.f;
                 for (int k = (lane & 31) * 4; k < Dp; k += 128) {
                     const float4 x = *reinterpret_cast<const float4*>(ar + k), y = load4(br, k, ET);
-                    const float dx = x.x - y.x, dy = x.y - y.y, dz = x.z - y.z, dw = x.w - y.w;
-                    part += dx * dx + dy * dy + dz * dz + dw * dw;
+                    if (DIST == DIST_L2) {
+                        const float dx = x.x - y.x, dy = x.y - y.y, dz = x.z - y.z, dw = x.w - y.w;
+                        part += dx * dx + dy * dy + dz * dz + dw * dw;
+                    } else {
+                        part += x.x * y.x + x.y * y.y + x.z * y.z + x.w * y.w;
+                    }
                 }
 #pragma unroll
                 for (int o = 16; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
@@ -215,7 +223,9 @@ __global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(Predict
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int m = q0 + 8 * (r >> 2) + 4 * hl + (r & 3);
-            const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(fmaxf(val[r], 0.f)) : val[r];
+            // (no squared distance is negative here: what is small was recomputed; a NaN stays one, and
+            // the merge takes none)
+            const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[r]) : val[r];
             if (m < p.n_query && n < p.n_row) p.scores[(size_t)m * p.ldc + n] = p.distance_value ? dist : p.gamma - dist;
         }
     }

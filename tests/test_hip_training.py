@@ -278,6 +278,60 @@ def test_predict_sweep_edges(score_fn, dim, dtype, n_query, n_entity):
     assert np.all(agree | close)
 
 
+@pytest.mark.parametrize("score_fn", ["TransE", "DistMult"])
+@pytest.mark.parametrize("dim,dtype", [(30, "float32"), (64, "float16"), (100, "float32"), (130, "float16"), (256, "float32")])
+def test_predict_sweep_nonfinite_rows(score_fn, dim, dtype):
+    """A row with an infinite element scores what its own terms add up to (L2: minus infinity; dot: the
+    infinity of the product's sign), a row with a NaN ranks nowhere, and no other row's or query's
+    list changes."""
+    import poplar_kge as kge
+
+    settings = kge.Settings.create_demo()
+    m, ex = settings.model, settings.execution
+    m.score_fn, m.distance_fn = score_fn, "L2" if score_fn == "TransE" else "MatMul"
+    m.n_shard, m.n_entity, m.embedding_size, m.entity_feature_size, m.n_relation_type = 1, 301, dim, 0, 4
+    settings.data.batch_size, settings.data.a2a_size, ex.rw_batch_size = 2, 2, 301
+    ex.dtype, ex.predict_hr_batch_size, ex.predict_n_best = dtype, 40, 300
+    settings.prepare()
+    engine = kge.Engine(settings, np.array([300]))
+    rng = np.random.default_rng(8)
+    rows = np.zeros((1, 301, 3 * dim), np.float32)
+    rows[0, :, :dim] = rng.integers(1, 5, (301, dim)) * rng.choice([-0.25, 0.25], (301, dim))  # exact, never 0
+    relation = rng.integers(1, 5, (4, dim)).astype(np.float32) * 0.25
+    for name in engine.uninitialized_variables.copy():
+        engine.write_variable(name, np.zeros(engine.variable_to_shape[name], engine.variable_to_dtype[name]))
+    engine.write_variable("relation_embedding", relation)
+    queries = np.stack([np.zeros(40), 1 + np.arange(40), np.arange(40) % 4], axis=1).astype(np.uint32)
+    engine.write_entity_raw(0, rows)
+    clean = engine.predict(queries)
+    for value in (np.inf, -np.inf, np.nan):
+        bad = rows.copy()
+        bad[0, 200, dim // 2] = value  # no query's head
+        bad[0, 299, dim - 1] = value
+        engine.write_entity_raw(0, bad)
+        found = engine.predict(queries)
+        head, rel = rows[0, queries[:, 1], :dim], relation[queries[:, 2]]
+        for i in range(40):
+            listed = found.score[i] > -1e6  # (unfilled slots)
+            got = dict(zip(found.shard_idx[i, listed, 1].tolist(), found.score[i, listed].tolist()))
+            want = dict(zip(clean.shard_idx[i, :, 1].tolist(), clean.score[i].tolist()))
+            for row, col in ((200, dim // 2), (299, dim - 1)):
+                want.pop(row)
+                if score_fn == "DistMult" and head[i, col] * rel[i, col] * value == np.inf:
+                    want[row] = np.inf
+            assert got == want
+    # a query that is not finite leaves the others alone
+    bad = rows.copy()
+    bad[0, 1, 0] = np.inf
+    engine.write_entity_raw(0, bad)
+    found = engine.predict(queries)
+    for i in range(1, 40):
+        keep = clean.shard_idx[i, :, 1] != 1
+        listed = (found.shard_idx[i, :, 1] != 1) & (found.score[i] > -1e6)
+        np.testing.assert_array_equal(found.shard_idx[i, listed], clean.shard_idx[i, keep])
+        np.testing.assert_array_equal(found.score[i, listed], clean.score[i, keep])
+
+
 @pytest.mark.parametrize("chunk_rows", [None, 4096])
 def test_predict_ties_go_to_the_lower_row(chunk_rows):
     """All embeddings zero: every tail scores the same, so each tail shard's n_best are its
