@@ -171,62 +171,73 @@ __global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(Predict
         // register r of lane l: query 8 (r / 4) + 4 (l / 32) + r % 4, row l % 32
         const int n = tile * PT_ROWS + (lane & 31), hl = lane >> 5;
         const float nb = DIST == DIST_L2 ? nb_s[buf][lane & 31] : 0.f;
-        float val[16];
-        uint32_t cancel = 0u;
+        auto put = [&](int q, int row, float v) __attribute__((always_inline)) {
+            const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(v) : v;  // (never negative; a NaN stays one)
+            p.scores[(size_t)q * p.ldc + row] = p.distance_value ? dist : p.gamma - dist;
+        };
+        uint32_t again = 0u;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int m = 8 * (r >> 2) + 4 * hl + (r & 3);
-            val[r] = acc[0][r] + acc[1][r];
-            bool good = fabsf(val[r]) < INFINITY;  // (dot)
+            float val = acc[0][r] + acc[1][r];
+            bool good = fabsf(val) < INFINITY;  // (dot)
             if (DIST == DIST_L2) {
                 const float ns = na_s[32 * wave + m] + nb;
-                val[r] = ns - 2.f * val[r];
-                good = val[r] >= kCancelRatio * ns;
+                val = ns - 2.f * val;
+                good = val >= kCancelRatio * ns;
             }
-            if (!good && n < p.n_row && q0 + m < p.n_query) cancel |= 1u << r;
+            if (n < p.n_row && q0 + m < p.n_query) {
+                if (good) put(q0 + m, n, val); else again |= 1u << r;
+            }
         }
-        // rare: the wave recomputes pairs directly, two at a time, 32 lanes to a pair: those that
-        // cancelled, and those that are not finite (an infinity's pieces are infinity and NaN; from the
-        // values themselves its distance is infinite and its row comes last, not, as NaN clamped to 0, first)
-        {
-            uint64_t owners;
-            while ((owners = __ballot(cancel != 0u)) != 0) {
-                const int l0 = __ffsll((long long)owners) - 1;
-                const uint64_t rest = owners & (owners - 1);
-                const int l1 = rest ? __ffsll((long long)rest) - 1 : l0;
-                const int src = hl ? l1 : l0;
-                const int fr = __ffs((int)__shfl(cancel, src, 64)) - 1;
-                const float* ar = p.a + (size_t)(q0 + 8 * (fr >> 2) + 4 * (src >> 5) + (fr & 3)) * Dp;
-                const char* br = p.b.base + (int64_t)(tile * PT_ROWS + (src & 31)) * p.b.pitch;
-                float part = 0.f;
-                for (int k = (lane & 31) * 4; k < Dp; k += 128) {
-                    const float4 x = *reinterpret_cast<const float4*>(ar + k), y = load4(br, k, ET);
+        // rare: the wave computes pairs directly, eight at a time, eight lanes to a pair (two pairs of each
+        // of four lanes; fewer lanes: the last one's again): those that cancelled, and those that are not
+        // finite (an infinity's pieces are infinity and NaN; from the values themselves its distance is
+        // infinite and its row comes last, a NaN's score is NaN and the merge takes none).  Each round is a
+        // ballot, a shuffle and trips to L2, one after the other, which four waves to a CU do not hide: at two
+        // pairs a round, through shuffles back to the lanes whose registers they were, a table whose rows lie
+        // close together (every pair cancelled; 200k x 256 float32, 128 queries) took 12.4 ms.
+        uint64_t owners;
+        while ((owners = __ballot(again != 0u)) != 0) {
+            int own[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                own[i] = owners ? __ffsll((long long)owners) - 1 : own[i ? i - 1 : 0];
+                owners &= owners - 1;
+            }
+            const int src = lane & 32 ? (lane & 16 ? own[3] : own[2]) : (lane & 16 ? own[1] : own[0]);
+            const uint32_t bits = __shfl(again, src, 64), upper = bits & (bits - 1);
+            const int fr = __ffs((int)((lane & 8) && upper ? upper : bits)) - 1;
+            const int q = q0 + 8 * (fr >> 2) + 4 * (src >> 5) + (fr & 3), row = tile * PT_ROWS + (src & 31);
+            const float* ar = p.a + (size_t)q * Dp;
+            const char* br = p.b.base + (int64_t)row * p.b.pitch;
+            float part = 0.f;
+#pragma unroll 1
+            for (int k0 = 4 * (lane & 7); k0 < Dp; k0 += 128) {
+                float4 x[4], y[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {  // four loads of each row under way
+                    const int k = k0 + 32 * i;
+                    x[i] = y[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (k < Dp) { x[i] = *reinterpret_cast<const float4*>(ar + k); y[i] = load4(br, k, ET); }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
                     if (DIST == DIST_L2) {
-                        const float dx = x.x - y.x, dy = x.y - y.y, dz = x.z - y.z, dw = x.w - y.w;
+                        const float dx = x[i].x - y[i].x, dy = x[i].y - y[i].y, dz = x[i].z - y[i].z, dw = x[i].w - y[i].w;
                         part += dx * dx + dy * dy + dz * dz + dw * dw;
                     } else {
-                        part += x.x * y.x + x.y * y.y + x.z * y.z + x.w * y.w;
+                        part += x[i].x * y[i].x + x[i].y * y[i].y + x[i].z * y[i].z + x[i].w * y[i].w;
                     }
                 }
-#pragma unroll
-                for (int o = 16; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
-                const float v0 = __shfl(part, 0, 64), v1 = __shfl(part, 32, 64);
-                if (lane == l0 || lane == l1) {
-                    const uint32_t bit = cancel & (0u - cancel);
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        if ((bit >> r) & 1u) val[r] = lane == l0 ? v0 : v1;
-                    cancel ^= bit;
-                }
             }
-        }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m = q0 + 8 * (r >> 2) + 4 * hl + (r & 3);
-            // (no squared distance is negative here: what is small was recomputed; a NaN stays one, and
-            // the merge takes none)
-            const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[r]) : val[r];
-            if (m < p.n_query && n < p.n_row) p.scores[(size_t)m * p.ldc + n] = p.distance_value ? dist : p.gamma - dist;
+            for (int o = 4; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
+            if ((lane & 7) == 0) put(q, row, part);
+            if (lane == own[0] || lane == own[1] || lane == own[2] || lane == own[3]) {
+                again &= again - 1;
+                again &= again - 1;
+            }
         }
     }
 }

@@ -278,6 +278,37 @@ def test_predict_sweep_edges(score_fn, dim, dtype, n_query, n_entity):
     assert np.all(agree | close)
 
 
+@pytest.mark.parametrize("dim,dtype,n_query,n_entity", [(2, "float32", 33, 40), (64, "float32", 1, 33), (130, "float16", 35, 100),
+                                                        (256, "float32", 130, 290)])
+def test_predict_sweep_close_rows(dim, dtype, n_query, n_entity):
+    """Rows and queries close together and far from zero: the product form cancels for every pair and all
+    are computed directly, for numbers of pairs that fill the kernel's rounds and ones that do not."""
+    import poplar_kge as kge
+    from oracle.kge_oracle import predict_reference
+
+    settings = kge.Settings.create_demo()
+    m, ex = settings.model, settings.execution
+    m.distance_fn, m.n_shard, m.n_entity, m.embedding_size, m.entity_feature_size = "L2", 1, n_entity, dim, 0
+    settings.data.batch_size, settings.data.a2a_size, ex.rw_batch_size = 2, 2, n_entity
+    ex.dtype, ex.predict_hr_batch_size, ex.predict_n_best = dtype, n_query, n_entity - 1
+    settings.prepare()
+    counts = np.array([n_entity - 1])
+    engine = kge.Engine(settings, counts)
+    engine.initialise_all(np.zeros((1, n_entity, 0), np.float16))
+    rng = np.random.default_rng(9)
+    rows = np.zeros((1, n_entity, 3 * dim), np.float32)
+    rows[0, :, :dim] = rng.normal(size=dim) + 0.02 * rng.normal(size=(n_entity, dim))
+    engine.write_entity_raw(0, rows)
+    engine.write_variable("relation_embedding", 0.01 * rng.normal(size=(m.n_relation_type, dim)).astype(np.float32))
+    state = _oracle_state(engine.read_all())
+    queries = _random_queries(engine, n_query)
+    found = engine.predict(queries)
+    _, want_score = predict_reference(_oracle_cfg(settings), state, queries, counts, n_entity - 1)
+    # gamma - dist: a float32 difference of scores near gamma
+    np.testing.assert_allclose(found.score, want_score, rtol=1e-5, atol=1e-5)
+    assert np.all(np.sort(found.shard_idx[:, :, 1], axis=1) == np.arange(1, n_entity))
+
+
 @pytest.mark.parametrize("score_fn", ["TransE", "DistMult"])
 @pytest.mark.parametrize("dim,dtype", [(30, "float32"), (64, "float16"), (100, "float32"), (130, "float16"), (256, "float32")])
 def test_predict_sweep_nonfinite_rows(score_fn, dim, dtype):
