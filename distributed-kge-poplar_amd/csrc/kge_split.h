@@ -34,16 +34,23 @@ DEVINL float swap2(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));
 }
 
-// four columns of a piece-matrix row, k % 4 == 0
+// four columns of a piece-matrix row, k % 4 == 0.  (An infinity's pieces are infinity, NaN, NaN: the first
+// alone is the value.)
 DEVINL float4 load_pieces4(const char* row, int k) {
     const char* p = row + (size_t)(k >> 5) * 192 + (k & 31) * 2;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    const uint2 hi = *reinterpret_cast<const uint2*>(p);
+    float4 v = make_float4(bf16_lo_f32(hi.x), bf16_hi_f32(hi.x), bf16_lo_f32(hi.y), bf16_hi_f32(hi.y));
+    const float4 first = v;
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
+    for (int q = 1; q < 3; ++q) {
         const uint2 raw = *reinterpret_cast<const uint2*>(p + 64 * q);
         v.x += bf16_lo_f32(raw.x); v.y += bf16_hi_f32(raw.x);
         v.z += bf16_lo_f32(raw.y); v.w += bf16_hi_f32(raw.y);
     }
+    if (!(fabsf(first.x) < INFINITY)) v.x = first.x;
+    if (!(fabsf(first.y) < INFINITY)) v.y = first.y;
+    if (!(fabsf(first.z) < INFINITY)) v.z = first.z;
+    if (!(fabsf(first.w) < INFINITY)) v.w = first.w;
     return v;
 }
 DEVINL float load_piece1(const char* row, int k) {

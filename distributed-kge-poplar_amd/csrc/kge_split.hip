@@ -315,18 +315,28 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 val[r] = acc[mi][ni][r];
+                const int m_loc = mb + 8 * (r >> 2) + 4 * hl + (r & 3);
+                const bool live = col_counts && m0 + m_loc < B;
+                bool good = fabsf(val[r]) < INFINITY;  // (dot)
                 if (DIST == DIST_L2) {
-                    const int m_loc = mb + 8 * (r >> 2) + 4 * hl + (r & 3);
                     const float ns = na_s[m_loc] + nb_s[nbk + cl];
                     val[r] = ns - 2.f * val[r];
-                    const bool live = col_counts && m0 + m_loc < B;
-                    if (live && val[r] < kCancelRatio * ns) cancel |= 1u << r;
+                    good = val[r] >= kCancelRatio * ns;
                     if (live && val[r] < kNearRatio * ns) near |= 1u << r;
                 }
+                if (!good) cancel |= 1u << r;
             }
-            // rare: the wave recomputes the cancelled pairs directly, two pairs of each of two lanes at
-            // a time, sixteen lanes to a pair
-            if (DIST == DIST_L2 && __ballot(cancel != 0u)) {
+            // rare: the wave recomputes pairs directly, two pairs of each of two lanes at a time, sixteen
+            // lanes to a pair: those that cancelled, and those that are not finite (an infinity's second
+            // piece is NaN, which the clamp below would make a distance of zero and a finite loss).  Pairs
+            // that do not count, a NaN among them, get any finite value.
+            if (__ballot(cancel != 0u)) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (!(col_counts && m0 + mb + 8 * (r >> 2) + 4 * hl + (r & 3) < B)) {
+                        val[r] = 0.f;
+                        cancel &= ~(1u << r);
+                    }
                 near = 0u;
                 uint32_t left = cancel;
                 uint64_t owners;
@@ -342,8 +352,12 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
                     float part = 0.f;
                     for (int k = (lane & 15) * 4; k < Kp; k += 64) {
                         const float4 x = load_pieces4(ar, k), y = load_pieces4(br, k);
-                        const float dx = x.x - y.x, dy = x.y - y.y, dz = x.z - y.z, dw = x.w - y.w;
-                        part += dx * dx + dy * dy + dz * dz + dw * dw;
+                        if (DIST == DIST_L2) {
+                            const float dx = x.x - y.x, dy = x.y - y.y, dz = x.z - y.z, dw = x.w - y.w;
+                            part += dx * dx + dy * dy + dz * dz + dw * dw;
+                        } else {
+                            part += x.x * y.x + x.y * y.y + x.z * y.z + x.w * y.w;
+                        }
                     }
 #pragma unroll
                     for (int o = 8; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
@@ -363,7 +377,8 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int m_loc = mb + 8 * (r >> 2) + 4 * hl + (r & 3);
-                    if (col_counts && m0 + m_loc < B && val[r] < kNearRatio * (na_s[m_loc] + nb_s[nbk + cl])) near |= 1u << r;
+                    if (DIST == DIST_L2 && col_counts && m0 + m_loc < B && val[r] < kNearRatio * (na_s[m_loc] + nb_s[nbk + cl]))
+                        near |= 1u << r;
                 }
             }
             const bool flagged = DIST == DIST_L2 && __ballot(near != 0u) != 0;

@@ -86,3 +86,34 @@ def test_nonfinite_row_stays_in_its_block(kind, loss_fn, merge, B, A, D):
             assert got[0][0] == clean[0][0]
             np.testing.assert_array_equal(got[1], clean[1])
             np.testing.assert_array_equal(got[2], clean[2])
+
+
+# An infinite element must show in the block's loss (L2: distances to it are infinite, dot: products
+# are; logsigmoid's sum holds 0 x infinity), and with whole columns that stand for no tail (repeats of the
+# block's first tail) the gradients' other columns stay finite
+@pytest.mark.parametrize("kind", ["L2", "MatMul"])
+@pytest.mark.parametrize("B,A,D", [(33, 21, 30), (8, 100, 64), (130, 65, 100)])
+def test_infinite_row_shows_in_the_loss(kind, B, A, D):
+    for role in ("head", "tail"):
+        for value in (np.inf, -np.inf):
+            loss = _two_disjoint_blocks(kind, "logsigmoid", B, A, D, (role, value), True)[0]
+            assert np.isfinite(loss[0]) and not np.isfinite(loss[1]), (role, value, loss)
+
+
+def test_infinite_first_tail_keeps_to_its_column(oracle64):
+    import libpoplar_kge
+
+    S, B, A, D = 1, 20, 70, 24
+    c = K.cfg_dict(score_fn="DistMult", distance_fn="MatMul", shared_table=True, n_shard=S, batch=B, a2a=A, dim=D, feature=0,
+                   n_entity=100, n_relation=20, gamma=4.0)
+    state = K.make_state(c, np.random.default_rng(3))
+    remote = np.concatenate([np.arange(60, 60 + B), np.resize(np.arange(1, 11), A)]).astype(np.uint32).reshape(1, 1, B + A)
+    batch = dict(remote=remote, a2a=(B + np.arange(A, dtype=np.uint32)).reshape(1, 1, 1, A),
+                 head=np.arange(B, dtype=np.uint32).reshape(1, 1, B), relation=np.arange(B, dtype=np.uint32).reshape(1, 1, B),
+                 tail=np.zeros((1, 1, B), np.uint32) + 3)
+    state["entity_data"][1, 5] = np.inf  # ten distinct tails of 70: the columns behind them repeat row 1
+    engine = libpoplar_kge.Engine(H.engine_settings(c, 1), "")
+    H.load_state(engine, c, state)
+    H.train(engine, c, 0.1, batch)
+    heads = H.read_state(engine, c)["entity_data"][60:60 + B, :D]
+    assert np.isfinite(np.delete(heads, 5, axis=1)).all()
