@@ -88,7 +88,7 @@ __global__ __launch_bounds__(NW * 64) void k_feature_fwd(FeatureArgs a, const ch
     using TB = ColTile<TN>;
     constexpr int kA = PA * TM * 64, kStage = kA + TB::kBytes, kEach = TB::kCopies / NW;
     __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
-    __shared__ uint32_t key_s[TM];
+    __shared__ __attribute__((aligned(16))) uint32_t key_s[TM];
     const int gx = (a.Dp + TN - 1) / TN;
     const int u0 = (int)blockIdx.x / gx * TM, n0 = (int)blockIdx.x % gx * TN;
     const int U = (int)a.counts[0];
@@ -119,27 +119,59 @@ __global__ __launch_bounds__(NW * 64) void k_feature_fwd(FeatureArgs a, const ch
     };
     const int n_slab = (a.Fp + 31) / 32;
     fill(0);
-    // the embeddings are what the accumulators start from: fetched after the loop, a chain of two round
-    // trips at a time, they took as long as the product (24k rows: 99 us, 55 without them)
     const int k = n0 + 32 * wave + (lane & 31);
     floatx16 acc[AM];
-    const bool add = a.emb_base && k < a.Dp, wide = a.emb_etype == ET_F32;
-    const char* const col = a.emb_base + (add ? k : 0) * (wide ? 4 : 2);
 #pragma unroll
     for (int m = 0; m < AM; ++m)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {  // as they lie: a conversion here would wait for each load
-            const char* at = col + (int64_t)key_s[32 * m + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)] * a.pitch;
-            acc[m][r] = !add ? 0.f : wide ? *reinterpret_cast<const float*>(at) : __uint_as_float(*reinterpret_cast<const uint16_t*>(at));
+        for (int r = 0; r < 16; ++r) acc[m][r] = 0.f;
+    auto multiply = [&](int slab) __attribute__((always_inline)) {
+        const char* ta = smem + (slab & 1) * kStage;
+        const char* tb = ta + kA;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            floatx4 fa[AM][PA], fb[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) fb[q] = TB::fragment(tb, q, 32 * wave, ks, lane);
+#pragma unroll
+            for (int m = 0; m < AM; ++m)
+#pragma unroll
+                for (int q = 0; q < PA; ++q) fa[m][q] = TA::fragment(ta, q, 32 * m, ks, lane);
+            feature_products<PA, AM>(fa, fb, acc);
         }
-    if (!wide)
+    };
+    // The embeddings: added once, to the finished sums (as what the accumulators start from they would
+    // make every instruction of the contraction round at their size, 240 times for 768 float16 features),
+    // and all asked for together: up front where they have registers, else under the last slab's products.
+    const bool wide = a.emb_etype == ET_F32;
+    floatx16 emb[AM];
+    auto fetch = [&](auto type) __attribute__((always_inline)) {  // as they lie
+        using T = decltype(type);
+        const T* const col = reinterpret_cast<const T*>(a.emb_base) + min(k, a.Dp - 1);
 #pragma unroll
         for (int m = 0; m < AM; ++m)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint16_t raw = (uint16_t)__float_as_uint(acc[m][r]);
-                acc[m][r] = load1(reinterpret_cast<const char*>(&raw), 0, a.emb_etype);
+            for (int g = 0; g < 4; ++g) {
+                const uint4 key4 = *reinterpret_cast<const uint4*>(&key_s[32 * m + 8 * g + 4 * (lane >> 5)]);
+                const uint32_t key[4] = {key4.x, key4.y, key4.z, key4.w};
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const T v = *reinterpret_cast<const T*>(reinterpret_cast<const char*>(col) + (uint64_t)key[r] * (uint32_t)a.pitch);
+                    if constexpr (sizeof(T) == 4) emb[m][4 * g + r] = v;
+                    else emb[m][4 * g + r] = __uint_as_float(v);
+                }
             }
+    };
+    auto fetch_embeddings = [&]() __attribute__((always_inline)) {
+        if (!a.emb_base) {
+#pragma unroll
+            for (int m = 0; m < AM; ++m)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) emb[m][r] = 0.f;
+        } else if (wide) fetch(float{});
+        else fetch(uint16_t{});
+    };
+    if constexpr (AM <= 2) fetch_embeddings();
     for (int s0 = 0; s0 < n_slab; s0 += KS) {
         Raw8<FT> raw[KS][NC];
 #pragma unroll
@@ -162,29 +194,24 @@ __global__ __launch_bounds__(NW * 64) void k_feature_fwd(FeatureArgs a, const ch
                         *reinterpret_cast<uint4*>(smem + (slab & 1) * kStage + q * (TM * 64) + dst[i]) = piece[q];
                 }
             wait_copies_and_barrier<0>();
-            if (slab + 1 < n_slab) fill(slab + 1);
-            const char* ta = smem + (slab & 1) * kStage;
-            const char* tb = ta + kA;
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                floatx4 fa[AM][PA], fb[3];
-#pragma unroll
-                for (int q = 0; q < 3; ++q) fb[q] = TB::fragment(tb, q, 32 * wave, ks, lane);
-#pragma unroll
-                for (int m = 0; m < AM; ++m)
-#pragma unroll
-                    for (int q = 0; q < PA; ++q) fa[m][q] = TA::fragment(ta, q, 32 * m, ks, lane);
-                feature_products<PA, AM>(fa, fb, acc);
+            if (slab + 1 < n_slab) {
+                fill(slab + 1);
+                multiply(slab);
             }
         });
     }
+    if constexpr (AM > 2) fetch_embeddings();
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(n_slab - 1);
     if (k >= a.Dp) return;
 #pragma unroll
     for (int m = 0; m < AM; ++m)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int u = u0 + 32 * m + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            if (u < U) hidden[(size_t)u * a.Dp + k] = acc[m][r];
+            const uint16_t raw = (uint16_t)__float_as_uint(emb[m][r]);
+            const float e = wide ? emb[m][r] : load1(reinterpret_cast<const char*>(&raw), 0, a.emb_etype);
+            if (u < U) hidden[(size_t)u * a.Dp + k] = acc[m][r] + e;
         }
 }
 
