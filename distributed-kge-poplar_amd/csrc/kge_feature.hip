@@ -58,18 +58,20 @@ DEVINL void split_raw8(const Raw8<FT>& r, uint4 (&piece)[Pieces<FT>::n]) {
 }
 
 // the products of one sixteen-step: AM accumulators, one fragment column of the other operand,
-// smallest terms first
+// smallest terms first.  `low`: where all but the largest term go (acc itself, or accumulators of their own)
 template <int PA, int AM>
-DEVINL void feature_products(const floatx4 (&fa)[AM][PA], const floatx4 (&fb)[3], floatx16 (&acc)[AM]) {
+DEVINL void feature_products(const floatx4 (&fa)[AM][PA], const floatx4 (&fb)[3], floatx16 (&acc)[AM], floatx16 (&low)[AM]) {
     constexpr int n = PA == 3 ? 6 : PA == 2 ? 5 : 3;
     constexpr int qa[6] = {PA == 3 ? 0 : PA == 2 ? 1 : 0, PA == 3 ? 2 : 0, PA == 3 ? 1 : PA == 2 ? 1 : 0, 0, PA == 3 ? 1 : 0, 0};
     constexpr int qb[6] = {PA == 3 ? 2 : PA == 2 ? 1 : 2, PA == 3 ? 0 : PA == 2 ? 2 : 1, PA == 3 ? 1 : 0, 1, 0, 0};
 #pragma unroll
     for (int x = 0; x < n; ++x)
 #pragma unroll
-        for (int m = 0; m < AM; ++m)
-            acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[m][qa[x]]),
-                                                             __builtin_bit_cast(bf16x8, fb[qb[x]]), acc[m], 0, 0, 0);
+        for (int m = 0; m < AM; ++m) {
+            floatx16& to = x + 1 < n ? low[m] : acc[m];
+            to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[m][qa[x]]),
+                                                         __builtin_bit_cast(bf16x8, fb[qb[x]]), to, 0, 0, 0);
+        }
 }
 
 // hidden.  A workgroup of NW waves takes 32 AM rows x 32 NW columns, every wave all of the rows and 32 of
@@ -137,7 +139,7 @@ __global__ __launch_bounds__(NW * 64) void k_feature_fwd(FeatureArgs a, const ch
             for (int m = 0; m < AM; ++m)
 #pragma unroll
                 for (int q = 0; q < PA; ++q) fa[m][q] = TA::fragment(ta, q, 32 * m, ks, lane);
-            feature_products<PA, AM>(fa, fb, acc);
+            feature_products<PA, AM>(fa, fb, acc, acc);
         }
     };
     // The embeddings: added once, to the finished sums (as what the accumulators start from they would
@@ -234,11 +236,14 @@ __global__ __launch_bounds__(NW * 64) void k_feature_grad(FeatureArgs a, const f
     const int share = ((U + n_split - 1) / n_split + 31) & ~31;
     const int ub = split * share, ue = min(U, ub + share), n_slab = ue > ub ? (ue - ub + 31) / 32 : 0;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    floatx16 acc[AM];
+    // the small terms in accumulators of their own: the large ones round once per sixteen rows, not five times
+    // (dW of 256 rows of 768 float16 features, against float64: 1.95e-7 off with one set, 1.5e-7 with two,
+    // most of it the gradient's; the time is the same, 60 us for 24k rows of 768 and 256 columns)
+    floatx16 acc[AM], low[AM];
 #pragma unroll
     for (int m = 0; m < AM; ++m)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[m][r] = 0.f;
+        for (int r = 0; r < 16; ++r) acc[m][r] = low[m][r] = 0.f;
     uint32_t key[NA];       // the next slab's rows
     Raw8<FT> raw[NA];
     float4 g[NB];
@@ -307,7 +312,7 @@ __global__ __launch_bounds__(NW * 64) void k_feature_grad(FeatureArgs a, const f
             for (int m = 0; m < AM; ++m)
 #pragma unroll
                 for (int q = 0; q < PA; ++q) fa[m][q] = TA::fragment(ta, q, 32 * m, ks, lane);
-            feature_products<PA, AM>(fa, fb, acc);
+            feature_products<PA, AM>(fa, fb, acc, low);
         }
     }
     const int k = n0 + 32 * wave + (lane & 31);
@@ -318,7 +323,7 @@ __global__ __launch_bounds__(NW * 64) void k_feature_grad(FeatureArgs a, const f
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int f = f0 + 32 * m + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            if (f < a.Fp) out[(size_t)f * a.Dp + k] = acc[m][r];
+            if (f < a.Fp) out[(size_t)f * a.Dp + k] = acc[m][r] + low[m][r];
         }
 }
 

@@ -42,3 +42,6 @@ def test_embeddings_larger_than_the_projection(oracle64, feature_dtype):
     got, want = _first_moments(oracle64, c, feature_dtype, 5, emb_scale=3.0)
     D = c["dim"]
     assert K.rel_l2(got["entity_data"][:, D:2 * D], want["entity_data"][:, D:2 * D]) < 2.5e-7
+    # dW over 256 rows: the gradient's own error, and one rounding of the large terms per sixteen rows (1.5e-7;
+    # 1.95e-7 when the small terms round into the same sum)
+    assert K.rel_l2(got["feature_projection/adam_m"], want["feature_projection/adam_m"]) < 1.75e-7
