@@ -12,6 +12,7 @@
 #include <condition_variable>
 #include <cstddef>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <memory>
 #include <mutex>
@@ -21,11 +22,16 @@
 namespace kge {
 
 // A handful of threads that all run one function at a time, woken once per transfer.  Created by
-// the first large transfer of its owner, joined with it.
+// the first large transfer of its owner, joined with it.  Where the system has no more threads to
+// give there are fewer of them, or none: the callers go by size().
 class CopyThreads {
    public:
     explicit CopyThreads(int n) {
-        for (int i = 0; i < n; ++i) threads_.emplace_back([this, i] { loop(i); });
+        threads_.reserve(n);
+        try {
+            for (int i = 0; i < n; ++i) threads_.emplace_back([this, i] { loop(i); });
+        } catch (const std::exception&) {
+        }
     }
     ~CopyThreads() {
         {
