@@ -808,7 +808,10 @@ void transfer(kge_engine& E, bool to_device, void* array, size_t units, size_t u
     const size_t per = std::min(units, E.io_slot / unit), n_chunk = (units + per - 1) / per;
     // below this a few threads' wake-up costs more than they save
     const bool threaded = units * unit >= (size_t)1 << 20;
-    if (threaded && !E.copy_threads) E.copy_threads.reset(new CopyThreads(7));
+    if (threaded && !E.copy_threads) {  // with this one eight, or as many as there are cores
+        const int cores = (int)std::thread::hardware_concurrency();
+        E.copy_threads.reset(new CopyThreads(cores ? std::min(7, cores - 1) : 7));
+    }
     SlottedCopy copy((char*)array, E.io_slots, units * unit, per * unit, (int)n_slots, to_device,
                      threaded ? E.copy_threads.get() : nullptr);
     auto start = [&](size_t k) {

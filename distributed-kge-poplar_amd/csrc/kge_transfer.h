@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstddef>
 #include <cstring>
@@ -85,6 +86,10 @@ class CopyThreads {
 // The copies of one transfer: chunk k of `n_chunks` is bytes [k * chunk, ...) of the caller's array
 // and lies in slot k % n_slots.  allow(k) lets the threads work on chunk k, wait(k) returns when it
 // is copied; the calling thread takes a share of every chunk inside wait().
+//
+// A slot's kernel takes some 40 us, a thread's wake-up about as long: whoever waits looks on for kLook,
+// giving its core to others meanwhile, and sleeps only after that, so that a transfer that stalls, or a
+// host with fewer cores than threads, is not kept busy by the waiting.
 class SlottedCopy {
    public:
     // to_slot: array -> slots, else slots -> array.  threads: null for a copy by the calling thread alone
@@ -95,29 +100,50 @@ class SlottedCopy {
         for (size_t k = 0; k < n_chunks(); ++k) left_[k].store(parts_ - 1, std::memory_order_relaxed);
         if (threads_) threads_->start([this](int i) {
             for (size_t k = 0; k < n_chunks(); ++k) {
-                while (allowed_.load(std::memory_order_acquire) <= k) {
-                    if (stop_.load(std::memory_order_relaxed)) return;
-                    std::this_thread::yield();
-                }
+                await(may_, [&] { return allowed_.load(std::memory_order_acquire) > k || stop_.load(std::memory_order_relaxed); });
+                if (allowed_.load(std::memory_order_acquire) <= k) return;  // stopped
                 copy_part(k, i + 1);
-                left_[k].fetch_sub(1, std::memory_order_release);
+                if (left_[k].fetch_sub(1, std::memory_order_acq_rel) == 1) signal(copied_);
             }
         });
     }
     ~SlottedCopy() {
         stop_.store(true);
+        signal(may_);
         if (threads_) threads_->wait();
     }
     SlottedCopy(const SlottedCopy&) = delete;
     SlottedCopy& operator=(const SlottedCopy&) = delete;
     size_t n_chunks() const { return (total_ + chunk_ - 1) / chunk_; }
-    void allow(size_t k) { allowed_.store(k + 1, std::memory_order_release); }
+    void allow(size_t k) {
+        allowed_.store(k + 1, std::memory_order_release);
+        signal(may_);
+    }
     void wait(size_t k) {
         copy_part(k, 0);
-        while (left_[k].load(std::memory_order_acquire)) std::this_thread::yield();
+        await(copied_, [&] { return left_[k].load(std::memory_order_acquire) == 0; });
     }
 
    private:
+    static constexpr std::chrono::microseconds kLook{200};
+    template <class Ready>
+    void await(std::condition_variable& cv, Ready&& ready) {
+        const auto until = std::chrono::steady_clock::now() + kLook;
+        while (!ready()) {
+            if (std::chrono::steady_clock::now() >= until) {
+                std::unique_lock<std::mutex> lock(mu_);
+                cv.wait(lock, ready);
+                return;
+            }
+            std::this_thread::yield();
+        }
+    }
+    // (what was waited for is stored before: a waiter that is about to sleep holds the mutex until it does)
+    void signal(std::condition_variable& cv) {
+        if (!threads_) return;
+        { std::lock_guard<std::mutex> lock(mu_); }
+        cv.notify_all();
+    }
     void copy_part(size_t k, int part) {
         const size_t n = std::min(chunk_, total_ - k * chunk_);
         // parts end on whole pages of the array, so that no two threads touch the same new page
@@ -138,6 +164,8 @@ class SlottedCopy {
     std::unique_ptr<std::atomic<int>[]> left_;
     std::atomic<size_t> allowed_{0};
     std::atomic<bool> stop_{false};
+    std::mutex mu_;
+    std::condition_variable may_, copied_;
 };
 
 }  // namespace kge

@@ -105,3 +105,9 @@ def test_every_byte_arrives(program, total, chunk, n_slots, offset, threads):
 def test_a_system_without_threads(program, granted):
     """The system refuses a thread: the copies go on with those there are."""
     _run(program, granted, 7, 3_000_001, 65_536, 4, 1, 0)
+
+
+def test_waiting_threads_sleep(program):
+    """Ten chunks of 20 ms each way, seven threads: they look on for 0.2 ms of each wait and sleep for
+    the rest (all of them on a core for the whole time would be 7 x 0.42 s where there are the cores)."""
+    assert _run(program, 7, 7, 1 << 20, 110_000, 4, 0, 20) < 0.2
