@@ -12,6 +12,7 @@
 #include <chrono>
 #include <condition_variable>
 #include <cstddef>
+#include <cstdint>
 #include <cstring>
 #include <exception>
 #include <functional>
@@ -146,8 +147,13 @@ class SlottedCopy {
     }
     void copy_part(size_t k, int part) {
         const size_t n = std::min(chunk_, total_ - k * chunk_);
-        // parts end on whole pages of the array, so that no two threads touch the same new page
-        auto cut = [&](int q) { return q == parts_ ? n : std::min(n, (n * q / parts_) & ~(size_t)4095); };
+        // a chunk's parts end on whole pages of the array, wherever it starts: no two threads touch the
+        // same new page of a chunk
+        const uintptr_t base = (uintptr_t)(array_ + k * chunk_);
+        auto cut = [&](int q) -> size_t {
+            const uintptr_t page = (base + n * q / parts_) & ~(uintptr_t)4095;
+            return q == parts_ ? n : page > base ? page - base : 0;
+        };
         const size_t a = cut(part), b = cut(part + 1);
         if (a >= b) return;
         char* arr = array_ + k * chunk_ + a;
