@@ -597,7 +597,8 @@ __global__ __launch_bounds__(NW * 64) void k_score_fwd_mfma(FwdParams p) {
     const bool col_counts = !sh.tcount || n < (int)sh.tcount[d];
 #pragma unroll
     for (int t = 0; t < AT; ++t) {
-        // phase 1 (straight-line): squared distances and which of them cancelled
+        // phase 1 (straight-line): squared distances (products) and which of them cancelled or are not
+        // finite (an infinity's second piece is NaN)
         float val[16];
         uint32_t cancel = 0u, near = 0u;
 #pragma unroll
@@ -605,18 +606,27 @@ __global__ __launch_bounds__(NW * 64) void k_score_fwd_mfma(FwdParams p) {
             const int m_loc = wm + 32 * t + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
             const bool live = col_counts && (ALIGNED || (m0 + m_loc < B && n < T));
             val[r] = acc[t][r];
+            bool good = fabsf(val[r]) < INFINITY;  // (dot)
             if (DIST == DIST_L2) {
                 const float na = na_s[m_loc];
                 val[r] = na + nb - 2.f * acc[t][r];
-                if (live && val[r] < kCancelRatio * (na + nb)) cancel |= 1u << r;
+                good = val[r] >= kCancelRatio * (na + nb);
                 if (live && val[r] < kNearRatio * (na + nb)) near |= 1u << r;
             }
+            if (!good) cancel |= 1u << r;
         }
-        // phase 2 (rare): the wave recomputes the cancelled pairs directly, four at a time: two pairs
+        // phase 2 (rare): the wave recomputes these pairs directly, four at a time: two pairs
         // of each of two lanes, sixteen lanes to a pair.  (Pairs come in runs: a popular row among
         // the heads against its own column puts them all on two lanes.  One pair at a time, each a
-        // round trip to memory, such a tile ran on alone for tens of us.)
-        if (DIST == DIST_L2 && __ballot(cancel != 0u)) {
+        // round trip to memory, such a tile ran on alone for tens of us.)  Pairs that do not count, a
+        // NaN among them, get any finite value.
+        if (__ballot(cancel != 0u)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (!(col_counts && (ALIGNED || (m0 + wm + 32 * t + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3) < B && n < T)))) {
+                    val[r] = 0.f;
+                    cancel &= ~(1u << r);
+                }
             near = 0u;
             uint32_t left = cancel;
             uint64_t owners;
@@ -645,8 +655,12 @@ __global__ __launch_bounds__(NW * 64) void k_score_fwd_mfma(FwdParams p) {
                     }
 #pragma unroll
                     for (int x = 0; x < 4; ++x) {
-                        const float dx = a[x].x - b[x].x, dy = a[x].y - b[x].y, dz = a[x].z - b[x].z, dw = a[x].w - b[x].w;
-                        part += dx * dx + dy * dy + dz * dz + dw * dw;
+                        if (DIST == DIST_L2) {
+                            const float dx = a[x].x - b[x].x, dy = a[x].y - b[x].y, dz = a[x].z - b[x].z, dw = a[x].w - b[x].w;
+                            part += dx * dx + dy * dy + dz * dz + dw * dw;
+                        } else {
+                            part += a[x].x * b[x].x + a[x].y * b[x].y + a[x].z * b[x].z + a[x].w * b[x].w;
+                        }
                     }
                 }
 #pragma unroll
@@ -669,7 +683,7 @@ __global__ __launch_bounds__(NW * 64) void k_score_fwd_mfma(FwdParams p) {
             for (int r = 0; r < 16; ++r) {
                 const int m_loc = wm + 32 * t + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                 const bool live = col_counts && (ALIGNED || (m0 + m_loc < B && n < T));
-                if (live && val[r] < kNearRatio * (na_s[m_loc] + nb)) near |= 1u << r;
+                if (DIST == DIST_L2 && live && val[r] < kNearRatio * (na_s[m_loc] + nb)) near |= 1u << r;
             }
         }
         // phase 3 (straight-line): distance, score, loss, backward coefficient
@@ -682,7 +696,7 @@ __global__ __launch_bounds__(NW * 64) void k_score_fwd_mfma(FwdParams p) {
             const int m_loc = wm + 32 * t + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
             const int m = m0 + m_loc;
             const bool live = ALIGNED || (m < B && n < T);
-            const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(fmaxf(val[r], 0.f)) : val[r];
+            const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[r]) : val[r];  // (never negative; a NaN stays one)
             float outv;
             if (OM == 2) {
                 outv = dist;

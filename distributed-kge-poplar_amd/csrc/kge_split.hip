@@ -328,8 +328,7 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
             }
             // rare: the wave recomputes pairs directly, two pairs of each of two lanes at a time, sixteen
             // lanes to a pair: those that cancelled, and those that are not finite (an infinity's second
-            // piece is NaN, which the clamp below would make a distance of zero and a finite loss).  Pairs
-            // that do not count, a NaN among them, get any finite value.
+            // piece is NaN).  Pairs that do not count, a NaN among them, get any finite value.
             if (__ballot(cancel != 0u)) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
@@ -390,7 +389,7 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int m = m0 + mb + 8 * (r >> 2) + 4 * hl + (r & 3);
-                    const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(fmaxf(val[r], 0.f)) : val[r];
+                    const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[r]) : val[r];  // (never negative; a NaN stays one)
                     if (m < B && n < T) {
                         out[(size_t)m * T + n] = score_is_distance_value(sh.score_fn) ? dist : sh.gamma - dist;
                         if (out_d) out_d[(size_t)m * T + n] = dist;
@@ -404,7 +403,7 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
             for (int r = 0; r < 16; ++r) {
                 const int m_loc = mb + 8 * (r >> 2) + 4 * hl + (r & 3);
                 const bool live = m0 + m_loc < B && n < T;
-                const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(fmaxf(val[r], 0.f)) : val[r];
+                const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[r]) : val[r];  // (never negative; a NaN stays one)
                 const float score = score_is_distance_value(sh.score_fn) ? dist : sh.gamma - dist;
                 float ds;
                 const float term = logsigmoid_column(score, (uint32_t)n == label_s[m_loc], mult, w_pos, w_neg, grad_scale, ds);

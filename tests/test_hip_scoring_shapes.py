@@ -92,7 +92,8 @@ def test_nonfinite_row_stays_in_its_block(kind, loss_fn, merge, B, A, D):
 # are; logsigmoid's sum holds 0 x infinity), and with whole columns that stand for no tail (repeats of the
 # block's first tail) the gradients' other columns stay finite
 @pytest.mark.parametrize("kind", ["L2", "MatMul"])
-@pytest.mark.parametrize("B,A,D", [(33, 21, 30), (8, 100, 64), (130, 65, 100)])
+@pytest.mark.parametrize("B,A,D", [(33, 21, 30), (8, 100, 64), (130, 65, 100),
+                                   (512, 512, 64)])  # whole 128-row tiles, enough of them: float32 operands, split while staged
 def test_infinite_row_shows_in_the_loss(kind, B, A, D):
     for role in ("head", "tail"):
         for value in (np.inf, -np.inf):

@@ -310,7 +310,8 @@ def test_predict_sweep_close_rows(dim, dtype, n_query, n_entity):
 
 
 @pytest.mark.parametrize("score_fn", ["TransE", "DistMult"])
-@pytest.mark.parametrize("dim,dtype", [(30, "float32"), (64, "float16"), (100, "float32"), (130, "float16"), (256, "float32")])
+@pytest.mark.parametrize("dim,dtype", [(30, "float32"), (64, "float16"), (100, "float32"), (130, "float16"), (256, "float32"),
+                                       (320, "float32"), (300, "float16")])
 def test_predict_sweep_nonfinite_rows(score_fn, dim, dtype):
     """A row with an infinite element scores what its own terms add up to (L2: minus infinity; dot: the
     infinity of the product's sign), a row with a NaN ranks nowhere, and no other row's or query's
