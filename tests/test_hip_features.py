@@ -11,9 +11,9 @@ from oracle.kge_oracle import make_cfg
 pytestmark = pytest.mark.gpu
 
 
-def _first_moments(oracle, c, feature_dtype, seed, emb_scale=None):
+def _first_moments(oracle, c, feature_dtype, seed, emb_scale=None, all_distinct=False):
     """One step from zero moments: the first moments are the gradients times (1 - beta_m).  Returns the
-    engine's and the oracle's state."""
+    engine's and the oracle's state.  `all_distinct` (one shard): every head and tail a row of its own."""
     import libpoplar_kge
 
     rng = np.random.default_rng(seed)
@@ -23,6 +23,9 @@ def _first_moments(oracle, c, feature_dtype, seed, emb_scale=None):
     if feature_dtype == "bfloat16":
         state["entity_data"][:, 3 * c["dim"]:] = oracle.round(state["entity_data"][:, 3 * c["dim"]:], "bfloat16_embedding")
     batch = K.random_batch(c, 1, rng)
+    if all_distinct:
+        batch["head"][:] = np.arange(c["batch"])
+        batch["a2a"][:] = c["batch"] + np.arange(c["a2a"])
     lr = np.full(c["n_shard"], 1e-3, np.float32)
     engine = libpoplar_kge.Engine(H.engine_settings(c, 1, **{"execution.feature_dtype": feature_dtype}), "")
     H.load_state(engine, c, state)
@@ -45,3 +48,36 @@ def test_embeddings_larger_than_the_projection(oracle64, feature_dtype):
     # dW over 256 rows: the gradient's own error, and one rounding of the large terms per sixteen rows (1.5e-7;
     # 1.95e-7 when the small terms round into the same sum)
     assert K.rel_l2(got["feature_projection/adam_m"], want["feature_projection/adam_m"]) < 1.75e-7
+
+
+def _small(dtype, F, D, rows):  # that many distinct rows, two of them tails
+    return pytest.param(dtype, F, D, rows - 2, True, id=f"{dtype}-F{F}-D{D}-{rows}rows")
+
+
+def _tall(dtype, F, D, batch):  # heads drawn with repeats: fewer distinct rows than the launches are sized for
+    return pytest.param(dtype, F, D, batch, False, id=f"{dtype}-F{F}-D{D}-batch{batch}")
+
+
+# Widths of two, four and eight waves (up to 64, 128, 256 columns) and of two workgroups; features that end in a
+# slab of 32 or fill it up; rows around a tile of 32; features that take the loads a second round (all but the
+# first line of either list: eight waves above 768 16-bit or 384 float32 features; fewer waves on tall
+# tiles, four times as many chunks per thread, above 192 and 96).  Batches of 10k, 20k and 30k rows with
+# eight waves, twice as many with four and four times with two, take tiles of 64, 96 and 128 rows; from 1152 rows on
+# dW's contraction has more than eight parts.
+@pytest.mark.parametrize("dtype,F,D,batch,all_distinct", [
+    _small("float32", 4, 30, 31), _small("float16", 4, 66, 33), _small("bfloat16", 130, 66, 32), _small("float32", 36, 260, 33),
+    _small("float16", 800, 130, 31), _small("float32", 388, 130, 33), _small("bfloat16", 800, 260, 65), _small("float32", 388, 256, 1200),
+    _tall("float16", 36, 30, 40000), _tall("float32", 36, 30, 80000), _tall("float16", 228, 30, 120000),
+    _tall("bfloat16", 36, 66, 20000), _tall("float16", 130, 66, 40000), _tall("float32", 132, 66, 60000),
+    _tall("float32", 36, 130, 10000), _tall("bfloat16", 130, 130, 20000), _tall("float16", 36, 130, 30000), _tall("float32", 100, 260, 15000),
+])
+def test_feature_shapes(oracle64, dtype, F, D, batch, all_distinct):
+    c = K.cfg_dict(distance_fn="L2", n_shard=1, batch=batch, a2a=2, dim=D, feature=F, n_entity=batch + 5, n_relation=6, gamma=4.0)
+    got, want = _first_moments(oracle64, c, dtype, 7, all_distinct=all_distinct)
+    # A step's dozen roundings of 2^-24 and the contraction over the features (800: 3.1e-7 measured); and the two
+    # tails' gradients, most of the norm on tall batches: one float32 sum over all positives, of 12 matrix
+    # instructions per 32, whose N roundings (0.29 of 2^-24 each, at a partial sum that grows evenly)
+    # add up to 0.29 / sqrt(3) 2^-24 sqrt(N): 2.1e-6 for 120000 positives.  Half as much again for the draw.
+    bound = 5e-7 + 1.5 * 0.29 / np.sqrt(3) * 2.0**-24 * np.sqrt(12 * batch / 32)
+    assert K.rel_l2(got["entity_data"][:, D:2 * D], want["entity_data"][:, D:2 * D]) < bound
+    assert K.rel_l2(got["feature_projection/adam_m"], want["feature_projection/adam_m"]) < bound
