@@ -740,13 +740,15 @@ void allocate(kge_engine& E) {
             E.proj_pieces_bytes = split_bytes(round_up(E.Fp, 32), E.Dp);
             E.projp.alloc(E.nets * E.proj_pieces_bytes);
             E.projp.zero(st);  // rows behind the last feature meet zeros
-        } else E.featd.alloc(R * E.Fp);
+        } else {
+            E.featd.alloc(R * E.Fp);
+            E.gproj.alloc(E.nets * proj_n);  // (on pieces the update adds up the parts itself)
+        }
         E.gproj_part.alloc((size_t)(E.split_feat ? feature_grad_parts((int)R, E.Fp, E.Dp) : 16) * E.Fp * E.Dp);
         if (E.score_bf16) {
             E.feat16.alloc(R * E.Fp);
             E.projR.alloc((size_t)E.Fp * E.Dp);
         }
-        E.gproj.alloc(E.nets * proj_n);
         if (E.mlp) {
             const size_t M = E.mlp, up_n = 2 * (size_t)E.Dp * M, down_n = M * E.Dp, N = E.nets;
             for (DevBuf<float>* b : {&E.up, &E.up_m, &E.up_v, &E.g_up}) { b->alloc(N * up_n); b->zero(st); }
@@ -1328,8 +1330,7 @@ void run_step(kge_engine& E, int i) {
         const SplitCoef sc = {E.coefp.p, E.rowpart.p, E.colpart.p, E.Bp, E.Tp};
         { KernelTimer t(E, K_FWD);
           SplitFwd f = {};
-          f.sh = sh; f.a = f.b = E.rowsp.p; f.norm_a = f.norm_b = E.row_norm.p;
-          f.a_c0 = 0; f.b_c0 = (int)SB; f.Kp = E.Kp; f.clabel = clabel;
+          f.sh = sh; f.rows = E.rowsp.p; f.norm = E.row_norm.p; f.b_c0 = (int)SB; f.Kp = E.Kp; f.clabel = clabel;
           f.coef = E.coef.p; f.dist = fused ? nullptr : E.dist.p; f.loss_part = loss_part; f.nearflag = E.nearflag.p;
           f.out = sc;
           launch_split_fwd(f, fused, st); }

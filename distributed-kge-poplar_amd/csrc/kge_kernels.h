@@ -262,9 +262,9 @@ void launch_gather_pieces(const RowSource& ent, const float* rel, const uint32_t
 struct SplitCoef { char* coefp; float* rowpart; float* colpart; int Bp, Tp; };
 struct SplitFwd {
     ScoreShape sh;
-    const char* a; const char* b;          // piece matrices of the rows; block d's from a_c0 + d B and b_c0 + d T
-    const float* norm_a; const float* norm_b;  // their squared norms
-    int a_c0, b_c0, Kp;
+    const char* rows;   // piece matrix: heads from row 0, tails from row b_c0
+    const float* norm;  // the rows' squared norms
+    int Kp, b_c0;
     const uint32_t* clabel;
     float* coef;        // [S, B, T] scores (without fused loss); the flagged sub-blocks' coefficients
     float* dist;        // or null

@@ -103,6 +103,10 @@ void launch_gather_pieces(const RowSource& ent, const float* rel, const uint32_t
 // --------------------------------------------------------------------------
 // products
 
+// Tiles of 64 x 64, four waves, three workgroups to a CU: at these sizes a launch is bound by the
+// latency of its slabs and by how many workgroups there are, not by the matrix cores.
+constexpr int kTile = 64, kWaves = 2;  // waves as kWaves x kWaves
+
 // The product loop of a TM x TN tile: n_slab slabs of 32 contraction steps, two tile copies in LDS
 // (one fills while the other is multiplied, one barrier per slab).  TA, TB: RowTile / ColTile;
 // a_step, b_step: bytes from slab to slab.  Waves as WM x WN, each (TM/WM) x (TN/WN) in 32 x 32
@@ -252,8 +256,9 @@ __global__ __launch_bounds__(256) void k_coef_pieces(ScoreShape sh, const float*
 // forward
 
 // (kCancelRatio, kNearRatio: kge_loss.h)
-template <int DIST, int OM, int TM, int TN, int WM, int WN>
-__global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_fwd(SplitFwd p) {
+template <int DIST, int OM>
+__global__ __launch_bounds__(kWaves * kWaves * 64, 2) void k_split_fwd(SplitFwd p) {
+    constexpr int TM = kTile, TN = kTile, WM = kWaves, WN = kWaves;
     using P = SplitProduct<RowTile<TM>, RowTile<TN>, TM, TN, WM, WN>;
     __shared__ __attribute__((aligned(16))) char smem[P::kLds];
     __shared__ float na_s[TM], nb_s[TN], mult_s[TN], red[WM * WN];
@@ -269,10 +274,10 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
         return;
     }
     const int n_live = sh.tcount ? (int)sh.tcount[d] : T;
-    const int a_row = p.a_c0 + d * B, b_row = p.b_c0 + d * T;
+    const int a_row = d * B, b_row = p.b_c0 + d * T;
     const int pitch = Kp * 6;
-    const char* a = p.a + (int64_t)(a_row + m0) * pitch;
-    const char* b = p.b + (int64_t)(b_row + n0) * pitch;
+    const char* a = p.rows + (int64_t)(a_row + m0) * pitch;
+    const char* b = p.rows + (int64_t)(b_row + n0) * pitch;
     floatx16 acc[P::AM][P::AN];
 #pragma unroll
     for (int m = 0; m < P::AM; ++m)
@@ -282,11 +287,11 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
             for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
     P::run(smem, a, pitch, 192, b, pitch, 192, Kp / 32, 0, acc, lane, wave, [&]() __attribute__((always_inline)) {
         for (int i = tid; i < TM; i += WM * WN * 64) {
-            if (DIST == DIST_L2) na_s[i] = p.norm_a[a_row + m0 + i];
+            if (DIST == DIST_L2) na_s[i] = p.norm[a_row + m0 + i];
             if (OM == 0) label_s[i] = m0 + i < B ? p.clabel[d * B + m0 + i] : 0u;
         }
         if (DIST == DIST_L2)
-            for (int i = tid; i < TN; i += WM * WN * 64) nb_s[i] = p.norm_b[b_row + n0 + i];
+            for (int i = tid; i < TN; i += WM * WN * 64) nb_s[i] = p.norm[b_row + n0 + i];
         if (OM == 0)
             for (int i = tid; i < TN; i += WM * WN * 64)
                 mult_s[i] = n0 + i < T ? (sh.tmult ? sh.tmult[(size_t)d * T + n0 + i] : 1.f) : 0.f;
@@ -441,8 +446,9 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN > 8192 ? 1 : 2) void k_split_
 // (L2: self[i, k] sum_j c[i, j] - the product).  Head side: i = heads, the coefficient rows lie along
 // the contraction.  Tail side: i = tails, they lie across it.  `other` always lies across it.
 
-template <int DIST, bool SIDE_B, int TM, int TN, int WM, int WN>
+template <int DIST, bool SIDE_B>
 DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, char* smem, float* csum_s) {
+    constexpr int TM = kTile, TN = kTile, WM = kWaves, WN = kWaves;
     using TA = std::conditional_t<SIDE_B, ColTile<TM>, RowTile<TM>>;
     using P = SplitProduct<TA, ColTile<TN>, TM, TN, WM, WN>;
     const int i0 = tile_y * TM, kt0 = tile_x * TN;
@@ -555,9 +561,10 @@ DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, cha
 
 // Both sides in one launch: the side whose tiles loop over more rows comes first, for every block, so
 // that the long tiles do not start last.  A block's tiles of one side stay together on one XCD.
-template <int DIST, int TM, int TN, int WM, int WN>
-__global__ __launch_bounds__(WM * WN * 64) void k_split_bwd(SplitBwd p) {
-    using PA = SplitProduct<RowTile<TM>, ColTile<TN>, TM, TN, WM, WN>;
+template <int DIST>
+__global__ __launch_bounds__(kWaves * kWaves * 64) void k_split_bwd(SplitBwd p) {
+    constexpr int TM = kTile, TN = kTile;
+    using PA = SplitProduct<RowTile<TM>, ColTile<TN>, TM, TN, kWaves, kWaves>;
     __shared__ __attribute__((aligned(16))) char smem[PA::kLds];
     __shared__ float csum_s[TM];
     const int gx = (p.Dp + TN - 1) / TN, ga = (p.B + TM - 1) / TM, gb = (p.T + TM - 1) / TM;
@@ -566,19 +573,15 @@ __global__ __launch_bounds__(WM * WN * 64) void k_split_bwd(SplitBwd p) {
     const int L = blockIdx.x;
     if ((L < n_first) == heads_first) {
         const TileId tile = xcd_tile(gx, ga, p.S, heads_first ? L : L - n_first);
-        split_bwd_tile<DIST, false, TM, TN, WM, WN>(p, tile.z, tile.x, tile.y, smem, csum_s);
+        split_bwd_tile<DIST, false>(p, tile.z, tile.x, tile.y, smem, csum_s);
     } else {
         const TileId tile = xcd_tile(gx, gb, p.S, heads_first ? L - n_first : L);
-        split_bwd_tile<DIST, true, TM, TN, WM, WN>(p, tile.z, tile.x, tile.y, smem, csum_s);
+        split_bwd_tile<DIST, true>(p, tile.z, tile.x, tile.y, smem, csum_s);
     }
 }
 
 // --------------------------------------------------------------------------
 // launches
-
-// Tiles of 64 x 64, four waves, three workgroups to a CU: at these sizes a launch is bound by the
-// latency of its slabs and by how many workgroups there are, not by the matrix cores.
-constexpr int kTile = 64;
 
 int split_fwd_parts(const ScoreShape& sh) {
     return ((sh.T + kTile - 1) / kTile) * ((sh.B + kTile - 1) / kTile);
@@ -588,7 +591,7 @@ void launch_split_fwd(const SplitFwd& p, bool fused_loss, hipStream_t stream) {
     const ScoreShape& sh = p.sh;
     const dim3 grid = tile_grid((sh.T + kTile - 1) / kTile, (sh.B + kTile - 1) / kTile, sh.S);
     const bool l2 = sh.dist_fn == DIST_L2 && sh.score_fn != SCORE_DISTMULT;
-#define KGE_FWD(D_, OM_) hipLaunchKernelGGL((k_split_fwd<D_, OM_, kTile, kTile, 2, 2>), grid, dim3(256), 0, stream, p)
+#define KGE_FWD(D_, OM_) hipLaunchKernelGGL((k_split_fwd<D_, OM_>), grid, dim3(256), 0, stream, p)
     if (l2) { if (fused_loss) KGE_FWD(DIST_L2, 0); else KGE_FWD(DIST_L2, 1); }
     else    { if (fused_loss) KGE_FWD(DIST_DOT, 0); else KGE_FWD(DIST_DOT, 1); }
 #undef KGE_FWD
@@ -604,8 +607,8 @@ void launch_coef_pieces(const ScoreShape& sh, const float* coef, const uint32_t*
 
 void launch_split_bwd(const SplitBwd& p, bool l2, hipStream_t stream) {
     const dim3 grid(((p.Dp + kTile - 1) / kTile) * ((p.B + kTile - 1) / kTile + (p.T + kTile - 1) / kTile) * p.S);
-    if (l2) hipLaunchKernelGGL((k_split_bwd<DIST_L2, kTile, kTile, 2, 2>), grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((k_split_bwd<DIST_DOT, kTile, kTile, 2, 2>), grid, dim3(256), 0, stream, p);
+    if (l2) hipLaunchKernelGGL(k_split_bwd<DIST_L2>, grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL(k_split_bwd<DIST_DOT>, grid, dim3(256), 0, stream, p);
 }
 
 // Where these kernels are taken.  At whole 128-row tiles and enough of them the kernels that split
@@ -614,7 +617,7 @@ void launch_split_bwd(const SplitBwd& p, bool l2, hipStream_t stream) {
 // piece matrices cost half as much memory traffic again, and with that many tiles the
 // staging's vector work hides behind other workgroups' matrix work.  Elsewhere - ragged sizes, which
 // those kernels take with bounds checks and float32 matrix instructions, and few tiles - these
-// are the faster ones: one block of 256 x 64, D = 64: forward 11.2 -> 10.5 us, backward 37 -> 12;
+// are the faster ones: one block of 256 x 64, D = 64: forward 11.2 -> 10.5 us, backward 37 -> 9.5;
 // four of 200 x 268, D = 100: 17.4 -> 7.8 and 49 -> 10.6.
 bool split_scoring(const ScoreShape& sh) {
     if (sh.use_mfma != 2 || sh.score_fn == SCORE_TRANSH) return false;
