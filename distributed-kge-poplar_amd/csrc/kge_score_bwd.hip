@@ -964,14 +964,25 @@ DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane,
 // `heads` pieces [heads][S * T][Dp].
 struct L1Split { int heads, tails; };
 static L1Split l1_pair_split(const ScoreShape& sh) {
-    // A workgroup of sixteen waves fills a CU.  Tails first (a group of 64 still gives every wave
-    // four), then heads, as long as the chip has CUs without work; more groups than CUs only add
-    // pieces.  16 blocks of 512 x 1536 with D = 256: 4 groups of 384 tails, 256 workgroups.
+    // A workgroup of sixteen waves fills a CU.  Of the group sizes that the kernel has loops for, with
+    // as many groups of heads (four chunks of eight at least) as the chip then has CUs left, the one whose
+    // workgroups are done first: heads of a group times tails per wave and kHead, what a head costs
+    // beside its tails, in tails (an estimate; 2 to 4 choose nearly the same).  16 blocks of 512 x 1536 with
+    // D = 256: 4 groups of 384 tails, 256 workgroups.  Against doubling the groups of tails, then those of heads,
+    // while there are CUs, 40 steps each: 4 blocks of 512 x 1024, D = 256: 8.0 -> 4.9 ms; 10 of 130 x 960,
+    // D = 128: 3.8 -> 3.3; 1000 x 2000, D = 128: 3.4 -> 3.2; 16 of 64 x 64 and 1024 x 300, D = 64: the same;
+    // 40 x 1500, D = 256: 2.75 -> 2.80.
+    constexpr int kHead = 3;
     const int base = sh.S * ((sh.Dp + 63) / 64);
-    L1Split k = {1, (sh.T + L1P_MAX_T - 1) / L1P_MAX_T};
-    if (k.tails == 3 && base * 4 <= 256) k.tails = 4;
-    while (base * k.tails * 2 <= 256 && sh.T >= 128 * k.tails) k.tails *= 2;
-    while (base * k.tails * k.heads * 2 <= 256 && sh.B >= 64 * k.heads) k.heads *= 2;
+    L1Split k = {};
+    int64_t least = INT64_MAX;
+    for (int size = L1P_MAX_T; size >= 64; size -= 32) {
+        const int tails = (sh.T + size - 1) / size, heads = std::max(1, std::min(256 / (base * tails), sh.B / 32));
+        const int h_size = ((sh.B + heads - 1) / heads + L1P_CB - 1) / L1P_CB * L1P_CB;
+        const int per_wave = std::min(size, (sh.T + 31) / 32 * 32) / L1P_WAVES;
+        const int64_t cost = (int64_t)((base * tails * heads + 255) / 256) * h_size * (per_wave + kHead);
+        if (cost < least) { least = cost; k.heads = heads; k.tails = tails; }
+    }
     return k;
 }
 size_t score_bwd_pieces(const ScoreShape& sh) {
