@@ -83,8 +83,10 @@ __global__ __launch_bounds__(NW * 64) void k_feature_fwd(FeatureArgs a, const ch
     constexpr int PA = Pieces<FT>::n, TM = 32 * AM, TN = 32 * NW, NT = NW * 64;
     constexpr int NC = (TM * 4 + NT - 1) / NT;  // 16-byte chunks of a slab per thread
     // Slabs whose features are asked for together: a row of the table is a round trip of microseconds
-    // (and its loads hold up the copies behind them: they return in order), so it is paid once for
-    // 768 16-bit features, not once per slab (94 us for 24k rows of 768 features and 256 columns).
+    // (and its loads hold up the copies behind them: they return in order), so it is paid once for as
+    // many slabs as 96 registers hold, not once per slab (24k rows of 768 float16 features, 256 columns, all
+    // in one round: 94 us with a round trip per slab, 60 so).  Wider rows pay it once per such a round: with
+    // one chunk per thread 768 16-bit or 384 float32 features, with four a quarter of that.
     constexpr int KS = (FT == ET_F32 ? 12 : 24) / NC;
     using TA = RowTile<TM>;
     using TB = ColTile<TN>;
@@ -344,7 +346,9 @@ static int feature_waves(int Dp) { return Dp > 128 ? 8 : Dp > 64 ? 4 : 2; }
 void launch_feature_fwd(const FeatureArgs& a, float* hidden, hipStream_t stream) {
     const int nw = feature_waves(a.Dp), gx = (a.Dp + 32 * nw - 1) / (32 * nw), w_pitch = (a.Dp + 31) / 32 * 192;
     // rows per workgroup: a workgroup of eight waves fills a CU, so the tile height is the one with the
-    // fewest rows per CU over all rounds (24k rows: 96, one round of 250)
+    // fewest rows per CU over all rounds of workgroups.  max_rows is what the step may have, all its
+    // contributions; the distinct rows, on the device, are fewer: 24k of 32k get tiles of 128 (189 of 256
+    // workgroups with work, 57 us), where 24k alone would get 96.
     int am = 1;
     int64_t best = INT64_MAX;
     const int slots = 256 * (8 / nw);
