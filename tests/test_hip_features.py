@@ -81,3 +81,29 @@ def test_feature_shapes(oracle64, dtype, F, D, batch, all_distinct):
     bound = 5e-7 + 1.5 * 0.29 / np.sqrt(3) * 2.0**-24 * np.sqrt(12 * batch / 32)
     assert K.rel_l2(got["entity_data"][:, D:2 * D], want["entity_data"][:, D:2 * D]) < bound
     assert K.rel_l2(got["feature_projection/adam_m"], want["feature_projection/adam_m"]) < bound
+
+
+# The loads of a row's last slab run on into the row behind it: nothing of that row may enter, a NaN included.
+@pytest.mark.parametrize("dtype,F", [("float32", 4), ("float32", 36), ("float16", 8), ("float16", 40), ("bfloat16", 40)])
+@pytest.mark.parametrize("D", [30, 66, 130])
+def test_row_behind_stays_out(dtype, F, D):
+    import libpoplar_kge
+
+    c = K.cfg_dict(distance_fn="L2", n_shard=1, batch=40, a2a=2, dim=D, feature=F, n_entity=300, n_relation=6, gamma=4.0)
+    rng = np.random.default_rng(3)
+    state, batch = K.make_state(c, rng, warm=False), K.random_batch(c, 1, rng)
+    used = np.unique(batch["remote"])
+    unused = np.setdiff1d(np.arange(c["n_entity"]), used)
+    assert np.isin(used + 1, unused).any()
+    after = []
+    for value in (0.0, np.nan):
+        start = K.copy_state(state)
+        start["entity_data"][unused] = value
+        engine = libpoplar_kge.Engine(H.engine_settings(c, 1, **{"execution.feature_dtype": dtype}), "")
+        H.load_state(engine, c, start)
+        loss = H.train(engine, c, np.full(1, 1e-3, np.float32), batch)
+        got = H.read_state(engine, c)
+        after.append((loss, got["entity_data"][used], got["feature_projection/adam_m"], got["relation_embedding"]))
+    for clean, beside in zip(*after):
+        assert np.isfinite(clean).all()
+        np.testing.assert_array_equal(clean, beside)
