@@ -798,15 +798,11 @@ void launch_bwd(const BwdParams& p, int dist_fn, hipStream_t stream) {
 // One workgroup of 16 waves per (block, 64-column slice, group of heads, group of at most 512
 // tails: l1_pair_split); a lane owns one column.  Wave w keeps tails [w*tw, (w+1)*tw) of the
 // group and their gradient sums in registers and walks over the group's heads; a head's sum over one wave's tails is a
-// partial, the 16 partials of a head meet in LDS and are added in wave order
-// (deterministic).  The coefficients of a (head, tail range) are the same for
-// every lane: the workgroup stages the coefficient rows of eight heads at a time
-// in LDS (one 16-byte load per thread, the next chunk's in flight under the
-// current one's arithmetic) and every wave reads its four at a time with one
-// LDS instruction whose lanes all name the same address (a broadcast, no bank
-// conflict).  As scalar loads (wave-uniform operands straight from memory) the
-// same coefficients bounded the kernel: each of a block's four column slices
-// pulled the whole coefficient matrix through the scalar caches.
+// partial, the 16 partials of a head meet in LDS and are added in a fixed order.
+// The coefficients of a (head, tail) are the same for every lane: a wave brings those of eight heads and
+// its own tails to LDS (one load of four per lane, the next chunk's in flight under the current one's
+// arithmetic) and reads them four at a time with one instruction whose lanes all name the same address (a broadcast:
+// 4 cycles per CU).  As scalar operands the same coefficients halve the rate of the instructions that take them.
 constexpr int L1P_CB = 8;      // heads per chunk
 constexpr int L1P_WAVES = 16;
 
@@ -814,14 +810,33 @@ constexpr int L1P_MAX_T = 512;  // tails per workgroup at most (32 per wave)
 
 // One workgroup's share of a block: its heads, its tails, its 64 columns.
 struct L1Pair {
-    const float* a_rows;  // the first head's value in this lane's column
+    const float* a_rows;  // the first head's value in the block's first column; rows Dp apart
     const float* b_rows;  // the first tail's
     const float* coef;    // coefficient of the first head and the first tail; rows `ldc` apart
-    float* grad_a;        // where the first head's gradient in this lane's column goes
+    float* grad_a;        // where the first head's gradient in the block's first column goes
     float* grad_b;
     int n_head, n_tail, ldc, Dp;
-    bool col;             // this lane has a column
+    int k0, kc;           // the slice's first column, this lane's column
+    bool col;             // this lane has a column (another lane's otherwise)
 };
+
+// What the workgroup keeps in LDS: every wave's coefficients of a chunk and half their column sums
+// (nobody else's business), and the heads' partial sums.
+struct L1PairLds {
+    float cs[L1P_WAVES][2][L1P_CB][L1P_MAX_T / L1P_WAVES];
+    float col_half[L1P_WAVES][L1P_MAX_T / L1P_WAVES];
+    float part[2][L1P_WAVES][L1P_CB][64];
+};
+
+template <int CTRL>
+DEVINL float dpp_f32(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+// this wave's LDS accesses before and after stay in that order (the hardware keeps a wave's order by itself)
+DEVINL void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 // the work of one wave with exactly TW tails (TW even): straight-line code over
 // its tails, their values and sums in registers.
@@ -836,126 +851,179 @@ struct L1Pair {
 //           sum c (p - 1/2) = (1/2) sum c signum;
 //   heads   each wave's partial 2 sum_j c p minus the sum of the coefficients of its own TW
 //           columns, before the 16 waves' values are added.
-// The column and row-part sums of a chunk come from the coefficient rows staged in LDS, by waves
-// 8 .. 15 while waves 0 .. 7 add the head partials of the chunk before.
-// FULL: whole chunks of heads, 16-byte coefficient loads, readable zero coefficients up to the next
+// Either linear part is summed in the order of the multiply-adds that it is taken from, so that a column in
+// which heads and tails are equal (p = 1/2 throughout: the padding, rows of zeros) comes out as exactly zero.
+// Bound by vector issue.  A head's sum runs in four chains: in one chain every multiply-add waits for
+// the one before, and four waves per SIMD do not fill that gap (a register-only loop of these
+// four instructions: 3.05 cycles of 2.4 GHz per instruction with one chain, 2.25 with four).  Everything
+// but the heads' partial sums belongs to a wave alone, is asked for a chunk ahead, and is worked off between the
+// heads; one barrier per chunk.  64 blocks of 256 x 512 (331 distinct tails each), D = 256: 147 -> 132 us; 16 of 512 x 1536:
+// 315 -> 284.  2.6 cycles per instruction, of which one in seven is not the pairs' own; the rest of the launch
+// is waiting for the block with the most distinct tails (7 % above their mean) and for its start and end.
+// FULL: whole chunks of heads, 8-byte coefficient loads, readable zero coefficients up to the next
 // multiple of 32 tails and a column in every lane: no bounds checks.
 template <int TW, bool FULL>
-DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane,
-                         float (*part)[L1P_WAVES][L1P_CB][64], float (*cs)[L1P_CB][L1P_MAX_T],
-                         float (*col_half)[L1P_MAX_T], float (*row_part)[L1P_CB][L1P_WAVES]) {
-    // In LDS a wave's TW columns start at a multiple of four (TWS apart): its reads stay 16-byte
-    // ones when TW is not a multiple of four.  Column c lies at lds_col(c).
-    constexpr int TWS = (TW + 3) & ~3;
-    constexpr int TL = TW * L1P_WAVES, T4 = TL / 4;  // tails of the workgroup, filled up
-    auto lds_col = [](int c) { return (c / TW) * TWS + c % TW; };
-    const int tid = threadIdx.x, l0 = w * TWS, Dp = q.Dp, n_head = q.n_head;
-    // staging: thread -> (head, four columns) of a chunk's coefficient rows, stored as two pairs
-    // (TW is even, so a pair never straddles two waves' columns)
-    const bool stager = tid < L1P_CB * T4;
-    const int s_head = tid / T4, s_col = (tid - s_head * T4) * 4;
-    const int s_lo = lds_col(s_col), s_hi = lds_col(s_col + 2);
+DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane, L1PairLds& lds) {
+    constexpr int TWM = L1P_MAX_T / L1P_WAVES;
+    const int n_head = q.n_head, t0 = w * TW;
+    const size_t Dp = q.Dp;
+    // staging: lane -> (head, four columns) of the wave's coefficients of a chunk.  Loads without a branch
+    // (a lane that has nothing to fetch fetches something else: a load that may not have been issued would be
+    // waited for together with what was asked for before it); what does not count becomes zero when it has come.
+    const int s_head = lane >> 3, s_col = (lane & 7) * 4;
+    const int s_n = (FULL ? TW : min(TW, q.n_tail - t0)) - s_col;  // columns of this lane that count
     auto fetch = [&](int b0) __attribute__((always_inline)) {
-        const float* src = q.coef + (size_t)(b0 + s_head) * q.ldc + s_col;
-        if constexpr (FULL) return *reinterpret_cast<const float4*>(src);
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (b0 + s_head < n_head) {
-            if (s_col + 0 < q.n_tail) v.x = src[0];
-            if (s_col + 1 < q.n_tail) v.y = src[1];
-            if (s_col + 2 < q.n_tail) v.z = src[2];
-            if (s_col + 3 < q.n_tail) v.w = src[3];
+        if constexpr (FULL) {
+            const float* src = q.coef + (size_t)(b0 + s_head) * q.ldc + t0;
+            const float2 lo = *reinterpret_cast<const float2*>(src + (s_n > 0 ? s_col : 0));
+            const float2 hi = *reinterpret_cast<const float2*>(src + (s_n > 2 ? s_col + 2 : 0));
+            return make_float4(lo.x, lo.y, hi.x, hi.y);
         }
-        return v;
+        const float* src = q.coef + (size_t)min(b0 + s_head, n_head - 1) * q.ldc;
+        const int last = q.n_tail - 1;
+        return make_float4(src[min(t0 + s_col, last)], src[min(t0 + s_col + 1, last)],
+                           src[min(t0 + s_col + 2, last)], src[min(t0 + s_col + 3, last)]);
     };
-    auto stage = [&](int buf, float4 v) __attribute__((always_inline)) {
-        *reinterpret_cast<float2*>(&cs[buf][s_head][s_lo]) = make_float2(v.x, v.y);
-        *reinterpret_cast<float2*>(&cs[buf][s_head][s_hi]) = make_float2(v.z, v.w);
+    // a chunk's coefficients into the wave's tile `buf`
+    auto stage = [&](int buf, int b0, float4 v) __attribute__((always_inline)) {
+        const int n = FULL || b0 + s_head < n_head ? s_n : 0;
+        if (n < 1) v.x = 0.f;
+        if (n < 2) v.y = 0.f;
+        if (n < 3) v.z = 0.f;
+        if (n < 4) v.w = 0.f;
+        *reinterpret_cast<float4*>(&lds.cs[w][buf][s_head][s_col]) = v;
     };
-    // linear parts: thread 512 + t -> column t; threads 512 .. 639 -> (head, wave)
-    const int u = tid - 512, u_lds = u >= 0 ? lds_col(u) : 0;
-    float4 c_next = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (stager) {
-        c_next = fetch(0);
-        stage(0, c_next);
-    }
+    // the sums of a chunk's coefficients per head (the same in the head's eight lanes)
+    constexpr int NG = (TW + 3) / 4;
+    auto row_sums = [&](int buf) __attribute__((always_inline)) {
+        const float* c = &lds.cs[w][buf][s_head][lane & 3];
+        float r = c[0];
+#pragma unroll
+        for (int g = 1; g < NG; ++g) r += c[4 * g];
+        r += dpp_f32<0xB1>(r);  // lane ^ 1
+        r += dpp_f32<0x4E>(r);  // lane ^ 2
+        return r;
+    };
+    // (the row's address in scalar registers: one 32-bit lane offset serves all loads)
+    auto head_value = [&](int b) __attribute__((always_inline)) {
+        typedef const __attribute__((address_space(1))) float* global_row;
+        global_row row = (global_row)q.a_rows + (size_t)__builtin_amdgcn_readfirstlane(FULL ? b : min(b, n_head - 1)) * Dp;
+        asm("" : "+s"(row));
+        return row[(uint32_t)q.kc];
+    };
     float bt[TW], gt[TW];
 #pragma unroll
     for (int j = 0; j < TW; ++j) {
-        const int t = w * TW + j;
-        bt[j] = q.b_rows[(size_t)(FULL ? t : min(t, q.n_tail - 1)) * Dp];
+        bt[j] = q.b_rows[(size_t)(FULL ? t0 + j : min(t0 + j, q.n_tail - 1)) * Dp + q.kc];
         gt[j] = 0.f;
     }
-    // the heads' values, asked for two heads ahead of their use (one ahead leaves the load's
-    // latency showing at the end of every head: 170 -> 161 us on the 22.8M-row L1 workload;
-    // three ahead measures the same as two)
-    float a_q0 = q.a_rows[0], a_q1 = q.a_rows[(size_t)min(1, n_head - 1) * Dp];
-    __syncthreads();
-    int buf = 0;
-    for (int b0 = 0; b0 < n_head; b0 += L1P_CB, buf ^= 1) {
-        const bool more = b0 + L1P_CB < n_head;
-        if (stager && more) c_next = fetch(b0 + L1P_CB);
-        if (b0 > 0) {
+    // sixteen partials of a head: wave w takes head w / 2 of the chunk and half of the columns, the lower lanes the
+    // first eight waves' partials, the upper ones the others'
+    const int r_head = w >> 1, r_col = (w & 1) * 32 + (lane & 31), r_wave = (lane >> 5) * 8;
+    const bool r_there = lane < 32 && (FULL || q.k0 + r_col < q.Dp);
+    float red[8];
+    auto ask = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int v = 0; v < 8; ++v) red[v] = lds.part[buf][r_wave + v][r_head][r_col];
+    };
+    auto give = [&](int b0) __attribute__((always_inline)) {
+        float sum = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
+        sum += __shfl_xor(sum, 32, 64);
+        const int b = b0 + r_head;
+        if (r_there && b >= 0 && (FULL || b < n_head)) q.grad_a[(size_t)b * Dp + q.k0 + r_col] = sum;
+    };
+    stage(0, 0, fetch(0));
+    wave_lds_fence();
+    float row_sum = row_sums(0);
+    lds.col_half[w][lane & (TWM - 1)] = 0.f;
+    float a[L1P_CB];
+#pragma unroll
+    for (int h = 0; h < L1P_CB; ++h) a[h] = head_value(h);
+    // (waited for here: the loop's waits then count on the loop's own order of loads)
+#pragma unroll
+    for (int h = 0; h < L1P_CB; ++h) asm volatile("" : "+v"(a[h]));
+#pragma unroll
+    for (int j = 0; j < TW; ++j) asm volatile("" : "+v"(bt[j]));
+    int buf = 0, b0 = 0;
+    for (; b0 < n_head; b0 += L1P_CB, buf ^= 1) {
+        const int next = FULL ? min(b0 + L1P_CB, n_head - L1P_CB) : b0 + L1P_CB;  // (past the end: never used)
+        float4 c_next = fetch(next);
+        float next_sum = 0.f;
+        wave_lds_fence();
+        // four tails at a time, their coefficients read two groups ahead; the order of the groups is kept
+        // (left to itself the scheduler runs the heads into one another and out of registers)
+        float4 c4[3];
+        c4[0] = *reinterpret_cast<const float4*>(&lds.cs[w][buf][0][0]);
+        c4[1] = *reinterpret_cast<const float4*>(&lds.cs[w][buf][1 / NG][(1 % NG) * 4]);
+        float col[L1P_CB];
+        float4 half = *reinterpret_cast<const float4*>(&lds.col_half[w][0]);
+#pragma unroll
+        for (int h = 0; h < L1P_CB; ++h) {
+            // A wave that is behind goes first: left to themselves a SIMD's waves finish the chunk one after the
+            // other, and the last one, alone, issues at half the rate (4.3 cycles per instruction against
+            // 2.3 with company).
+            if (h == 0) __builtin_amdgcn_s_setprio(3);
+            if (h == 3) __builtin_amdgcn_s_setprio(2);
+            if (h == 6) __builtin_amdgcn_s_setprio(1);
+            if (h == 7) __builtin_amdgcn_s_setprio(0);
+            // what is not the pairs' own work, each part's operands asked for a head before they are used, so that
+            // nothing but the barrier stands between two chunks: the heads' sums of the chunk before, this
+            // chunk's column sums, the next chunk's coefficients
+            if (h == 1) ask(buf ^ 1);
+            if (h == 2) give(b0 - L1P_CB);
+            if (h == 3)
+#pragma unroll
+                for (int i = 0; i < L1P_CB; ++i) col[i] = lds.cs[w][buf][i][lane & (TWM - 1)];
+            if (h == 4) {  // (both halves of the wave: the same value)
+                lds.col_half[w][lane & (TWM - 1)] =
+                    0.5f * (((((((col[0] + col[1]) + col[2]) + col[3]) + col[4]) + col[5]) + col[6]) + col[7]);
+            }
+            if (h == 6) {
+                asm volatile("" : "+v"(c_next.x), "+v"(c_next.y), "+v"(c_next.z), "+v"(c_next.w));  // (not before)
+                stage(buf ^ 1, next, c_next);
+                wave_lds_fence();
+            }
+            if (h == 7) next_sum = row_sums(buf ^ 1);
+            float gp[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int j4 = 0; j4 < TW; j4 += 4) {
-                const float4 h4 = *reinterpret_cast<const float4*>(&col_half[buf ^ 1][l0 + j4]);
-                const float hv[4] = {h4.x, h4.y, h4.z, h4.w};
+                const int g = h * NG + j4 / 4, ahead = min(g + 2, L1P_CB * NG - 1);
+                c4[(g + 2) % 3] = *reinterpret_cast<const float4*>(&lds.cs[w][buf][ahead / NG][(ahead % NG) * 4]);
+                const float cv[4] = {c4[g % 3].x, c4[g % 3].y, c4[g % 3].z, c4[g % 3].w};
+                float d[4], p[4];
+                if (h == 0) {  // the chunk before's
+                    const float hv[4] = {half.x, half.y, half.z, half.w};
 #pragma unroll
-                for (int x = 0; x < 4; ++x)
-                    if (j4 + x < TW) gt[j4 + x] -= hv[x];
-            }
-        }
-        if (u >= 0) {
-            if (u < TL) {
-                float sum = 0.f;
+                    for (int x = 0; x < 4; ++x) if (j4 + x < TW) gt[j4 + x] -= hv[x];
+                    half = *reinterpret_cast<const float4*>(&lds.col_half[w][min(j4 + 4, TWM - 4)]);
+                }
 #pragma unroll
-                for (int h = 0; h < L1P_CB; ++h) sum += cs[buf][h][u_lds];
-                col_half[buf][u_lds] = 0.5f * sum;
-            }
-            if (u < L1P_CB * L1P_WAVES) {
-                const int h = u / L1P_WAVES, v = u % L1P_WAVES;
-                float sum = 0.f;
+                for (int x = 0; x < 4; ++x) d[x] = a[h] - bt[min(j4 + x, TW - 1)];
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int j = 0; j < TW; ++j) sum += cs[buf][h][v * TWS + j];
-                row_part[buf][h][v] = sum;
-            }
-        }
-#pragma unroll 1
-        for (int bi = 0; bi < L1P_CB; ++bi) {
-            const float a = a_q0;
-            a_q0 = a_q1;
-            a_q1 = q.a_rows[(size_t)min(b0 + bi + 2, n_head - 1) * Dp];
-            const float* c = &cs[buf][bi][l0];
-            float gp = 0.f;
-#pragma unroll
-            for (int j4 = 0; j4 < TW; j4 += 4) {
-                const float4 c4 = *reinterpret_cast<const float4*>(c + j4);
-                const float cv[4] = {c4.x, c4.y, c4.z, c4.w};
+                for (int x = 0; x < 4; ++x) p[x] = __builtin_amdgcn_fmed3f(fmaf(d[x], 0x1p126f, 0.5f), 0.f, 1.f);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int x = 0; x < 4; ++x) {
                     if (j4 + x >= TW) continue;
-                    const float p = __builtin_amdgcn_fmed3f(fmaf(a - bt[j4 + x], 0x1p126f, 0.5f), 0.f, 1.f);
-                    gp = fmaf(cv[x], p, gp);
-                    gt[j4 + x] = fmaf(cv[x], p, gt[j4 + x]);
+                    gp[x] = fmaf(cv[x], p[x], gp[x]);
+                    gt[j4 + x] = fmaf(cv[x], p[x], gt[j4 + x]);
+                    asm volatile("" : "+v"(gt[j4 + x]));  // (not put off to the end of the chunk)
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            part[buf][w][bi][lane] = gp;
+            a[h] = head_value(next + h);  // the next chunk's: a chunk's time to arrive
+            const float rs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(row_sum), h * 8));
+            lds.part[buf][w][h][lane] = fmaf(2.f, (gp[0] + gp[1]) + (gp[2] + gp[3]), -rs);
         }
-        if (stager && more) stage(buf ^ 1, c_next);
+        row_sum = next_sum;
         __syncthreads();
-        // waves 0 .. 7 add the 16 partials of head b0 + w
-        if (w < L1P_CB && (FULL || (b0 + w < n_head && q.col))) {
-            float sum = 0.f;
-#pragma unroll
-            for (int v = 0; v < L1P_WAVES; ++v) sum += fmaf(2.f, part[buf][v][w][lane], -row_part[buf][w][v]);
-            q.grad_a[(size_t)(b0 + w) * Dp] = sum;
-        }
     }
-    const int last = buf ^ 1;
+    ask(buf ^ 1);
+    give(b0 - L1P_CB);
 #pragma unroll
-    for (int j = 0; j < TW; ++j) {
-        const int t = w * TW + j;
-        if (FULL || (t < q.n_tail && q.col)) q.grad_b[(size_t)t * Dp] = -2.f * (gt[j] - col_half[last][l0 + j]);
-    }
+    for (int j = 0; j < TW; ++j)
+        if (FULL || (t0 + j < q.n_tail && q.col)) q.grad_b[(size_t)(t0 + j) * Dp + q.kc] = -2.f * (gt[j] - lds.col_half[w][j]);
 }
 
 // How a block's pairs are divided: `heads` x `tails` groups, every group a workgroup per 64 columns.
@@ -998,14 +1066,7 @@ __global__ __launch_bounds__(1024) void k_score_bwd_l1_pair(const float* __restr
                                                             int S, int B, int T, int Dp, int a_c0, int b_c0,
                                                             int h_groups, int t_groups, int h_size,
                                                             const uint32_t* __restrict__ tcount) {
-    // the coefficient rows first: their reads in the inner loop then carry the whole address
-    // offset in the instruction
-    __shared__ __attribute__((aligned(16))) struct {
-        float cs[2][L1P_CB][L1P_MAX_T];
-        float col_half[2][L1P_MAX_T];
-        float row_part[2][L1P_CB][L1P_WAVES];
-        float part[2][L1P_WAVES][L1P_CB][64];
-    } lds;
+    __shared__ __attribute__((aligned(16))) L1PairLds lds;
     const TileId tile = xcd_tile((Dp + 63) / 64, h_groups * t_groups, S);
     const int d = tile.z, lane = threadIdx.x & 63, k = tile.x * 64 + lane;
     const int hg = tile.y / t_groups, tg = tile.y - hg * t_groups;
@@ -1022,23 +1083,24 @@ __global__ __launch_bounds__(1024) void k_score_bwd_l1_pair(const float* __restr
     q.n_tail = __builtin_amdgcn_readfirstlane(min(t_size, live - t0));
     q.n_head = __builtin_amdgcn_readfirstlane(min(h_size, B - h0));
     q.col = FULL || k < Dp;
-    const int kc = FULL ? k : min(k, Dp - 1);
+    q.k0 = tile.x * 64;
+    q.kc = FULL ? k : min(k, Dp - 1);
     q.Dp = Dp; q.ldc = T;
-    q.grad_a = grad_heads + ((size_t)(t_groups > 1 ? tg : 0) * S * B + (size_t)d * B + h0) * Dp + kc;
-    q.grad_b = grad_tails + ((size_t)(h_groups > 1 ? hg : 0) * S * T + (size_t)d * T + t0) * Dp + kc;
+    q.grad_a = grad_heads + ((size_t)(t_groups > 1 ? tg : 0) * S * B + (size_t)d * B + h0) * Dp;
+    q.grad_b = grad_tails + ((size_t)(h_groups > 1 ? hg : 0) * S * T + (size_t)d * T + t0) * Dp;
     if (q.n_head <= 0 || q.n_tail <= 0) {  // rounding left this group empty: its pieces of the sums are zero
         if (q.col) {
-            for (int b = w; b < q.n_head; b += L1P_WAVES) q.grad_a[(size_t)b * Dp] = 0.f;
-            for (int t = w; t < q.n_tail; t += L1P_WAVES) q.grad_b[(size_t)t * Dp] = 0.f;
+            for (int b = w; b < q.n_head; b += L1P_WAVES) q.grad_a[(size_t)b * Dp + q.kc] = 0.f;
+            for (int t = w; t < q.n_tail; t += L1P_WAVES) q.grad_b[(size_t)t * Dp + q.kc] = 0.f;
         }
         return;
     }
-    q.a_rows = operands + (size_t)(a_c0 + d * B + h0) * Dp + kc;
-    q.b_rows = operands + (size_t)(b_c0 + d * T + t0) * Dp + kc;
+    q.a_rows = operands + (size_t)(a_c0 + d * B + h0) * Dp;
+    q.b_rows = operands + (size_t)(b_c0 + d * T + t0) * Dp;
     q.coef = coef + ((size_t)d * B + h0) * T + t0;
     const int tw = ((q.n_tail + 31) & ~31) / L1P_WAVES;
 #define KGE_L1P(TW_) \
-    case TW_: l1_pair_wave<TW_, FULL>(q, w, lane, lds.part, lds.cs, lds.col_half, lds.row_part); break;
+    case TW_: l1_pair_wave<TW_, FULL>(q, w, lane, lds); break;
     switch (tw) {  // one of sixteen copies of the loop, chosen per group
         KGE_L1P(2) KGE_L1P(4) KGE_L1P(6) KGE_L1P(8) KGE_L1P(10) KGE_L1P(12) KGE_L1P(14) KGE_L1P(16)
         KGE_L1P(18) KGE_L1P(20) KGE_L1P(22) KGE_L1P(24) KGE_L1P(26) KGE_L1P(28) KGE_L1P(30) KGE_L1P(32)

@@ -29,6 +29,34 @@ def test_l1_shapes(oracle64, S, B, A, D, merge):
                             n_relation=16, gamma=4.0), n_step=2, **{"execution.merge_tails": merge})
 
 
+# L1 backward without bounds checks (tails in steps of 32, heads of 8, columns of 64): tails per wave that are
+# and are not a multiple of four, one chunk of heads and several
+@pytest.mark.parametrize("B,A,D", [(8, 32, 64), (16, 96, 128), (24, 160, 64), (64, 352, 64), (8, 512, 64), (264, 544, 64)])
+def test_l1_whole_groups(oracle64, B, A, D):
+    run_case(oracle64, dict(distance_fn="L1", n_shard=1, batch=B, a2a=A, dim=D, feature=0, n_entity=4000, n_relation=16,
+                            gamma=4.0), n_step=2, **{"execution.merge_tails": False})
+
+
+# Columns in which every head equals every tail have signum 0 throughout: their gradients are exactly zero
+@pytest.mark.parametrize("B,A,D", [(33, 90, 30), (64, 352, 64)])
+def test_l1_equal_columns_have_zero_gradient(B, A, D):
+    import libpoplar_kge
+
+    c = K.cfg_dict(distance_fn="L1", n_shard=1, batch=B, a2a=A, dim=D, feature=0, n_entity=2000, n_relation=9, gamma=4.0)
+    rng = np.random.default_rng(5)
+    state = K.make_state(c, rng, warm=False)
+    equal = np.arange(0, D, 3)
+    state["entity_data"][:, equal] = 0.25
+    state["relation_embedding"][:, equal] = 0.0
+    engine = libpoplar_kge.Engine(H.engine_settings(c, 2, **{"execution.merge_tails": False}), "")
+    H.load_state(engine, c, state)
+    H.train(engine, c, 0.1, K.random_batch(c, 2, rng))
+    after = H.read_state(engine, c)
+    np.testing.assert_array_equal(after["entity_data"][:, equal], state["entity_data"][:, equal])
+    np.testing.assert_array_equal(after["relation_embedding"][:, equal], state["relation_embedding"][:, equal])
+    np.testing.assert_array_equal(after["entity_data"][:, D + equal], 0.0)
+
+
 # L2 and dot on three-piece operands: tiles of 64 x 64 over slabs of 32, matrices filled up to 32
 @pytest.mark.parametrize("merge", [True, False])
 @pytest.mark.parametrize("score_fn,distance_fn", [("TransE", "L2"), ("DistMult", "MatMul"), ("ComplEx", "L2")])
