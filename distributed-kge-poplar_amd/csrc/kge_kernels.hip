@@ -20,6 +20,7 @@
 
 namespace kge {
 
+
 // --------------------------------------------------------------------------
 // operand gather: one wave per contribution copies its entity (or hidden) row,
 // converted to float32 and with the relation already applied for the heads
@@ -156,8 +157,7 @@ constexpr int BK = 32;         // embedding columns staged per iteration
 
 // ALIGNED: whole tiles and slabs of dense float32 operands with the relation already applied:
 // the staging loads carry no bounds checks, and the next slab's are in flight while the current
-// slab is worked on (86 -> 84 us on the 22.8M-row L1 workload: the other workgroups of a CU hide
-// most of that latency already).
+// slab is worked on.
 template <int DIST, int OM, bool ALIGNED = false>  // OM: FwdParams::out_mode, fixed at compile time
 __global__ __launch_bounds__(256) void k_score_fwd(FwdParams p) {
     __shared__ __attribute__((aligned(16))) float As[BK][LDP];
@@ -299,6 +299,207 @@ __global__ __launch_bounds__(256) void k_score_fwd(FwdParams p) {
                 (red[0] + red[1] + red[2] + red[3]) * inv_norm;
         }
     }
+}
+
+// --------------------------------------------------------------------------
+// L1 forward.  Tiles of 64 heads x 32 tails, four waves; a wave takes every fourth slab of eight columns for the whole
+// tile, a lane 8 x 4 pairs, and the four waves' sums meet at the end.  A slab is its wave's alone: it goes from
+// memory through registers (asked for a slab ahead) into the wave's own part of LDS, without a barrier.
+// Bound by vector issue: two instructions per pair and column, of which a SIMD takes one every 2.65 cycles.  64 blocks of 256
+// heads against 331 distinct tails on average, D = 256: 77 -> 69.5 us (49 of them the pairs' instructions; the loss terms 3, the
+// rest the waves' start and end), 16 of 512 x 1536: 131 -> 123 (108).  Against 64 x 64 tiles with 4 x 4 pairs per lane (the kernel
+// above) LDS is read three times per 64 instructions and not twice per 32, blocks end on 32 columns, and a block's
+// columns are summed in four parts.  64 x 64 tiles with 8 x 8 pairs per lane: 71 and 126 us, three or four waves
+// per SIMD where these have five.
+constexpr int L1F_K = 8;            // columns per slab (the four waves' slabs of a round are one 128-byte line of every row)
+constexpr int L1F_TN = 32;
+// a column's rows; a store instruction's two columns fall on different banks
+constexpr int L1F_LDA = kScoreTile + 8, L1F_LDB = L1F_TN + 8;
+
+struct L1FwdLds {
+    union {
+        struct { float a[L1F_K][L1F_LDA], b[L1F_K][L1F_LDB]; } slab[4];
+        float4 part[4][2][2][64];  // partial sums of two of the four waves' shares
+    };
+    float red[4];
+};
+
+template <int OM>
+DEVINL float l1_fwd_tile(const FwdParams& p, const int d, const int m0, const int n0, L1FwdLds& lds) {
+    const ScoreShape& sh = p.sh;
+    const int B = sh.B, T = sh.T, Dp = sh.Dp;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tx = lane & 7, ty = lane >> 3;  // rows 4 ty + 32 h .. + 3, columns 4 tx + 32 h .. + 3
+    // loads: rows lane / 2 + 32 i, columns 4 (lane % 2) .. + 3 of a slab
+    const int r0 = lane >> 1, kq = (lane & 1) * 4;
+    const char* const a_base = p.ent_a.base + (int64_t)(p.a_c0 + d * B + m0) * p.ent_a.pitch;
+    const char* const b_base = p.ent_b.base + (int64_t)(p.b_c0 + d * T + n0) * p.ent_b.pitch;
+    uint32_t a_off[2], b_off[1];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) a_off[i] = (uint32_t)min(r0 + 32 * i, B - 1 - m0) * (uint32_t)p.ent_a.pitch;
+#pragma unroll
+    for (int i = 0; i < 1; ++i) b_off[i] = (uint32_t)min(r0 + 32 * i, T - 1 - n0) * (uint32_t)p.ent_b.pitch;
+    float acc[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+    float4 ra[2], rb[1];
+    auto prefetch = [&](int slab) __attribute__((always_inline)) {  // (past the last column: that row's last four again)
+        const uint32_t at = (uint32_t)min(slab * L1F_K + kq, Dp - 4) * 4u;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) ra[i] = *reinterpret_cast<const float4*>(a_base + (a_off[i] + at));
+#pragma unroll
+        for (int i = 0; i < 1; ++i) rb[i] = *reinterpret_cast<const float4*>(b_base + (b_off[i] + at));
+    };
+    float (&As)[L1F_K][L1F_LDA] = lds.slab[wave].a;
+    float (&Bs)[L1F_K][L1F_LDB] = lds.slab[wave].b;
+    const int n_slab = (Dp + L1F_K - 1) / L1F_K;
+    // what the loss needs, asked for together and ahead of everything else: this lane's pairs at the end are rows m, m + 1
+    // and columns n .. n + 3
+    const int m = m0 + 4 * ty + 32 * (wave >> 1) + 2 * (wave & 1), n = n0 + 4 * tx;
+    uint32_t label[2];
+    float mult[4];
+    if (OM == 0) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) label[i] = p.clabel[d * B + min(m + i, B - 1)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mult[j] = sh.tmult ? sh.tmult[(size_t)d * T + min(n + j, T - 1)] : 1.f;
+    }
+    prefetch(wave);
+    for (int slab = wave; slab < n_slab; slab += 4) {
+        if ((slab + 1) * L1F_K > Dp && slab * L1F_K + kq >= Dp) {  // columns that do not exist: no difference
+#pragma unroll
+            for (int i = 0; i < 2; ++i) ra[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int i = 0; i < 1; ++i) rb[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        wave_lds_fence();
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            As[kq][r0 + 32 * i] = ra[i].x; As[kq + 1][r0 + 32 * i] = ra[i].y;
+            As[kq + 2][r0 + 32 * i] = ra[i].z; As[kq + 3][r0 + 32 * i] = ra[i].w;
+        }
+#pragma unroll
+        for (int i = 0; i < 1; ++i) {
+            Bs[kq][r0 + 32 * i] = rb[i].x; Bs[kq + 1][r0 + 32 * i] = rb[i].y;
+            Bs[kq + 2][r0 + 32 * i] = rb[i].z; Bs[kq + 3][r0 + 32 * i] = rb[i].w;
+        }
+        wave_lds_fence();
+        prefetch(slab + 4);
+        // A column's pairs in quarters of 4 x 4, in an order in which the operands of the next column take the place of
+        // this one's a quarter or more before they are needed.  Four differences, then their four sums: an
+        // instruction that follows on the one it depends on waits.  The order is kept (left to itself the scheduler pairs
+        // them up and asks for a column's operands when it needs them).
+        float a[2][4], b[2][4];
+        auto ask_a = [&](int kk, int h) __attribute__((always_inline)) {
+            *reinterpret_cast<float4*>(a[h]) = *reinterpret_cast<const float4*>(&As[min(kk, L1F_K - 1)][4 * ty + 32 * h]);
+        };
+        auto ask_b = [&](int kk) __attribute__((always_inline)) {
+            *reinterpret_cast<float4*>(b[kk & 1]) = *reinterpret_cast<const float4*>(&Bs[min(kk, L1F_K - 1)][4 * tx]);
+        };
+        auto half = [&](int kk, int ah) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float t[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) t[j] = a[ah][i] - b[kk & 1][j];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[4 * ah + i][j] += fabsf(t[j]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        ask_a(0, 0);
+        ask_b(0);
+        ask_a(0, 1);
+#pragma unroll
+        for (int kk = 0; kk < L1F_K; ++kk) {
+            ask_b(kk + 1);
+            half(kk, 0);
+            ask_a(kk + 1, 0);
+            half(kk, 1);
+            ask_a(kk + 1, 1);
+        }
+    }
+    // wave w ends up with the sums of every lane's rows 2 w and 2 w + 1 of eight
+    float sum[2][4];
+#pragma unroll
+    for (int round = 0; round < 2; ++round) {
+        __syncthreads();
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                lds.part[wave][x][i][lane] = *reinterpret_cast<const float4*>(&acc[4 * round + 2 * x + i][0]);
+        __syncthreads();
+        if (wave >> 1 == round)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                float4 v[4];
+#pragma unroll
+                for (int w = 0; w < 4; ++w) v[w] = lds.part[w][wave & 1][i][lane];
+                *reinterpret_cast<float4*>(sum[i]) = f4add(f4add(v[0], v[1]), f4add(v[2], v[3]));
+            }
+    }
+
+    const float Tn = (float)T;
+    const float w_pos = uniform_f32(0.5f * Tn), w_neg = uniform_f32((0.5f * Tn) / (float)(T - 1));
+    const float grad_scale = uniform_f32(1.f / ((float)sh.S * (float)B * Tn) * sh.loss_scale);
+    float loss_acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        if (m + i >= B) continue;
+        float* const crow = p.coef + ((size_t)d * B + m + i) * T;
+        float out[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float dist = sum[i][j];
+            const float score = score_is_distance_value(sh.score_fn) ? dist : sh.gamma - dist;
+            if (OM == 2) out[j] = dist;
+            else if (OM == 1) out[j] = score;
+            else {
+                float ds;  // d loss / d score, times the loss scale
+                const float term = logsigmoid_column(score, (uint32_t)(n + j) == label[i], mult[j], w_pos, w_neg, grad_scale, ds);
+                if (n + j < T) loss_acc += term;
+                out[j] = score_is_distance_value(sh.score_fn) ? ds : -ds;
+            }
+        }
+        if (n + 3 < T && (T & 3) == 0) *reinterpret_cast<float4*>(crow + n) = make_float4(out[0], out[1], out[2], out[3]);
+        else
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (n + j < T) crow[n + j] = out[j];
+    }
+    return loss_acc;
+}
+
+template <int OM>
+__global__ __launch_bounds__(256, 5) void k_score_fwd_l1(FwdParams p) {
+    __shared__ __attribute__((aligned(16))) L1FwdLds lds;
+    const ScoreShape& sh = p.sh;
+    const int B = sh.B, T = sh.T;
+    const TileId tile = xcd_tile((T + L1F_TN - 1) / L1F_TN, (B + kScoreTile - 1) / kScoreTile, sh.S);
+    const int d = tile.z, m0 = tile.y * kScoreTile, n0 = tile.x * L1F_TN, part = d * (tile.gx * tile.gy) + tile.y * tile.gx + tile.x;
+    // merged tails: no columns behind the limit; and with the fused loss those behind the distinct tails, which stand for
+    // none, have zeros for coefficients without a look at the distance
+    const int limit = tail_limit(sh.tcount, d, T, sh.tpad), live = OM == 0 && sh.tcount ? min(limit, (int)sh.tcount[d]) : limit;
+    if (n0 >= live) {
+        if (OM == 0 && threadIdx.x == 0) p.loss_part[part] = 0.f;
+        if (n0 < limit) {
+            const int n = n0 + (threadIdx.x & 31);
+            for (int m = m0 + (threadIdx.x >> 5); m < min(m0 + kScoreTile, B); m += 8)
+                if (n < T) p.coef[((size_t)d * B + m) * T + n] = 0.f;
+        }
+        return;
+    }
+    float loss = l1_fwd_tile<OM>(p, d, m0, n0, lds);
+    if (OM != 0) return;
+    loss = wave_sum(loss);
+    if ((threadIdx.x & 63) == 0) lds.red[threadIdx.x >> 6] = loss;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        p.loss_part[part] = (lds.red[0] + lds.red[1] + lds.red[2] + lds.red[3]) * (1.f / ((float)sh.S * (float)B * (float)T));
 }
 
 // --------------------------------------------------------------------------
@@ -741,9 +942,15 @@ static bool fwd_uses_mfma(const FwdParams& p) {
     return p.sh.use_mfma && p.sh.dist_fn != DIST_L1 && p.ent_a.vec && p.ent_b.vec && (p.sh.Dp & 3) == 0;
 }
 
+// Shapes of k_score_fwd_l1: four slabs, one for every wave, are 32 columns; below 64 the loop is too short for what the
+// waves' sums cost.
+static bool fwd_l1_shape(const ScoreShape& sh) {
+    return sh.dist_fn == DIST_L1 && sh.score_fn != SCORE_DISTMULT && sh.score_fn != SCORE_TRANSH && sh.Dp >= 64 && (sh.Dp & 3) == 0;
+}
+
 int score_fwd_parts(const ScoreShape& sh) {
     const bool mfma = sh.use_mfma && !(sh.score_fn != SCORE_DISTMULT && sh.dist_fn == DIST_L1);
-    const int tm = mfma ? FM_TM : kScoreTile, tn = mfma ? FM_TN : kScoreTile;
+    const int tm = mfma ? FM_TM : kScoreTile, tn = mfma ? FM_TN : fwd_l1_shape(sh) ? L1F_TN : kScoreTile;
     return ((sh.T + tn - 1) / tn) * ((sh.B + tm - 1) / tm);
 }
 
@@ -784,7 +991,15 @@ static void launch_fwd(const FwdParams& p, hipStream_t stream) {
         else if (p.out_mode == 1) hipLaunchKernelGGL((k_score_fwd<D_, 1>), grid, dim3(256), 0, stream, p);    \
         else hipLaunchKernelGGL((k_score_fwd<D_, 2>), grid, dim3(256), 0, stream, p);                         \
     } while (0)
-    if (p.sh.dist_fn == DIST_L1) KGE_FWD_VALU(DIST_L1);
+    const bool dense = p.ent_a.etype == ET_F32 && p.ent_b.etype == ET_F32 && p.ent_a.vec && p.ent_b.vec && !p.ent_a.index &&
+                       !p.ent_b.index && p.a_rel_mode == 0;
+    if (dense && fwd_l1_shape(p.sh)) {
+        const dim3 grid = tile_grid((p.sh.T + L1F_TN - 1) / L1F_TN, (p.sh.B + kScoreTile - 1) / kScoreTile, p.sh.S);
+        if (p.out_mode == 0) hipLaunchKernelGGL(k_score_fwd_l1<0>, grid, dim3(256), 0, stream, p);
+        else if (p.out_mode == 1) hipLaunchKernelGGL(k_score_fwd_l1<1>, grid, dim3(256), 0, stream, p);
+        else hipLaunchKernelGGL(k_score_fwd_l1<2>, grid, dim3(256), 0, stream, p);
+    }
+    else if (p.sh.dist_fn == DIST_L1) KGE_FWD_VALU(DIST_L1);
     else if (p.sh.dist_fn == DIST_L2) KGE_FWD_VALU(DIST_L2);
     else KGE_FWD_VALU(DIST_DOT);
 #undef KGE_FWD_VALU

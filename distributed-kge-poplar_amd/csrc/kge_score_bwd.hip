@@ -832,11 +832,6 @@ template <int CTRL>
 DEVINL float dpp_f32(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
 }
-// this wave's LDS accesses before and after stay in that order (the hardware keeps a wave's order by itself)
-DEVINL void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 
 // the work of one wave with exactly TW tails (TW even): straight-line code over
 // its tails, their values and sums in registers.

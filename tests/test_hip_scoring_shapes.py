@@ -37,6 +37,16 @@ def test_l1_whole_groups(oracle64, B, A, D):
                             gamma=4.0), n_step=2, **{"execution.merge_tails": False})
 
 
+# L1 forward: tiles of 64 heads x 32 tails, four waves over slabs of eight columns (from 64 columns on): around a tile's
+# edges, a last slab of four columns, waves with and without one, distinct tails that end on a tile
+@pytest.mark.parametrize("merge", [True, False])
+@pytest.mark.parametrize("loss_fn", ["logsigmoid", "softmax"])
+@pytest.mark.parametrize("S,B,A,D", [(1, 1, 2, 64), (1, 63, 31, 68), (2, 64, 16, 72), (1, 65, 33, 100), (3, 130, 43, 260), (1, 8, 96, 128)])
+def test_l1_forward_tiles(oracle64, loss_fn, S, B, A, D, merge):
+    run_case(oracle64, dict(distance_fn="L1", loss_fn=loss_fn, n_shard=S, batch=B, a2a=A, dim=D, feature=0, n_entity=1500,
+                            n_relation=6, gamma=4.0), n_step=2, **{"execution.merge_tails": merge})
+
+
 # Columns in which every head equals every tail have signum 0 throughout: their gradients are exactly zero
 @pytest.mark.parametrize("B,A,D", [(33, 90, 30), (64, 352, 64)])
 def test_l1_equal_columns_have_zero_gradient(B, A, D):
