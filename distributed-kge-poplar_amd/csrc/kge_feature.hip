@@ -91,9 +91,19 @@ DEVINL void feature_products(const floatx4 (&fa)[AM][PA], const floatx4 (&fb)[3]
 // the columns: with D <= 256 a row's features come from memory once.  W lies as a piece matrix
 // (launch_split_matrix) and goes straight into LDS.
 template <int FT, int AM, int NW>
-__global__ __launch_bounds__(NW * 64) void k_feature_fwd(FeatureArgs a, const char* __restrict__ wp, int w_pitch,
-                                                         float* __restrict__ hidden) {
-    constexpr int PA = Pieces<FT>::n, TM = 32 * AM, TN = 32 * NW, NT = NW * 64;
+struct FeatureFwd {
+    static constexpr int PA = Pieces<FT>::n, TM = 32 * AM, TN = 32 * NW, NT = NW * 64;
+    using TA = RowTile<TM>;
+    using TB = ColTile<TN>;
+    static constexpr int kA = PA * TM * 64, kStage = kA + TB::kBytes;
+};
+template <int FT, int AM, int NW>
+DEVINL void feature_fwd_tile(const FeatureArgs& a, const char* __restrict__ wp, int w_pitch, float* __restrict__ hidden,
+                             char* const smem, uint32_t* const key_s) {
+    using Tile = FeatureFwd<FT, AM, NW>;
+    using TA = typename Tile::TA;
+    using TB = typename Tile::TB;
+    constexpr int PA = Tile::PA, TM = Tile::TM, TN = Tile::TN, NT = Tile::NT;
     constexpr int NC = (TM * 4 + NT - 1) / NT;  // 16-byte chunks of a slab per thread
     // Slabs whose features are asked for together: a row of the table is a round trip of microseconds
     // (and its loads hold up the copies behind them: they return in order), so it is paid once for as
@@ -101,11 +111,7 @@ __global__ __launch_bounds__(NW * 64) void k_feature_fwd(FeatureArgs a, const ch
     // in one round: 94 us with a round trip per slab, 60 so).  Wider rows pay it once per such a round: with
     // one chunk per thread 768 16-bit or 384 float32 features, with four a quarter of that.
     constexpr int KS = (FT == ET_F32 ? 12 : 24) / NC;
-    using TA = RowTile<TM>;
-    using TB = ColTile<TN>;
-    constexpr int kA = PA * TM * 64, kStage = kA + TB::kBytes, kEach = TB::kCopies / NW;
-    __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
-    __shared__ __attribute__((aligned(16))) uint32_t key_s[TM];
+    constexpr int kA = Tile::kA, kStage = Tile::kStage, kEach = TB::kCopies / NW;
     const int gx = (a.Dp + TN - 1) / TN;
     const int u0 = (int)blockIdx.x / gx * TM, n0 = (int)blockIdx.x % gx * TN;
     const int U = (int)a.counts[0];
@@ -244,6 +250,37 @@ __global__ __launch_bounds__(NW * 64) void k_feature_fwd(FeatureArgs a, const ch
         }
 }
 
+// Tile height (in 32 rows) for `rows` rows: the one with the fewest rows per CU over all rounds of workgroups.
+__host__ DEVINL uint32_t feature_tiles(uint32_t rows, int t, int gx) { return (rows + 32 * t - 1) / (32 * t) * gx; }
+__host__ DEVINL int feature_tile(uint32_t rows, int gx, uint32_t slots) {
+    int am = 1;
+    uint32_t best = UINT32_MAX;
+#pragma unroll
+    for (int t = 1; t <= 4; ++t) {
+        const uint32_t cost = (feature_tiles(rows, t, gx) + slots - 1) / slots * (2 + 3 * t);  // (a tile's W slabs cost as much as some rows)
+        if (cost < best) { best = cost; am = t; }
+    }
+    return am;
+}
+
+// AM = 0: the height is the one for the distinct rows, which only the device knows
+template <int FT, int AM, int NW>
+__global__ __launch_bounds__(NW * 64) void k_feature_fwd(FeatureArgs a, const char* __restrict__ wp, int w_pitch,
+                                                         float* __restrict__ hidden) {
+    using Most = FeatureFwd<FT, AM ? AM : 4, NW>;
+    __shared__ __attribute__((aligned(16))) char smem[2 * Most::kStage];
+    __shared__ __attribute__((aligned(16))) uint32_t key_s[Most::TM];
+    if constexpr (AM != 0) {
+        feature_fwd_tile<FT, AM, NW>(a, wp, w_pitch, hidden, smem, key_s);
+    } else {
+        const int am = feature_tile(a.counts[0], (a.Dp + 32 * NW - 1) / (32 * NW), 256 * (8 / NW));
+        if (am == 1) feature_fwd_tile<FT, 1, NW>(a, wp, w_pitch, hidden, smem, key_s);
+        else if (am == 2) feature_fwd_tile<FT, 2, NW>(a, wp, w_pitch, hidden, smem, key_s);
+        else if (am == 3) feature_fwd_tile<FT, 3, NW>(a, wp, w_pitch, hidden, smem, key_s);
+        else feature_fwd_tile<FT, 4, NW>(a, wp, w_pitch, hidden, smem, key_s);
+    }
+}
+
 // dW.  A workgroup takes 32 AM features x 32 NW columns over its share of the rows (the output has
 // few tiles: the contraction is split, the parts are added up by the update's kernel).  Both
 // operands lie across the contraction and are split while staged.
@@ -376,26 +413,28 @@ static int feature_waves(int Dp) { return Dp > 128 ? 8 : Dp > 64 ? 4 : 2; }
 
 void launch_feature_fwd(const FeatureArgs& a, float* hidden, hipStream_t stream) {
     const int nw = feature_waves(a.Dp), gx = (a.Dp + 32 * nw - 1) / (32 * nw), w_pitch = (a.Dp + 31) / 32 * 192;
-    // rows per workgroup: a workgroup of eight waves fills a CU, so the tile height is the one with the
-    // fewest rows per CU over all rounds of workgroups.  max_rows is what the step may have, all its
-    // contributions; the distinct rows, on the device, are fewer: 24k of 32k get tiles of 128 (189 of 256
-    // workgroups with work, 57 us), where 24k alone would get 96.
-    int am = 1;
-    int64_t best = INT64_MAX;
-    const int slots = 256 * (8 / nw);
-    for (int t = 1; t <= 4; ++t) {
-        const int64_t tiles = (int64_t)((a.max_rows + 32 * t - 1) / (32 * t)) * gx;
-        const int64_t cost = (tiles + slots - 1) / slots * (2 + 3 * t);  // (a tile's W slabs cost as much as some rows)
-        if (cost < best) { best = cost; am = t; }
+    // A workgroup of eight waves fills a CU whatever its height, so the kernel chooses it for the rows that it finds: 24k
+    // distinct ones of 32k contributions, 768 float16 features and 256 columns take 61 us in tiles of 128, which 32k
+    // rows would get, and 56 in tiles of 96, one for every CU.  The grid holds the most workgroups that any number of
+    // rows up to max_rows needs: that one, or one of those behind which a height takes another round.  Smaller
+    // workgroups share a CU by their LDS: theirs is the height for max_rows.
+    const uint32_t slots = 256 * (8 / nw), rows = a.max_rows;
+    int am = feature_tile(rows, gx, slots);
+    uint32_t most = feature_tiles(rows, am, gx);
+    if (nw == 8) {
+        for (int t = 1; t <= 4; ++t)
+            for (uint32_t round = 1, r; (r = round * slots / gx * (32 * t)) < rows; ++round)
+                most = std::max(most, feature_tiles(r, feature_tile(r, gx, slots), gx));
+        am = 0;
     }
-    const dim3 grid((unsigned)(((a.max_rows + 32 * am - 1) / (32 * am)) * gx));
+    const dim3 grid(most);
 #define KGE_FF(F_, A_, W_) hipLaunchKernelGGL((k_feature_fwd<F_, A_, W_>), grid, dim3(W_ * 64), 0, stream, a, (const char*)a.wp, w_pitch, hidden)
 #define KGE_FF_A(F_, W_)                                                                             \
     do {                                                                                             \
         if (am == 1) KGE_FF(F_, 1, W_); else if (am == 2) KGE_FF(F_, 2, W_);                         \
         else if (am == 3) KGE_FF(F_, 3, W_); else KGE_FF(F_, 4, W_);                                 \
     } while (0)
-#define KGE_FF_W(F_) do { if (nw == 8) KGE_FF_A(F_, 8); else if (nw == 4) KGE_FF_A(F_, 4); else KGE_FF_A(F_, 2); } while (0)
+#define KGE_FF_W(F_) do { if (nw == 8) KGE_FF(F_, 0, 8); else if (nw == 4) KGE_FF_A(F_, 4); else KGE_FF_A(F_, 2); } while (0)
     if (a.feat_etype == ET_F16) KGE_FF_W(ET_F16);
     else if (a.feat_etype == ET_BF16) KGE_FF_W(ET_BF16);
     else KGE_FF_W(ET_F32);
