@@ -125,6 +125,12 @@ DEVINL float wave_max(float v) {
 }
 
 
+// this wave's LDS accesses before and after stay in that order (the hardware keeps a wave's order by itself)
+DEVINL void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // --------------------------------------------------------------------------
 // Tile order.  The scoring kernels run gx * gy tiles for each of gz blocks; a
 // block's tiles all read that block's operand rows (and coefficient matrix).
@@ -132,12 +138,6 @@ DEVINL float wave_max(float v) {
 // L2, so with the plain (x, y, z) order each XCD would fetch every block's
 // operands.  Launching a 1-D grid and decoding it this way keeps a block's
 // tiles on one XCD (block z on XCD z % 8), in consecutive slots of that XCD.
-// this wave's LDS accesses before and after stay in that order (the hardware keeps a wave's order by itself)
-DEVINL void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 struct TileId { int x, y, z, gx, gy; };
 constexpr int kXcdGroup = 2;
 DEVINL TileId xcd_tile(int gx, int gy, int gz, int L) {

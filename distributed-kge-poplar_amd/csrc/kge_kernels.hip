@@ -20,7 +20,6 @@
 
 namespace kge {
 
-
 // --------------------------------------------------------------------------
 // operand gather: one wave per contribution copies its entity (or hidden) row,
 // converted to float32 and with the relation already applied for the heads
@@ -334,23 +333,21 @@ DEVINL float l1_fwd_tile(const FwdParams& p, const int d, const int m0, const in
     const int r0 = lane >> 1, kq = (lane & 1) * 4;
     const char* const a_base = p.ent_a.base + (int64_t)(p.a_c0 + d * B + m0) * p.ent_a.pitch;
     const char* const b_base = p.ent_b.base + (int64_t)(p.b_c0 + d * T + n0) * p.ent_b.pitch;
-    uint32_t a_off[2], b_off[1];
+    uint32_t a_off[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) a_off[i] = (uint32_t)min(r0 + 32 * i, B - 1 - m0) * (uint32_t)p.ent_a.pitch;
-#pragma unroll
-    for (int i = 0; i < 1; ++i) b_off[i] = (uint32_t)min(r0 + 32 * i, T - 1 - n0) * (uint32_t)p.ent_b.pitch;
+    const uint32_t b_off = (uint32_t)min(r0, T - 1 - n0) * (uint32_t)p.ent_b.pitch;
     float acc[8][4];
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-    float4 ra[2], rb[1];
+    float4 ra[2], rb;
     auto prefetch = [&](int slab) __attribute__((always_inline)) {  // (past the last column: that row's last four again)
         const uint32_t at = (uint32_t)min(slab * L1F_K + kq, Dp - 4) * 4u;
 #pragma unroll
         for (int i = 0; i < 2; ++i) ra[i] = *reinterpret_cast<const float4*>(a_base + (a_off[i] + at));
-#pragma unroll
-        for (int i = 0; i < 1; ++i) rb[i] = *reinterpret_cast<const float4*>(b_base + (b_off[i] + at));
+        rb = *reinterpret_cast<const float4*>(b_base + (b_off + at));
     };
     float (&As)[L1F_K][L1F_LDA] = lds.slab[wave].a;
     float (&Bs)[L1F_K][L1F_LDB] = lds.slab[wave].b;
@@ -371,8 +368,7 @@ DEVINL float l1_fwd_tile(const FwdParams& p, const int d, const int m0, const in
         if ((slab + 1) * L1F_K > Dp && slab * L1F_K + kq >= Dp) {  // columns that do not exist: no difference
 #pragma unroll
             for (int i = 0; i < 2; ++i) ra[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int i = 0; i < 1; ++i) rb[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            rb = make_float4(0.f, 0.f, 0.f, 0.f);
         }
         wave_lds_fence();
 #pragma unroll
@@ -380,11 +376,7 @@ DEVINL float l1_fwd_tile(const FwdParams& p, const int d, const int m0, const in
             As[kq][r0 + 32 * i] = ra[i].x; As[kq + 1][r0 + 32 * i] = ra[i].y;
             As[kq + 2][r0 + 32 * i] = ra[i].z; As[kq + 3][r0 + 32 * i] = ra[i].w;
         }
-#pragma unroll
-        for (int i = 0; i < 1; ++i) {
-            Bs[kq][r0 + 32 * i] = rb[i].x; Bs[kq + 1][r0 + 32 * i] = rb[i].y;
-            Bs[kq + 2][r0 + 32 * i] = rb[i].z; Bs[kq + 3][r0 + 32 * i] = rb[i].w;
-        }
+        Bs[kq][r0] = rb.x; Bs[kq + 1][r0] = rb.y; Bs[kq + 2][r0] = rb.z; Bs[kq + 3][r0] = rb.w;
         wave_lds_fence();
         prefetch(slab + 4);
         // A column's pairs in quarters of 4 x 4, in an order in which the operands of the next column take the place of
