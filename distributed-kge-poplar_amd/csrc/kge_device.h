@@ -125,6 +125,13 @@ DEVINL float wave_max(float v) {
 }
 
 
+// the lane's number, formed where it stands: it and what follows from it hold no register before
+DEVINL uint32_t lane_here() {
+    uint32_t from = 0;
+    asm volatile("" : "+v"(from));
+    return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, from));
+}
+
 // this wave's LDS accesses before and after stay in that order (the hardware keeps a wave's order by itself)
 DEVINL void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");

@@ -352,12 +352,14 @@ DEVINL float l1_fwd_tile(const FwdParams& p, const int d, const int m0, const in
     float (&As)[L1F_K][L1F_LDA] = lds.slab[wave].a;
     float (&Bs)[L1F_K][L1F_LDB] = lds.slab[wave].b;
     const int n_slab = (Dp + L1F_K - 1) / L1F_K;
-    // what the loss needs, asked for together and ahead of everything else: this lane's pairs at the end are rows m, m + 1
-    // and columns n .. n + 3
-    const int m = m0 + 4 * ty + 32 * (wave >> 1) + 2 * (wave & 1), n = n0 + 4 * tx;
+    // this lane's pairs at the end: rows m, m + 1 and columns n .. n + 3 (numbers that the loop has no registers for)
+    auto end_row = [&](int l) __attribute__((always_inline)) { return m0 + 4 * (l >> 3) + 32 * (wave >> 1) + 2 * (wave & 1); };
+    auto end_column = [&](int l) __attribute__((always_inline)) { return n0 + 4 * (l & 7); };
+    // what the loss needs, asked for together and ahead of everything else
     uint32_t label[2];
     float mult[4];
     if (OM == 0) {
+        const int m = end_row(lane), n = end_column(lane);
 #pragma unroll
         for (int i = 0; i < 2; ++i) label[i] = p.clabel[d * B + min(m + i, B - 1)];
 #pragma unroll
@@ -435,6 +437,7 @@ DEVINL float l1_fwd_tile(const FwdParams& p, const int d, const int m0, const in
             }
     }
 
+    const int m = end_row(lane_here()), n = end_column(lane_here());
     const float Tn = (float)T;
     const float w_pos = uniform_f32(0.5f * Tn), w_neg = uniform_f32((0.5f * Tn) / (float)(T - 1));
     const float grad_scale = uniform_f32(1.f / ((float)sh.S * (float)B * Tn) * sh.loss_scale);

@@ -800,7 +800,7 @@ void launch_bwd(const BwdParams& p, int dist_fn, hipStream_t stream) {
 // group and their gradient sums in registers and walks over the group's heads; a head's sum over one wave's tails is a
 // partial, the 16 partials of a head meet in LDS and are added in a fixed order.
 // The coefficients of a (head, tail) are the same for every lane: a wave brings those of eight heads and
-// its own tails to LDS (one load of four per lane, the next chunk's in flight under the current one's
+// its own tails to LDS (four per lane, in two loads or, with bounds checks, four; the next chunk's in flight under the current one's
 // arithmetic) and reads them four at a time with one instruction whose lanes all name the same address (a broadcast:
 // 4 cycles per CU).  As scalar operands the same coefficients halve the rate of the instructions that take them.
 constexpr int L1P_CB = 8;      // heads per chunk
@@ -860,6 +860,12 @@ DEVINL float dpp_f32(float v) {
 template <int TW, bool FULL>
 DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane, L1PairLds& lds) {
     constexpr int TWM = L1P_MAX_T / L1P_WAVES;
+    // The widest copies have no register for what can be had again: heads' values are asked for eight (a chunk), four or
+    // two heads ahead, and places that follow from the lane are formed where they are used.  (Copies
+    // that have the registers are up to 7 % slower so.)  Nothing goes to scratch: 64 blocks of 250 x 512 distinct tails,
+    // D = 256: 243 -> 221 us, 32 of 250 x 480: 118 -> 110; of whole groups the same as with scratch.
+    constexpr int AHEAD = TW < 28 ? L1P_CB : TW < 32 ? 4 : 2;
+    auto lane_again = [&]() __attribute__((always_inline)) { return TW < 30 ? (uint32_t)lane : lane_here(); };
     const int n_head = q.n_head, t0 = w * TW;
     const size_t Dp = q.Dp;
     // staging: lane -> (head, four columns) of the wave's coefficients of a chunk.  Loads without a branch
@@ -868,16 +874,20 @@ DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane, L1PairLds& lds) {
     const int s_head = lane >> 3, s_col = (lane & 7) * 4;
     const int s_n = (FULL ? TW : min(TW, q.n_tail - t0)) - s_col;  // columns of this lane that count
     auto fetch = [&](int b0) __attribute__((always_inline)) {
+        const uint32_t l = lane_again(), head = l >> 3, col = (l & 7) * 4;
+        // the chunk's first row and the wave's first column in scalar registers, what is the lane's in 32 bits
         if constexpr (FULL) {
-            const float* src = q.coef + (size_t)(b0 + s_head) * q.ldc + t0;
-            const float2 lo = *reinterpret_cast<const float2*>(src + (s_n > 0 ? s_col : 0));
-            const float2 hi = *reinterpret_cast<const float2*>(src + (s_n > 2 ? s_col + 2 : 0));
+            const float* src = q.coef + (size_t)b0 * q.ldc + t0;
+            const uint32_t row = head * (uint32_t)q.ldc;
+            const float2 lo = *reinterpret_cast<const float2*>(src + (row + (col < TW ? col : 0u)));
+            const float2 hi = *reinterpret_cast<const float2*>(src + (row + (col + 2 < TW ? col + 2 : 0u)));
             return make_float4(lo.x, lo.y, hi.x, hi.y);
         }
-        const float* src = q.coef + (size_t)min(b0 + s_head, n_head - 1) * q.ldc;
-        const int last = q.n_tail - 1;
-        return make_float4(src[min(t0 + s_col, last)], src[min(t0 + s_col + 1, last)],
-                           src[min(t0 + s_col + 2, last)], src[min(t0 + s_col + 3, last)]);
+        const int b = min(b0, n_head - 1), t = min(t0, q.n_tail - 1);
+        const float* src = q.coef + (size_t)b * q.ldc + t;
+        const uint32_t row = min(head, (uint32_t)(n_head - 1 - b)) * (uint32_t)q.ldc, last = q.n_tail - 1 - t;
+        return make_float4(src[row + min(col, last)], src[row + min(col + 1, last)],
+                           src[row + min(col + 2, last)], src[row + min(col + 3, last)]);
     };
     // a chunk's coefficients into the wave's tile `buf`
     auto stage = [&](int buf, int b0, float4 v) __attribute__((always_inline)) {
@@ -909,34 +919,36 @@ DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane, L1PairLds& lds) {
     float bt[TW], gt[TW];
 #pragma unroll
     for (int j = 0; j < TW; ++j) {
-        bt[j] = q.b_rows[(size_t)(FULL ? t0 + j : min(t0 + j, q.n_tail - 1)) * Dp + q.kc];
+        bt[j] = (q.b_rows + (size_t)(FULL ? t0 + j : min(t0 + j, q.n_tail - 1)) * Dp)[(uint32_t)q.kc];
         gt[j] = 0.f;
     }
     // sixteen partials of a head: wave w takes head w / 2 of the chunk and half of the columns, the lower lanes the
     // first eight waves' partials, the upper ones the others'
-    const int r_head = w >> 1, r_col = (w & 1) * 32 + (lane & 31), r_wave = (lane >> 5) * 8;
-    const bool r_there = lane < 32 && (FULL || q.k0 + r_col < q.Dp);
+    const int r_head = w >> 1;
     float red[8];
     auto ask = [&](int buf) __attribute__((always_inline)) {
+        const uint32_t l = lane_again(), r_wave = (l >> 5) * 8, r_col = (w & 1) * 32 + (l & 31);
 #pragma unroll
         for (int v = 0; v < 8; ++v) red[v] = lds.part[buf][r_wave + v][r_head][r_col];
     };
     auto give = [&](int b0) __attribute__((always_inline)) {
         float sum = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
         sum += __shfl_xor(sum, 32, 64);
+        const uint32_t l = lane_again(), r_col = (w & 1) * 32 + (l & 31);
         const int b = b0 + r_head;
-        if (r_there && b >= 0 && (FULL || b < n_head)) q.grad_a[(size_t)b * Dp + q.k0 + r_col] = sum;
+        if (l < 32 && (FULL || q.k0 + (int)r_col < q.Dp) && b >= 0 && (FULL || b < n_head))
+            (q.grad_a + (size_t)b * Dp + q.k0)[r_col] = sum;
     };
     stage(0, 0, fetch(0));
     wave_lds_fence();
     float row_sum = row_sums(0);
     lds.col_half[w][lane & (TWM - 1)] = 0.f;
-    float a[L1P_CB];
+    float a[AHEAD];
 #pragma unroll
-    for (int h = 0; h < L1P_CB; ++h) a[h] = head_value(h);
+    for (int h = 0; h < AHEAD; ++h) a[h] = head_value(h);
     // (waited for here: the loop's waits then count on the loop's own order of loads)
 #pragma unroll
-    for (int h = 0; h < L1P_CB; ++h) asm volatile("" : "+v"(a[h]));
+    for (int h = 0; h < AHEAD; ++h) asm volatile("" : "+v"(a[h]));
 #pragma unroll
     for (int j = 0; j < TW; ++j) asm volatile("" : "+v"(bt[j]));
     int buf = 0, b0 = 0;
@@ -993,7 +1005,7 @@ DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane, L1PairLds& lds) {
                     half = *reinterpret_cast<const float4*>(&lds.col_half[w][min(j4 + 4, TWM - 4)]);
                 }
 #pragma unroll
-                for (int x = 0; x < 4; ++x) d[x] = a[h] - bt[min(j4 + x, TW - 1)];
+                for (int x = 0; x < 4; ++x) d[x] = a[h % AHEAD] - bt[min(j4 + x, TW - 1)];
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int x = 0; x < 4; ++x) p[x] = __builtin_amdgcn_fmed3f(fmaf(d[x], 0x1p126f, 0.5f), 0.f, 1.f);
@@ -1007,7 +1019,7 @@ DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane, L1PairLds& lds) {
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            a[h] = head_value(next + h);  // the next chunk's: a chunk's time to arrive
+            a[h % AHEAD] = head_value(h + AHEAD < L1P_CB ? b0 + h + AHEAD : next + h + AHEAD - L1P_CB);
             const float rs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(row_sum), h * 8));
             lds.part[buf][w][h][lane] = fmaf(2.f, (gp[0] + gp[1]) + (gp[2] + gp[3]), -rs);
         }
@@ -1016,9 +1028,11 @@ DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane, L1PairLds& lds) {
     }
     ask(buf ^ 1);
     give(b0 - L1P_CB);
+    const uint32_t kl = lane_again();
 #pragma unroll
     for (int j = 0; j < TW; ++j)
-        if (FULL || (t0 + j < q.n_tail && q.col)) q.grad_b[(size_t)(t0 + j) * Dp + q.kc] = -2.f * (gt[j] - lds.col_half[w][j]);
+        if (FULL || (t0 + j < q.n_tail && q.k0 + (int)kl < q.Dp))
+            (q.grad_b + (size_t)(t0 + j) * Dp + q.k0)[kl] = -2.f * (gt[j] - lds.col_half[w][j]);
 }
 
 // How a block's pairs are divided: `heads` x `tails` groups, every group a workgroup per 64 columns.

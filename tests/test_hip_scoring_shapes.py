@@ -37,6 +37,14 @@ def test_l1_whole_groups(oracle64, B, A, D):
                             gamma=4.0), n_step=2, **{"execution.merge_tails": False})
 
 
+# L1 backward with bounds checks, one group of 512, 480, 448 and 416 tails: 32, 30, 28 and 26 per wave, whose heads'
+# values are asked for two, four, four and eight heads ahead
+@pytest.mark.parametrize("S,B,A,D", [(64, 9, 8, 200), (32, 19, 15, 452), (64, 12, 7, 250), (32, 9, 13, 450)])
+def test_l1_wide_groups(oracle64, S, B, A, D):
+    run_case(oracle64, dict(distance_fn="L1", n_shard=S, batch=B, a2a=A, dim=D, feature=0, n_entity=1500, n_relation=S,
+                            gamma=4.0), n_step=1, **{"execution.merge_tails": False})
+
+
 # L1 forward: tiles of 64 heads x 32 tails, four waves over slabs of eight columns (from 64 columns on): around a tile's
 # edges, a last slab of four columns, waves with and without one, distinct tails that end on a tile
 @pytest.mark.parametrize("merge", [True, False])

@@ -158,3 +158,42 @@ def test_bench_reads_traffic_of_the_most_launched_kernel_variant():
     most = max(rows.values(), key=lambda r: r[1])
     assert measured_traffic("c2")[0]["adam_entity"] == pytest.approx(most[0])
     assert measured_traffic("no_such_workload") == (None, None)
+
+
+def _library_kernels():
+    """Metadata of every gfx950 kernel in the library: its offload bundles' code objects carry it as a
+    msgpack note (AMDGPU code object metadata, note type 32)."""
+    import struct
+
+    import msgpack
+
+    data, kernels = H.LIB_PATH.read_bytes(), []
+    at = data.find(b"__CLANG_OFFLOAD_BUNDLE__")
+    while at >= 0:
+        entry = at + 32
+        for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):
+            offset, size, n_id = struct.unpack_from("<QQQ", data, entry)
+            target, entry = data[entry + 24:entry + 24 + n_id], entry + 24 + n_id
+            if b"gfx950" not in target:
+                continue
+            elf = data[at + offset:at + offset + size]
+            headers, = struct.unpack_from("<Q", elf, 32)
+            header_size, n_header = struct.unpack_from("<HH", elf, 54)
+            for header in range(headers, headers + n_header * header_size, header_size):
+                if struct.unpack_from("<I", elf, header)[0] != 4:  # PT_NOTE
+                    continue
+                note, = struct.unpack_from("<Q", elf, header + 8)
+                n_name, n_desc, kind = struct.unpack_from("<III", elf, note)
+                if kind == 32:
+                    desc = note + 12 + (n_name + 3) // 4 * 4
+                    kernels += msgpack.unpackb(elf[desc:desc + n_desc])["amdhsa.kernels"]
+        at = data.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 1)
+    return kernels
+
+
+def test_no_kernel_spills_registers():
+    """A kernel that needs more registers than its launch bounds leave goes to scratch, in all of its launches."""
+    kernels = _library_kernels()
+    assert any("k_score_bwd_l1_pair" in k[".name"] for k in kernels)
+    spilled = {k[".name"]: k[".vgpr_spill_count"] for k in kernels if k.get(".vgpr_spill_count")}
+    assert not spilled
