@@ -800,7 +800,7 @@ void launch_bwd(const BwdParams& p, int dist_fn, hipStream_t stream) {
 // group and their gradient sums in registers and walks over the group's heads; a head's sum over one wave's tails is a
 // partial, the 16 partials of a head meet in LDS and are added in a fixed order.
 // The coefficients of a (head, tail) are the same for every lane: a wave brings those of eight heads and
-// its own tails to LDS (four per lane, in two loads or, with bounds checks, four; the next chunk's in flight under the current one's
+// its own tails to LDS (one to four per lane; the next chunk's in flight under the current one's
 // arithmetic) and reads them four at a time with one instruction whose lanes all name the same address (a broadcast:
 // 4 cycles per CU).  As scalar operands the same coefficients halve the rate of the instructions that take them.
 constexpr int L1P_CB = 8;      // heads per chunk
@@ -868,35 +868,51 @@ DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane, L1PairLds& lds) {
     auto lane_again = [&]() __attribute__((always_inline)) { return TW < 30 ? (uint32_t)lane : lane_here(); };
     const int n_head = q.n_head, t0 = w * TW;
     const size_t Dp = q.Dp;
-    // staging: lane -> (head, four columns) of the wave's coefficients of a chunk.  Loads without a branch
+    // staging: lane -> (head, CPL columns) of the wave's coefficients of a chunk.  Loads without a branch
     // (a lane that has nothing to fetch fetches something else: a load that may not have been issued would be
     // waited for together with what was asked for before it); what does not count becomes zero when it has come.
-    const int s_head = lane >> 3, s_col = (lane & 7) * 4;
+    // A narrow copy's eight lanes per head take as many columns as the wave has tails for: with four each, most lanes of
+    // most loads brought nothing, and the loads' addresses bounded the short loops (one block of 40 x 1500,
+    // D = 256, up to 8 tails per wave: 13.5 -> 11.7 us; 4 of 200 x 268, D = 100: 14.5 -> 13.0; 33 x 90, D = 30: 11.7 -> 10.3).
+    constexpr int CPL = TW <= 8 ? 1 : TW <= 16 ? 2 : 4;
+    const int s_head = lane >> 3, s_col = (lane & 7) * CPL;
     const int s_n = (FULL ? TW : min(TW, q.n_tail - t0)) - s_col;  // columns of this lane that count
+    struct Coefs { float v[CPL]; };
     auto fetch = [&](int b0) __attribute__((always_inline)) {
-        const uint32_t l = lane_again(), head = l >> 3, col = (l & 7) * 4;
+        const uint32_t l = lane_again(), head = l >> 3, col = (l & 7) * CPL;
+        Coefs c;
         // the chunk's first row and the wave's first column in scalar registers, what is the lane's in 32 bits
         if constexpr (FULL) {
             const float* src = q.coef + (size_t)b0 * q.ldc + t0;
             const uint32_t row = head * (uint32_t)q.ldc;
-            const float2 lo = *reinterpret_cast<const float2*>(src + (row + (col < TW ? col : 0u)));
-            const float2 hi = *reinterpret_cast<const float2*>(src + (row + (col + 2 < TW ? col + 2 : 0u)));
-            return make_float4(lo.x, lo.y, hi.x, hi.y);
+            constexpr int N = CPL > 1 ? 2 : 1;
+#pragma unroll
+            for (int i = 0; i < CPL; i += N) {
+                const float* at = src + (row + (col + i < TW ? col + i : 0u));
+                if constexpr (N == 1) c.v[0] = at[0];
+                else {
+                    const float2 two = *reinterpret_cast<const float2*>(at);
+                    c.v[i] = two.x; c.v[i + 1] = two.y;
+                }
+            }
+        } else {
+            const int b = min(b0, n_head - 1), t = min(t0, q.n_tail - 1);
+            const float* src = q.coef + (size_t)b * q.ldc + t;
+            const uint32_t row = min(head, (uint32_t)(n_head - 1 - b)) * (uint32_t)q.ldc, last = q.n_tail - 1 - t;
+#pragma unroll
+            for (int i = 0; i < CPL; ++i) c.v[i] = src[row + min(col + i, last)];
         }
-        const int b = min(b0, n_head - 1), t = min(t0, q.n_tail - 1);
-        const float* src = q.coef + (size_t)b * q.ldc + t;
-        const uint32_t row = min(head, (uint32_t)(n_head - 1 - b)) * (uint32_t)q.ldc, last = q.n_tail - 1 - t;
-        return make_float4(src[row + min(col, last)], src[row + min(col + 1, last)],
-                           src[row + min(col + 2, last)], src[row + min(col + 3, last)]);
+        return c;
     };
     // a chunk's coefficients into the wave's tile `buf`
-    auto stage = [&](int buf, int b0, float4 v) __attribute__((always_inline)) {
+    auto stage = [&](int buf, int b0, Coefs c) __attribute__((always_inline)) {
         const int n = FULL || b0 + s_head < n_head ? s_n : 0;
-        if (n < 1) v.x = 0.f;
-        if (n < 2) v.y = 0.f;
-        if (n < 3) v.z = 0.f;
-        if (n < 4) v.w = 0.f;
-        *reinterpret_cast<float4*>(&lds.cs[w][buf][s_head][s_col]) = v;
+        float* const to = &lds.cs[w][buf][s_head][s_col];
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) if (n <= i) c.v[i] = 0.f;
+        if constexpr (CPL == 4) *reinterpret_cast<float4*>(to) = make_float4(c.v[0], c.v[1], c.v[2], c.v[3]);
+        else if constexpr (CPL == 2) *reinterpret_cast<float2*>(to) = make_float2(c.v[0], c.v[1]);
+        else *to = c.v[0];
     };
     // the sums of a chunk's coefficients per head (the same in the head's eight lanes)
     constexpr int NG = (TW + 3) / 4;
@@ -954,7 +970,7 @@ DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane, L1PairLds& lds) {
     int buf = 0, b0 = 0;
     for (; b0 < n_head; b0 += L1P_CB, buf ^= 1) {
         const int next = FULL ? min(b0 + L1P_CB, n_head - L1P_CB) : b0 + L1P_CB;  // (past the end: never used)
-        float4 c_next = fetch(next);
+        Coefs c_next = fetch(next);
         float next_sum = 0.f;
         wave_lds_fence();
         // four tails at a time, their coefficients read two groups ahead; the order of the groups is kept
@@ -986,7 +1002,8 @@ DEVINL void l1_pair_wave(const L1Pair& q, int w, int lane, L1PairLds& lds) {
                     0.5f * (((((((col[0] + col[1]) + col[2]) + col[3]) + col[4]) + col[5]) + col[6]) + col[7]);
             }
             if (h == 6) {
-                asm volatile("" : "+v"(c_next.x), "+v"(c_next.y), "+v"(c_next.z), "+v"(c_next.w));  // (not before)
+#pragma unroll
+                for (int i = 0; i < CPL; ++i) asm volatile("" : "+v"(c_next.v[i]));  // (not before)
                 stage(buf ^ 1, next, c_next);
                 wave_lds_fence();
             }

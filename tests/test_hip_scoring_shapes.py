@@ -45,6 +45,13 @@ def test_l1_wide_groups(oracle64, S, B, A, D):
                             gamma=4.0), n_step=1, **{"execution.merge_tails": False})
 
 
+# the same with 4, 8, 10 and 16 tails per wave: one, one, two and two columns of coefficients per lane
+@pytest.mark.parametrize("S,B,A,D", [(50, 9, 1, 250), (50, 17, 2, 250), (50, 9, 3, 250), (50, 8, 5, 250)])
+def test_l1_narrow_groups(oracle64, S, B, A, D):
+    run_case(oracle64, dict(distance_fn="L1", n_shard=S, batch=B, a2a=A, dim=D, feature=0, n_entity=1000, n_relation=S,
+                            gamma=4.0), n_step=1, **{"execution.merge_tails": False})
+
+
 # L1 forward: tiles of 64 heads x 32 tails, four waves over slabs of eight columns (from 64 columns on): around a tile's
 # edges, a last slab of four columns, waves with and without one, distinct tails that end on a tile
 @pytest.mark.parametrize("merge", [True, False])
