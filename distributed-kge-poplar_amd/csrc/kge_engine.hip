@@ -591,6 +591,14 @@ void parse_settings(kge_engine& E, const Items& s) {
     }
 }
 
+// rows of Dp float32 values as the scoring kernels' operands
+RowSource operand_rows(const kge_engine& E, const float* rows) {
+    RowSource r;
+    r.base = (const char*)rows; r.pitch = (int64_t)E.Dp * 4; r.etype = ET_F32;
+    r.index = nullptr; r.count = E.Dp; r.vec = 1;
+    return r;
+}
+
 void allocate(kge_engine& E) {
     int n_dev = 0;
     const hipError_t dev_err = hipGetDeviceCount(&n_dev);
@@ -764,7 +772,8 @@ void allocate(kge_engine& E) {
         }
     }
     if (E.score_fn != SCORE_TRANSH) E.bwd_pieces.alloc(score_bwd_pieces(sh));
-    E.n_part = !fused ? E.B : E.split ? split_fwd_parts(sh) : score_fwd_parts(sh);
+    sh.operands_dense = 1;
+    E.n_part = !fused ? E.B : E.split ? split_fwd_parts(sh) : score_fwd_parts(sh, operand_rows(E, E.opnd.p));
     if (E.use_mfma && E.dist_fn == DIST_L2) {
         E.nearflag.alloc(nearflag_words(sh));
         E.nearflag.zero(st);
@@ -1247,9 +1256,7 @@ void run_step(kge_engine& E, int i) {
       else
       launch_gather_operands(ent, E.rel.p, crel, rel_mode_of(E), E.D / 2, (int)SB, (int)R, E.Dp,
                              E.opnd.p, E.score_bf16 ? E.opnd16.p : nullptr, st, &tc); }
-    RowSource dense;
-    dense.base = (const char*)E.opnd.p; dense.pitch = (int64_t)E.Dp * 4; dense.etype = ET_F32;
-    dense.index = nullptr; dense.count = E.Dp; dense.vec = 1;
+    const RowSource dense = operand_rows(E, E.opnd.p);
     sh.operands_dense = 1;
     const bool transh = E.score_fn == SCORE_TRANSH;
     if (transh) {
@@ -1989,9 +1996,7 @@ void run_predict(kge_engine& E, const Items& in) {
     sh.S = 1; sh.B = Qp; sh.T = chunk; sh.Dp = Dp;
     sh.score_fn = E.score_fn; sh.dist_fn = E.dist_fn; sh.loss_fn = E.loss_fn;
     sh.gamma = E.gamma; sh.loss_scale = 1.f; sh.use_mfma = E.use_mfma; sh.operands_dense = 1;
-    RowSource dense;
-    dense.base = (const char*)E.p_opnd.p; dense.pitch = (int64_t)Dp * 4; dense.etype = ET_F32;
-    dense.index = nullptr; dense.count = Dp; dense.vec = 1;
+    const RowSource dense = operand_rows(E, E.p_opnd.p);
     RowSource dense_n = dense;
     dense_n.base = (const char*)E.p_opnd_n.p;
     const bool sweep = predict_scores_takes(sh);

@@ -228,7 +228,7 @@ void launch_gemm_nt_bf16(const GemmNT& g, hipStream_t stream);
 // contribution S*B + d*T + t.  With `fused_loss` the logsigmoid loss and the
 // backward coefficient are produced in the epilogue; otherwise the raw score is
 // stored in `coef` (and the L2 distance in `dist`) for launch_loss_rows.
-// loss_part receives S * n_part partial sums (n_part = tiles per block).
+// loss_part receives S * n_part partial sums (score_fwd_parts).
 void launch_score_fwd(const ScoreShape& sh, const RowSource& ent, const float* rel,
                       const uint32_t* crel, const uint32_t* clabel, float* coef, float* dist,
                       uint32_t* nearflag, float* loss_part, bool fused_loss, hipStream_t stream);
@@ -244,7 +244,7 @@ void launch_predict_scores(const ScoreShape& sh, const float* a, const RowSource
 inline size_t nearflag_words(const ScoreShape& sh) {
     return (size_t)sh.S * ((sh.B + 31) / 32) * ((sh.T + 31) / 32);
 }
-int score_fwd_parts(const ScoreShape& sh);
+int score_fwd_parts(const ScoreShape& sh, const RowSource& ent);  // n_part of such a launch
 
 // ---- scoring on three-piece operands (kge_split.hip; L2 and dot, any shape) ----
 // Piece matrices hold every float32 value as three bfloat16 pieces, rows of 6 * Kp bytes (columns

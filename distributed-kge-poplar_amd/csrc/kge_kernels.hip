@@ -933,28 +933,48 @@ __global__ __launch_bounds__(NW * 64) void k_score_fwd_mfma(FwdParams p) {
     }
 }
 
-static bool fwd_uses_mfma(const FwdParams& p) {
-    return p.sh.use_mfma && p.sh.dist_fn != DIST_L1 && p.ent_a.vec && p.ent_b.vec && (p.sh.Dp & 3) == 0;
+// Which kernel a launch takes and the tiles into which it divides a block: the one rule for the launch itself and for
+// whoever lays out its parts of the loss.
+enum FwdKernel { FWD_MFMA, FWD_L1, FWD_VALU };
+struct FwdChoice {
+    FwdKernel kernel;
+    int tm, tn;
+    bool dense;  // float32 rows in their place, 16-byte aligned, the relation applied
+    int parts(const ScoreShape& sh) const { return ((sh.T + tn - 1) / tn) * ((sh.B + tm - 1) / tm); }
+    dim3 grid(const ScoreShape& sh) const { return tile_grid((sh.T + tn - 1) / tn, (sh.B + tm - 1) / tm, sh.S); }
+};
+static FwdChoice fwd_choice(const FwdParams& p) {
+    const ScoreShape& sh = p.sh;
+    const bool vec = p.ent_a.vec && p.ent_b.vec;
+    const bool dense = p.ent_a.etype == ET_F32 && p.ent_b.etype == ET_F32 && vec && !p.ent_a.index && !p.ent_b.index &&
+                       p.a_rel_mode == 0;
+    if (sh.use_mfma && sh.dist_fn != DIST_L1 && vec && (sh.Dp & 3) == 0) return {FWD_MFMA, FM_TM, FM_TN, dense};
+    // Four slabs, one for every wave, are 32 columns; below 64 the loop is too short for what the waves' sums cost.
+    // (TransH's own forward has tiles of 64 x 64.)
+    if (dense && sh.dist_fn == DIST_L1 && sh.score_fn != SCORE_TRANSH && sh.Dp >= 64 && (sh.Dp & 3) == 0)
+        return {FWD_L1, kScoreTile, L1F_TN, dense};
+    return {FWD_VALU, kScoreTile, kScoreTile, dense};
 }
 
-// Shapes of k_score_fwd_l1: four slabs, one for every wave, are 32 columns; below 64 the loop is too short for what the
-// waves' sums cost.
-static bool fwd_l1_shape(const ScoreShape& sh) {
-    return sh.dist_fn == DIST_L1 && sh.score_fn != SCORE_DISTMULT && sh.score_fn != SCORE_TRANSH && sh.Dp >= 64 && (sh.Dp & 3) == 0;
+static FwdParams fwd_params(const ScoreShape& sh, const RowSource& a, const RowSource& b, int a_rel_mode) {
+    FwdParams p = {};
+    p.sh = sh;
+    if (sh.score_fn == SCORE_DISTMULT) p.sh.dist_fn = DIST_DOT;
+    p.ent_a = a; p.ent_b = b;
+    p.a_rel_mode = a_rel_mode;
+    return p;
+}
+static FwdParams fwd_params(const ScoreShape& sh, const RowSource& ent) {
+    return fwd_params(sh, ent, ent, sh.operands_dense ? 0 : (sh.score_fn == SCORE_DISTMULT ? 2 : 1));
 }
 
-int score_fwd_parts(const ScoreShape& sh) {
-    const bool mfma = sh.use_mfma && !(sh.score_fn != SCORE_DISTMULT && sh.dist_fn == DIST_L1);
-    const int tm = mfma ? FM_TM : kScoreTile, tn = mfma ? FM_TN : fwd_l1_shape(sh) ? L1F_TN : kScoreTile;
-    return ((sh.T + tn - 1) / tn) * ((sh.B + tm - 1) / tm);
-}
+int score_fwd_parts(const ScoreShape& sh, const RowSource& ent) { return fwd_choice(fwd_params(sh, ent)).parts(sh); }
 
 static void launch_fwd(const FwdParams& p, hipStream_t stream) {
-    if (fwd_uses_mfma(p)) {
-        const dim3 grid = tile_grid((p.sh.T + FM_TN - 1) / FM_TN, (p.sh.B + FM_TM - 1) / FM_TM, p.sh.S);
-        const bool f32 = p.ent_a.etype == ET_F32 && p.ent_b.etype == ET_F32;
-        const bool aligned = f32 && p.a_rel_mode == 0 && !p.ent_a.index && !p.ent_b.index &&
-                             p.sh.B % FM_TM == 0 && p.sh.T % FM_TN == 0;
+    const FwdChoice choice = fwd_choice(p);
+    const dim3 grid = choice.grid(p.sh);
+    if (choice.kernel == FWD_MFMA) {
+        const bool aligned = choice.dense && p.sh.B % FM_TM == 0 && p.sh.T % FM_TN == 0;
 #define KGE_FWD_OM(D_, OM_)                                                                                  \
     do {                                                                                                     \
         if (aligned && p.sh.Dp % 64 == 0 && p.sh.use_mfma == 2) {                                            \
@@ -975,10 +995,7 @@ static void launch_fwd(const FwdParams& p, hipStream_t stream) {
 #undef KGE_FWD
         return;
     }
-    const dim3 grid = tile_grid((p.sh.T + kScoreTile - 1) / kScoreTile, (p.sh.B + kScoreTile - 1) / kScoreTile, p.sh.S);
-    const bool valu_aligned = p.ent_a.etype == ET_F32 && p.ent_b.etype == ET_F32 && p.ent_a.vec && p.ent_b.vec &&
-                              !p.ent_a.index && !p.ent_b.index && p.a_rel_mode == 0 &&
-                              p.sh.B % kScoreTile == 0 && p.sh.T % kScoreTile == 0 && p.sh.Dp % BK == 0;
+    const bool valu_aligned = choice.dense && p.sh.B % kScoreTile == 0 && p.sh.T % kScoreTile == 0 && p.sh.Dp % BK == 0;
 #define KGE_FWD_VALU(D_)                                                                                     \
     do {                                                                                                     \
         if (p.out_mode == 0 && valu_aligned) hipLaunchKernelGGL((k_score_fwd<D_, 0, true>), grid, dim3(256), 0, stream, p); \
@@ -986,10 +1003,7 @@ static void launch_fwd(const FwdParams& p, hipStream_t stream) {
         else if (p.out_mode == 1) hipLaunchKernelGGL((k_score_fwd<D_, 1>), grid, dim3(256), 0, stream, p);    \
         else hipLaunchKernelGGL((k_score_fwd<D_, 2>), grid, dim3(256), 0, stream, p);                         \
     } while (0)
-    const bool dense = p.ent_a.etype == ET_F32 && p.ent_b.etype == ET_F32 && p.ent_a.vec && p.ent_b.vec && !p.ent_a.index &&
-                       !p.ent_b.index && p.a_rel_mode == 0;
-    if (dense && fwd_l1_shape(p.sh)) {
-        const dim3 grid = tile_grid((p.sh.T + L1F_TN - 1) / L1F_TN, (p.sh.B + kScoreTile - 1) / kScoreTile, p.sh.S);
+    if (choice.kernel == FWD_L1) {
         if (p.out_mode == 0) hipLaunchKernelGGL(k_score_fwd_l1<0>, grid, dim3(256), 0, stream, p);
         else if (p.out_mode == 1) hipLaunchKernelGGL(k_score_fwd_l1<1>, grid, dim3(256), 0, stream, p);
         else hipLaunchKernelGGL(k_score_fwd_l1<2>, grid, dim3(256), 0, stream, p);
@@ -1003,13 +1017,10 @@ static void launch_fwd(const FwdParams& p, hipStream_t stream) {
 void launch_score_fwd(const ScoreShape& sh, const RowSource& ent, const float* rel,
                       const uint32_t* crel, const uint32_t* clabel, float* coef, float* dist,
                       uint32_t* nearflag, float* loss_part, bool fused_loss, hipStream_t stream) {
-    FwdParams p;
+    FwdParams p = fwd_params(sh, ent);
     p.nearflag = nearflag;
-    p.sh = sh;
-    if (sh.score_fn == SCORE_DISTMULT) p.sh.dist_fn = DIST_DOT;
-    p.ent_a = ent; p.ent_b = ent; p.rel = rel; p.crel = crel; p.clabel = clabel;
+    p.rel = rel; p.crel = crel; p.clabel = clabel;
     p.coef = coef; p.dist = dist; p.loss_part = loss_part;
-    p.a_rel_mode = sh.operands_dense ? 0 : (sh.score_fn == SCORE_DISTMULT ? 2 : 1);
     p.out_mode = fused_loss ? 0 : 1;
     p.a_c0 = 0; p.b_c0 = sh.S * sh.B;
     launch_fwd(p, stream);
@@ -1019,14 +1030,9 @@ void launch_score_fwd(const ScoreShape& sh, const RowSource& ent, const float* r
 // source, e.g. consecutive rows of the table itself: no copy of the b side is made.
 void launch_score_fwd_rows(const ScoreShape& sh, const RowSource& a, const RowSource& b, float* scores,
                            hipStream_t stream) {
-    FwdParams p;
-    p.nearflag = nullptr;
-    p.sh = sh;
-    if (sh.score_fn == SCORE_DISTMULT) p.sh.dist_fn = DIST_DOT;
-    p.ent_a = a; p.ent_b = b; p.rel = nullptr; p.crel = nullptr; p.clabel = nullptr;
-    p.coef = scores; p.dist = nullptr; p.loss_part = nullptr;
-    p.a_rel_mode = 0; p.out_mode = 1;
-    p.a_c0 = 0; p.b_c0 = 0;
+    FwdParams p = fwd_params(sh, a, b, 0);
+    p.coef = scores;
+    p.out_mode = 1;
     launch_fwd(p, stream);
 }
 

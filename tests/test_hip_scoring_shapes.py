@@ -1,6 +1,8 @@
 """The scoring kernels away from whole tiles, against the float64 oracle through the training step:
 sizes around the edges of tiles and groups, one row, splits of a side over several workgroups."""
 
+import ctypes as C
+
 import hip_harness as H
 import kge_cases as K
 import numpy as np
@@ -171,3 +173,50 @@ def test_infinite_first_tail_keeps_to_its_column(oracle64):
     H.train(engine, c, 0.1, batch)
     heads = H.read_state(engine, c)["entity_data"][60:60 + B, :D]
     assert np.isfinite(np.delete(heads, 5, axis=1)).all()
+
+
+class _ScoreShape(C.Structure):  # kge::ScoreShape, kge::RowSource
+    _fields_ = ([(k, C.c_int) for k in ("S", "B", "T", "Dp", "score_fn", "dist_fn", "loss_fn")] +
+                [(k, C.c_float) for k in ("gamma", "loss_scale", "softmax_correction", "negative_adversarial_scale")] +
+                [("use_mfma", C.c_int), ("operands_dense", C.c_int), ("tcount", C.c_void_p), ("tmult", C.c_void_p),
+                 ("tpad", C.c_int)])
+
+
+class _RowSource(C.Structure):
+    _fields_ = [("base", C.c_void_p), ("pitch", C.c_int64), ("etype", C.c_int), ("index", C.c_void_p), ("count", C.c_int),
+                ("vec", C.c_int)]
+
+
+# The parts of the loss that the fused L1 forward leaves are as many as score_fwd_parts says, whichever kernel
+# takes the operands: prepared ones, or the table's rows with the relation still to be added.
+@pytest.mark.parametrize("prepared", [True, False])
+@pytest.mark.parametrize("S,B,T,D", [(2, 70, 100, 64), (1, 64, 32, 128)])
+def test_l1_fused_forward_fills_its_parts(S, B, T, D, prepared):
+    import torch
+
+    rng = np.random.default_rng(3)
+    rows = rng.normal(0, 0.3, (S * (B + T), D)).astype(np.float32)
+    rel = rng.normal(0, 0.3, (5, D)).astype(np.float32)
+    crel, label = rng.integers(0, 5, S * B).astype(np.int32), rng.integers(0, T, S * B).astype(np.int32)
+    head = rows[:S * B].astype(np.float64) + (0 if prepared else rel[crel])
+    dist = np.abs(head.reshape(S, B, 1, D) - rows[S * B:].reshape(S, 1, T, D)).sum(-1)
+    score, positive = 4.0 - dist, label.reshape(S, B, 1) == np.arange(T)
+    weight = np.where(positive, 0.5 * T, 0.5 * T / (T - 1))
+    loss = np.mean(weight * np.logaddexp(0, np.where(positive, -score, score)))
+    coef = np.where(positive, 1 / (1 + np.exp(score)), -1 / (1 + np.exp(-score))) * weight / (S * B * T)
+
+    lib, dev = H.lib(), lambda a: torch.from_numpy(a).cuda()
+    shape = _ScoreShape(S=S, B=B, T=T, Dp=D, score_fn=0, dist_fn=0, loss_fn=0, gamma=4.0, loss_scale=1.0, use_mfma=1,
+                        operands_dense=int(prepared), tpad=64)
+    table, drel, dcrel, dlabel = dev(rows), dev(rel), dev(crel), dev(label)
+    source = _RowSource(base=table.data_ptr(), pitch=4 * D, etype=0, index=None, count=D, vec=1)
+    n_part = lib._ZN3kge15score_fwd_partsERKNS_10ScoreShapeERKNS_9RowSourceE(C.byref(shape), C.byref(source))
+    out, parts = torch.zeros(S, B, T, device="cuda"), torch.full((S * n_part + 256,), float("nan"), device="cuda")
+    lib._ZN3kge16launch_score_fwdERKNS_10ScoreShapeERKNS_9RowSourceEPKfPKjS9_PfSA_PjSA_bP12ihipStream_t(
+        C.byref(shape), C.byref(source), H.dptr(drel), H.dptr(dcrel), H.dptr(dlabel), H.dptr(out), None, None, H.dptr(parts),
+        C.c_bool(True), None)
+    torch.cuda.synchronize()
+    parts = parts.cpu().numpy()
+    assert np.isnan(parts[S * n_part:]).all()
+    np.testing.assert_allclose(parts[:S * n_part].sum(dtype=np.float64), loss, rtol=1e-5)
+    assert K.rel_l2(out.cpu().numpy(), coef) < 1e-5
