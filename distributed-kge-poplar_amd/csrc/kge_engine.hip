@@ -773,6 +773,7 @@ void allocate(kge_engine& E) {
     }
     if (E.score_fn != SCORE_TRANSH) E.bwd_pieces.alloc(score_bwd_pieces(sh));
     sh.operands_dense = 1;
+    sh.tcount = E.merge_tails ? E.tcount.p : nullptr;
     E.n_part = !fused ? E.B : E.split ? split_fwd_parts(sh) : score_fwd_parts(sh, operand_rows(E, E.opnd.p));
     if (E.use_mfma && E.dist_fn == DIST_L2) {
         E.nearflag.alloc(nearflag_words(sh));

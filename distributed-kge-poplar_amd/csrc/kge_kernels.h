@@ -244,7 +244,7 @@ void launch_predict_scores(const ScoreShape& sh, const float* a, const RowSource
 inline size_t nearflag_words(const ScoreShape& sh) {
     return (size_t)sh.S * ((sh.B + 31) / 32) * ((sh.T + 31) / 32);
 }
-int score_fwd_parts(const ScoreShape& sh, const RowSource& ent);  // n_part of such a launch
+int score_fwd_parts(const ScoreShape& sh, const RowSource& ent);  // n_part of such a launch (of `sh.tcount`, only whether it is there counts)
 
 // ---- scoring on three-piece operands (kge_split.hip; L2 and dot, any shape) ----
 // Piece matrices hold every float32 value as three bfloat16 pieces, rows of 6 * Kp bytes (columns

@@ -949,26 +949,40 @@ static FwdChoice fwd_choice(const FwdParams& p) {
     const bool dense = p.ent_a.etype == ET_F32 && p.ent_b.etype == ET_F32 && vec && !p.ent_a.index && !p.ent_b.index &&
                        p.a_rel_mode == 0;
     if (sh.use_mfma && sh.dist_fn != DIST_L1 && vec && (sh.Dp & 3) == 0) return {FWD_MFMA, FM_TM, FM_TN, dense};
-    // Four slabs, one for every wave, are 32 columns; below 64 the loop is too short for what the waves' sums cost.
-    // (TransH's own forward has tiles of 64 x 64.)
-    if (dense && sh.dist_fn == DIST_L1 && sh.score_fn != SCORE_TRANSH && sh.Dp >= 64 && (sh.Dp & 3) == 0)
-        return {FWD_L1, kScoreTile, L1F_TN, dense};
+    // k_score_fwd_l1: from 64 columns on, where each of its waves has two slabs (TransH's own forward has tiles of 64 x 64).
+    // Not the fused forward of whole tiles with eight workgroups of them for every CU, while the loop is short against the
+    // waves' sums.  us per launch in k_score_fwd, in k_score_fwd_l1:
+    //   D                                            64        96       128        160        192        256
+    //   16 of 512 x 1536, all tails distinct     53, 60    70, 75    86, 92   100, 104   117, 121   148, 150
+    //   64 of 256 x 512, all distinct            39, 43    51, 54    63, 66     72, 74     84, 86   109, 109
+    //   32 of 256 x 512 (half the workgroups)    23, 23    29, 29    36, 35     42, 40     48, 46     62, 58
+    //   64 of 256 x 512, merged, power law       31, 31    41, 39    51, 47     58, 54     67, 62     87, 77
+    //   1 of 4096 x 2048, merged, power law      32, 25    42, 30    51, 36     60, 41     70, 47     89, 58
+    // How many merged tails are distinct only the device knows: the line for them lies where neither kernel loses more
+    // than the other gains, which is nowhere with a single block (k_score_fwd's dead tiles share CUs).
+    if (dense && sh.dist_fn == DIST_L1 && sh.score_fn != SCORE_TRANSH && sh.Dp >= 64 && (sh.Dp & 3) == 0) {
+        const int64_t whole = sh.B % kScoreTile == 0 && sh.T % kScoreTile == 0 && sh.Dp % BK == 0
+                                  ? (int64_t)sh.S * (sh.B / kScoreTile) * (sh.T / kScoreTile) : 0;
+        const int columns = !sh.tcount ? 192 : sh.S > 1 ? 96 : 0;
+        if (p.out_mode != 0 || whole < 8 * 256 || sh.Dp >= columns) return {FWD_L1, kScoreTile, L1F_TN, dense};
+    }
     return {FWD_VALU, kScoreTile, kScoreTile, dense};
 }
 
-static FwdParams fwd_params(const ScoreShape& sh, const RowSource& a, const RowSource& b, int a_rel_mode) {
+static FwdParams fwd_params(const ScoreShape& sh, const RowSource& a, const RowSource& b, int a_rel_mode, int out_mode) {
     FwdParams p = {};
     p.sh = sh;
     if (sh.score_fn == SCORE_DISTMULT) p.sh.dist_fn = DIST_DOT;
     p.ent_a = a; p.ent_b = b;
     p.a_rel_mode = a_rel_mode;
+    p.out_mode = out_mode;
     return p;
 }
-static FwdParams fwd_params(const ScoreShape& sh, const RowSource& ent) {
-    return fwd_params(sh, ent, ent, sh.operands_dense ? 0 : (sh.score_fn == SCORE_DISTMULT ? 2 : 1));
+static FwdParams fwd_params(const ScoreShape& sh, const RowSource& ent, bool fused) {
+    return fwd_params(sh, ent, ent, sh.operands_dense ? 0 : (sh.score_fn == SCORE_DISTMULT ? 2 : 1), fused ? 0 : 1);
 }
 
-int score_fwd_parts(const ScoreShape& sh, const RowSource& ent) { return fwd_choice(fwd_params(sh, ent)).parts(sh); }
+int score_fwd_parts(const ScoreShape& sh, const RowSource& ent) { return fwd_choice(fwd_params(sh, ent, true)).parts(sh); }
 
 static void launch_fwd(const FwdParams& p, hipStream_t stream) {
     const FwdChoice choice = fwd_choice(p);
@@ -1017,11 +1031,10 @@ static void launch_fwd(const FwdParams& p, hipStream_t stream) {
 void launch_score_fwd(const ScoreShape& sh, const RowSource& ent, const float* rel,
                       const uint32_t* crel, const uint32_t* clabel, float* coef, float* dist,
                       uint32_t* nearflag, float* loss_part, bool fused_loss, hipStream_t stream) {
-    FwdParams p = fwd_params(sh, ent);
+    FwdParams p = fwd_params(sh, ent, fused_loss);
     p.nearflag = nearflag;
     p.rel = rel; p.crel = crel; p.clabel = clabel;
     p.coef = coef; p.dist = dist; p.loss_part = loss_part;
-    p.out_mode = fused_loss ? 0 : 1;
     p.a_c0 = 0; p.b_c0 = sh.S * sh.B;
     launch_fwd(p, stream);
 }
@@ -1030,9 +1043,8 @@ void launch_score_fwd(const ScoreShape& sh, const RowSource& ent, const float* r
 // source, e.g. consecutive rows of the table itself: no copy of the b side is made.
 void launch_score_fwd_rows(const ScoreShape& sh, const RowSource& a, const RowSource& b, float* scores,
                            hipStream_t stream) {
-    FwdParams p = fwd_params(sh, a, b, 0);
+    FwdParams p = fwd_params(sh, a, b, 0, 1);
     p.coef = scores;
-    p.out_mode = 1;
     launch_fwd(p, stream);
 }
 

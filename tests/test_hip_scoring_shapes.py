@@ -64,6 +64,15 @@ def test_l1_forward_tiles(oracle64, loss_fn, S, B, A, D, merge):
                             n_relation=6, gamma=4.0), n_step=2, **{"execution.merge_tails": merge})
 
 
+# L1 forward on whole tiles of 64 x 64 and slabs of 32 columns, the next slab's loads in flight: below 64 columns, and
+# where short loops meet 2048 tiles or more (64 columns with merged tails, 96 without)
+@pytest.mark.parametrize("S,B,A,D,merge", [(2, 64, 64, 32, True), (1, 128, 64, 32, False), (32, 256, 32, 64, True),
+                                           (32, 512, 16, 96, False)])
+def test_l1_forward_whole_tiles(oracle64, S, B, A, D, merge):
+    run_case(oracle64, dict(distance_fn="L1", n_shard=S, batch=B, a2a=A, dim=D, feature=0, n_entity=2000, n_relation=S,
+                            gamma=4.0), n_step=1, **{"execution.merge_tails": merge})
+
+
 # Columns in which every head equals every tail have signum 0 throughout: their gradients are exactly zero
 @pytest.mark.parametrize("B,A,D", [(33, 90, 30), (64, 352, 64)])
 def test_l1_equal_columns_have_zero_gradient(B, A, D):
