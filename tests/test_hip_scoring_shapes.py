@@ -55,13 +55,35 @@ def test_l1_narrow_groups(oracle64, S, B, A, D):
 
 
 # L1 forward: tiles of 64 heads x 32 tails, four waves over slabs of eight columns (from 64 columns on): around a tile's
-# edges, a last slab of four columns, waves with and without one, distinct tails that end on a tile
+# edges, a last slab of four columns, waves with and without one
 @pytest.mark.parametrize("merge", [True, False])
 @pytest.mark.parametrize("loss_fn", ["logsigmoid", "softmax"])
 @pytest.mark.parametrize("S,B,A,D", [(1, 1, 2, 64), (1, 63, 31, 68), (2, 64, 16, 72), (1, 65, 33, 100), (3, 130, 43, 260), (1, 8, 96, 128)])
 def test_l1_forward_tiles(oracle64, loss_fn, S, B, A, D, merge):
     run_case(oracle64, dict(distance_fn="L1", loss_fn=loss_fn, n_shard=S, batch=B, a2a=A, dim=D, feature=0, n_entity=1500,
                             n_relation=6, gamma=4.0), n_step=2, **{"execution.merge_tails": merge})
+
+
+# Merged tails: limits are whole groups of 64 columns, the L1 forward's tiles are 32 wide, so the last 32 columns in front of
+# a limit can lie behind the distinct tails.  The forward leaves zeros there; the vector backward, a launch per side, adds
+# them up.  Fewer distinct tails from step to step: what the step before left there would show.
+@pytest.mark.parametrize("B,T,D", [(70, 192, 64), (33, 180, 100)])
+def test_l1_dead_columns_in_front_of_the_limit(oracle64, B, T, D):
+    counts = [(T, T - 1), (160, 129), (96, 70), (32, 20)]  # distinct tails of the two blocks, step by step
+
+    def batch_fn(c, n_step, rng):
+        batch = K.raw_batch(c, n_step, rng, zipf=False)
+        for step in range(n_step):
+            for d in range(2):
+                pool = rng.choice(np.arange(1, c["n_entity"]), counts[step][d], replace=False).astype(np.uint32)
+                rows = np.concatenate([pool, pool[rng.integers(0, len(pool), T - len(pool))]])
+                rng.shuffle(rows)
+                # block d's tails: slots B + d A .. + A - 1 of either source shard's `remote`
+                batch["remote"][:, step, B + d * T // 2:B + (d + 1) * T // 2] = rows.reshape(2, T // 2)
+        return batch
+
+    run_case(oracle64, dict(distance_fn="L1", n_shard=2, batch=B, a2a=T // 2, dim=D, feature=0, n_entity=1500, n_relation=6,
+                            gamma=4.0, shared_table=True), n_step=4, batch_fn=batch_fn, **{"execution.scoring": "valu"})
 
 
 # L1 forward on whole tiles of 64 x 64 and slabs of 32 columns, the next slab's loads in flight: below 64 columns, and

@@ -35,8 +35,7 @@ CASES = {
     # tile-aligned shapes (positives % 128, tails % 128, dim % 64): the matrix-core fast path
     "aligned_l2": dict(distance_fn="L2", n_shard=2, batch=128, a2a=64, dim=64, feature=0,
                        n_entity=3000, n_relation=8, gamma=6.0),
-    # L1 on whole 64 x 64 tiles and 32-column slabs: the vector forward kernel's form with the next
-    # slab's loads in flight
+    # L1 on whole tiles and slabs
     "aligned_l1": dict(distance_fn="L1", n_shard=2, batch=128, a2a=64, dim=64, feature=0,
                        n_entity=3000, n_relation=8, gamma=6.0),
     "aligned_l2_wide": dict(distance_fn="L2", n_shard=4, batch=256, a2a=64, dim=128, feature=0,
