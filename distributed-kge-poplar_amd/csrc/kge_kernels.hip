@@ -949,7 +949,9 @@ static FwdChoice fwd_choice(const FwdParams& p) {
     const bool dense = p.ent_a.etype == ET_F32 && p.ent_b.etype == ET_F32 && vec && !p.ent_a.index && !p.ent_b.index &&
                        p.a_rel_mode == 0;
     if (sh.use_mfma && sh.dist_fn != DIST_L1 && vec && (sh.Dp & 3) == 0) return {FWD_MFMA, FM_TM, FM_TN, dense};
-    // k_score_fwd_l1: from 64 columns on, where each of its waves has two slabs (TransH's own forward has tiles of 64 x 64).
+    // k_score_fwd_l1: from 64 columns on, where each of its waves has two slabs.  (TransH's own forward has tiles of 64 x 64.
+    // Below 64 no line is drawn yet.  k_score_fwd, k_score_fwd_l1 at D = 48: 4 of 256 x 256 12.8, 7.8 us, 16 of 512 x 1536
+    // 51.9, 51.5; at D = 32 8.9, 6.8 and 35.6, 42.7.)
     // Not the fused forward of whole tiles with eight workgroups of them for every CU, while the loop is short against the
     // waves' sums.  us per launch in k_score_fwd, in k_score_fwd_l1:
     //   D                                            64        96       128        160        192        256

@@ -1061,12 +1061,11 @@ static L1Split l1_pair_split(const ScoreShape& sh) {
     // A workgroup of sixteen waves fills a CU.  Of the group sizes that the kernel has loops for, with
     // as many groups of heads (four chunks of eight at least) as the chip then has CUs left, the one whose
     // workgroups are done first: heads of a group times tails per wave and kHead, what a head costs
-    // beside its tails, in tails (an estimate; 2 to 4 choose nearly the same).  16 blocks of 512 x 1536 with
-    // D = 256: 4 groups of 384 tails, 256 workgroups.  Against doubling the groups of tails, then those of heads,
-    // while there are CUs, 40 steps each: 4 blocks of 512 x 1024, D = 256: 8.0 -> 4.9 ms; 10 of 130 x 960,
-    // D = 128: 3.8 -> 3.3; 1000 x 2000, D = 128: 3.4 -> 3.2; 16 of 64 x 64 and 1024 x 300, D = 64: the same;
-    // 40 x 1500, D = 256: 2.75 -> 2.80.
-    constexpr int kHead = 3;
+    // beside its tails, in tails.  16 blocks of 512 x 1536 with D = 256: 4 groups of 384 tails, 256 workgroups.
+    // kHead 1, 2, 3, 4, 6 choose differently for few shapes; us with the pieces' sums: 8 blocks of 200 x 1000, D = 256: 57, 56,
+    // 59, 60, 60; 32 of 200 x 512, D = 100: 57, 57, 59, 59, 59; 16 of 200 x 256, D = 256: 38, 35, 35, 35, 35; 10 of
+    // 130 x 960, D = 128: 34, 33, 33, 35, 35; 8 of 1000 x 256, D = 64: 31, 31, 31, 31, 33.
+    constexpr int kHead = 2;
     const int base = sh.S * ((sh.Dp + 63) / 64);
     L1Split k = {};
     int64_t least = INT64_MAX;
@@ -1100,8 +1099,7 @@ __global__ __launch_bounds__(1024) void k_score_bwd_l1_pair(const float* __restr
     // merged tails: the block's distinct tails alone.  The columns between them and the forward
     // pass's limit stand for no tail position: their coefficients are zero and nothing reads
     // their gradient rows.  The groups share the live tails evenly, in steps of 32 (an even number
-    // per wave: 331 instead of 343 columns per block on average on the 22.8M-row workload, and
-    // the launch's time follows that average (158.6 -> 155 us), not its largest block).
+    // per wave: 331 instead of 343 columns per block on average on the 22.8M-row workload).
     const int live = tcount ? min(T, (int)tcount[d]) : T;
     const int t_size = ((live + t_groups - 1) / t_groups + 31) & ~31;
     const int t0 = tg * t_size, h0 = hg * h_size;
