@@ -197,3 +197,17 @@ def test_no_kernel_spills_registers():
     assert any("k_score_bwd_l1_pair" in k[".name"] for k in kernels)
     spilled = {k[".name"]: k[".vgpr_spill_count"] for k in kernels if k.get(".vgpr_spill_count")}
     assert not spilled
+
+
+def test_profiled_step_kernels_are_the_librarys():
+    """The committed summaries of the step's traffic, which bench.py reads, name kernels that the library still has;
+    the L1 workload of D = 256 the forward that it launches."""
+    have = {re.sub(r"^_ZN3kge\d+", "", k[".name"]) for k in _library_kernels()}
+    named = {}
+    for path in sorted((ROOT / "profiles").glob("*_step_hbm_traffic.md")):
+        named[path.name] = re.findall(r"^\| `kge::(\w+)(?:<([^>`]*)>)?` \|", path.read_text(), re.M)
+        for name, args in named[path.name]:
+            coded = "".join(f"Lb{int(a == 'true')}E" if a in ("true", "false") else f"Li{a}E" for a in args.split(", ")) if args else ""
+            assert any(k.startswith(name + (f"I{coded}E" if coded else "E")) for k in have), (path.name, name, args)
+    assert len(named) == 5
+    assert ("k_score_fwd_l1", "0") in named["c3_step_hbm_traffic.md"]
