@@ -63,7 +63,8 @@ def _tall(dtype, F, D, batch):  # heads drawn with repeats: fewer distinct rows 
 # first line of either list: eight waves above 768 16-bit or 384 float32 features; fewer waves on tall
 # tiles, four times as many chunks per thread, above 192 and 96).  Batches of 40k and 80k, 120k rows with four and
 # two waves take tiles of 64 to 128 rows; eight waves take theirs by the distinct rows, 0.63 of a batch: 32, 64, 96 and 128
-# for 10k, 20k, 30k and 40k, and for 25.5k 64 in more workgroups than the 128 of the batch itself; from 1152 rows on
+# for 10k, 20k, 30k and 40k, and for 25.5k 64 in more workgroups than the 128 of the batch itself (up to 8192 contributions
+# in all there is nothing to choose); from 1152 rows on
 # dW's contraction has more than eight parts.
 @pytest.mark.parametrize("dtype,F,D,batch,all_distinct", [
     _small("float32", 4, 30, 31), _small("float16", 4, 66, 33), _small("bfloat16", 130, 66, 32), _small("float32", 36, 260, 33),
@@ -72,6 +73,7 @@ def _tall(dtype, F, D, batch):  # heads drawn with repeats: fewer distinct rows 
     _tall("bfloat16", 36, 66, 20000), _tall("float16", 130, 66, 40000), _tall("float32", 132, 66, 60000),
     _tall("float32", 36, 130, 10000), _tall("bfloat16", 130, 130, 20000), _tall("float16", 36, 130, 30000), _tall("float32", 100, 260, 15000),
     _tall("float16", 36, 130, 25500), _tall("float16", 36, 130, 40000), _tall("float32", 36, 130, 40000),
+    _tall("float16", 36, 130, 8190), _tall("float16", 36, 130, 8191),
 ])
 def test_feature_shapes(oracle64, dtype, F, D, batch, all_distinct):
     c = K.cfg_dict(distance_fn="L2", n_shard=1, batch=batch, a2a=2, dim=D, feature=F, n_entity=batch + 5, n_relation=6, gamma=4.0)
