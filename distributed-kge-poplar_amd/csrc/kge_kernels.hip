@@ -952,21 +952,28 @@ static FwdChoice fwd_choice(const FwdParams& p) {
     // k_score_fwd_l1: from 64 columns on, where each of its waves has two slabs.  (TransH's own forward has tiles of 64 x 64.
     // Below 64 no line is drawn yet.  k_score_fwd, k_score_fwd_l1 at D = 48: 4 of 256 x 256 12.8, 7.8 us, 16 of 512 x 1536
     // 51.9, 51.5; at D = 32 8.9, 6.8 and 35.6, 42.7.)
-    // Not the fused forward of whole tiles with eight workgroups of them for every CU, while the loop is short against the
+    // Not launches of whole slabs with eight workgroups of k_score_fwd for every CU, while the loop is short against the
     // waves' sums.  us per launch in k_score_fwd, in k_score_fwd_l1:
     //   D                                            64        96       128        160        192        256
+    //   fused loss, whole tiles:
     //   16 of 512 x 1536, all tails distinct     53, 60    70, 75    86, 92   100, 104   117, 121   148, 150
     //   64 of 256 x 512, all distinct            39, 43    51, 54    63, 66     72, 74     84, 86   109, 109
     //   32 of 256 x 512 (half the workgroups)    23, 23    29, 29    36, 35     42, 40     48, 46     62, 58
     //   64 of 256 x 512, merged, power law       31, 31    41, 39    51, 47     58, 54     67, 62     87, 77
     //   1 of 4096 x 2048, merged, power law      32, 25    42, 30    51, 36     60, 41     70, 47     89, 58
+    //   raw scores:
+    //   16 of 512 x 1536, all distinct           42, 46    59, 64    76, 77                112, 107
+    //   64 of 256 x 512, all distinct            31, 33    43, 43    54, 53                 77, 75
+    //   64 of 256 x 512, merged, power law       28, 26    39, 33    48, 41                 69, 56
+    //   a sweep of 1M rows, ms                0.70, 0.73 .80, .80  .92, .95              1.22, 1.24
     // How many merged tails are distinct only the device knows: the line for them lies where neither kernel loses more
     // than the other gains, which is nowhere with a single block (k_score_fwd's dead tiles share CUs).
     if (dense && sh.dist_fn == DIST_L1 && sh.score_fn != SCORE_TRANSH && sh.Dp >= 64 && (sh.Dp & 3) == 0) {
-        const int64_t whole = sh.B % kScoreTile == 0 && sh.T % kScoreTile == 0 && sh.Dp % BK == 0
-                                  ? (int64_t)sh.S * (sh.B / kScoreTile) * (sh.T / kScoreTile) : 0;
-        const int columns = !sh.tcount ? 192 : sh.S > 1 ? 96 : 0;
-        if (p.out_mode != 0 || whole < 8 * 256 || sh.Dp >= columns) return {FWD_L1, kScoreTile, L1F_TN, dense};
+        const bool raw = p.out_mode != 0, whole = sh.B % kScoreTile == 0 && sh.T % kScoreTile == 0;
+        const FwdChoice squares = {FWD_VALU, kScoreTile, kScoreTile, dense};
+        const int columns = sh.tcount ? (sh.S > 1 ? 96 : 0) : raw ? 160 : 192;
+        if (!(sh.Dp < columns && sh.Dp % BK == 0 && (raw || whole) && (int64_t)sh.S * squares.parts(sh) >= 8 * 256))
+            return {FWD_L1, kScoreTile, L1F_TN, dense};
     }
     return {FWD_VALU, kScoreTile, kScoreTile, dense};
 }
