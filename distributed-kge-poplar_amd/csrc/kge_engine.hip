@@ -195,9 +195,8 @@ struct kge_engine {
     int predict_chunk_rows = 0;  // additive setting execution.predict_chunk_rows: tails scored per launch (0: chosen from the number of queries)
     int stream_kind;  // KGE_F32 or KGE_F16: dtype of the entity read/write streams
     bool profile_kernels = false;
-    // additive setting execution.scoring: "mfma_bf16x3" (2, the default: matrix cores, the forward
-    // products from six bfloat16 instructions on three-piece float32 operands where shapes are
-    // aligned), "mfma" (1: float32 matrix instructions only), "valu" (0)
+    // additive setting execution.scoring: "mfma_bf16x3" (2, the default: matrix cores, float32 products
+    // from 16-bit instructions on split operands), "mfma" (1: float32 matrix instructions only), "valu" (0)
     int use_mfma = 2;
     bool score_bf16 = false;  // additive setting execution.scoring_dtype = "float32" | "bfloat16"
     int chunk = 64;       // contributions per first-level chunk (rows with many contributions; 256 measured no faster)
@@ -271,11 +270,13 @@ struct kge_engine {
     DevBuf<float> up, up_m, up_v, down, down_m, down_v, g_up, g_down;
     DevBuf<float> mlp_fproj, mlp_concat, mlp_pre, mlp_gpre, mlp_gfp, mlp_gval, p_fproj, p_concat, p_pre;
     DevBuf<float> opnd_n, cmat, dcm, transh_mm, relgrad;  // TransH: [n | tails], c, d loss / d c, its products, relation contributions
-    // L2 and dot scoring on three-piece operands (kge_split.hip)
+    // L2 and dot scoring on float16 halves (kge_split.hip)
     bool split = false;
     int Kp = 0, Bp = 0, Tp = 0;
     DevBuf<char> rowsp, coefp;
-    DevBuf<float> row_norm, rowpart, colpart;
+    DevBuf<int> coef_exp;
+    DevBuf<uint32_t> row_lost;
+    DevBuf<float> row_norm, row_scale, rowpart, colpart;
     // feature products on pieces (kge_feature.hip): W of every network as a piece matrix, kept by
     // the update and formed afresh after a write from outside
     bool split_feat = false, proj_pieces_fresh = false;
@@ -711,11 +712,15 @@ void allocate(kge_engine& E) {
         E.Kp = round_up(E.Dp, 32); E.Bp = round_up(E.B, 32); E.Tp = round_up(E.T, 32);
         // rows and columns that no kernel writes are read and dropped, or (columns filled up to whole
         // slabs) multiplied by each other: zeros
-        E.rowsp.alloc(split_bytes(R, E.Kp));
+        E.rowsp.alloc(half_bytes(R, E.Kp));
         E.rowsp.zero(st);
-        E.coefp.alloc(split_bytes(S * E.Bp, E.Tp));
+        E.row_lost.alloc((R + kSplitSpareRows) * E.Kp / 32);
+        E.coefp.alloc(half_bytes(S * E.Bp, E.Tp));
         E.coefp.zero(st);
+        E.coef_exp.alloc(S * (E.Bp / 32) * (E.Tp / 32));
         E.row_norm.alloc(R + kSplitSpareRows);
+        E.row_scale.alloc(R + kSplitSpareRows);
+        E.row_scale.zero(st);
         E.rowpart.alloc(S * E.Bp * (E.Tp / 32));
         E.colpart.alloc(S * (E.Bp / 32) * E.Tp);
     } else E.opnd.alloc(R * E.Dp);
@@ -1249,11 +1254,10 @@ void run_step(kge_engine& E, int i) {
     }
 
     // dense operands: every contribution's row, float32, relation applied to the heads
+    const SplitRows split_rows = {(int)SB, (int)R, E.Dp, E.Kp, E.rowsp.p, E.row_lost.p, E.row_scale.p, E.row_norm.p};
     { KernelTimer t(E, K_GATHER);
       TailCols tc = {sh.tcount, E.T, E.tpad};
-      if (E.split)
-          launch_gather_pieces(ent, E.rel.p, crel, rel_mode_of(E), E.D / 2, (int)SB, (int)R, E.Dp, E.Kp, E.rowsp.p,
-                               E.row_norm.p, st, &tc);
+      if (E.split) launch_gather_halves(ent, E.rel.p, crel, rel_mode_of(E), E.D / 2, split_rows, sh, st);
       else
       launch_gather_operands(ent, E.rel.p, crel, rel_mode_of(E), E.D / 2, (int)SB, (int)R, E.Dp,
                              E.opnd.p, E.score_bf16 ? E.opnd16.p : nullptr, st, &tc); }
@@ -1335,22 +1339,22 @@ void run_step(kge_engine& E, int i) {
           launch_transh_bwd(tb, st);
           launch_transh_back(ent, E.rel.p, crel, E.n_rel, (int)SB, E.Dp, E.grad.p, E.transh_mm.p, E.relgrad.p, st); }
     } else if (E.split) {
-        const SplitCoef sc = {E.coefp.p, E.rowpart.p, E.colpart.p, E.Bp, E.Tp};
+        const SplitCoef sc = {E.coefp.p, E.coef_exp.p, E.rowpart.p, E.colpart.p, E.Bp, E.Tp};
         { KernelTimer t(E, K_FWD);
           SplitFwd f = {};
-          f.sh = sh; f.rows = E.rowsp.p; f.norm = E.row_norm.p; f.b_c0 = (int)SB; f.Kp = E.Kp; f.clabel = clabel;
+          f.sh = sh; f.rows = split_rows; f.clabel = clabel;
           f.coef = E.coef.p; f.dist = fused ? nullptr : E.dist.p; f.loss_part = loss_part; f.nearflag = E.nearflag.p;
           f.out = sc;
           launch_split_fwd(f, fused, st); }
         if (!fused) {
             KernelTimer t(E, K_LOSS);
             launch_loss_rows(sh, clabel, E.coef.p, E.dist.p, loss_part, nullptr, st);
-            launch_coef_pieces(sh, E.coef.p, E.nearflag.p, sc, st);
+            launch_coef_halves(sh, E.coef.p, E.nearflag.p, split_rows, sc, st);
         }
         { KernelTimer t(E, K_BWD);
           SplitBwd b = {};
-          b.rows = E.rowsp.p; b.Kp = E.Kp; b.b_c0 = (int)SB; b.in = sc; b.coef = E.coef.p; b.nearflag = E.nearflag.p;
-          b.grad = E.grad.p; b.S = E.S; b.B = E.B; b.T = E.T; b.Dp = E.Dp; b.tcount = sh.tcount; b.tpad = sh.tpad;
+          b.rows = split_rows; b.in = sc; b.coef = E.coef.p; b.nearflag = E.nearflag.p;
+          b.grad = E.grad.p; b.S = E.S; b.B = E.B; b.T = E.T; b.tcount = sh.tcount; b.tpad = sh.tpad;
           launch_split_bwd(b, E.dist_fn == DIST_L2 && E.score_fn != SCORE_DISTMULT, st); }
     } else {
         { KernelTimer t(E, K_FWD);

@@ -246,25 +246,38 @@ inline size_t nearflag_words(const ScoreShape& sh) {
 }
 int score_fwd_parts(const ScoreShape& sh, const RowSource& ent);  // n_part of such a launch (of `sh.tcount`, only whether it is there counts)
 
-// ---- scoring on three-piece operands (kge_split.hip; L2 and dot, any shape) ----
-// Piece matrices hold every float32 value as three bfloat16 pieces, rows of 6 * Kp bytes (columns
+// ---- scoring on float16 halves (kge_split.hip; L2 and dot, any shape) ----
+// Matrices of halves hold every float32 value as two scaled float16 numbers, rows of half_pitch(cols) bytes (columns
 // filled up to a multiple of 32 with zeros).  The product kernels read whole tiles: kSplitSpareRows
-// rows behind a matrix's last must be readable and finite.
+// rows behind a matrix's last must be readable.
 constexpr int kSplitSpareRows = 128;
+// The workgroups on an XCD read the same 128 bytes of many rows at about the same time: a pitch that is an odd
+// number of 128-byte lines spreads those over the L2's channels, a power of two does not.
+inline __host__ __device__ int half_pitch(int cols) { return (cols / 32 | 1) * 128; }
+inline size_t half_bytes(size_t rows, size_t cols) { return (rows + kSplitSpareRows) * half_pitch((int)cols) + 128 * 4; }
+// bytes of a matrix of three bfloat16 pieces
 inline size_t split_bytes(size_t rows, size_t cols) {
     return (rows + kSplitSpareRows) * ((cols + 31) / 32 * 32) * 6 + 128 * 6;
 }
-void launch_gather_pieces(const RowSource& ent, const float* rel, const uint32_t* crel, int rel_mode, int half,
-                          int n_head, int n_rows, int Dp, int Kp, void* out, float* norm, hipStream_t stream,
-                          const TailCols* tail_cols);
-// The coefficient matrices [S][Bp][Tp] (B and T filled up to multiples of 32) as pieces, and their
-// sums over the 32 x 32 sub-blocks: rowpart [S][Bp][Tp / 32], colpart [S][Bp / 32][Tp] (L2 only)
-struct SplitCoef { char* coefp; float* rowpart; float* colpart; int Bp, Tp; };
+inline __host__ __device__ int lost_at(int k) { return (k & 3) * 8 + ((k & 31) >> 2); }
+// The contributions' rows, heads first.
+struct SplitRows {
+    int n_head, n_rows, Dp, Kp;
+    char* halves;    // [n_rows + kSplitSpareRows][Kp] as halves
+    uint32_t* lost;  // [n_rows + kSplitSpareRows][Kp / 32]: the bits that they lack, column k's at lost_at(k)
+    float* scale;    // the rows' scales and squared norms, [n_rows + kSplitSpareRows]
+    float* norm;
+};
+void launch_gather_halves(const RowSource& ent, const float* rel, const uint32_t* crel, int rel_mode, int half,
+                          const SplitRows& rows, const ScoreShape& sh, hipStream_t stream);
+// The coefficient matrices [S][Bp][Tp] (B and T filled up to multiples of 32) times the scales of their head and
+// tail as halves, the exponents of the 32 x 32 sub-blocks' own scales [S][Bp / 32][Tp / 32] (kNoExponent: all
+// zeros), and the coefficients' sums over the sub-blocks: rowpart [S][Bp][Tp / 32], colpart [S][Bp / 32][Tp] (L2 only)
+struct SplitCoef { char* coefp; int* exponent; float* rowpart; float* colpart; int Bp, Tp; };
+constexpr int kNoExponent = 1 << 20;
 struct SplitFwd {
     ScoreShape sh;
-    const char* rows;   // piece matrix: heads from row 0, tails from row b_c0
-    const float* norm;  // the rows' squared norms
-    int Kp, b_c0;
+    SplitRows rows;     // heads from row 0, tails from row n_head
     const uint32_t* clabel;
     float* coef;        // [S, B, T] scores (without fused loss); the flagged sub-blocks' coefficients
     float* dist;        // or null
@@ -275,16 +288,16 @@ struct SplitFwd {
 bool split_scoring(const ScoreShape& sh);  // whether a step's scoring takes this form
 int split_fwd_parts(const ScoreShape& sh);
 void launch_split_fwd(const SplitFwd& p, bool fused_loss, hipStream_t stream);
-// `coef` as launch_loss_rows leaves it -> pieces and sums
-void launch_coef_pieces(const ScoreShape& sh, const float* coef, const uint32_t* nearflag, const SplitCoef& out,
-                        hipStream_t stream);
+// `coef` as launch_loss_rows leaves it -> halves and sums
+void launch_coef_halves(const ScoreShape& sh, const float* coef, const uint32_t* nearflag, const SplitRows& rows,
+                        const SplitCoef& out, hipStream_t stream);
 struct SplitBwd {
-    const char* rows; int Kp, b_c0;  // heads from row 0, tails from row b_c0
+    SplitRows rows;
     SplitCoef in;
     const float* coef;               // float32 coefficients of the flagged sub-blocks
     const uint32_t* nearflag;
     float* grad;                     // [R, Dp]
-    int S, B, T, Dp;
+    int S, B, T;
     const uint32_t* tcount; int tpad;
 };
 void launch_split_bwd(const SplitBwd& p, bool l2, hipStream_t stream);

@@ -32,29 +32,31 @@ DEVINL void log_sigmoid_both(float z, float& value, float& grad) {
     grad = z >= 0.f ? g_pos : rw;
 }
 
-// The same for both signs of one score: exp(-|z|) serves z = s and z = -s alike.
-DEVINL void log_sigmoid_pair(float s, float& v_pos, float& g_pos, float& v_neg, float& g_neg) {
-    const float u = __builtin_amdgcn_exp2f(-1.44269504089f * fabsf(s));
-    const float w = 1.f + u;
-    const float rw = __builtin_amdgcn_rcpf(w);
-    const float l1p = 0.69314718056f * __builtin_amdgcn_logf(w) - ((w - 1.f) - u) * rw;
-    const float g_big = fmaxf(u * rw, 1.670142184e-5f);  // e^-11 / (1 + e^-11)
-    v_pos = fminf(s, 0.f) - (s > -11.f ? l1p : 0.f);
-    v_neg = fminf(-s, 0.f) - (s < 11.f ? l1p : 0.f);
-    g_pos = s >= 0.f ? g_big : rw;
-    g_neg = s <= 0.f ? g_big : rw;
-}
+// The same for both signs of one score: exp(-|s|) serves z = s and z = -s alike.
+struct LogSigmoid {
+    float s, rw, l1p, g_big;
+    DEVINL explicit LogSigmoid(float score) : s(score) {
+        const float u = __builtin_amdgcn_exp2f(-1.44269504089f * fabsf(s));
+        const float w = 1.f + u;
+        rw = __builtin_amdgcn_rcpf(w);
+        l1p = 0.69314718056f * __builtin_amdgcn_logf(w) - ((w - 1.f) - u) * rw;
+        g_big = fmaxf(u * rw, 1.670142184e-5f);  // e^-11 / (1 + e^-11)
+    }
+    DEVINL float plus_value() const { return fminf(s, 0.f) - (s > -11.f ? l1p : 0.f); }
+    DEVINL float minus_value() const { return fminf(-s, 0.f) - (s < 11.f ? l1p : 0.f); }
+    DEVINL float plus_grad() const { return s >= 0.f ? g_big : rw; }
+    DEVINL float minus_grad() const { return s <= 0.f ? g_big : rw; }
+};
 
 // The logsigmoid loss of one score column that stands for `mult` tail positions, one of them the
 // positive's label if `pos` (src/poplar_kge.cpp:615-636 summed over the positions that share the
 // row): returns the loss term (before the normalisation) and sets d loss / d score (times grad_scale).
 DEVINL float logsigmoid_column(float score, bool pos, float mult, float w_pos, float w_neg, float grad_scale,
                                float& dscore) {
-    float v_pos, g_pos, v_neg, g_neg;
-    log_sigmoid_pair(score, v_pos, g_pos, v_neg, g_neg);
+    const LogSigmoid z(score);
     const float wp = pos ? w_pos : 0.f, wn = (mult - (pos ? 1.f : 0.f)) * w_neg;
-    dscore = (wn * g_neg - wp * g_pos) * grad_scale;
-    return -(wp * v_pos + wn * v_neg);
+    dscore = (wn * z.minus_grad() - wp * z.plus_grad()) * grad_scale;
+    return -(wp * z.plus_value() + wn * z.minus_value());
 }
 
 constexpr float kCancelRatio = 0.125f;  // recompute when d^2 < ratio * (|a|^2 + |b|^2)

@@ -1,9 +1,10 @@
-// Device functions of the kernels that multiply float32 values as three bfloat16 pieces each: piece
-// matrices in memory, their tiles in LDS, and the copies from one to the other.
+// Device functions of the kernels that multiply float32 values as pieces of 16 bits: piece matrices in
+// memory, their tiles in LDS, and the copies from one to the other.  A value is three bfloat16 pieces, or
+// two float16 halves (below).
 //
-// Piece matrix: row r, column k, piece q at  r * pitch + (k / 32) * 192 + q * 64 + (k % 32) * 2  bytes:
-// the three pieces of 32 columns lie together, and a slab of a row is 192 consecutive bytes.  Columns
-// are filled with zeros to a multiple of 32.
+// Piece matrix of NP pieces: row r, column k, piece q at  r * pitch + (k / 32) * 64 NP + q * 64 + (k % 32) * 2
+// bytes: the pieces of 32 columns lie together, and a slab of a row is 64 NP consecutive bytes.
+// Columns are filled with zeros to a multiple of 32.
 #pragma once
 
 #include "kge_device.h"
@@ -26,40 +27,20 @@ DEVINL uint32_t lds_address(const void* p) {
     return (uint32_t)(size_t)(const __attribute__((address_space(3))) char*)p;
 }
 
-// neighbouring lanes' values (lane ^ 1)
+// neighbouring lanes' values (lane ^ 1, lane ^ 2); the lane's mirror image in its half row of eight, in its row of 16
+template <int CTRL>
+DEVINL float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+DEVINL float mirror8(float v) { return dpp<0x141>(v); }
+DEVINL float mirror16(float v) { return dpp<0x140>(v); }
 DEVINL float swap1(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));
+    return dpp<0xB1>(v);
 }
 DEVINL float swap2(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));
+    return dpp<0x4E>(v);
 }
 
-// four columns of a piece-matrix row, k % 4 == 0.  (An infinity's pieces are infinity, NaN, NaN: the first
-// alone is the value.)
-DEVINL float4 load_pieces4(const char* row, int k) {
-    const char* p = row + (size_t)(k >> 5) * 192 + (k & 31) * 2;
-    const uint2 hi = *reinterpret_cast<const uint2*>(p);
-    float4 v = make_float4(bf16_lo_f32(hi.x), bf16_hi_f32(hi.x), bf16_lo_f32(hi.y), bf16_hi_f32(hi.y));
-    const float4 first = v;
-#pragma unroll
-    for (int q = 1; q < 3; ++q) {
-        const uint2 raw = *reinterpret_cast<const uint2*>(p + 64 * q);
-        v.x += bf16_lo_f32(raw.x); v.y += bf16_hi_f32(raw.x);
-        v.z += bf16_lo_f32(raw.y); v.w += bf16_hi_f32(raw.y);
-    }
-    if (!(fabsf(first.x) < INFINITY)) v.x = first.x;
-    if (!(fabsf(first.y) < INFINITY)) v.y = first.y;
-    if (!(fabsf(first.z) < INFINITY)) v.z = first.z;
-    if (!(fabsf(first.w) < INFINITY)) v.w = first.w;
-    return v;
-}
-DEVINL float load_piece1(const char* row, int k) {
-    const char* p = row + (size_t)(k >> 5) * 192 + (k & 31) * 2;
-    float v = 0.f;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) v += bf16_to_f32(*reinterpret_cast<const uint16_t*>(p + 64 * q));
-    return v;
-}
 DEVINL void store_pieces4(char* row, int k, float4 v) {
     uint2 piece[3];
     split4_bf16(as_x4(v), piece);
@@ -67,14 +48,98 @@ DEVINL void store_pieces4(char* row, int k, float4 v) {
 #pragma unroll
     for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2*>(p + 64 * q) = piece[q];
 }
-// two neighbouring values -> three words of two pieces each
-DEVINL void split2(float a, float b, uint32_t w[3]) {
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        w[q] = pack_bf16(a, b);
-        if (q < 2) { a -= bf16_lo_f32(w[q]); b -= bf16_hi_f32(w[q]); }
-    }
+
+// --------------------------------------------------------------------------
+// Float16 halves.  x = s (h0 + h1 / 2048), h0 = float16(x / s), h1 = float16(2048 (x / s - h0)): 11 bits
+// each, the rounding of h0 to either side worth one more, so the sum differs from x by at most one unit in its
+// 24th bit, and for three values of four by nothing.  The scale s is a power of two that brings the largest of a
+// row (or of a block of coefficients) to 2^14; with the second half 2^11 times as large as it counts, both are
+// normal float16 numbers down to 2^-28 of that largest value, and what is smaller is off by 2^-49 of it at most.
+//   a b = sa sb (a0 b0 + (a0 b1 + a1 b0) / 2048 + O(2^-24 |a0 b0|)):
+// three matrix instructions where three bfloat16 pieces take six, two fragments of an operand where they take
+// three, and a row of halves is as long as the float32 row.  The cross products have an accumulator of their own.
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+constexpr float kHalfStep = 1.f / 2048.f;
+constexpr int kHalfBytes = 128;  // of 32 columns of a row
+
+// the scale for a largest magnitude (not negative; infinities and NaN take some scale, their halves say the rest).
+// Rows below 2^-40 share one, so that the product of two rows' scales stays a normal number.
+DEVINL float half_scale(float largest) {
+    const int e = min(max((int)(__float_as_uint(largest) >> 23) - 127, -40), 100);
+    return __uint_as_float((uint32_t)(e - 14 + 127) << 23);
 }
+// the reciprocal of a power of two
+DEVINL float pow2_inverse(float s) { return __uint_as_float(0x7f000000u - __float_as_uint(s)); }
+// two values, scaled already -> two words of two halves each
+DEVINL void split2_f16(float a, float b, uint32_t w[2]) {
+    const f16x2 h = {(_Float16)a, (_Float16)b};
+    const f16x2 l = {(_Float16)((a - (float)h.x) * 2048.f), (_Float16)((b - (float)h.y) * 2048.f)};
+    w[0] = __builtin_bit_cast(uint32_t, h);
+    w[1] = __builtin_bit_cast(uint32_t, l);
+}
+// Four columns of a row of halves, k % 4 == 0.  The second halves are cut off here, not rounded, and what that leaves
+// is one bit: whether the value has a twelfth bit there.  A whole wave at once; lost[i]: bit l for lane l's column k + i.
+DEVINL void store_halves4(char* row, int k, float4 v, bool live, uint64_t (&lost)[4]) {
+    const float x[4] = {v.x, v.y, v.z, v.w};
+    uint32_t w[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const f16x2 h = {(_Float16)x[2 * i], (_Float16)x[2 * i + 1]};
+        const float a = (x[2 * i] - (float)h.x) * 2048.f, b = (x[2 * i + 1] - (float)h.y) * 2048.f;
+        const auto cut = __builtin_amdgcn_cvt_pkrtz(a, b);
+        const f16x2 l = __builtin_bit_cast(f16x2, cut);
+        lost[2 * i] = __ballot(a != (float)l.x);
+        lost[2 * i + 1] = __ballot(b != (float)l.y);
+        w[0][i] = __builtin_bit_cast(uint32_t, h);
+        w[1][i] = __builtin_bit_cast(uint32_t, l);
+    }
+    if (!live) return;
+    char* p = row + (size_t)(k >> 5) * kHalfBytes + (k & 31) * 2;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) *reinterpret_cast<uint2*>(p + 64 * q) = make_uint2(w[q][0], w[q][1]);
+}
+// The rows of a gather as they were (values below 2^-28 of their row's largest to 2^-49 of that).
+DEVINL float join_lost(_Float16 h, _Float16 l, uint32_t bit) {  // (of a finite value, without its scale)
+    return fmaf(__uint_as_float(__float_as_uint((float)l) + (bit << 12)), kHalfStep, (float)h);
+}
+DEVINL float with_lost(_Float16 h, _Float16 l, bool lost, float scale) {
+    if (!(fabsf((float)h) < INFINITY)) return (float)h;
+    return join_lost(h, l, lost) * scale;
+}
+// eight columns k .. k + 7 of row c (k % 8 == 0), all loads in one go
+struct Row8 {
+    uint4 h, l;
+    uint32_t lost;
+    float scale;
+    DEVINL void load(const SplitRows& s, int c, int k) {
+        const char* p = s.halves + (size_t)c * half_pitch(s.Kp) + (size_t)(k >> 5) * kHalfBytes + (k & 31) * 2;
+        h = *reinterpret_cast<const uint4*>(p);
+        l = *reinterpret_cast<const uint4*>(p + 64);
+        lost = s.lost[(size_t)c * (s.Kp >> 5) + (k >> 5)] >> ((k & 31) >> 2);
+        scale = s.scale[c];
+    }
+    template <int I>
+    DEVINL float value() const {
+        constexpr int W = I >> 1;
+        const f16x2 hw = __builtin_bit_cast(f16x2, W == 0 ? h.x : W == 1 ? h.y : W == 2 ? h.z : h.w);
+        const f16x2 lw = __builtin_bit_cast(f16x2, W == 0 ? l.x : W == 1 ? l.y : W == 2 ? l.z : l.w);
+        return with_lost(I & 1 ? hw.y : hw.x, I & 1 ? lw.y : lw.x, (lost >> lost_at(I)) & 1u, scale);
+    }
+};
+struct Row1 {  // one column
+    _Float16 h, l;
+    uint32_t lost;
+    float scale;
+    DEVINL void load(const SplitRows& s, int c, int k) {
+        const char* p = s.halves + (size_t)c * half_pitch(s.Kp) + (size_t)(k >> 5) * kHalfBytes + (k & 31) * 2;
+        h = *reinterpret_cast<const _Float16*>(p);
+        l = *reinterpret_cast<const _Float16*>(p + 64);
+        lost = s.lost[(size_t)c * (s.Kp >> 5) + (k >> 5)];
+        scale = s.scale[c];
+    }
+    DEVINL float value(int k) const { return with_lost(h, l, (lost >> lost_at(k)) & 1u, scale); }
+};
 
 // --------------------------------------------------------------------------
 // tiles in LDS
@@ -82,9 +147,9 @@ DEVINL void split2(float a, float b, uint32_t w[3]) {
 // Contraction-innermost operand: R rows x 32 columns of a piece matrix as [piece][row][32], a row's
 // four 16-byte chunks at position chunk ^ ((row / 4) % 4): sixteen rows' reads of one chunk fall on
 // all banks.  One copy instruction moves sixteen rows of one piece.
-template <int R>
+template <int R, int NP = 3>
 struct RowTile {
-    static constexpr int kBytes = 3 * R * 64, kCopies = 3 * R / 16;
+    static constexpr int kBytes = NP * R * 64, kCopies = NP * R / 16;
     // offset of copy x's bytes for this lane, from the tile's first row and slab
     static DEVINL uint32_t source(int x, int lane, int pitch) {
         const int piece = x / (R / 16), row = (x % (R / 16)) * 16 + (lane >> 2);
@@ -103,9 +168,9 @@ struct RowTile {
 // each receives one column of it).  A row's 32-byte units sit at position unit ^ 2 (row % 4): the four
 // rows that a read instruction's half takes fall on different banks.  One copy instruction moves
 // 512 / C rows of one piece.
-template <int C>
+template <int C, int NP = 3>
 struct ColTile {
-    static constexpr int kBytes = 3 * 32 * C * 2, kCopies = 3 * C / 16;
+    static constexpr int kBytes = NP * 32 * C * 2, kCopies = NP * C / 16;
     static constexpr int kKey = C >= 128 ? 3 : 1;  // (a row of 64 columns has four units)
     // (rows past `last` repeat it)
     static DEVINL uint32_t source(int x, int lane, int pitch, int last = 31) {
@@ -113,7 +178,7 @@ struct ColTile {
         const int piece = x / (C / 16), row = (x % (C / 16)) * rows + lane / chunks, pos = lane % chunks;
         const int chunk = pos ^ ((row & kKey) << 2);  // 16-byte chunks: two to a unit
         const int col = chunk * 8;
-        return (uint32_t)(min(row, last) * pitch + (col >> 5) * 192 + piece * 64 + (col & 31) * 2);
+        return (uint32_t)(min(row, last) * pitch + (col >> 5) * (64 * NP) + piece * 64 + (col & 31) * 2);
     }
     // columns col0 .. col0 + 31 over the sixteen rows of step `ks` (this lane: column
     // col0 + lane % 32, rows 8 (lane / 32) .. + 7)

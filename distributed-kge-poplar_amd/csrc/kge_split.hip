@@ -1,14 +1,11 @@
-// gfx950 scoring kernels on three-piece operands (L2 and dot): the operand gather, the forward
-// scores with the fused loss, and both sides of the backward.
+// gfx950 scoring kernels on float16 halves (L2 and dot): the operand gather, the forward scores with the
+// fused loss, and both sides of the backward.
 //
-// Every float32 value is the exact sum of three bfloat16 pieces, and a float32 product is six
-// products of pieces (split4_bf16, mfma_split6's order).  Splitting while staging, as a kernel
-// that reads float32 operands must, costs more vector instructions than the products cost matrix
-// instructions, and every tile that reads a row splits it again.  Here every value is split once,
-// by the kernel that makes it: the gather writes the operand rows as pieces, the forward writes the
-// backward's coefficients as pieces, and the product kernels copy tiles straight from memory into
-// LDS (global_load_lds, no registers, no vector instructions), so that their waves do little else
-// than read fragments and multiply.
+// A float32 value is a scale and two float16 halves, and a float32 product is three products of halves
+// (kge_split.h).  Every value is split once, by the kernel that makes it: the gather writes the
+// operand rows as halves, the forward writes the backward's coefficients as halves, and the product
+// kernels copy tiles straight from memory into LDS (global_load_lds, no registers, no vector
+// instructions), so that their waves do little else than read fragments and multiply.
 //
 #include "kge_device.h"
 #include "kge_loss.h"
@@ -20,111 +17,173 @@
 namespace kge {
 
 // --------------------------------------------------------------------------
+// reductions over a wave without a way through LDS: the result is in lane 63 (rows of 16 by DPP, then across them)
+template <class Op>
+DEVINL float wave_reduce63(float v, Op&& op) {
+    v = op(v, swap1(v));
+    v = op(v, swap2(v));
+    v = op(v, mirror8(v));
+    v = op(v, mirror16(v));
+    const int x = __float_as_int(v);
+    v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(x, x, 0x142, 0xa, 0xf, false)));  // row 0's to 1, 2's to 3
+    const int y = __float_as_int(v);
+    return op(v, __int_as_float(__builtin_amdgcn_update_dpp(y, y, 0x143, 0xc, 0xf, false)));  // 1's to 2 and 3
+}
+// the largest of a wave's magnitudes, as its bits
+DEVINL uint32_t wave_max_bits(float v) {
+    v = wave_reduce63(v, [](float a, float b) { return fmaxf(a, b); });
+    return (uint32_t)__builtin_amdgcn_readlane(__float_as_int(v), 63);
+}
+
+// --------------------------------------------------------------------------
 // operand gather: RPW contributions per wave, their entity (or hidden) rows with the relation
-// applied for the heads, as pieces; and the rows' squared norms.
-template <int RPW, bool XF>  // XF: the complex product and the rotation compiled in
-__global__ __launch_bounds__(256) void k_gather_pieces(RowSource ent, const float* __restrict__ rel,
-                                                       const uint32_t* __restrict__ crel, int rel_mode, int half,
-                                                       int n_head, int n_rows, int Dp, int Kp, char* __restrict__ out,
-                                                       float* __restrict__ norm, TailCols tc) {
-    const int lane = threadIdx.x & 63;
-    const int c0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW;
-    if (c0 >= n_rows) return;
+// applied for the heads, as halves; and the rows' scales and squared norms.  Workgroup (d, y): the y-th lot of
+// block d's B heads and then T tails, which finds its XCD (d % 8) where the block's tiles will run.
+// ET: the rows' element type, or -1: as `ent` says, the complex product and the rotation among the
+// relations; ONE: rows of at most 256 columns, which stay in their registers between the largest value and the halves.
+template <int RPW, int ET, bool ONE>
+__global__ __launch_bounds__(256) void k_gather_halves(RowSource ent, const float* __restrict__ rel, const uint32_t* __restrict__ crel,
+                                                       int rel_mode, int half, SplitRows s, const uint32_t* __restrict__ tcount,
+                                                       int B, int T, int tpad) {
+    constexpr bool XF = ET < 0;
+    const int lane = threadIdx.x & 63, d = blockIdx.x;
+    const int i0 = (blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * RPW;
     // the row numbers are asked for together with the block's tail count (rows past it are
-    // never used, but their slots hold valid numbers): one round trip instead of two
+    // never used, but their slots hold valid numbers): one round trip instead of two.  (All of them
+    // are the wave's, and scalar loads: a lane has an offset into its rows and no addresses.)
+    int c[RPW];
     uint32_t key[RPW], rkey[RPW];
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
-        const int c = min(c0 + r, n_rows - 1);  // a row past the end repeats the last one
-        key[r] = ent.index ? ent.index[c] : (uint32_t)c;
-        rkey[r] = (c < n_head && rel_mode) ? crel[c] : 0u;
+        const int i = min(i0 + r, B + T - 1);  // a row past the end repeats the last one
+        c[r] = i < B ? d * B + i : s.n_head + d * T + i - B;
+        key[r] = ent.index ? ent.index[c[r]] : (uint32_t)c[r];
+        rkey[r] = (i < B && rel_mode) ? crel[c[r]] : 0u;
     }
-    bool live[RPW], any = false;
+    const int end = B + tail_limit(tcount, d, T, tpad);
 #pragma unroll
-    for (int r = 0; r < RPW; ++r) {
-        live[r] = c0 + r < n_rows && tc.live(c0 + r - n_head);
-        any = any || live[r];
-    }
-#pragma unroll
-    for (int r = 0; r < RPW; ++r) asm volatile("" : "+v"(key[r]), "+v"(rkey[r]));
-    if (!any) return;
+    for (int r = 0; r < RPW; ++r) asm volatile("" : "+s"(key[r]), "+s"(rkey[r]));
+    if (i0 >= end) return;
     const char* row[RPW];
     const float* rrow[RPW];
-    float sq[RPW];
+    float sq[RPW], top[RPW];
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
         row[r] = ent.base + (int64_t)key[r] * ent.pitch;
-        rrow[r] = (c0 + r < n_head && rel_mode) ? rel + (size_t)rkey[r] * Dp : nullptr;
-        sq[r] = 0.f;
+        rrow[r] = (i0 + r < B && rel_mode) ? rel + (size_t)rkey[r] * s.Dp : nullptr;
+        sq[r] = top[r] = 0.f;
     }
-    for (int k = lane * 4; k < Kp; k += 256) {
-        float4 v[RPW], w[RPW];
+    float4 v[RPW];
+    auto fetch = [&](int k) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < RPW; ++r) {  // all loads first
-            v[r] = w[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (k < Dp) {
-                v[r] = load4(row[r], k, ent);
-                if (rrow[r] && rel_mode <= 2) w[r] = *reinterpret_cast<const float4*>(rrow[r] + k);
-            }
-        }
+        for (int r = 0; r < RPW; ++r) v[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (k >= s.Dp) return;
 #pragma unroll
-        for (int r = 0; r < RPW; ++r) {
-            if (rrow[r] && k < Dp) {
+        for (int r = 0; r < RPW; ++r) v[r] = XF ? load4(row[r], k, ent) : load4(row[r], k, ET);  // all loads first
+        float4 w[RPW];
+#pragma unroll
+        for (int r = 0; r < RPW; ++r)
+            if (rrow[r] && !(XF && rel_mode >= 3)) w[r] = *reinterpret_cast<const float4*>(rrow[r] + k);
+#pragma unroll
+        for (int r = 0; r < RPW; ++r)
+            if (rrow[r]) {
                 if (XF && rel_mode >= 3) v[r] = relation_xf(v[r], row[r], ent.etype, rrow[r], k, half, rel_mode);
                 else v[r] = rel_mode == 1 ? f4add(v[r], w[r]) : f4mul(v[r], w[r]);
             }
+    };
+    const int k_end = ONE ? 256 : (s.Kp + 255) & ~255;  // (the whole wave stays together)
+    for (int k = lane * 4; k < k_end; k += 256) {
+        fetch(k);
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {
             sq[r] += v[r].x * v[r].x + v[r].y * v[r].y + v[r].z * v[r].z + v[r].w * v[r].w;
-            if (live[r]) store_pieces4(out + (size_t)(c0 + r) * Kp * 6, k, v[r]);
+            top[r] = fmaxf(fmaxf(top[r], fmaxf(fabsf(v[r].x), fabsf(v[r].y))), fmaxf(fabsf(v[r].z), fabsf(v[r].w)));
         }
     }
+    float up[RPW];
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
-        const float s = wave_sum(sq[r]);
-        if (lane == 0 && live[r]) norm[c0 + r] = s;
+        const float sum = wave_reduce63(sq[r], [](float a, float b) { return a + b; });
+        const float scale = half_scale(__uint_as_float(wave_max_bits(top[r])));
+        up[r] = pow2_inverse(scale);
+        if (lane == 63 && i0 + r < end) {
+            s.norm[c[r]] = sum;
+            s.scale[c[r]] = scale;
+        }
+    }
+    for (int k = lane * 4; k < k_end; k += 256) {
+        if (!ONE) fetch(k);
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {
+            uint64_t lost[4];
+            store_halves4(s.halves + (size_t)c[r] * half_pitch(s.Kp), k,
+                          make_float4(v[r].x * up[r], v[r].y * up[r], v[r].z * up[r], v[r].w * up[r]), i0 + r < end && k < s.Kp, lost);
+            // a slab's 32 bits: a byte of each ballot, by one lane
+            uint32_t word = 0u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) word |= (((uint32_t)(lane & 4 ? lost[i] >> 32 : lost[i]) >> (8 * (lane & 3))) & 255u) << (8 * i);
+            const int slab = ((k - 4 * lane) >> 5) + lane;
+            if (lane < 8 && slab < s.Kp >> 5 && i0 + r < end) s.lost[(size_t)c[r] * (s.Kp >> 5) + slab] = word;
+        }
     }
 }
 
-void launch_gather_pieces(const RowSource& ent, const float* rel, const uint32_t* crel, int rel_mode, int half,
-                          int n_head, int n_rows, int Dp, int Kp, void* out, float* norm, hipStream_t stream,
-                          const TailCols* tail_cols) {
-    TailCols tc = {};
-    if (tail_cols) tc = *tail_cols;
+void launch_gather_halves(const RowSource& ent, const float* rel, const uint32_t* crel, int rel_mode, int half,
+                          const SplitRows& s, const ScoreShape& sh, hipStream_t stream) {
     // two rows per wave where that leaves enough waves: the kernel is resident waves over the
     // latency of the chain row number -> row -> store, and a wave may as well keep two chains going
-#define KGE_GATHER(N_, X_)                                                                                            \
-    hipLaunchKernelGGL((k_gather_pieces<N_, X_>), dim3((n_rows + 4 * N_ - 1) / (4 * N_)), dim3(256), 0, stream, ent, rel, \
-                       crel, rel_mode, half, n_head, n_rows, Dp, Kp, (char*)out, norm, tc)
-    if (rel_mode >= 3) KGE_GATHER(1, true);
-    else if (n_rows >= 8192) KGE_GATHER(2, false);
-    else KGE_GATHER(1, false);
+    const int n = sh.B + sh.T;
+#define KGE_GATHER(N_, ET_, ONE_)                                                                                       \
+    hipLaunchKernelGGL((k_gather_halves<N_, ET_, ONE_>), dim3(sh.S, (n + 4 * N_ - 1) / (4 * N_)), dim3(256), 0, stream, \
+                       ent, rel, crel, rel_mode, half, s, sh.tcount, sh.B, sh.T, sh.tpad)
+#define KGE_GATHER_ET(ET_)                                                                                      \
+    do {                                                                                                        \
+        if (s.Kp > 256) KGE_GATHER(1, ET_, false);                                                              \
+        else if (s.n_rows >= 8192) KGE_GATHER(2, ET_, true);                                                    \
+        else KGE_GATHER(1, ET_, true);                                                                          \
+    } while (0)
+    if (rel_mode >= 3 || !ent.vec) { if (s.Kp > 256) KGE_GATHER(1, -1, false); else KGE_GATHER(1, -1, true); }
+    else if (ent.etype == ET_F32) KGE_GATHER_ET(ET_F32);
+    else if (ent.etype == ET_BF16) KGE_GATHER_ET(ET_BF16);
+    else KGE_GATHER_ET(ET_F16);
+#undef KGE_GATHER_ET
 #undef KGE_GATHER
 }
 
 // --------------------------------------------------------------------------
 // products
 
-// Tiles of 64 x 64, four waves, three workgroups to a CU: at these sizes a launch is bound by the
-// latency of its slabs and by how many workgroups there are, not by the matrix cores.
-constexpr int kTile = 64, kWaves = 2;  // waves as kWaves x kWaves
+// Tiles of TM x TN, waves as WM x WN of them, 32 x 32 of the tile to a wave: EU waves to a SIMD, whose registers allow as many
+// workgroups as LDS has room for (three of 128 x 64, four of 64 x 64).  What a launch spends its time on is the first slab's
+// way from memory, the loop and the epilogue of every workgroup, one after the other; workgroups beside it fill
+// the gaps, and a third of 128 x 64 is worth more than a third tile copy (64 blocks of 256 x 512, 331 distinct tails, D = 256:
+// forward 32.9 us with two workgroups of three copies, 27.2 with three of two; backward 48.2 and 46.3).
+template <int TM_, int TN_, int WM_, int WN_, int EU_>
+struct SplitTile { static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, EU = EU_, threads = WM_ * WN_ * 64; };
+using TileSmall = SplitTile<64, 64, 2, 2, 4>;
+using TileLarge = SplitTile<128, 64, 4, 2, 6>;
 
-// The product loop of a TM x TN tile: n_slab slabs of 32 contraction steps, two tile copies in LDS
-// (one fills while the other is multiplied, one barrier per slab).  TA, TB: RowTile / ColTile;
+// The product loop of a tile: n_slab slabs of 32 contraction steps, three tile copies in LDS
+// (two fill while the third is multiplied, one barrier per slab).  TA, TB: RowTile / ColTile;
 // a_step, b_step: bytes from slab to slab.  Waves as WM x WN, each (TM/WM) x (TN/WN) in 32 x 32
-// accumulators.
+// accumulators: `big` the products of first halves, `small` the cross products.
 // b_rows: rows of `b` along the contraction where it lies across it (ColTile).  The last slab's rows past them
 // repeat the last one: their coefficients are zero, but what lies behind a block's rows are other
 // blocks', and zero times a neighbour's infinity or NaN would be this block's NaN.
-template <class TA, class TB, int TM, int TN, int WM, int WN>
+template <class TA, class TB, class Tile>
 struct SplitProduct {
-    static constexpr int NW = WM * WN, AM = TM / WM / 32, AN = TN / WN / 32;
-    static constexpr int kStage = TA::kBytes + TB::kBytes, kLds = 2 * kStage;
+    static constexpr int kStages = 2;
+    static constexpr int NW = Tile::WM * Tile::WN, AM = Tile::TM / Tile::WM / 32, AN = Tile::TN / Tile::WN / 32;
+    static constexpr int kStage = TA::kBytes + TB::kBytes, kLds = kStages * kStage;
     static constexpr int kCopies = TA::kCopies + TB::kCopies, kEach = kCopies / NW;
     static_assert(kCopies % NW == 0, "every wave issues the same number of copies");
 
-    // meanwhile(): what the caller has to fetch for itself, under the first slab's way from memory
-    template <class Meanwhile>
+    // meanwhile(): what the caller has to fetch for itself, under the first slab's way from memory;
+    // before(slab): ahead of the slab's products, whether to form them
+    template <class Meanwhile, class Before>
     static DEVINL void run(char* smem, const char* a, int a_pitch, size_t a_step, const char* b, int b_pitch, size_t b_step,
-                           int n_slab, int b_rows, floatx16 (&acc)[AM][AN], int lane, int wave, Meanwhile&& meanwhile) {
+                           int n_slab, int b_rows, floatx16 (&big)[AM][AN], floatx16 (&small)[AM][AN], int lane, int wave,
+                           Meanwhile&& meanwhile, Before&& before) {
         uint32_t off[kEach];
 #pragma unroll
         for (int i = 0; i < kEach; ++i) {
@@ -135,14 +194,14 @@ struct SplitProduct {
         auto fill = [&](int slab) __attribute__((always_inline)) {
             const char* as = a + slab * a_step;
             const char* bs = b + slab * b_step;
-            const uint32_t to = lds0 + (slab & 1) * kStage;
-            if constexpr (!std::is_same_v<TB, RowTile<TN>>) {
+            const uint32_t to = lds0 + slab % kStages * kStage;
+            if constexpr (!std::is_same_v<TB, RowTile<Tile::TN, 2>>) {
                 const int last = b_rows - 32 * slab - 1;
                 if (last < 31)  // the last slab's offsets take the others' place
 #pragma unroll
                     for (int i = 0; i < kEach; ++i) {
                         const int x = wave + NW * i;
-                        if (x >= TA::kCopies) off[i] = TB::source(x - TA::kCopies, lane, b_pitch, last);
+                        if (x >= TA::kCopies) off[i] = TB::source(x - TA::kCopies, (int)lane_here(), b_pitch, last);
                     }
             }
 #pragma unroll
@@ -152,90 +211,117 @@ struct SplitProduct {
             }
         };
         fill(0);
+        if (kStages > 2 && n_slab > 1) fill(1);
         meanwhile();
-        const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
+#pragma unroll
+        for (int m = 0; m < AM; ++m)
+#pragma unroll
+            for (int n = 0; n < AN; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) big[m][n][r] = small[m][n][r] = 0.f;
+        const int wm = (wave / Tile::WN) * (Tile::TM / Tile::WM), wn = (wave % Tile::WN) * (Tile::TN / Tile::WN);
         for (int slab = 0; slab < n_slab; ++slab) {
-            wait_copies_and_barrier<0>();
-            if (slab + 1 < n_slab) fill(slab + 1);
-            const char* ta = smem + (slab & 1) * kStage;
+            // (a wave's copies arrive in order: all but the next slab's are there)
+            if (kStages > 2 && slab + 1 < n_slab) wait_copies_and_barrier<kEach>();
+            else wait_copies_and_barrier<0>();
+            if (slab + kStages - 1 < n_slab) fill(slab + kStages - 1);
+            if (!before(slab)) continue;
+            const char* ta = smem + slab % kStages * kStage;
             const char* tb = ta + TA::kBytes;
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
-                floatx4 fa[AM][3], fb[AN][3];
+                floatx4 fa[AM][2], fb[AN][2];
 #pragma unroll
-                for (int q = 0; q < 3; ++q) {
+                for (int q = 0; q < 2; ++q) {
 #pragma unroll
                     for (int m = 0; m < AM; ++m) fa[m][q] = TA::fragment(ta, q, wm + 32 * m, ks, lane);
 #pragma unroll
                     for (int n = 0; n < AN; ++n) fb[n][q] = TB::fragment(tb, q, wn + 32 * n, ks, lane);
                 }
-                // six products, smallest first; the accumulators in turn, so that an instruction
-                // does not wait for the one before it
-                constexpr int qa[6] = {0, 2, 1, 0, 1, 0}, qb[6] = {2, 0, 1, 1, 0, 0};
-#pragma unroll
-                for (int x = 0; x < 6; ++x)
-#pragma unroll
-                    for (int m = 0; m < AM; ++m)
-#pragma unroll
-                        for (int n = 0; n < AN; ++n)
-                            acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                                __builtin_bit_cast(bf16x8, fa[m][qa[x]]), __builtin_bit_cast(bf16x8, fb[n][qb[x]]),
-                                acc[m][n], 0, 0, 0);
+#define KGE_MM(acc_, qa_, qb_)                                                                                   \
+    _Pragma("unroll") for (int m = 0; m < AM; ++m) _Pragma("unroll") for (int n = 0; n < AN; ++n) acc_[m][n] =    \
+        __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fa[m][qa_]),                            \
+                                               __builtin_bit_cast(f16x8, fb[n][qb_]), acc_[m][n], 0, 0, 0)
+                KGE_MM(big, 0, 0);
+                KGE_MM(small, 0, 1);
+                KGE_MM(small, 1, 0);
+#undef KGE_MM
             }
         }
     }
 };
 
 // --------------------------------------------------------------------------
-// the coefficient matrix as pieces
+// the coefficient matrix as halves
 
 // A 32 x 32 block of coefficients in accumulator layout (register r of lane l: row
-// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32) to its place in the piece matrix, block corner
-// (m0, n0) of block d.  Neighbouring lanes swap values so that a lane stores two columns of one row as
-// one word.  For L2 also the block's row sums and column sums.
-template <int DIST>
-DEVINL void store_coef_block(const float (&c)[16], const SplitCoef& p, int d, int m0, int n0, int lane) {
+// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32) to its place in the matrix of halves, block corner
+// (m0, n0) of block d.  sa[r], sb: the scales of the rows and of the column.  The backward multiplies rows of
+// halves that lack their scales, the heads' on one side and the tails' on the other: a coefficient takes
+// both along, and the backward takes its own row's out of the finished sum.  The block's own scale is 2^exponent,
+// a multiple of four, so that the backward seldom meets another one in the next block; its largest comes to 2^11 at least, and
+// what is below 2^-25 of that (a softmax's e^-17) is off by 2^-47 of it at most.  Neighbouring lanes swap values
+// so that a lane stores two columns of one row as one word.  For L2 also the block's row sums and column sums.
+template <int DIST, class Scales>
+DEVINL void store_coef_block(float (&c)[16], Scales&& scale_of_row, float sb, const SplitCoef& p, int d, int m0, int n0, int lane) {
     const int Bp = p.Bp, Tp = p.Tp;
     if (m0 >= Bp || n0 >= Tp) return;
     const int cl = lane & 31, hl = lane >> 5;
-    const bool odd = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
-    char* const base = p.coefp + ((size_t)d * Bp + m0) * Tp * 6 + (size_t)(n0 >> 5) * 192 + (cl & ~1) * 2;
-    float s[8];
+    const bool odd = lane & 1;
+    if (DIST == DIST_L2) {
+        const bool b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
+        // row sums: at each step a lane keeps half of its rows and hands the other half's sums over
+        float s[8], t[4], u[2];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s[i] = (odd ? c[2 * i + 1] : c[2 * i]) + swap1(odd ? c[2 * i] : c[2 * i + 1]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) t[i] = (b1 ? s[2 * i + 1] : s[2 * i]) + swap2(b1 ? s[2 * i] : s[2 * i + 1]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) u[i] = (b2 ? t[2 * i + 1] : t[2 * i]) + __shfl_xor(b2 ? t[2 * i] : t[2 * i + 1], 4, 64);
+        float v = (b3 ? u[1] : u[0]) + __shfl_xor(b3 ? u[0] : u[1], 8, 64);
+        v += __shfl_xor(v, 16, 64);
+        const int r = lane & 15;
+        if (!(lane & 16))
+            p.rowpart[((size_t)d * Bp + m0 + 8 * (r >> 2) + 4 * hl + (r & 3)) * (Tp >> 5) + (n0 >> 5)] = v;
+        float col = 0.f;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) col += c[k];
+        col += __shfl_xor(col, 32, 64);
+        if (lane < 32) p.colpart[((size_t)d * (Bp >> 5) + (m0 >> 5)) * Tp + n0 + lane] = col;
+        __builtin_amdgcn_sched_barrier(0);  // (from here on no sums beside the coefficients)
+    }
+    float top = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        c[r] *= scale_of_row(r) * sb;
+        top = fmaxf(top, fabsf(c[r]));
+    }
+    const uint32_t bits = wave_max_bits(top);
+    const int exponent = min(max(((int)(bits >> 23) - 127 - 14 + 3) & ~3, -120), 120);
+    const float up = __uint_as_float((uint32_t)(127 - exponent) << 23);
+    if (lane == 0) p.exponent[((size_t)d * (Bp >> 5) + (m0 >> 5)) * (Tp >> 5) + (n0 >> 5)] = bits ? exponent : kNoExponent;
+    const int pitch = half_pitch(Tp);
+    char* const base = p.coefp + ((size_t)d * Bp + m0) * pitch + (size_t)(n0 >> 5) * kHalfBytes;
+    const uint32_t off = (uint32_t)((4 * hl + odd) * pitch + (cl & ~1) * 2);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
+        // row 2 i + odd of this lane's half
         const float got = swap1(odd ? c[2 * i] : c[2 * i + 1]);
-        const float x = odd ? got : c[2 * i], y = odd ? c[2 * i + 1] : got;  // row 2 i + odd of this lane's half
-        s[i] = x + y;
-        uint32_t w[3];
-        split2(x, y, w);
-        char* const q = base + (size_t)(8 * (i >> 1) + 4 * hl + 2 * (i & 1) + odd) * Tp * 6;
+        const float x = odd ? got : c[2 * i], y = odd ? c[2 * i + 1] : got;
+        uint32_t w[2];
+        split2_f16(x * up, y * up, w);
+        char* const q = base + (size_t)(8 * (i >> 1) + 2 * (i & 1)) * pitch;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) *reinterpret_cast<uint32_t*>(q + 64 * k) = w[k];
+        for (int k = 0; k < 2; ++k) *reinterpret_cast<uint32_t*>(q + off + 64 * k) = w[k];
     }
-    if (DIST != DIST_L2) return;
-    // row sums: at each step a lane keeps half of its rows and hands the other half's sums over
-    float t[4], u[2];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) t[i] = (b1 ? s[2 * i + 1] : s[2 * i]) + swap2(b1 ? s[2 * i] : s[2 * i + 1]);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) u[i] = (b2 ? t[2 * i + 1] : t[2 * i]) + __shfl_xor(b2 ? t[2 * i] : t[2 * i + 1], 4, 64);
-    float v = (b3 ? u[1] : u[0]) + __shfl_xor(b3 ? u[0] : u[1], 8, 64);
-    v += __shfl_xor(v, 16, 64);
-    const int r = lane & 15;
-    if (!(lane & 16))
-        p.rowpart[((size_t)d * Bp + m0 + 8 * (r >> 2) + 4 * hl + (r & 3)) * (Tp >> 5) + (n0 >> 5)] = v;
-    float col = 0.f;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) col += c[k];
-    col += __shfl_xor(col, 32, 64);
-    if (lane < 32) p.colpart[((size_t)d * (Bp >> 5) + (m0 >> 5)) * Tp + n0 + lane] = col;
 }
 
 // The same from float32 coefficients in memory (the losses that are formed row by row): one wave
 // per 32 x 32 block.
 template <int DIST>
-__global__ __launch_bounds__(256) void k_coef_pieces(ScoreShape sh, const float* __restrict__ coef,
-                                                     const uint32_t* __restrict__ nearflag, SplitCoef p) {
+__global__ __launch_bounds__(256) void k_coef_halves(ScoreShape sh, const float* __restrict__ coef,
+                                                     const uint32_t* __restrict__ nearflag, const float* __restrict__ scale,
+                                                     int n_head, SplitCoef p) {
     const int lane = threadIdx.x & 63, MT = p.Bp >> 5, NT = p.Tp >> 5;
     const int g = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int d = g / (MT * NT), mt = (g - d * MT * NT) / NT, nt = g % NT;
@@ -243,67 +329,68 @@ __global__ __launch_bounds__(256) void k_coef_pieces(ScoreShape sh, const float*
     const float* src = coef + (size_t)d * sh.B * sh.T;
     const bool skip = DIST == DIST_L2 && nearflag[((size_t)d * MT + mt) * NT + nt] != 0u;  // direct form
     const int n = 32 * nt + (lane & 31);
-    float c[16];
+    const float sb = scale[n_head + d * sh.T + n];
+    float c[16], sa[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int m = 32 * mt + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        sa[r] = scale[d * sh.B + m];
         c[r] = (!skip && m < sh.B && n < sh.T) ? src[(size_t)m * sh.T + n] : 0.f;
     }
-    store_coef_block<DIST>(c, p, d, 32 * mt, 32 * nt, lane);
+    store_coef_block<DIST>(c, [&](int r) { return sa[r]; }, sb, p, d, 32 * mt, 32 * nt, lane);
 }
 
 // --------------------------------------------------------------------------
 // forward
 
 // (kCancelRatio, kNearRatio: kge_loss.h)
-template <int DIST, int OM>
-__global__ __launch_bounds__(kWaves * kWaves * 64, 2) void k_split_fwd(SplitFwd p) {
-    constexpr int TM = kTile, TN = kTile, WM = kWaves, WN = kWaves;
-    using P = SplitProduct<RowTile<TM>, RowTile<TN>, TM, TN, WM, WN>;
+template <int DIST, int OM, class Tile>
+__global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(Tile::EU, Tile::EU))) void k_split_fwd(SplitFwd p) {
+    constexpr int TM = Tile::TM, TN = Tile::TN, WM = Tile::WM, WN = Tile::WN;
+    using P = SplitProduct<RowTile<TM, 2>, RowTile<TN, 2>, Tile>;
     __shared__ __attribute__((aligned(16))) char smem[P::kLds];
-    __shared__ float na_s[TM], nb_s[TN], mult_s[TN], red[WM * WN];
+    __shared__ float na_s[TM], nb_s[TN], sa_s[TM], sb_s[TN], mult_s[TN], red[WM * WN];
     __shared__ uint32_t label_s[TM];
+    __shared__ int n_redo;
     const ScoreShape& sh = p.sh;
-    const int B = sh.B, T = sh.T, Kp = p.Kp;
+    const int B = sh.B, T = sh.T, Kp = p.rows.Kp;
     const TileId tile = xcd_tile((T + TN - 1) / TN, (B + TM - 1) / TM, sh.S);
     const int d = tile.z, m0 = tile.y * TM, n0 = tile.x * TN;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tid = threadIdx.x, lane = tid & 63;
     const int t_live = tail_limit(sh.tcount, d, T, sh.tpad);
     if (n0 >= t_live) {  // merged tails: the block has no such column
         if (OM == 0 && tid == 0) p.loss_part[(size_t)d * (tile.gx * tile.gy) + tile.y * tile.gx + tile.x] = 0.f;
         return;
     }
     const int n_live = sh.tcount ? (int)sh.tcount[d] : T;
-    const int a_row = d * B, b_row = p.b_c0 + d * T;
-    const int pitch = Kp * 6;
-    const char* a = p.rows + (int64_t)(a_row + m0) * pitch;
-    const char* b = p.rows + (int64_t)(b_row + n0) * pitch;
-    floatx16 acc[P::AM][P::AN];
-#pragma unroll
-    for (int m = 0; m < P::AM; ++m)
-#pragma unroll
-        for (int n = 0; n < P::AN; ++n)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
-    P::run(smem, a, pitch, 192, b, pitch, 192, Kp / 32, 0, acc, lane, wave, [&]() __attribute__((always_inline)) {
-        for (int i = tid; i < TM; i += WM * WN * 64) {
-            if (DIST == DIST_L2) na_s[i] = p.norm[a_row + m0 + i];
+    const int a_row = d * B, b_row = p.rows.n_head + d * T;
+    const int pitch = half_pitch(Kp);
+    const char* a = p.rows.halves + (int64_t)(a_row + m0) * pitch;
+    const char* b = p.rows.halves + (int64_t)(b_row + n0) * pitch;
+    floatx16 big[P::AM][P::AN], small[P::AM][P::AN];
+    P::run(smem, a, pitch, kHalfBytes, b, pitch, kHalfBytes, Kp / 32, 0, big, small, lane, wave, [&]() __attribute__((always_inline)) {
+        for (int i = tid; i < TM; i += Tile::threads) {
+            if (DIST == DIST_L2) na_s[i] = p.rows.norm[a_row + m0 + i];
+            sa_s[i] = m0 + i < B ? p.rows.scale[a_row + m0 + i] : 0.f;  // (no row that counts has scale 0)
             if (OM == 0) label_s[i] = m0 + i < B ? p.clabel[d * B + m0 + i] : 0u;
         }
-        if (DIST == DIST_L2)
-            for (int i = tid; i < TN; i += WM * WN * 64) nb_s[i] = p.norm[b_row + n0 + i];
-        if (OM == 0)
-            for (int i = tid; i < TN; i += WM * WN * 64)
-                mult_s[i] = n0 + i < T ? (sh.tmult ? sh.tmult[(size_t)d * T + n0 + i] : 1.f) : 0.f;
-    });
+        for (int i = tid; i < TN; i += Tile::threads) {
+            if (DIST == DIST_L2) nb_s[i] = p.rows.norm[b_row + n0 + i];
+            sb_s[i] = n0 + i < T ? p.rows.scale[b_row + n0 + i] : 0.f;
+            if (OM == 0) mult_s[i] = n0 + i < T ? (sh.tmult ? sh.tmult[(size_t)d * T + n0 + i] : 1.f) : 0.f;
+        }
+    }, [](int) { return true; });
 
     // epilogue.  Register r of lane l holds row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
     const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
-    const int cl = lane & 31, hl = lane >> 5;
+    const int lane1 = (int)lane_here(), tid1 = 64 * wave + lane1, cl = lane1 & 31, hl = lane1 >> 5;
     const float Tn = (float)T;
     const float w_pos = uniform_f32(0.5f * Tn), w_neg = uniform_f32((0.5f * Tn) / (float)(T - 1));
     const float inv_norm = uniform_f32(1.f / ((float)sh.S * (float)B * Tn));
-    const float grad_scale = uniform_f32(inv_norm * sh.loss_scale);
+    // score = base + sign * (distance or product); a coefficient is sign * dL/dscore
+    const bool plain = score_is_distance_value(sh.score_fn);
+    const float score_sign = plain ? 1.f : -1.f, score_base = plain ? 0.f : sh.gamma;
+    const float coef_scale = uniform_f32(inv_norm * sh.loss_scale * score_sign);
     const int Bp = p.out.Bp, Tp = p.out.Tp, MT = Bp >> 5, NT = Tp >> 5;
     float loss_acc = 0.f;
 #pragma unroll
@@ -315,78 +402,84 @@ __global__ __launch_bounds__(kWaves * kWaves * 64, 2) void k_split_fwd(SplitFwd 
             // columns behind a block's distinct tails repeat its first row, the most popular one more
             // often than not: no pair of theirs is worth a second look
             const bool col_counts = n < n_live;
+            const float sb = sb_s[nbk + cl];
             float val[16];
-            uint32_t cancel = 0u, near = 0u;
+            const float* const sa = sa_s + mb + 4 * hl;
+            auto scale_a = [&](int r) __attribute__((always_inline)) { return sa[8 * (r >> 2) + (r & 3)]; };
+            const float nb = DIST == DIST_L2 ? nb_s[nbk + cl] : 0.f;
+            const float* const na = na_s + mb + 4 * hl;
+            auto norms = [&](int r) __attribute__((always_inline)) { return na[8 * (r >> 2) + (r & 3)] + nb; };
+            uint64_t redo = 0u;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                val[r] = acc[mi][ni][r];
-                const int m_loc = mb + 8 * (r >> 2) + 4 * hl + (r & 3);
-                const bool live = col_counts && m0 + m_loc < B;
-                bool good = fabsf(val[r]) < INFINITY;  // (dot)
+                const float product = fmaf(small[mi][ni][r], kHalfStep, big[mi][ni][r]);
                 if (DIST == DIST_L2) {
-                    const float ns = na_s[m_loc] + nb_s[nbk + cl];
-                    val[r] = ns - 2.f * val[r];
-                    good = val[r] >= kCancelRatio * ns;
-                    if (live && val[r] < kNearRatio * ns) near |= 1u << r;
+                    const float ns = norms(r);
+                    val[r] = fmaf(product, -2.f * sb * scale_a(r), ns);
+                    redo |= __ballot(!(val[r] > kCancelRatio * ns));
+                } else {
+                    val[r] = product * scale_a(r) * sb;
+                    redo |= __ballot(!(fabsf(val[r]) < INFINITY));
                 }
-                if (!good) cancel |= 1u << r;
             }
-            // rare: the wave recomputes pairs directly, two pairs of each of two lanes at a time, sixteen
-            // lanes to a pair: those that cancelled, and those that are not finite (an infinity's second
-            // piece is NaN).  Pairs that do not count, a NaN among them, get any finite value.
-            if (__ballot(cancel != 0u)) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (!(col_counts && m0 + mb + 8 * (r >> 2) + 4 * hl + (r & 3) < B)) {
-                        val[r] = 0.f;
-                        cancel &= ~(1u << r);
-                    }
-                near = 0u;
-                uint32_t left = cancel;
-                uint64_t owners;
-                while ((owners = __ballot(left != 0u)) != 0) {
-                    const int l0 = __ffsll((long long)owners) - 1;
-                    const uint64_t rest = owners & (owners - 1);
-                    const int l1 = rest ? __ffsll((long long)rest) - 1 : l0;
-                    const int src = lane & 32 ? l1 : l0;
-                    const uint32_t bits = __shfl(left, src, 64), upper = bits & (bits - 1);
-                    const int fr = __ffs((int)((lane & 16) && upper ? upper : bits)) - 1;
-                    const char* ar = a + (int64_t)(mb + 8 * (fr >> 2) + 4 * (src >> 5) + (fr & 3)) * pitch;
-                    const char* br = b + (int64_t)(nbk + (src & 31)) * pitch;
-                    float part = 0.f;
-                    for (int k = (lane & 15) * 4; k < Kp; k += 64) {
-                        const float4 x = load_pieces4(ar, k), y = load_pieces4(br, k);
-                        if (DIST == DIST_L2) {
-                            const float dx = x.x - y.x, dy = x.y - y.y, dz = x.z - y.z, dw = x.w - y.w;
-                            part += dx * dx + dy * dy + dz * dz + dw * dw;
-                        } else {
-                            part += x.x * y.x + x.y * y.y + x.z * y.z + x.w * y.w;
-                        }
-                    }
-#pragma unroll
-                    for (int o = 8; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
-                    const int at = (lane == l0) ? 0 : 32;
-                    const float v0 = __shfl(part, at, 64), v1 = __shfl(part, at + 16, 64);
-                    if (lane == l0 || lane == l1) {
-                        const uint32_t up = left & (left - 1);
-                        const uint32_t b0 = left ^ up, b1 = up & (0u - up);
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            if ((b0 >> r) & 1u) val[r] = v0;
-                            if ((b1 >> r) & 1u) val[r] = v1;
-                        }
-                        left = up & (up - 1);
-                    }
-                }
+            bool flagged = false;
+            // rare: pairs are recomputed directly, half a wave to a pair, by all of the workgroup (a popular row's
+            // come together in one wave's block): those that cancelled, and those that are not finite (an infinity's
+            // second half is NaN).  Pairs that do not count, a NaN among them, get any finite value.
+            static_assert(P::AM == 1 && P::AN == 1, "one block to a wave");
+            if (__syncthreads_or(redo != 0u)) {
+                float* const result = reinterpret_cast<float*>(smem);  // [TM][TN]; the tiles are no longer needed
+                uint16_t* const list = reinterpret_cast<uint16_t*>(smem + TM * TN * 4);
+                static_assert(TM * TN * 6 <= P::kLds, "the tile's pairs as a list and as results");
+                if (tid1 == 0) n_redo = 0;
+                __syncthreads();
+                uint32_t cancel = 0u, near = 0u;
+                const int at = (mb + 4 * hl) * TN + nbk + cl;  // of register 0
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int m_loc = mb + 8 * (r >> 2) + 4 * hl + (r & 3);
-                    if (DIST == DIST_L2 && col_counts && m0 + m_loc < B && val[r] < kNearRatio * (na_s[m_loc] + nb_s[nbk + cl]))
-                        near |= 1u << r;
+                    const bool live = col_counts && scale_a(r) != 0.f;
+                    if (!live) val[r] = 0.f;
+                    else if (DIST == DIST_L2 ? !(val[r] > kCancelRatio * norms(r)) : !(fabsf(val[r]) < INFINITY)) cancel |= 1u << r;
+                    result[at + (8 * (r >> 2) + (r & 3)) * TN] = val[r];  // (their registers are wanted meanwhile)
                 }
+                for (uint32_t left = cancel; left; left &= left - 1) {
+                    const int r = __ffs((int)left) - 1;
+                    list[atomicAdd(&n_redo, 1)] = (uint16_t)(at + (8 * (r >> 2) + (r & 3)) * TN);
+                }
+                __syncthreads();
+#pragma unroll 1
+                for (int q = tid1 >> 5; q < n_redo; q += Tile::threads / 32) {
+                    const int pos = list[q];
+                    float part = 0.f;
+#pragma unroll 1
+                    for (int k = (lane1 & 31) * 8; k < Kp; k += 256) {
+                        Row8 x, y;
+                        x.load(p.rows, a_row + m0 + pos / TN, k);
+                        y.load(p.rows, b_row + n0 + pos % TN, k);
+                        static_for<8>([&](auto I) {
+                            const float u = x.template value<I>(), v = y.template value<I>();
+                            part = DIST == DIST_L2 ? fmaf(u - v, u - v, part) : fmaf(u, v, part);
+                        });
+                    }
+                    part += swap1(part);
+                    part += swap2(part);
+                    part += mirror8(part);
+                    part += mirror16(part);
+                    part += __shfl_xor(part, 16, 64);
+                    if ((lane1 & 31) == 0) result[pos] = part;
+                }
+                __syncthreads();
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    val[r] = result[at + (8 * (r >> 2) + (r & 3)) * TN];
+                    if (DIST == DIST_L2 && ((cancel >> r) & 1u) && val[r] < kNearRatio * norms(r)) near |= 1u << r;
+                }
+                flagged = DIST == DIST_L2 && __ballot(near != 0u) != 0;
+                if (OM == 0)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) loss_acc += val[r] - val[r];  // a pair that is not finite shows in the loss
             }
-            const bool flagged = DIST == DIST_L2 && __ballot(near != 0u) != 0;
-            if (DIST == DIST_L2 && p.nearflag && lane == 0 && m0 + mb < Bp && n0 + nbk < Tp)
+            if (DIST == DIST_L2 && p.nearflag && lane1 == 0 && m0 + mb < Bp && n0 + nbk < Tp)
                 p.nearflag[((size_t)d * MT + ((m0 + mb) >> 5)) * NT + ((n0 + nbk) >> 5)] = flagged ? 1u : 0u;
             if (OM != 0) {  // raw scores (and distances)
                 float* const out = p.coef + (size_t)d * B * T;
@@ -402,37 +495,48 @@ __global__ __launch_bounds__(kWaves * kWaves * 64, 2) void k_split_fwd(SplitFwd 
                 }
                 continue;
             }
-            const float mult = mult_s[nbk + cl];
+            // a column's negatives: mult of them, or one less where one is the row's label (src/poplar_kge.cpp:615-636)
+            const float mult = mult_s[nbk + cl], w_all = mult * w_neg, w_less = (mult - 1.f) * w_neg;
+            const bool whole = m0 + mb + 32 <= B && n0 + nbk + 32 <= T;
+            const uint32_t* const label = label_s + mb + 4 * hl;
             float c[16];
+            asm volatile("" ::: "memory");  // what stands in LDS is read again, not kept in registers
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int m_loc = mb + 8 * (r >> 2) + 4 * hl + (r & 3);
-                const bool live = m0 + m_loc < B && n < T;
                 const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[r]) : val[r];  // (never negative; a NaN stays one)
-                const float score = score_is_distance_value(sh.score_fn) ? dist : sh.gamma - dist;
-                float ds;
-                const float term = logsigmoid_column(score, (uint32_t)n == label_s[m_loc], mult, w_pos, w_neg, grad_scale, ds);
-                if (live) loss_acc += term;
-                float v = score_is_distance_value(sh.score_fn) ? ds : -ds;
+                const float score = fmaf(dist, score_sign, score_base);
+                const bool pos = (uint32_t)n == label[8 * (r >> 2) + (r & 3)];
+                LogSigmoid z(score);
+                const float w = pos ? w_less : w_all;
+                float term = -(w * z.minus_value()), ds = w * z.minus_grad();
+                if (__ballot(pos)) {  // one pair of a positive's row
+                    term -= pos ? w_pos * z.plus_value() : 0.f;
+                    ds -= pos ? w_pos * z.plus_grad() : 0.f;
+                }
+                float v = ds * coef_scale;
                 if (DIST == DIST_L2) v = dist != 0.f ? v * __builtin_amdgcn_rcpf(dist) : 0.f;
-                c[r] = live ? v : 0.f;
+                if (!whole && !(scale_a(r) != 0.f && sb != 0.f)) term = v = 0.f;
+                loss_acc += term;
+                c[r] = v;
+                if ((r & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // no more rows' intermediate values at once
             }
             if (flagged) {  // the backward takes this block in the direct form, from the coefficients as they are
-                float* const out = p.coef + (size_t)d * B * T;
+                char* const out = (char*)(p.coef + ((size_t)d * B + m0 + mb) * T + n0 + nbk);
+                const uint32_t off = (uint32_t)(4 * hl * T + cl) * 4;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + mb + 8 * (r >> 2) + 4 * hl + (r & 3);
-                    if (m < B && n < T) out[(size_t)m * T + n] = c[r];
+                    if (scale_a(r) != 0.f && sb != 0.f) *reinterpret_cast<float*>(out + (size_t)(8 * (r >> 2) + (r & 3)) * T * 4 + off) = c[r];
                     c[r] = 0.f;
                 }
             }
-            store_coef_block<DIST>(c, p.out, d, m0 + mb, n0 + nbk, lane);
+            asm volatile("" ::: "memory");
+            store_coef_block<DIST>(c, scale_a, sb, p.out, d, m0 + mb, n0 + nbk, lane1);
         }
     if (OM == 0) {
         loss_acc = wave_sum(loss_acc);
-        if (lane == 0) red[wave] = loss_acc;
+        if (lane1 == 0) red[wave] = loss_acc;
         __syncthreads();
-        if (tid == 0) {
+        if (tid1 == 0) {
             float tot = 0.f;
 #pragma unroll
             for (int w = 0; w < WM * WN; ++w) tot += red[w];
@@ -446,184 +550,276 @@ __global__ __launch_bounds__(kWaves * kWaves * 64, 2) void k_split_fwd(SplitFwd 
 // (L2: self[i, k] sum_j c[i, j] - the product).  Head side: i = heads, the coefficient rows lie along
 // the contraction.  Tail side: i = tails, they lie across it.  `other` always lies across it.
 
-template <int DIST, bool SIDE_B>
-DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, char* smem, float* csum_s) {
-    constexpr int TM = kTile, TN = kTile, WM = kWaves, WN = kWaves;
-    using TA = std::conditional_t<SIDE_B, ColTile<TM>, RowTile<TM>>;
-    using P = SplitProduct<TA, ColTile<TN>, TM, TN, WM, WN>;
+template <int DIST, bool SIDE_B, class Tile>
+DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, char* smem, float* csum_s, float* scale_s) {
+    constexpr int TM = Tile::TM, TN = Tile::TN, WM = Tile::WM, WN = Tile::WN, kSums = Tile::threads / TM;
+    using TA = std::conditional_t<SIDE_B, ColTile<TM, 2>, RowTile<TM, 2>>;
+    using P = SplitProduct<TA, ColTile<TN, 2>, Tile>;
     const int i0 = tile_y * TM, kt0 = tile_x * TN;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int B = p.B, T = p.T, Bp = p.in.Bp, Tp = p.in.Tp, MT = Bp >> 5, NT = Tp >> 5, pitch = p.Kp * 6;
+    const int B = p.B, T = p.T, Dp = p.rows.Dp, Kp = p.rows.Kp, Bp = p.in.Bp, Tp = p.in.Tp, MT = Bp >> 5, NT = Tp >> 5, pitch = half_pitch(Kp);
     const int t_live = tail_limit(p.tcount, d, T, p.tpad);  // merged tails: the block's live columns
     const int n_self = SIDE_B ? t_live : B, n_other = SIDE_B ? B : t_live, n_slab = (n_other + 31) >> 5;
     if (i0 >= n_self) return;
-    const int head0 = d * B, tail0 = p.b_c0 + d * T, self0 = SIDE_B ? tail0 : head0, other0 = SIDE_B ? head0 : tail0;
-    const char* const coef = p.in.coefp + (size_t)d * Bp * Tp * 6;
-    const char* const a = SIDE_B ? coef + (size_t)(i0 >> 5) * 192 : coef + (size_t)i0 * Tp * 6;
-    const char* const other = p.rows + (int64_t)other0 * pitch;
-    const char* const b = other + (size_t)(kt0 >> 5) * 192;
+    const int head0 = d * B, tail0 = p.rows.n_head + d * T, self0 = SIDE_B ? tail0 : head0, other0 = SIDE_B ? head0 : tail0;
+    const int coef_pitch = half_pitch(Tp);
+    const char* const coef = p.in.coefp + (size_t)d * Bp * coef_pitch;
+    const char* const a = SIDE_B ? coef + (size_t)(i0 >> 5) * kHalfBytes : coef + (size_t)i0 * coef_pitch;
+    const char* const b = p.rows.halves + (int64_t)other0 * pitch + (size_t)(kt0 >> 5) * kHalfBytes;
     const uint32_t* const nflag = DIST == DIST_L2 ? p.nearflag + (size_t)d * MT * NT : nullptr;
-    floatx16 acc[P::AM][P::AN];
-#pragma unroll
-    for (int m = 0; m < P::AM; ++m)
-#pragma unroll
-        for (int n = 0; n < P::AN; ++n)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
-    uint32_t seen = 0u;  // flagged blocks among the tile's
-    P::run(smem, a, Tp * 6, SIDE_B ? (size_t)32 * Tp * 6 : 192, b, pitch, (size_t)32 * pitch, n_slab, n_other, acc, lane, wave,
-           [&]() __attribute__((always_inline)) {
-               if (DIST != DIST_L2) return;
-               // the self rows' coefficient sums, from the sub-blocks' in a fixed order
-               for (int i = tid; i < TM; i += WM * WN * 64) {
-                   float s = 0.f;
-                   if (SIDE_B) {
-                       if (i0 + i < Tp)
-                           for (int q = 0; q < MT; ++q) s += p.in.colpart[((size_t)d * MT + q) * Tp + i0 + i];
-                   } else if (i0 + i < Bp) {
-                       for (int q = 0; q < n_slab; ++q) s += p.in.rowpart[((size_t)d * Bp + i0 + i) * NT + q];
-                   }
-                   csum_s[i] = s;
-               }
-               for (int x = tid; x < TM / 32 * n_slab; x += WM * WN * 64) {
-                   const int st = (i0 >> 5) + x / n_slab, ot = x % n_slab;
-                   if (SIDE_B ? st < NT : st < MT) seen |= SIDE_B ? nflag[(size_t)ot * NT + st] : nflag[(size_t)st * NT + ot];
-               }
-           });
     const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
-    const int cl = lane & 31, hl = lane >> 5;
-    const char* const self = p.rows + (int64_t)(self0 + i0) * pitch;
-    if (DIST == DIST_L2 && __syncthreads_or(seen != 0u)) {
-        // slabs in which some pair of a sub-block is nearly identical: c (self - other) directly, as
-        // the reference codelet does (their coefficients went into the product as zeros; acc holds
-        // the negated sum)
-        const float* const cf = p.coef + (size_t)d * B * T;
+    // a sub-block's exponent: of the self rows' group st and of slab ot
+    const int* const exps = p.in.exponent + (size_t)d * MT * NT;
+    const int st0 = (i0 + wm) >> 5, st_last = (SIDE_B ? NT : MT) - 1;
+    int exp_reg[P::AM], exp_now[P::AM];  // of slab 64 n + lane; what the accumulators are in
+    auto load_exps = [&](int slab0) __attribute__((always_inline)) {
+        const int ot = min(slab0 + lane, n_slab - 1);
 #pragma unroll
-        for (int mi = 0; mi < P::AM; ++mi)
-            for (int ot = 0; ot < n_slab; ++ot) {
-                const int st = (i0 + wm + 32 * mi) >> 5;
-                if (st >= (SIDE_B ? NT : MT)) continue;
-                if ((SIDE_B ? nflag[(size_t)ot * NT + st] : nflag[(size_t)st * NT + ot]) == 0u) continue;
+        for (int m = 0; m < P::AM; ++m) {
+            const int st = min(st0 + m, st_last);  // (rows past the last are dropped)
+            exp_reg[m] = exps[SIDE_B ? (size_t)ot * NT + st : (size_t)st * NT + ot];
+        }
+    };
+    floatx16 big[P::AM][P::AN], small[P::AM][P::AN];
+    bool seen = false;  // a flagged block among the tile's (the wave's share of them)
+    exp_now[0] = 0;
+    P::run(smem, a, coef_pitch, SIDE_B ? (size_t)32 * coef_pitch : kHalfBytes, b, pitch, (size_t)32 * pitch, n_slab, n_other, big, small, lane, wave,
+           [&]() __attribute__((always_inline)) {
+               load_exps(0);
+               if (tid < TM) scale_s[tid] = p.rows.scale[self0 + i0 + tid];
+               if (DIST != DIST_L2) return;
+               // the self rows' coefficient sums, from the sub-blocks' in a fixed order: kSums threads to a row, four
+               // loads of each under way
+               const int i = tid % TM, n = SIDE_B ? MT : n_slab;
+               if (i0 + i < (SIDE_B ? Tp : Bp)) {
+                   const float* part = SIDE_B ? p.in.colpart + (size_t)d * MT * Tp + i0 + i : p.in.rowpart + ((size_t)d * Bp + i0 + i) * NT;
+                   const size_t step = SIDE_B ? Tp : 1;
+                   float s = 0.f;
+                   for (int q = tid / TM; q < n; q += 4 * kSums) {
+                       float v[4];
 #pragma unroll
-                for (int ni = 0; ni < P::AN; ++ni) {
-                    const int k = kt0 + wn + 32 * ni + cl;
-                    if (kt0 + wn + 32 * ni >= p.Kp) continue;
-                    float sv[16];
+                       for (int x = 0; x < 4; ++x) v[x] = q + x * kSums < n ? part[(q + x * kSums) * step] : 0.f;
+                       s += (v[0] + v[1]) + (v[2] + v[3]);
+                   }
+                   csum_s[tid] = s;
+               } else {
+                   csum_s[tid] = 0.f;
+               }
+               uint32_t flags = 0u;
+               for (int x = tid; x < TM / 32 * n_slab; x += Tile::threads) {
+                   const int st = (i0 >> 5) + x / n_slab, ot = x % n_slab;
+                   if (SIDE_B ? st < NT : st < MT) flags |= SIDE_B ? nflag[(size_t)ot * NT + st] : nflag[(size_t)st * NT + ot];
+               }
+               seen = __ballot(flags != 0u) != 0u;
+           },
+           [&](int slab) __attribute__((always_inline)) {
+               if (slab && !(slab & 63)) load_exps(slab);
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        sv[r] = load_piece1(self + (int64_t)(wm + 32 * mi + 8 * (r >> 2) + 4 * hl + (r & 3)) * pitch, k);
-                    for (int j = 32 * ot; j < min(32 * ot + 32, n_other); ++j) {
-                        const float o = load_piece1(other + (int64_t)j * pitch, k);
+               for (int m = 0; m < P::AM; ++m) {
+                   const int e = __builtin_amdgcn_readlane(exp_reg[m], slab & 63);
+                   if (e != exp_now[m] && e != kNoExponent) {  // seldom: what is there is brought to the slab's scale
+                       // (a slab 2^80 below what is there counts for nothing, and that would not fit its scale)
+                       static_assert(P::AM == 1, "one exponent to a wave's slab");
+                       if (exp_now[m] - e > 80) return false;
+                       const float by = __uint_as_float((uint32_t)(127 + max(exp_now[m] - e, -126)) << 23);
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            const int i = i0 + wm + 32 * mi + 8 * (r >> 2) + 4 * hl + (r & 3);
-                            const float c = i < n_self ? (SIDE_B ? cf[(size_t)j * T + i] : cf[(size_t)i * T + j]) : 0.f;
-                            acc[mi][ni][r] = fmaf(-c, sv[r] - o, acc[mi][ni][r]);
-                        }
-                    }
-                }
-            }
+                       for (int n = 0; n < P::AN; ++n)
+#pragma unroll
+                           for (int r = 0; r < 16; ++r) {
+                               big[m][n][r] *= by;
+                               small[m][n][r] *= by;
+                           }
+                       exp_now[m] = e;
+                   }
+               }
+               return true;
+           });
+    const int lane1 = (int)lane_here(), cl = lane1 & 31, hl = lane1 >> 5;
+    // the self rows' own scales leave the sums
+#pragma unroll
+    for (int m = 0; m < P::AM; ++m) {
+        const float scale = __uint_as_float((uint32_t)(127 + exp_now[m]) << 23);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float up = pow2_inverse(scale_s[wm + 32 * m + 8 * (r >> 2) + 4 * hl + (r & 3)]);
+#pragma unroll
+            for (int n = 0; n < P::AN; ++n) big[m][n][r] = fmaf(small[m][n][r], kHalfStep, big[m][n][r]) * scale * up;
+        }
     }
+    const char* const self = p.rows.halves + (int64_t)(self0 + i0) * pitch;
     // neighbouring lanes swap values: a lane stores two columns of one row
-    const bool odd = lane & 1;
-    float* const out = p.grad + (size_t)(self0 + i0) * p.Dp;
+    const bool odd = lane1 & 1;
+    float* const out = p.grad + (size_t)(self0 + i0) * Dp;
 #pragma unroll
     for (int mi = 0; mi < P::AM; ++mi)
 #pragma unroll
         for (int ni = 0; ni < P::AN; ++ni) {
             const int k = kt0 + wn + 32 * ni + (cl & ~1);
-            if (k >= p.Dp) continue;
-            const char* const sp = self + (size_t)(k >> 5) * 192 + (k & 31) * 2;
+            if (k >= Dp) continue;
+            // (a row: the wave's part, in scalars, and the lane's, in one offset for all of them)
+            const uint32_t in_off = (uint32_t)((4 * hl + odd) * pitch + (k >> 5) * kHalfBytes + (k & 31) * 2);
+            const uint32_t lost_off = (uint32_t)((4 * hl + odd) * (Kp >> 5) + (k >> 5)) * 4;
+            const uint32_t out_off = (uint32_t)((4 * hl + odd) * Dp + k) * 4;
+            auto wave_row = [&](int i) __attribute__((always_inline)) { return wm + 32 * mi + 8 * (i >> 1) + 2 * (i & 1); };
             uint32_t w[DIST == DIST_L2 ? 8 : 1][3];
             if (DIST == DIST_L2)
 #pragma unroll
-                for (int i = 0; i < 8; ++i)  // all loads before any use, rows past the last among them
+                for (int i = 0; i < 8; ++i) {  // all loads before any use, rows past the last among them
+                    const char* const row = self + (int64_t)wave_row(i) * pitch;
 #pragma unroll
-                    for (int q = 0; q < 3; ++q)
-                        w[i][q] = *reinterpret_cast<const uint32_t*>(
-                            sp + (int64_t)(wm + 32 * mi + 8 * (i >> 1) + 4 * hl + 2 * (i & 1) + odd) * pitch + 64 * q);
+                    for (int q = 0; q < 2; ++q) w[i][q] = *reinterpret_cast<const uint32_t*>(row + in_off + 64 * q);
+                    w[i][2] = *reinterpret_cast<const uint32_t*>((const char*)(p.rows.lost + (int64_t)(self0 + i0 + wave_row(i)) * (Kp >> 5)) + lost_off);
+                }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float got = swap1(odd ? acc[mi][ni][2 * i] : acc[mi][ni][2 * i + 1]);
-                float x = odd ? got : acc[mi][ni][2 * i], y = odd ? acc[mi][ni][2 * i + 1] : got;
-                const int row = wm + 32 * mi + 8 * (i >> 1) + 4 * hl + 2 * (i & 1) + odd;
+                const float got = swap1(odd ? big[mi][ni][2 * i] : big[mi][ni][2 * i + 1]);
+                float x = odd ? got : big[mi][ni][2 * i], y = odd ? big[mi][ni][2 * i + 1] : got;
+                const int row = wave_row(i) + 4 * hl + odd;
                 if (DIST == DIST_L2) {
-                    float sx = 0.f, sy = 0.f;
+                    const f16x2 h = __builtin_bit_cast(f16x2, w[i][0]), l = __builtin_bit_cast(f16x2, w[i][1]);
+                    float sum = csum_s[row];
 #pragma unroll
-                    for (int q = 0; q < 3; ++q) { sx += bf16_lo_f32(w[i][q]); sy += bf16_hi_f32(w[i][q]); }
-                    x = sx * csum_s[row] - x;
-                    y = sy * csum_s[row] - y;
+                    for (int q = 1; q < kSums; ++q) sum += csum_s[row + q * TM];
+                    sum *= scale_s[row];
+                    // (every bit of the self row: against this product the other one is small)
+                    const uint32_t lost = w[i][2] >> lost_at(k);
+                    x = join_lost(h.x, l.x, lost & 1u) * sum - x;
+                    y = join_lost(h.y, l.y, (lost >> 8) & 1u) * sum - y;
                 }
-                if (i0 + row < n_self) *reinterpret_cast<float2*>(out + (size_t)row * p.Dp + k) = make_float2(x, y);
+                if (i0 + row < n_self) *reinterpret_cast<float2*>((char*)(out + (size_t)wave_row(i) * Dp) + out_off) = make_float2(x, y);
             }
         }
+    if (DIST != DIST_L2 || !__syncthreads_or(seen)) return;
+    __syncthreads();
+    // sub-blocks in which some pair is nearly identical: c (self - other) directly, as the reference codelet
+    // does (their coefficients went into the product as zeros), added to what the workgroup has just
+    // stored.  A wave takes four rows at a time, a lane a column.
+    static_assert(TN == 64, "a lane per column");
+    const float* const cf = p.coef + (size_t)d * B * T;
+    const int k = kt0 + (int)lane_here();
+    if (k >= Dp) return;
+    for (int i = i0 + 4 * wave; i < min(i0 + TM, n_self); i += 4 * WM * WN) {
+        float add[4] = {0.f, 0.f, 0.f, 0.f};
+        int row[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) row[x] = min(i + x, n_self - 1);
+        bool any = false;
+        for (int ot = 0; ot < n_slab; ++ot) {
+            if (nflag[SIDE_B ? (size_t)ot * NT + (i >> 5) : (size_t)(i >> 5) * NT + ot] == 0u) continue;
+            any = true;
+            float sv[4];
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                Row1 raw;
+                raw.load(p.rows, self0 + row[x], k);
+                sv[x] = raw.value(k);
+            }
+#pragma unroll 1
+            for (int j0 = 32 * ot; j0 < min(32 * ot + 32, n_other); j0 += 4) {
+                Row1 raw[4];
+                float c[4][4];
+#pragma unroll
+                for (int y = 0; y < 4; ++y) {
+                    const int j = min(j0 + y, n_other - 1);
+                    raw[y].load(p.rows, other0 + j, k);
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) c[y][x] = j0 + y < n_other ? (SIDE_B ? cf[(size_t)j * T + row[x]] : cf[(size_t)row[x] * T + j]) : 0.f;
+                }
+#pragma unroll
+                for (int y = 0; y < 4; ++y)
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) add[x] = fmaf(c[y][x], sv[x] - raw[y].value(k), add[x]);
+            }
+        }
+        if (!any) continue;
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+            if (i + x < n_self) p.grad[(size_t)(self0 + i + x) * Dp + k] += add[x];
+    }
 }
 
 // Both sides in one launch: the side whose tiles loop over more rows comes first, for every block, so
 // that the long tiles do not start last.  A block's tiles of one side stay together on one XCD.
-template <int DIST>
-__global__ __launch_bounds__(kWaves * kWaves * 64) void k_split_bwd(SplitBwd p) {
-    constexpr int TM = kTile, TN = kTile;
-    using PA = SplitProduct<RowTile<TM>, ColTile<TN>, TM, TN, kWaves, kWaves>;
+template <int DIST, class Tile>
+__global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(Tile::EU, Tile::EU))) void k_split_bwd(SplitBwd p) {
+    constexpr int TM = Tile::TM, TN = Tile::TN;
+    using PA = SplitProduct<RowTile<TM, 2>, ColTile<TN, 2>, Tile>;
     __shared__ __attribute__((aligned(16))) char smem[PA::kLds];
-    __shared__ float csum_s[TM];
-    const int gx = (p.Dp + TN - 1) / TN, ga = (p.B + TM - 1) / TM, gb = (p.T + TM - 1) / TM;
+    __shared__ float csum_s[Tile::threads], scale_s[TM];
+    const int gx = (p.rows.Dp + TN - 1) / TN, ga = (p.B + TM - 1) / TM, gb = (p.T + TM - 1) / TM;
     const bool heads_first = p.T >= p.B;
     const int n_first = gx * (heads_first ? ga : gb) * p.S;
     const int L = blockIdx.x;
     if ((L < n_first) == heads_first) {
         const TileId tile = xcd_tile(gx, ga, p.S, heads_first ? L : L - n_first);
-        split_bwd_tile<DIST, false>(p, tile.z, tile.x, tile.y, smem, csum_s);
+        split_bwd_tile<DIST, false, Tile>(p, tile.z, tile.x, tile.y, smem, csum_s, scale_s);
     } else {
         const TileId tile = xcd_tile(gx, gb, p.S, heads_first ? L - n_first : L);
-        split_bwd_tile<DIST, true>(p, tile.z, tile.x, tile.y, smem, csum_s);
+        split_bwd_tile<DIST, true, Tile>(p, tile.z, tile.x, tile.y, smem, csum_s, scale_s);
     }
 }
 
 // --------------------------------------------------------------------------
 // launches
 
+// Which tiles.  128 x 64 read a third less, 64 x 64 are twice as many.  Forward, us, 64 x 64 and 128 x 64: 64 blocks of 256 x 512
+// (1024 large tiles) 34.4, 29.8; 32 of 256 x 256 (256) 13.6, 14.3; 4 of 200 x 268, D = 100 (40) 6.4, 6.8; one of 256 x 64,
+// D = 64 (2) 8.9, 10.5.  Backward: 49.8, 46.6; 17.2, 17.1 (512); 9.8, 11.6; 11.0, 11.3.
+static bool large_tiles(const ScoreShape& sh) {
+    return (int64_t)sh.S * ((sh.B + 127) / 128) * ((sh.T + 63) / 64) >= 512;
+}
+static bool large_tiles_bwd(const SplitBwd& p) {
+    return (int64_t)p.S * ((p.B + 127) / 128 + (p.T + 127) / 128) * ((p.rows.Dp + 63) / 64) >= 512;
+}
+
 int split_fwd_parts(const ScoreShape& sh) {
-    return ((sh.T + kTile - 1) / kTile) * ((sh.B + kTile - 1) / kTile);
+    const int tm = large_tiles(sh) ? TileLarge::TM : TileSmall::TM;
+    return ((sh.T + 63) / 64) * ((sh.B + tm - 1) / tm);
 }
 
-void launch_split_fwd(const SplitFwd& p, bool fused_loss, hipStream_t stream) {
+template <int DIST, int OM>
+static void split_fwd(const SplitFwd& p, hipStream_t stream) {
     const ScoreShape& sh = p.sh;
-    const dim3 grid = tile_grid((sh.T + kTile - 1) / kTile, (sh.B + kTile - 1) / kTile, sh.S);
-    const bool l2 = sh.dist_fn == DIST_L2 && sh.score_fn != SCORE_DISTMULT;
-#define KGE_FWD(D_, OM_) hipLaunchKernelGGL((k_split_fwd<D_, OM_>), grid, dim3(256), 0, stream, p)
-    if (l2) { if (fused_loss) KGE_FWD(DIST_L2, 0); else KGE_FWD(DIST_L2, 1); }
-    else    { if (fused_loss) KGE_FWD(DIST_DOT, 0); else KGE_FWD(DIST_DOT, 1); }
-#undef KGE_FWD
+    if (large_tiles(sh))
+        hipLaunchKernelGGL((k_split_fwd<DIST, OM, TileLarge>), tile_grid((sh.T + 63) / 64, (sh.B + 127) / 128, sh.S),
+                           dim3(TileLarge::threads), 0, stream, p);
+    else
+        hipLaunchKernelGGL((k_split_fwd<DIST, OM, TileSmall>), tile_grid((sh.T + 63) / 64, (sh.B + 63) / 64, sh.S),
+                           dim3(TileSmall::threads), 0, stream, p);
+}
+void launch_split_fwd(const SplitFwd& p, bool fused_loss, hipStream_t stream) {
+    const bool l2 = p.sh.dist_fn == DIST_L2 && p.sh.score_fn != SCORE_DISTMULT;
+    if (l2) fused_loss ? split_fwd<DIST_L2, 0>(p, stream) : split_fwd<DIST_L2, 1>(p, stream);
+    else fused_loss ? split_fwd<DIST_DOT, 0>(p, stream) : split_fwd<DIST_DOT, 1>(p, stream);
 }
 
-void launch_coef_pieces(const ScoreShape& sh, const float* coef, const uint32_t* nearflag, const SplitCoef& out,
-                        hipStream_t stream) {
+void launch_coef_halves(const ScoreShape& sh, const float* coef, const uint32_t* nearflag, const SplitRows& rows,
+                        const SplitCoef& out, hipStream_t stream) {
     const int n = sh.S * (out.Bp / 32) * (out.Tp / 32);
     const bool l2 = sh.dist_fn == DIST_L2 && sh.score_fn != SCORE_DISTMULT;
-    if (l2) hipLaunchKernelGGL(k_coef_pieces<DIST_L2>, dim3((n + 3) / 4), dim3(256), 0, stream, sh, coef, nearflag, out);
-    else hipLaunchKernelGGL(k_coef_pieces<DIST_DOT>, dim3((n + 3) / 4), dim3(256), 0, stream, sh, coef, nearflag, out);
+#define KGE_COEF(D_) \
+    hipLaunchKernelGGL(k_coef_halves<D_>, dim3((n + 3) / 4), dim3(256), 0, stream, sh, coef, nearflag, rows.scale, rows.n_head, out)
+    if (l2) KGE_COEF(DIST_L2);
+    else KGE_COEF(DIST_DOT);
+#undef KGE_COEF
 }
 
+template <int DIST, class Tile>
+static void split_bwd(const SplitBwd& p, hipStream_t stream) {
+    const dim3 grid(((p.rows.Dp + Tile::TN - 1) / Tile::TN) * ((p.B + Tile::TM - 1) / Tile::TM + (p.T + Tile::TM - 1) / Tile::TM) * p.S);
+    hipLaunchKernelGGL((k_split_bwd<DIST, Tile>), grid, dim3(Tile::threads), 0, stream, p);
+}
 void launch_split_bwd(const SplitBwd& p, bool l2, hipStream_t stream) {
-    const dim3 grid(((p.Dp + kTile - 1) / kTile) * ((p.B + kTile - 1) / kTile + (p.T + kTile - 1) / kTile) * p.S);
-    if (l2) hipLaunchKernelGGL(k_split_bwd<DIST_L2>, grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL(k_split_bwd<DIST_DOT>, grid, dim3(256), 0, stream, p);
+    if (large_tiles_bwd(p)) l2 ? split_bwd<DIST_L2, TileLarge>(p, stream) : split_bwd<DIST_DOT, TileLarge>(p, stream);
+    else l2 ? split_bwd<DIST_L2, TileSmall>(p, stream) : split_bwd<DIST_DOT, TileSmall>(p, stream);
 }
 
-// Where these kernels are taken.  At whole 128-row tiles and enough of them the kernels that split
-// float32 operands while staging are as fast or faster (22.8M-row workload, 64 blocks of 256 x 512:
-// forward 40 against 42 us, backward 57 against 67, and the gather writes a third less): the
-// piece matrices cost half as much memory traffic again, and with that many tiles the
-// staging's vector work hides behind other workgroups' matrix work.  Elsewhere - ragged sizes, which
-// those kernels take with bounds checks and float32 matrix instructions, and few tiles - these
-// are the faster ones: one block of 256 x 64, D = 64: forward 11.2 -> 10.5 us, backward 37 -> 9.5;
-// four of 200 x 268, D = 100: 17.4 -> 7.8 and 49 -> 10.6.
+// Where these kernels are taken: L2 and dot of every shape.  (Kernels that split float32 operands into bfloat16 pieces while
+// staging took 38 + 55 us for the forward and backward of 64 blocks of 256 x 512, these take 28 + 46; 32 of 256 x 256: 15 + 21
+// and 13 + 17.)
 bool split_scoring(const ScoreShape& sh) {
     if (sh.use_mfma != 2 || sh.score_fn == SCORE_TRANSH) return false;
-    if (sh.dist_fn == DIST_L1 && sh.score_fn != SCORE_DISTMULT) return false;
-    const bool whole = sh.B % 128 == 0 && sh.T % 128 == 0 && sh.Dp % 64 == 0;
-    return !whole || (int64_t)sh.S * (sh.B / 128) * (sh.T / 64) < 128;
+    return !(sh.dist_fn == DIST_L1 && sh.score_fn != SCORE_DISTMULT);
 }
 
 }  // namespace kge

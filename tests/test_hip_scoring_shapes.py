@@ -119,7 +119,7 @@ def test_l1_equal_columns_have_zero_gradient(B, A, D):
     np.testing.assert_array_equal(after["entity_data"][:, D + equal], 0.0)
 
 
-# L2 and dot on three-piece operands: tiles of 64 x 64 over slabs of 32, matrices filled up to 32
+# L2 and dot on float16 halves: tiles of 64 x 64 over slabs of 32, matrices filled up to 32
 @pytest.mark.parametrize("merge", [True, False])
 @pytest.mark.parametrize("score_fn,distance_fn", [("TransE", "L2"), ("DistMult", "MatMul"), ("ComplEx", "L2")])
 @pytest.mark.parametrize("loss_fn", ["logsigmoid", "softmax"])
@@ -134,6 +134,41 @@ def test_l1_equal_columns_have_zero_gradient(B, A, D):
 def test_l2_and_dot_shapes(oracle64, score_fn, distance_fn, loss_fn, S, B, A, D, merge):
     run_case(oracle64, dict(score_fn=score_fn, distance_fn=distance_fn, loss_fn=loss_fn, n_shard=S, batch=B, a2a=A, dim=D,
                             feature=0, n_entity=1500, n_relation=6, gamma=4.0), n_step=2, **{"execution.merge_tails": merge})
+
+
+@pytest.mark.parametrize("score_fn,distance_fn", [("TransE", "L2"), ("DistMult", "MatMul")])
+@pytest.mark.parametrize("loss_fn", ["logsigmoid", "softmax"])
+@pytest.mark.parametrize("S,B,A,D", [
+    (1, 40, 2080, 260),    # more than 64 slabs of tails, rows of more than 256 columns
+    (1, 2100, 40, 36),     # more than 64 slabs of heads
+    (64, 129, 9, 66),      # tiles of 128 x 64, none of them whole
+])
+def test_halves_of_rows_of_many_sizes(oracle64, score_fn, distance_fn, loss_fn, S, B, A, D):
+    """Rows whose lengths are spread over a factor of a thousand and more, so that the scales of rows and of sub-blocks of
+    coefficients differ from one to the next.  The first moments are the gradients (from zero, times 1 - beta_m): 1e-5
+    of their norm, the bar of every float32 gradient here (measured: 2e-7), and the same of every row's own with 2^-36 of the
+    largest row's: a coefficient is right to 2^-47 of the largest of its sub-block, which a row of 2^11 times the length
+    (four standard deviations to either side) multiplies."""
+    import libpoplar_kge
+    from oracle.kge_oracle import make_cfg
+
+    c = K.cfg_dict(score_fn=score_fn, distance_fn=distance_fn, loss_fn=loss_fn, n_shard=S, batch=B, a2a=A, dim=D, feature=0,
+                   n_entity=3000, n_relation=6, gamma=4.0, shared_table=True)
+    rng = np.random.default_rng(S + B)
+    state = K.make_state(c, rng, warm=False)
+    state["entity_data"][:, :D] *= np.exp(rng.normal(0, 1.5, (c["n_entity"], 1))).astype(np.float32)
+    batch = K.raw_batch(c, 1, rng)
+    lr = np.full(S, 0.01, np.float32)
+    engine = libpoplar_kge.Engine(H.engine_settings(c, 1), "")
+    H.load_state(engine, c, state)
+    loss = H.train(engine, c, lr, batch)
+    after = K.copy_state(state)
+    want_loss = oracle64.train_step_loop(make_cfg(**c), after, lr, batch)
+    np.testing.assert_allclose(loss, want_loss, rtol=1e-5)
+    got, want = H.read_state(engine, c)["entity_data"][:, D:2 * D], after["entity_data"][:, D:2 * D]
+    assert K.rel_l2(got, want) < 1e-5
+    norm = np.linalg.norm(want, axis=1)
+    assert np.all(np.linalg.norm(got - want, axis=1) <= 1e-5 * norm + 2.0**-36 * norm.max())
 
 
 def _two_disjoint_blocks(kind, loss_fn, B, A, D, bad, merge):
