@@ -35,6 +35,7 @@ DEVINL void log_sigmoid_both(float z, float& value, float& grad) {
 // The same for both signs of one score: exp(-|s|) serves z = s and z = -s alike.
 struct LogSigmoid {
     float s, rw, l1p, g_big;
+    DEVINL LogSigmoid() {}
     DEVINL explicit LogSigmoid(float score) : s(score) {
         const float u = __builtin_amdgcn_exp2f(-1.44269504089f * fabsf(s));
         const float w = 1.f + u;

@@ -350,7 +350,7 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
     using P = SplitProduct<RowTile<TM, 2>, RowTile<TN, 2>, Tile>;
     __shared__ __attribute__((aligned(16))) char smem[P::kLds];
     __shared__ float na_s[TM], nb_s[TN], sa_s[TM], sb_s[TN], mult_s[TN], red[WM * WN];
-    __shared__ uint32_t label_s[TM];
+    __shared__ __attribute__((aligned(16))) uint32_t label_s[TM];
     __shared__ int n_redo;
     const ScoreShape& sh = p.sh;
     const int B = sh.B, T = sh.T, Kp = p.rows.Kp;
@@ -498,27 +498,39 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
             // a column's negatives: mult of them, or one less where one is the row's label (src/poplar_kge.cpp:615-636)
             const float mult = mult_s[nbk + cl], w_all = mult * w_neg, w_less = (mult - 1.f) * w_neg;
             const bool whole = m0 + mb + 32 <= B && n0 + nbk + 32 <= T;
-            const uint32_t* const label = label_s + mb + 4 * hl;
             float c[16];
             asm volatile("" ::: "memory");  // what stands in LDS is read again, not kept in registers
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[r]) : val[r];  // (never negative; a NaN stays one)
-                const float score = fmaf(dist, score_sign, score_base);
-                const bool pos = (uint32_t)n == label[8 * (r >> 2) + (r & 3)];
-                LogSigmoid z(score);
-                const float w = pos ? w_less : w_all;
-                float term = -(w * z.minus_value()), ds = w * z.minus_grad();
-                if (__ballot(pos)) {  // one pair of a positive's row
-                    term -= pos ? w_pos * z.plus_value() : 0.f;
-                    ds -= pos ? w_pos * z.plus_grad() : 0.f;
+            for (int g = 0; g < 16; g += 4) {  // four rows at a time: their chains of dependent instructions side by side
+                const uint4 label4 = *reinterpret_cast<const uint4*>(&label_s[mb + 4 * hl + 2 * g]);
+                const uint32_t label[4] = {label4.x, label4.y, label4.z, label4.w};
+                float dist[4], term[4], ds[4];
+                LogSigmoid z[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    dist[r] = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[g + r]) : val[g + r];  // (never negative; a NaN stays one)
+                    z[r] = LogSigmoid(fmaf(dist[r], score_sign, score_base));
+                    const float w = (uint32_t)n == label[r] ? w_less : w_all;
+                    term[r] = -(w * z[r].minus_value());
+                    ds[r] = w * z[r].minus_grad();
                 }
-                float v = ds * coef_scale;
-                if (DIST == DIST_L2) v = dist != 0.f ? v * __builtin_amdgcn_rcpf(dist) : 0.f;
-                if (!whole && !(scale_a(r) != 0.f && sb != 0.f)) term = v = 0.f;
-                loss_acc += term;
-                c[r] = v;
-                if ((r & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // no more rows' intermediate values at once
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const bool pos = (uint32_t)n == label[r];
+                    if (__ballot(pos)) {  // one pair of a positive's row
+                        term[r] -= pos ? w_pos * z[r].plus_value() : 0.f;
+                        ds[r] -= pos ? w_pos * z[r].plus_grad() : 0.f;
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float v = ds[r] * coef_scale;
+                    if (DIST == DIST_L2) v = dist[r] != 0.f ? v * __builtin_amdgcn_rcpf(dist[r]) : 0.f;
+                    if (!whole && !(scale_a(g + r) != 0.f && sb != 0.f)) term[r] = v = 0.f;
+                    loss_acc += term[r];
+                    c[g + r] = v;
+                }
+                __builtin_amdgcn_sched_barrier(0);  // no more rows' intermediate values at once
             }
             if (flagged) {  // the backward takes this block in the direct form, from the coefficients as they are
                 char* const out = (char*)(p.coef + ((size_t)d * B + m0 + mb) * T + n0 + nbk);
