@@ -157,7 +157,7 @@ void launch_gather_halves(const RowSource& ent, const float* rel, const uint32_t
 // workgroups as LDS has room for (three of 128 x 64, four of 64 x 64).  What a launch spends its time on is the first slab's
 // way from memory, the loop and the epilogue of every workgroup, one after the other; workgroups beside it fill
 // the gaps, and a third of 128 x 64 is worth more than a third tile copy (64 blocks of 256 x 512, 331 distinct tails, D = 256:
-// forward 32.9 us with two workgroups of three copies, 27.2 with three of two; backward 48.2 and 46.3).
+// forward 35.5 us with two workgroups of three copies, 30.2 with three of two; backward 49.9 and 43.8).
 template <int TM_, int TN_, int WM_, int WN_, int EU_>
 struct SplitTile { static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, EU = EU_, threads = WM_ * WN_ * 64; };
 using TileSmall = SplitTile<64, 64, 2, 2, 4>;
@@ -224,8 +224,10 @@ struct SplitProduct {
             // (a wave's copies arrive in order: all but the next slab's are there)
             if (kStages > 2 && slab + 1 < n_slab) wait_copies_and_barrier<kEach>();
             else wait_copies_and_barrier<0>();
+            const bool count = before(slab);  // (ahead of the copies: behind them, its wait for
+            // exponents that it may have loaded was one for the next slab, 55 -> 44 us of 16 blocks of 256 x 1536)
             if (slab + kStages - 1 < n_slab) fill(slab + kStages - 1);
-            if (!before(slab)) continue;
+            if (!count) continue;
             const char* ta = smem + slab % kStages * kStage;
             const char* tb = ta + TA::kBytes;
 #pragma unroll
