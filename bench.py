@@ -181,17 +181,11 @@ def cpu_torch_run(prepared, settings, n_check, budget_s=10.0):
                        f"path, {threads} threads of {os.cpu_count()} host cpus"), loss
 
 
-def split_forward(w):
-    """Whether the forward kernel takes the three-piece bfloat16 path: the engine's default for
-    L2 / dot scoring on float32 operands at shapes aligned to its tiles."""
+def halves_scoring(w):
+    """Whether the scoring kernels multiply float16 halves: the engine's default for L2 / dot scoring on
+    float32 operands."""
     return (w.get("scoring") in (None, "mfma_bf16x3") and w.get("distance_fn", "L2") != "L1"
-            and w.get("scoring_dtype") != "bfloat16"
-            and w["batch"] % 128 == 0 and w["tails"] % 64 == 0 and w["dim"] % 64 == 0)
-
-
-def split_backward(w):
-    """The same for the backward kernel (its tiles are 128 rows on either side)."""
-    return split_forward(w) and w["tails"] % 128 == 0
+            and w.get("scoring_dtype") != "bfloat16")
 
 
 # kernels whose working set (a few tens of MB, just written by the kernel before) is served by the
@@ -243,13 +237,13 @@ def kernel_table(w, timing, n_steps, uniq_rows, contributions):
                          peak=PEAK_HBM_GBPS, unit="GB/s")
         else:
             # the published peak of the instruction the kernel issues: float32 matrix / vector
-            # instructions 157.3; bfloat16 matrix instructions 2500, of which the float32-product
-            # kernels issue six per product (three-piece operands)
+            # instructions 157.3; 16-bit matrix instructions 2500, of which the float32-product
+            # kernels issue three per product (two float16 halves an operand)
             peak, instr = PEAK_FP32_TFLOPS, "f32"
             if w.get("scoring_dtype") == "bfloat16":
                 peak, instr = PEAK_BF16_TFLOPS, "bf16"
-            elif (name == "score_fwd" and split_forward(w)) or (name == "score_bwd" and split_backward(w)):
-                peak, instr = PEAK_BF16_TFLOPS / 6.0, "bf16 x6 (float32 products)"
+            elif name in ("score_fwd", "score_bwd") and halves_scoring(w):
+                peak, instr = PEAK_BF16_TFLOPS / 3.0, "f16 x3 (float32 products)"
             entry.update(bound="mfma", achieved=amount / (ms * 1e-3) / 1e12, peak=peak, unit="TFLOP/s",
                          instructions=instr)
         entry["frac"] = entry["achieved"] / entry["peak"]
@@ -335,12 +329,12 @@ def predict_bench(args, w, kge, torch):
     flop = 3.0 * pairs * D
     emb_bytes = 2 if w.get("embedding_dtype") == "bfloat16" else 4
     table_bytes = float(m.n_entity - 1) * D * emb_bytes
-    # L2 with the default scoring runs as six bfloat16 matrix products per float32 product
-    # (12 executed flop per pair-dim, priced against the bfloat16 peak); L1 is float32 vector work
+    # L2 with the default scoring runs as three float16 matrix products per float32 product up to 256 columns,
+    # as six bfloat16 ones beyond (6 and 12 executed flop per pair-dim, priced against the 16-bit peak); L1 is float32 vector work
     # (3 flop per pair-dim against the float32 peak)
     pieces = m.distance_fn == "L2" and (args.scoring or "mfma_bf16x3") == "mfma_bf16x3"
     peak = PEAK_BF16_TFLOPS if pieces else PEAK_FP32_TFLOPS
-    done = (12.0 if pieces else 3.0) * pairs * D
+    done = ((6.0 if D <= 256 else 12.0) if pieces else 3.0) * pairs * D
     frac_flop, frac_hbm = done / dt / 1e12 / peak, table_bytes / dt / 1e9 / PEAK_HBM_GBPS
     roof = (dict(bound="mfma", achieved=done / dt / 1e12, peak=peak, unit="TFLOP/s", frac=frac_flop)
             if frac_flop >= frac_hbm else

@@ -777,8 +777,8 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
 // launches
 
 // Which tiles.  128 x 64 read a third less, 64 x 64 are twice as many.  Forward, us, 64 x 64 and 128 x 64: 64 blocks of 256 x 512
-// (1024 large tiles) 34.4, 29.8; 32 of 256 x 256 (256) 13.6, 14.3; 4 of 200 x 268, D = 100 (40) 6.4, 6.8; one of 256 x 64,
-// D = 64 (2) 8.9, 10.5.  Backward: 49.8, 46.6; 17.2, 17.1 (512); 9.8, 11.6; 11.0, 11.3.
+// (1024 large tiles) 33.4, 28.7; 32 of 256 x 256 (256) 13.5, 14.2; 4 of 200 x 268, D = 100 (40) 6.3, 6.8; one of 256 x 64,
+// D = 64 (2) 8.8, 9.9.  Backward: 45.2, 42.6; 16.5, 16.0 (512); 8.3, 8.5; 9.2, 9.2.
 static bool large_tiles(const ScoreShape& sh) {
     return (int64_t)sh.S * ((sh.B + 127) / 128) * ((sh.T + 63) / 64) >= 512;
 }
@@ -829,8 +829,8 @@ void launch_split_bwd(const SplitBwd& p, bool l2, hipStream_t stream) {
 }
 
 // Where these kernels are taken: L2 and dot of every shape.  (Kernels that split float32 operands into bfloat16 pieces while
-// staging took 38 + 55 us for the forward and backward of 64 blocks of 256 x 512, these take 28 + 46; 32 of 256 x 256: 15 + 21
-// and 13 + 17.)
+// staging took 38 + 55 us for the forward and backward of 64 blocks of 256 x 512, these take 28 + 44; 32 of 256 x 256: 15 + 21
+// and 13 + 16.)
 bool split_scoring(const ScoreShape& sh) {
     if (sh.use_mfma != 2 || sh.score_fn == SCORE_TRANSH) return false;
     return !(sh.dist_fn == DIST_L1 && sh.score_fn != SCORE_DISTMULT);
