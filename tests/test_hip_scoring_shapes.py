@@ -218,7 +218,7 @@ def test_nonfinite_row_stays_in_its_block(kind, loss_fn, merge, B, A, D):
 # block's first tail) the gradients' other columns stay finite
 @pytest.mark.parametrize("kind", ["L2", "MatMul"])
 @pytest.mark.parametrize("B,A,D", [(33, 21, 30), (8, 100, 64), (130, 65, 100),
-                                   (512, 512, 64)])  # whole 128-row tiles, enough of them: float32 operands, split while staged
+                                   (512, 512, 64)])  # whole tiles
 def test_infinite_row_shows_in_the_loss(kind, B, A, D):
     for role in ("head", "tail"):
         for value in (np.inf, -np.inf):

@@ -314,7 +314,7 @@ def test_step_vs_oracle_valu_scoring(oracle64, name):
                                   "bf16_embedding_l2", "l2_feat", "mid_l2"])
 def test_step_vs_oracle_matrix_scoring(oracle64, name, scoring):
     # the two matrix-core forms of the float32 products, named explicitly: float32 instructions
-    # ("mfma"), and six bfloat16 instructions on three-piece operands ("mfma_bf16x3", the default, ragged
+    # ("mfma"), and 16-bit instructions on split operands ("mfma_bf16x3", the default, ragged
     # shapes included): same bars
     run_case(oracle64, CASES[name], **{"execution.scoring": scoring})
 
