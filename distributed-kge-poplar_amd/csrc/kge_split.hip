@@ -37,8 +37,8 @@ DEVINL uint32_t wave_max_bits(float v) {
 
 // --------------------------------------------------------------------------
 // operand gather: RPW contributions per wave, their entity (or hidden) rows with the relation
-// applied for the heads, as halves; and the rows' scales and squared norms.  Workgroup (d, y): the y-th lot of
-// block d's B heads and then T tails, which finds its XCD (d % 8) where the block's tiles will run.
+// applied for the heads, as halves; and the rows' scales and squared norms.  Workgroup (d, y, z): a lot of
+// block d's B heads and then T tails (z: a grid's y ends at 65535), which finds its XCD (d % 8) where the block's tiles will run.
 // ET: the rows' element type, or -1: as `ent` says, the complex product and the rotation among the
 // relations; ONE: rows of at most 256 columns, which stay in their registers between the largest value and the halves.
 template <int RPW, int ET, bool ONE>
@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256) void k_gather_halves(RowSource ent, const floa
                                                        int B, int T, int tpad) {
     constexpr bool XF = ET < 0;
     const int lane = threadIdx.x & 63, d = blockIdx.x;
-    const int i0 = (blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * RPW;
+    const int i0 = ((blockIdx.z * gridDim.y + blockIdx.y) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * RPW;
     // the row numbers are asked for together with the block's tail count (rows past it are
     // never used, but their slots hold valid numbers): one round trip instead of two.  (All of them
     // are the wave's, and scalar loads: a lane has an offset into its rows and no addresses.)
@@ -132,9 +132,12 @@ void launch_gather_halves(const RowSource& ent, const float* rel, const uint32_t
                           const SplitRows& s, const ScoreShape& sh, hipStream_t stream) {
     // two rows per wave where that leaves enough waves: the kernel is resident waves over the
     // latency of the chain row number -> row -> store, and a wave may as well keep two chains going
-    const int n = sh.B + sh.T;
+    auto grid = [&](int rows) {
+        const unsigned lots = (unsigned)((sh.B + sh.T + rows - 1) / rows), y = std::min(lots, 32768u);
+        return dim3((unsigned)sh.S, y, (lots + y - 1) / y);
+    };
 #define KGE_GATHER(N_, ET_, ONE_)                                                                                       \
-    hipLaunchKernelGGL((k_gather_halves<N_, ET_, ONE_>), dim3(sh.S, (n + 4 * N_ - 1) / (4 * N_)), dim3(256), 0, stream, \
+    hipLaunchKernelGGL((k_gather_halves<N_, ET_, ONE_>), grid(4 * N_), dim3(256), 0, stream, \
                        ent, rel, crel, rel_mode, half, s, sh.tcount, sh.B, sh.T, sh.tpad)
 #define KGE_GATHER_ET(ET_)                                                                                      \
     do {                                                                                                        \
