@@ -588,7 +588,7 @@ DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, cha
     // a sub-block's exponent: of the self rows' group st and of slab ot
     const int* const exps = p.in.exponent + (size_t)d * MT * NT;
     const int st0 = (i0 + wm) >> 5, st_last = (SIDE_B ? NT : MT) - 1;
-    int exp_reg[P::AM], exp_now[P::AM];  // of slab 64 n + lane; what the accumulators are in
+    int exp_reg[P::AM], exp_now[P::AM];  // of slab 64 n + lane; what the accumulators are in (kNoExponent: they are empty)
     auto load_exps = [&](int slab0) __attribute__((always_inline)) {
         const int ot = min(slab0 + lane, n_slab - 1);
 #pragma unroll
@@ -599,7 +599,7 @@ DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, cha
     };
     floatx16 big[P::AM][P::AN], small[P::AM][P::AN];
     bool seen = false;  // a flagged block among the tile's (the wave's share of them)
-    exp_now[0] = 0;
+    exp_now[0] = kNoExponent;
     P::run(smem, a, coef_pitch, SIDE_B ? (size_t)32 * coef_pitch : kHalfBytes, b, pitch, (size_t)32 * pitch, n_slab, n_other, big, small, lane, wave,
            [&]() __attribute__((always_inline)) {
                load_exps(0);
@@ -635,8 +635,12 @@ DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, cha
                for (int m = 0; m < P::AM; ++m) {
                    const int e = __builtin_amdgcn_readlane(exp_reg[m], slab & 63);
                    if (e != exp_now[m] && e != kNoExponent) {  // seldom: what is there is brought to the slab's scale
-                       // (a slab 2^80 below what is there counts for nothing, and that would not fit its scale)
                        static_assert(P::AM == 1, "one exponent to a wave's slab");
+                       if (exp_now[m] == kNoExponent) {  // nothing yet
+                           exp_now[m] = e;
+                           continue;
+                       }
+                       // (a slab 2^80 below what has been summed counts for nothing, and that would not fit its scale)
                        if (exp_now[m] - e > 80) return false;
                        const float by = __uint_as_float((uint32_t)(127 + max(exp_now[m] - e, -126)) << 23);
 #pragma unroll
@@ -655,7 +659,7 @@ DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, cha
     // the self rows' own scales leave the sums
 #pragma unroll
     for (int m = 0; m < P::AM; ++m) {
-        const float scale = __uint_as_float((uint32_t)(127 + exp_now[m]) << 23);
+        const float scale = exp_now[m] == kNoExponent ? 1.f : __uint_as_float((uint32_t)(127 + exp_now[m]) << 23);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const float up = pow2_inverse(scale_s[wm + 32 * m + 8 * (r >> 2) + 4 * hl + (r & 3)]);

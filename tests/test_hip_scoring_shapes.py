@@ -171,6 +171,75 @@ def test_halves_of_rows_of_many_sizes(oracle64, score_fn, distance_fn, loss_fn, 
     assert np.all(np.linalg.norm(got - want, axis=1) <= 1e-5 * norm + 2.0**-36 * norm.max())
 
 
+def _first_moments(c, state, batch, loss_scale, oracle64, **extra):
+    """One step from moments of zero: (engine, oracle) x (the loss, the entities' first moments, the relations'), which are
+    the gradients times 1 - beta_m."""
+    import libpoplar_kge
+    from oracle.kge_oracle import make_cfg
+
+    c = dict(c, loss_scale=float(loss_scale))
+    lr = np.full(c["n_shard"], 0.01, np.float32)
+    engine = libpoplar_kge.Engine(H.engine_settings(c, 1, **extra), "")
+    H.load_state(engine, c, state)
+    loss = H.train(engine, c, lr, batch)
+    got, want = H.read_state(engine, c), K.copy_state(state)
+    want_loss = oracle64.train_step_loop(make_cfg(**c), want, lr, batch)
+    D = c["dim"]
+    return [(l, s["entity_data"][:, D:2 * D].astype(np.float64), s["relation_embedding/adam_m"].astype(np.float64))
+            for l, s in ((loss, got), (want_loss, want))]
+
+
+def _assert_each_row(got, want, rel=1e-5):
+    """1e-5, the bar of every float32 gradient here, of the whole and of every row by its own norm."""
+    np.testing.assert_allclose(got[0], want[0], rtol=rel)
+    for g, w in zip(got[1:], want[1:]):
+        assert K.rel_l2(g, w) < rel
+        norm, error = np.linalg.norm(w, axis=1), np.linalg.norm(g - w, axis=1)
+        worst = np.argmax(error - rel * norm)
+        assert error[worst] <= rel * norm[worst], (worst, error[worst], norm[worst])
+
+
+# Coefficients times the scales of their rows far below 1 (a small initialisation, a loss scale that is not the default
+# one): no slab of them may be left out of the sums
+@pytest.mark.parametrize("score_fn,distance_fn", [("TransE", "L2"), ("DistMult", "MatMul"), ("ComplEx", "MatMul")])
+@pytest.mark.parametrize("loss_fn", ["logsigmoid", "softmax"])
+@pytest.mark.parametrize("S,B,A,D,sigma,loss_scale", [
+    (64, 256, 8, 256, 1 / 256, 1),
+    (16, 512, 96, 128, 1 / 128, 1),
+    (4, 200, 64, 100, 1e-3, 1),
+    (4, 200, 64, 100, 1e-4, 2.0**-12),
+])
+def test_small_coefficients_reach_the_gradient(oracle64, score_fn, distance_fn, loss_fn, S, B, A, D, sigma, loss_scale):
+    c = K.cfg_dict(score_fn=score_fn, distance_fn=distance_fn, loss_fn=loss_fn, n_shard=S, batch=B, a2a=A, dim=D, feature=0,
+                   n_entity=3000, n_relation=S * 6, gamma=4.0, shared_table=True)
+    rng = np.random.default_rng(7)
+    state = K.make_state(c, rng, warm=False, scale=sigma)
+    _assert_each_row(*_first_moments(c, state, K.raw_batch(c, 1, rng), loss_scale, oracle64))
+
+
+def _one_block(c, state, sizes, rng):
+    """One block whose heads, and then tails in their slots' order, are rows 1 .. with standard deviations `sizes`
+    ([B + A]); relations of size 1 of their own."""
+    B, A, D = c["batch"], c["a2a"], c["dim"]
+    state["entity_data"][1:1 + B + A, :D] = rng.normal(0, 1, (B + A, D)) * np.asarray(sizes)[:, None]
+    return dict(remote=(1 + np.arange(B + A, dtype=np.uint32)).reshape(1, 1, B + A),
+                a2a=(B + np.arange(A, dtype=np.uint32)).reshape(1, 1, 1, A), head=np.arange(B, dtype=np.uint32).reshape(1, 1, B),
+                relation=np.arange(B, dtype=np.uint32).reshape(1, 1, B), tail=rng.integers(0, A, (1, 1, B)).astype(np.uint32))
+
+
+# The first slab of heads and of tails is sixteen times shorter than the others: whatever the loss scale, it counts
+@pytest.mark.parametrize("power", range(-40, 41, 4))
+def test_short_first_slab_counts(oracle64, power):
+    B, A, D = 96, 96, 64
+    c = K.cfg_dict(score_fn="DistMult", distance_fn="MatMul", n_shard=1, batch=B, a2a=A, dim=D, feature=0, n_entity=300,
+                   n_relation=B, gamma=4.0, shared_table=True)
+    rng = np.random.default_rng(7)
+    state = K.make_state(c, rng, warm=False, scale=2.0**-3)
+    sizes = np.where(np.arange(B + A) % 96 < 32, 2.0**-7, 2.0**-3)
+    batch = _one_block(c, state, sizes, rng)
+    _assert_each_row(*_first_moments(c, state, batch, 2.0**power, oracle64, **{"execution.merge_tails": False}))
+
+
 def _two_disjoint_blocks(kind, loss_fn, B, A, D, bad, merge):
     """One step of two blocks that share no row (entity or relation); `bad`: (role, value) of block 1's
     first head or tail, or None.  Returns the losses and block 0's rows afterwards."""
