@@ -240,6 +240,27 @@ def test_short_first_slab_counts(oracle64, power):
     _assert_each_row(*_first_moments(c, state, batch, 2.0**power, oracle64, **{"execution.merge_tails": False}))
 
 
+# Rows of zeros, one head and one tail, among others of one size: their gradients are as right as their neighbours'
+@pytest.mark.parametrize("score_fn,distance_fn,loss_fn,sigma", [
+    ("TransE", "L2", "logsigmoid", 1 / 16), ("TransE", "L2", "logsigmoid", 1), ("TransE", "L2", "logsigmoid", 64),
+    ("TransE", "L2", "softmax", 1 / 16), ("DistMult", "MatMul", "logsigmoid", 1 / 16), ("DistMult", "MatMul", "logsigmoid", 1),
+    ("DistMult", "MatMul", "logsigmoid", 64), ("DistMult", "MatMul", "softmax", 1), ("DistMult", "MatMul", "softmax", 64),
+])
+def test_rows_of_zeros(oracle64, score_fn, distance_fn, loss_fn, sigma):
+    B, A, D = 70, 100, 64
+    c = K.cfg_dict(score_fn=score_fn, distance_fn=distance_fn, loss_fn=loss_fn, n_shard=1, batch=B, a2a=A, dim=D, feature=0,
+                   n_entity=300, n_relation=B, gamma=4.0, shared_table=True)
+    rng = np.random.default_rng(7)
+    state = K.make_state(c, rng, warm=False, scale=sigma)
+    sizes = np.full(B + A, float(sigma))
+    sizes[[3, B + 37]] = 0.0
+    if score_fn == "DistMult":  # (scores of a few units)
+        state["relation_embedding"] *= sigma**-3 / 4
+    else:
+        state["relation_embedding"][3] = 0.0
+    _assert_each_row(*_first_moments(c, state, _one_block(c, state, sizes, rng), B * A, oracle64))
+
+
 def _two_disjoint_blocks(kind, loss_fn, B, A, D, bad, merge):
     """One step of two blocks that share no row (entity or relation); `bad`: (role, value) of block 1's
     first head or tail, or None.  Returns the losses and block 0's rows afterwards."""
