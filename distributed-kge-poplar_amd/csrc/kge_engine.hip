@@ -273,7 +273,7 @@ struct kge_engine {
     // L2 and dot scoring on float16 halves (kge_split.hip)
     bool split = false;
     int Kp = 0, Bp = 0, Tp = 0;
-    DevBuf<char> rowsp, coefp;
+    DevBuf<char> rowsp, coefp, coef_small;
     DevBuf<int> coef_exp;
     DevBuf<uint32_t> row_lost;
     DevBuf<float> row_norm, row_scale, rowpart, colpart;
@@ -717,6 +717,7 @@ void allocate(kge_engine& E) {
         E.row_lost.alloc((R + kSplitSpareRows) * E.Kp / 32);
         E.coefp.alloc(half_bytes(S * E.Bp, E.Tp));
         E.coefp.zero(st);
+        E.coef_small.alloc(half_bytes(S * E.Bp, E.Tp));
         E.coef_exp.alloc(S * (E.Bp / 32) * (E.Tp / 32));
         E.row_norm.alloc(R + kSplitSpareRows);
         E.row_scale.alloc(R + kSplitSpareRows);
@@ -780,7 +781,7 @@ void allocate(kge_engine& E) {
     sh.operands_dense = 1;
     sh.tcount = E.merge_tails ? E.tcount.p : nullptr;
     E.n_part = !fused ? E.B : E.split ? split_fwd_parts(sh) : score_fwd_parts(sh, operand_rows(E, E.opnd.p));
-    if (E.use_mfma && E.dist_fn == DIST_L2) {
+    if (E.use_mfma && E.dist_fn == DIST_L2 && !E.split) {
         E.nearflag.alloc(nearflag_words(sh));
         E.nearflag.zero(st);
     }
@@ -1339,21 +1340,21 @@ void run_step(kge_engine& E, int i) {
           launch_transh_bwd(tb, st);
           launch_transh_back(ent, E.rel.p, crel, E.n_rel, (int)SB, E.Dp, E.grad.p, E.transh_mm.p, E.relgrad.p, st); }
     } else if (E.split) {
-        const SplitCoef sc = {E.coefp.p, E.coef_exp.p, E.rowpart.p, E.colpart.p, E.Bp, E.Tp};
+        const SplitCoef sc = {E.coefp.p, E.coef_small.p, E.coef_exp.p, E.rowpart.p, E.colpart.p, E.Bp, E.Tp};
         { KernelTimer t(E, K_FWD);
           SplitFwd f = {};
           f.sh = sh; f.rows = split_rows; f.clabel = clabel;
-          f.coef = E.coef.p; f.dist = fused ? nullptr : E.dist.p; f.loss_part = loss_part; f.nearflag = E.nearflag.p;
+          f.coef = E.coef.p; f.dist = fused ? nullptr : E.dist.p; f.loss_part = loss_part;
           f.out = sc;
           launch_split_fwd(f, fused, st); }
         if (!fused) {
             KernelTimer t(E, K_LOSS);
             launch_loss_rows(sh, clabel, E.coef.p, E.dist.p, loss_part, nullptr, st);
-            launch_coef_halves(sh, E.coef.p, E.nearflag.p, split_rows, sc, st);
+            launch_coef_halves(sh, E.coef.p, split_rows, sc, st);
         }
         { KernelTimer t(E, K_BWD);
           SplitBwd b = {};
-          b.rows = split_rows; b.in = sc; b.coef = E.coef.p; b.nearflag = E.nearflag.p;
+          b.rows = split_rows; b.in = sc; b.coef = E.coef.p;
           b.grad = E.grad.p; b.S = E.S; b.B = E.B; b.T = E.T; b.tcount = sh.tcount; b.tpad = sh.tpad;
           launch_split_bwd(b, E.dist_fn == DIST_L2 && E.score_fn != SCORE_DISTMULT, st); }
     } else {

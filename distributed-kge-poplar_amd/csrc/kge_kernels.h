@@ -271,31 +271,30 @@ struct SplitRows {
 void launch_gather_halves(const RowSource& ent, const float* rel, const uint32_t* crel, int rel_mode, int half,
                           const SplitRows& rows, const ScoreShape& sh, hipStream_t stream);
 // The coefficient matrices [S][Bp][Tp] (B and T filled up to multiples of 32) times the scales of their head and
-// tail as halves, the exponents of the 32 x 32 sub-blocks' own scales [S][Bp / 32][Tp / 32] (kNoExponent: all
-// zeros), and the coefficients' sums over the sub-blocks: rowpart [S][Bp][Tp / 32], colpart [S][Bp / 32][Tp] (L2 only)
-struct SplitCoef { char* coefp; int* exponent; float* rowpart; float* colpart; int Bp, Tp; };
-constexpr int kNoExponent = 1 << 20;
+// tail as halves, the exponents of the 32 x 32 sub-blocks' own scales [S][Bp / 32][Tp / 32], multiples of four (plus one:
+// the sub-block's small coefficients are in `small`, laid out alike; kNoExponent: all zeros; kDirect: to be taken in
+// the direct form, from float32 coefficients), and the coefficients' sums over the sub-blocks: rowpart [S][Bp][Tp / 32],
+// colpart [S][Bp / 32][Tp] (L2 only)
+struct SplitCoef { char* coefp; char* small; int* exponent; float* rowpart; float* colpart; int Bp, Tp; };
+constexpr int kNoExponent = 1 << 20, kDirect = 1 << 21;
 struct SplitFwd {
     ScoreShape sh;
     SplitRows rows;     // heads from row 0, tails from row n_head
     const uint32_t* clabel;
-    float* coef;        // [S, B, T] scores (without fused loss); the flagged sub-blocks' coefficients
+    float* coef;        // [S, B, T] scores (without fused loss); the coefficients of the direct form's sub-blocks
     float* dist;        // or null
     float* loss_part;   // split_fwd_parts per block
-    uint32_t* nearflag; // [S, Bp / 32, Tp / 32]
     SplitCoef out;      // written with the fused loss
 };
 bool split_scoring(const ScoreShape& sh);  // whether a step's scoring takes this form
 int split_fwd_parts(const ScoreShape& sh);
 void launch_split_fwd(const SplitFwd& p, bool fused_loss, hipStream_t stream);
 // `coef` as launch_loss_rows leaves it -> halves and sums
-void launch_coef_halves(const ScoreShape& sh, const float* coef, const uint32_t* nearflag, const SplitRows& rows,
-                        const SplitCoef& out, hipStream_t stream);
+void launch_coef_halves(const ScoreShape& sh, const float* coef, const SplitRows& rows, const SplitCoef& out, hipStream_t stream);
 struct SplitBwd {
     SplitRows rows;
     SplitCoef in;
-    const float* coef;               // float32 coefficients of the flagged sub-blocks
-    const uint32_t* nearflag;
+    const float* coef;               // float32 coefficients of the direct form's sub-blocks
     float* grad;                     // [R, Dp]
     int S, B, T;
     const uint32_t* tcount; int tpad;

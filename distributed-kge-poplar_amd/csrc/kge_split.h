@@ -70,8 +70,13 @@ DEVINL float half_scale(float largest) {
     const int e = largest == 0.f ? 0 : min(max((int)(__float_as_uint(largest) >> 23) - 127, -40), 100);
     return __uint_as_float((uint32_t)(e - 14 + 127) << 23);
 }
-// the reciprocal of a power of two
+// a power of two's exponent, its reciprocal
+DEVINL int pow2_exponent(float s) { return (int)(__float_as_uint(s) >> 23) - 127; }
 DEVINL float pow2_inverse(float s) { return __uint_as_float(0x7f000000u - __float_as_uint(s)); }
+// Coefficients are halves with a scale per block, whose largest comes to 2^11 .. 2^15; those below kSmallCoef can go to a
+// matrix of their own, 2^kSmallShift times as large.
+constexpr float kSmallCoef = 0x1p-13f;
+constexpr int kSmallShift = 28;
 // two values, scaled already -> two words of two halves each
 DEVINL void split2_f16(float a, float b, uint32_t w[2]) {
     const f16x2 h = {(_Float16)a, (_Float16)b};

@@ -181,6 +181,14 @@ struct SplitProduct {
     static constexpr int kCopies = TA::kCopies + TB::kCopies, kEach = kCopies / NW;
     static_assert(kCopies % NW == 0, "every wave issues the same number of copies");
 
+    static DEVINL void products(const floatx4 (&fa)[2], const floatx4 (&fb)[2], floatx16& big, floatx16& small) {
+        auto one = [&](int qa, int qb, floatx16& acc) __attribute__((always_inline)) {
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fa[qa]), __builtin_bit_cast(f16x8, fb[qb]), acc, 0, 0, 0);
+        };
+        one(0, 0, big);
+        one(0, 1, small);
+        one(1, 0, small);
+    }
     // meanwhile(): what the caller has to fetch for itself, under the first slab's way from memory;
     // before(slab): ahead of the slab's products, whether to form them
     template <class Meanwhile, class Before>
@@ -243,14 +251,10 @@ struct SplitProduct {
 #pragma unroll
                     for (int n = 0; n < AN; ++n) fb[n][q] = TB::fragment(tb, q, wn + 32 * n, ks, lane);
                 }
-#define KGE_MM(acc_, qa_, qb_)                                                                                   \
-    _Pragma("unroll") for (int m = 0; m < AM; ++m) _Pragma("unroll") for (int n = 0; n < AN; ++n) acc_[m][n] =    \
-        __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fa[m][qa_]),                            \
-                                               __builtin_bit_cast(f16x8, fb[n][qb_]), acc_[m][n], 0, 0, 0)
-                KGE_MM(big, 0, 0);
-                KGE_MM(small, 0, 1);
-                KGE_MM(small, 1, 0);
-#undef KGE_MM
+#pragma unroll
+                for (int m = 0; m < AM; ++m)
+#pragma unroll
+                    for (int n = 0; n < AN; ++n) products(fa[m], fb[n], big[m][n], small[m][n]);
             }
         }
     }
@@ -259,80 +263,136 @@ struct SplitProduct {
 // --------------------------------------------------------------------------
 // the coefficient matrix as halves
 
-// A 32 x 32 block of coefficients in accumulator layout (register r of lane l: row
-// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32) to its place in the matrix of halves, block corner
-// (m0, n0) of block d.  sa[r], sb: the scales of the rows and of the column.  The backward multiplies rows of
-// halves that lack their scales, the heads' on one side and the tails' on the other: a coefficient takes
-// both along, and the backward takes its own row's out of the finished sum.  The block's own scale is 2^exponent,
-// a multiple of four, so that the backward seldom meets another one in the next block; its largest comes to 2^11 at least, and
-// what is below 2^-25 of that (a softmax's e^-17) is off by 2^-47 of it at most.  Neighbouring lanes swap values
-// so that a lane stores two columns of one row as one word.  For L2 also the block's row sums and column sums.
+// A 32 x 32 block of coefficients lies in accumulator layout: register r of lane l is row
+// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.  The backward multiplies rows of halves that lack their scales, the
+// heads' on one side and the tails' on the other: a coefficient takes both along, and the backward takes its own
+// row's out of the finished sum.  The block's own scale is 2^exponent, a multiple of four, so that the backward seldom
+// meets another one in the next block; its largest comes to 2^11 at least.  Halves hold 22 bits down to 2^-14, and what a
+// row's or a column's gradient is made of is its own largest: where one's lies below 2^-13 (an odd row out, a tail that no
+// head's softmax gives a probability worth mentioning), the coefficients below that go to a matrix of their own, 2^28 times
+// as large.  Where even that is not enough, the block is taken in the direct form.
+
+// sums (or maxima) of a block's rows: at each step a lane keeps half of its rows and hands the other half's over.  The
+// result's row is the one that register lane % 16 holds, in all lanes of that row's half.
+template <class Value, class Op>
+DEVINL float block_rows(Value&& value, int lane, Op&& op) {
+    const bool odd = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
+    float s[8], t[4], u[2];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float even_row = value(2 * i), odd_row = value(2 * i + 1);
+        s[i] = op(odd ? odd_row : even_row, swap1(odd ? even_row : odd_row));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) t[i] = op(b1 ? s[2 * i + 1] : s[2 * i], swap2(b1 ? s[2 * i] : s[2 * i + 1]));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) u[i] = op(b2 ? t[2 * i + 1] : t[2 * i], __shfl_xor(b2 ? t[2 * i] : t[2 * i + 1], 4, 64));
+    const float v = op(b3 ? u[1] : u[0], __shfl_xor(b3 ? u[0] : u[1], 8, 64));
+    return op(v, __shfl_xor(v, 16, 64));
+}
+
+// What stands for a block among the exponents.  sa[r], sb: the scales of the rows and of the column.
+template <class Scales>
+DEVINL int coef_block_exponent(const float (&c)[16], Scales&& scale_of_row, float sb, int lane) {
+    constexpr float kTiny = 0x1p-100f;
+    float top = 0.f, least = INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const float t = fabsf(c[r] * scale_of_row(r));
+        top = fmaxf(top, t);
+        least = fminf(least, t);
+    }
+    const int col = pow2_exponent(sb);
+    const uint32_t bits = wave_max_bits(ldexpf(top, col));
+    const int e = ((int)(bits >> 23) - 127 - 14 + 3) & ~3;
+    const bool fits = bits >= __float_as_uint(kTiny) && bits < __float_as_uint(0x1p100f);
+    if (fits && !__ballot(least < kTiny || ldexpf(least, col - e) < kSmallCoef)) return e;
+    // seldom (zeros among them: columns behind a block's last tail)
+    asm volatile("" ::: "memory");  // (scales that stand in LDS are read again, not kept)
+    uint64_t gone = 0u;  // a coefficient that is not zero, but is with its scales, or nearly
+    float most = 0.f;
+    const auto larger = [](float a, float b) { return fmaxf(a, b); };
+    const float row = block_rows([&](int r) __attribute__((always_inline)) {
+        const float t = fabsf(c[r] * scale_of_row(r)), x = ldexpf(t, col - e);
+        gone |= __ballot(c[r] != 0.f && !(t >= kTiny));
+        most = fmaxf(most, x);
+        return x;
+    }, lane, larger);
+    if (!fits) return (__ballot(top != 0.f) | gone) ? kDirect : kNoExponent;
+    most = fmaxf(most, __shfl_xor(most, 32, 64));
+    auto below = [&](float limit) { return __ballot((row != 0.f && row < limit) || (most != 0.f && most < limit)); };
+    if (gone | below(kSmallCoef / (float)(1 << kSmallShift))) return kDirect;
+    return e | (below(kSmallCoef) ? 1 : 0);
+}
+
+// The block to its place in the matrix of halves, block corner (m0, n0) of block d; `word`: coef_block_exponent's.
+// Neighbouring lanes swap values so that a lane stores two columns of one row as one word.  For L2 also the block's row
+// sums and column sums (zeros where the direct form takes the block).
 template <int DIST, class Scales>
-DEVINL void store_coef_block(float (&c)[16], Scales&& scale_of_row, float sb, const SplitCoef& p, int d, int m0, int n0, int lane) {
+DEVINL void store_coef_block(float (&c)[16], Scales&& scale_of_row, float sb, int word, const SplitCoef& p, int d, int m0, int n0,
+                             int lane) {
     const int Bp = p.Bp, Tp = p.Tp;
     if (m0 >= Bp || n0 >= Tp) return;
     const int cl = lane & 31, hl = lane >> 5;
-    const bool odd = lane & 1;
+    const bool odd = lane & 1, empty = word >= kNoExponent;
+    if (lane == 0) p.exponent[((size_t)d * (Bp >> 5) + (m0 >> 5)) * (Tp >> 5) + (n0 >> 5)] = word;
     if (DIST == DIST_L2) {
-        const bool b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
-        // row sums: at each step a lane keeps half of its rows and hands the other half's sums over
-        float s[8], t[4], u[2];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) s[i] = (odd ? c[2 * i + 1] : c[2 * i]) + swap1(odd ? c[2 * i] : c[2 * i + 1]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) t[i] = (b1 ? s[2 * i + 1] : s[2 * i]) + swap2(b1 ? s[2 * i] : s[2 * i + 1]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) u[i] = (b2 ? t[2 * i + 1] : t[2 * i]) + __shfl_xor(b2 ? t[2 * i] : t[2 * i + 1], 4, 64);
-        float v = (b3 ? u[1] : u[0]) + __shfl_xor(b3 ? u[0] : u[1], 8, 64);
-        v += __shfl_xor(v, 16, 64);
+        const float v = block_rows([&](int r) { return c[r]; }, lane, [](float a, float b) { return a + b; });
         const int r = lane & 15;
         if (!(lane & 16))
-            p.rowpart[((size_t)d * Bp + m0 + 8 * (r >> 2) + 4 * hl + (r & 3)) * (Tp >> 5) + (n0 >> 5)] = v;
+            p.rowpart[((size_t)d * Bp + m0 + 8 * (r >> 2) + 4 * hl + (r & 3)) * (Tp >> 5) + (n0 >> 5)] = empty ? 0.f : v;
         float col = 0.f;
 #pragma unroll
         for (int k = 0; k < 16; ++k) col += c[k];
         col += __shfl_xor(col, 32, 64);
-        if (lane < 32) p.colpart[((size_t)d * (Bp >> 5) + (m0 >> 5)) * Tp + n0 + lane] = col;
+        if (lane < 32) p.colpart[((size_t)d * (Bp >> 5) + (m0 >> 5)) * Tp + n0 + lane] = empty ? 0.f : col;
         __builtin_amdgcn_sched_barrier(0);  // (from here on no sums beside the coefficients)
     }
-    float top = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        c[r] *= scale_of_row(r) * sb;
-        top = fmaxf(top, fabsf(c[r]));
-    }
-    const uint32_t bits = wave_max_bits(top);
-    const int exponent = min(max(((int)(bits >> 23) - 127 - 14 + 3) & ~3, -120), 120);
-    const float up = __uint_as_float((uint32_t)(127 - exponent) << 23);
-    if (lane == 0) p.exponent[((size_t)d * (Bp >> 5) + (m0 >> 5)) * (Tp >> 5) + (n0 >> 5)] = bits ? exponent : kNoExponent;
-    const int pitch = half_pitch(Tp);
-    char* const base = p.coefp + ((size_t)d * Bp + m0) * pitch + (size_t)(n0 >> 5) * kHalfBytes;
+    if (empty) return;  // (the backward leaves the block's halves alone)
+    asm volatile("" ::: "memory");
+    const int shift = pow2_exponent(sb) - (word & ~3), pitch = half_pitch(Tp);
+    const size_t corner = ((size_t)d * Bp + m0) * pitch + (size_t)(n0 >> 5) * kHalfBytes;
     const uint32_t off = (uint32_t)((4 * hl + odd) * pitch + (cl & ~1) * 2);
+    auto pack = [&](char* base, auto one_by_one, auto&& value) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        // row 2 i + odd of this lane's half
-        const float got = swap1(odd ? c[2 * i] : c[2 * i + 1]);
-        const float x = odd ? got : c[2 * i], y = odd ? c[2 * i + 1] : got;
-        uint32_t w[2];
-        split2_f16(x * up, y * up, w);
-        char* const q = base + (size_t)(8 * (i >> 1) + 2 * (i & 1)) * pitch;
+        for (int i = 0; i < 8; ++i) {
+            if (decltype(one_by_one)::value) __builtin_amdgcn_sched_barrier(0);
+            // row 2 i + odd of this lane's half
+            const float even_row = value(2 * i), odd_row = value(2 * i + 1);
+            const float got = swap1(odd ? even_row : odd_row);
+            const float x = odd ? got : even_row, y = odd ? odd_row : got;
+            uint32_t w[2];
+            split2_f16(x, y, w);
+            char* const q = base + (size_t)(8 * (i >> 1) + 2 * (i & 1)) * pitch;
 #pragma unroll
-        for (int k = 0; k < 2; ++k) *reinterpret_cast<uint32_t*>(q + off + 64 * k) = w[k];
-    }
+            for (int k = 0; k < 2; ++k) *reinterpret_cast<uint32_t*>(q + off + 64 * k) = w[k];
+        }
+    };
+    auto scaled = [&](int r) __attribute__((always_inline)) { return ldexpf(c[r] * scale_of_row(r), shift); };
+    pack(p.coefp + corner, std::false_type{}, scaled);
+    if (!(word & 1)) return;
+    // seldom: once more, in two parts (and from the coefficients, instead of what would have to be kept for it)
+    auto apart = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) asm volatile("" : "+v"(c[r])::"memory");
+    };
+    apart();
+    pack(p.coefp + corner, std::true_type{}, [&](int r) { const float v = scaled(r); return fabsf(v) < kSmallCoef ? 0.f : v; });
+    apart();
+    pack(p.small + corner, std::true_type{}, [&](int r) { const float v = scaled(r); return fabsf(v) < kSmallCoef ? ldexpf(v, kSmallShift) : 0.f; });
 }
 
 // The same from float32 coefficients in memory (the losses that are formed row by row): one wave
 // per 32 x 32 block.
 template <int DIST>
-__global__ __launch_bounds__(256) void k_coef_halves(ScoreShape sh, const float* __restrict__ coef,
-                                                     const uint32_t* __restrict__ nearflag, const float* __restrict__ scale,
+__global__ __launch_bounds__(256) void k_coef_halves(ScoreShape sh, const float* __restrict__ coef, const float* __restrict__ scale,
                                                      int n_head, SplitCoef p) {
     const int lane = threadIdx.x & 63, MT = p.Bp >> 5, NT = p.Tp >> 5;
     const int g = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int d = g / (MT * NT), mt = (g - d * MT * NT) / NT, nt = g % NT;
     if (d >= sh.S || 32 * nt >= tail_limit(sh.tcount, d, sh.T, sh.tpad)) return;
     const float* src = coef + (size_t)d * sh.B * sh.T;
-    const bool skip = DIST == DIST_L2 && nearflag[((size_t)d * MT + mt) * NT + nt] != 0u;  // direct form
+    const bool near = DIST == DIST_L2 && p.exponent[((size_t)d * MT + mt) * NT + nt] == kDirect;  // as the forward left it
     const int n = 32 * nt + (lane & 31);
     const float sb = scale[n_head + d * sh.T + n];
     float c[16], sa[16];
@@ -340,9 +400,10 @@ __global__ __launch_bounds__(256) void k_coef_halves(ScoreShape sh, const float*
     for (int r = 0; r < 16; ++r) {
         const int m = 32 * mt + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
         sa[r] = scale[d * sh.B + m];
-        c[r] = (!skip && m < sh.B && n < sh.T) ? src[(size_t)m * sh.T + n] : 0.f;
+        c[r] = m < sh.B && n < sh.T ? src[(size_t)m * sh.T + n] : 0.f;
     }
-    store_coef_block<DIST>(c, [&](int r) { return sa[r]; }, sb, p, d, 32 * mt, 32 * nt, lane);
+    auto scale_a = [&](int r) __attribute__((always_inline)) { return sa[r]; };
+    store_coef_block<DIST>(c, scale_a, sb, near ? kDirect : coef_block_exponent(c, scale_a, sb, lane), p, d, 32 * mt, 32 * nt, lane);
 }
 
 // --------------------------------------------------------------------------
@@ -484,9 +545,9 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
 #pragma unroll
                     for (int r = 0; r < 16; ++r) loss_acc += val[r] - val[r];  // a pair that is not finite shows in the loss
             }
-            if (DIST == DIST_L2 && p.nearflag && lane1 == 0 && m0 + mb < Bp && n0 + nbk < Tp)
-                p.nearflag[((size_t)d * MT + ((m0 + mb) >> 5)) * NT + ((n0 + nbk) >> 5)] = flagged ? 1u : 0u;
-            if (OM != 0) {  // raw scores (and distances)
+            if (OM != 0) {  // raw scores (and distances), and which blocks the direct form is to take
+                if (DIST == DIST_L2 && lane1 == 0 && m0 + mb < Bp && n0 + nbk < Tp)
+                    p.out.exponent[((size_t)d * MT + ((m0 + mb) >> 5)) * NT + ((n0 + nbk) >> 5)] = flagged ? kDirect : kNoExponent;
                 float* const out = p.coef + (size_t)d * B * T;
                 float* const out_d = (DIST == DIST_L2 && p.dist) ? p.dist + (size_t)d * B * T : nullptr;
 #pragma unroll
@@ -537,17 +598,17 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
                 }
                 __builtin_amdgcn_sched_barrier(0);  // no more rows' intermediate values at once
             }
-            if (flagged) {  // the backward takes this block in the direct form, from the coefficients as they are
+            asm volatile("" ::: "memory");
+            const int word = flagged ? kDirect : coef_block_exponent(c, scale_a, sb, lane1);
+            if (word == kDirect) {  // the backward takes this block in the direct form, from the coefficients as they are
                 char* const out = (char*)(p.coef + ((size_t)d * B + m0 + mb) * T + n0 + nbk);
                 const uint32_t off = (uint32_t)(4 * hl * T + cl) * 4;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     if (scale_a(r) != 0.f && sb != 0.f) *reinterpret_cast<float*>(out + (size_t)(8 * (r >> 2) + (r & 3)) * T * 4 + off) = c[r];
-                    c[r] = 0.f;
                 }
             }
-            asm volatile("" ::: "memory");
-            store_coef_block<DIST>(c, scale_a, sb, p.out, d, m0 + mb, n0 + nbk, lane1);
+            store_coef_block<DIST>(c, scale_a, sb, word, p.out, d, m0 + mb, n0 + nbk, lane1);
         }
     if (OM == 0) {
         loss_acc = wave_sum(loss_acc);
@@ -566,198 +627,209 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
 // backward.  out[i, k] = sum_j c[i, j] phi(self[i, k], other[j, k]), phi = other (dot) or self - other
 // (L2: self[i, k] sum_j c[i, j] - the product).  Head side: i = heads, the coefficient rows lie along
 // the contraction.  Tail side: i = tails, they lie across it.  `other` always lies across it.
+//
+// The sub-blocks' own scales: a wave's sums stand in that of the last slab, and are brought to the next one's where that
+// differs.  Sums a long way above a slab's scale would not fit it, so a pass takes the slabs within 2^32 of the wave's
+// first.  What that leaves, the matrix of small coefficients and the sub-blocks of the direct form are added to the
+// results by passes of their own.  They are rare (a table of ordinary rows has none), and all of their code stands behind the main
+// pass's, from the kernel's arguments on: in one loop with it, it cost that registers and, through what lay between its
+// instructions, 1.5 of 8 us (4 blocks of 200 x 268, D = 100).
+constexpr int kMainPass = 8, kSmallPass = 24;  // pass: that of the slabs around the wave's first, plus the distance / 2^64
+constexpr uint32_t kDirectPass = 1u << 31;
 
 template <int DIST, bool SIDE_B, class Tile>
-DEVINL void split_bwd_tile(const SplitBwd& p, int d, int tile_x, int tile_y, char* smem, float* csum_s, float* scale_s) {
-    constexpr int TM = Tile::TM, TN = Tile::TN, WM = Tile::WM, WN = Tile::WN, kSums = Tile::threads / TM;
+struct SplitBwdTile {
+    static constexpr int TM = Tile::TM, TN = Tile::TN, WM = Tile::WM, WN = Tile::WN, kSums = Tile::threads / TM;
     using TA = std::conditional_t<SIDE_B, ColTile<TM, 2>, RowTile<TM, 2>>;
     using P = SplitProduct<TA, ColTile<TN, 2>, Tile>;
-    const int i0 = tile_y * TM, kt0 = tile_x * TN;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int B = p.B, T = p.T, Dp = p.rows.Dp, Kp = p.rows.Kp, Bp = p.in.Bp, Tp = p.in.Tp, MT = Bp >> 5, NT = Tp >> 5, pitch = half_pitch(Kp);
+    static_assert(P::AM == 1 && P::AN == 1, "one sub-block to a wave and slab");
+    const SplitBwd& p;
+    char* const smem;
+    float* const csum_s;
+    int* const exp_s;
+    const int tid, d, i0, kt0;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
+    const int B = p.B, T = p.T, Dp = p.rows.Dp, Kp = p.rows.Kp, Bp = p.in.Bp, Tp = p.in.Tp, MT = Bp >> 5, NT = Tp >> 5;
+    const int pitch = half_pitch(Kp), coef_pitch = half_pitch(Tp);
     const int t_live = tail_limit(p.tcount, d, T, p.tpad);  // merged tails: the block's live columns
     const int n_self = SIDE_B ? t_live : B, n_other = SIDE_B ? B : t_live, n_slab = (n_other + 31) >> 5;
-    if (i0 >= n_self) return;
-    const int head0 = d * B, tail0 = p.rows.n_head + d * T, self0 = SIDE_B ? tail0 : head0, other0 = SIDE_B ? head0 : tail0;
-    const int coef_pitch = half_pitch(Tp);
-    const char* const coef = p.in.coefp + (size_t)d * Bp * coef_pitch;
-    const char* const a = SIDE_B ? coef + (size_t)(i0 >> 5) * kHalfBytes : coef + (size_t)i0 * coef_pitch;
-    const char* const b = p.rows.halves + (int64_t)other0 * pitch + (size_t)(kt0 >> 5) * kHalfBytes;
-    const uint32_t* const nflag = DIST == DIST_L2 ? p.nearflag + (size_t)d * MT * NT : nullptr;
-    const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
+    const int self0 = SIDE_B ? p.rows.n_head + d * T : d * B, other0 = SIDE_B ? d * B : p.rows.n_head + d * T;
+
+    DEVINL SplitBwdTile(const SplitBwd& p_, char* smem_, float* csum, int* exps, int tid_, int d_, int tile_x, int tile_y)
+        : p(p_), smem(smem_), csum_s(csum), exp_s(exps), tid(tid_), d(d_), i0(tile_y * TM), kt0(tile_x * TN) {}
+
     // a sub-block's exponent: of the self rows' group st and of slab ot
-    const int* const exps = p.in.exponent + (size_t)d * MT * NT;
-    const int st0 = (i0 + wm) >> 5, st_last = (SIDE_B ? NT : MT) - 1;
-    int exp_reg[P::AM], exp_now[P::AM];  // of slab 64 n + lane; what the accumulators are in (kNoExponent: they are empty)
-    auto load_exps = [&](int slab0) __attribute__((always_inline)) {
-        const int ot = min(slab0 + lane, n_slab - 1);
+    DEVINL int exponent_of(int st, int ot) const { return p.in.exponent[(size_t)d * MT * NT + (SIDE_B ? (size_t)ot * NT + st : (size_t)st * NT + ot)]; }
+
+    // MAIN: the main pass, what this wave leaves to `todo`, whether any of the workgroup's does; or pass `pass`, added to the results
+    template <bool MAIN>
+    DEVINL bool sums(int pass, uint32_t& todo) const {
+        const size_t corner = (size_t)d * Bp * coef_pitch + (SIDE_B ? (size_t)(i0 >> 5) * kHalfBytes : (size_t)i0 * coef_pitch);
+        const char* const a = (MAIN || pass < 16 ? p.in.coefp : p.in.small) + corner;
+        const char* const b = p.rows.halves + (int64_t)other0 * pitch + (size_t)(kt0 >> 5) * kHalfBytes;
+        const bool alive = i0 + wm < n_self;  // any of the wave's rows
+        const int st0 = min((i0 + wm) >> 5, (SIDE_B ? NT : MT) - 1);  // (rows past the last are dropped)
+        int exp_reg;  // of slab 64 n + lane
+        auto load_exps = [&](int slab0) __attribute__((always_inline)) { exp_reg = exponent_of(st0, min(slab0 + lane, n_slab - 1)); };
+        constexpr int kNone = kDirect + 4;
+        int first = kNone, now = kNone;  // the wave's first slab's exponent; what the sums are in
+        floatx16 big[1][1], small[1][1];
+        P::run(smem, a, coef_pitch, SIDE_B ? (size_t)32 * coef_pitch : kHalfBytes, b, pitch, (size_t)32 * pitch, n_slab, n_other, big, small, lane, wave,
+               [&]() __attribute__((always_inline)) {
+                   load_exps(0);
+                   if (!MAIN) return;
+                   if (tid < TM) exp_s[tid] = pow2_exponent(p.rows.scale[self0 + i0 + tid]);
+                   if (DIST != DIST_L2) return;
+                   // the self rows' coefficient sums, from the sub-blocks' in a fixed order: kSums threads to a row, four
+                   // loads of each under way
+                   const int i = tid % TM, n = SIDE_B ? MT : n_slab;
+                   if (i0 + i < (SIDE_B ? Tp : Bp)) {
+                       const float* part = SIDE_B ? p.in.colpart + (size_t)d * MT * Tp + i0 + i : p.in.rowpart + ((size_t)d * Bp + i0 + i) * NT;
+                       const size_t step = SIDE_B ? Tp : 1;
+                       float s = 0.f;
+                       for (int q = tid / TM; q < n; q += 4 * kSums) {
+                           float v[4];
 #pragma unroll
-        for (int m = 0; m < P::AM; ++m) {
-            const int st = min(st0 + m, st_last);  // (rows past the last are dropped)
-            exp_reg[m] = exps[SIDE_B ? (size_t)ot * NT + st : (size_t)st * NT + ot];
-        }
-    };
-    floatx16 big[P::AM][P::AN], small[P::AM][P::AN];
-    bool seen = false;  // a flagged block among the tile's (the wave's share of them)
-    exp_now[0] = kNoExponent;
-    P::run(smem, a, coef_pitch, SIDE_B ? (size_t)32 * coef_pitch : kHalfBytes, b, pitch, (size_t)32 * pitch, n_slab, n_other, big, small, lane, wave,
-           [&]() __attribute__((always_inline)) {
-               load_exps(0);
-               if (tid < TM) scale_s[tid] = p.rows.scale[self0 + i0 + tid];
-               if (DIST != DIST_L2) return;
-               // the self rows' coefficient sums, from the sub-blocks' in a fixed order: kSums threads to a row, four
-               // loads of each under way
-               const int i = tid % TM, n = SIDE_B ? MT : n_slab;
-               if (i0 + i < (SIDE_B ? Tp : Bp)) {
-                   const float* part = SIDE_B ? p.in.colpart + (size_t)d * MT * Tp + i0 + i : p.in.rowpart + ((size_t)d * Bp + i0 + i) * NT;
-                   const size_t step = SIDE_B ? Tp : 1;
-                   float s = 0.f;
-                   for (int q = tid / TM; q < n; q += 4 * kSums) {
-                       float v[4];
-#pragma unroll
-                       for (int x = 0; x < 4; ++x) v[x] = q + x * kSums < n ? part[(q + x * kSums) * step] : 0.f;
-                       s += (v[0] + v[1]) + (v[2] + v[3]);
-                   }
-                   csum_s[tid] = s;
-               } else {
-                   csum_s[tid] = 0.f;
-               }
-               uint32_t flags = 0u;
-               for (int x = tid; x < TM / 32 * n_slab; x += Tile::threads) {
-                   const int st = (i0 >> 5) + x / n_slab, ot = x % n_slab;
-                   if (SIDE_B ? st < NT : st < MT) flags |= SIDE_B ? nflag[(size_t)ot * NT + st] : nflag[(size_t)st * NT + ot];
-               }
-               seen = __ballot(flags != 0u) != 0u;
-           },
-           [&](int slab) __attribute__((always_inline)) {
-               if (slab && !(slab & 63)) load_exps(slab);
-#pragma unroll
-               for (int m = 0; m < P::AM; ++m) {
-                   const int e = __builtin_amdgcn_readlane(exp_reg[m], slab & 63);
-                   if (e != exp_now[m] && e != kNoExponent) {  // seldom: what is there is brought to the slab's scale
-                       static_assert(P::AM == 1, "one exponent to a wave's slab");
-                       if (exp_now[m] == kNoExponent) {  // nothing yet
-                           exp_now[m] = e;
-                           continue;
+                           for (int x = 0; x < 4; ++x) v[x] = q + x * kSums < n ? part[(q + x * kSums) * step] : 0.f;
+                           s += (v[0] + v[1]) + (v[2] + v[3]);
                        }
-                       // (a slab 2^80 below what has been summed counts for nothing, and that would not fit its scale)
-                       if (exp_now[m] - e > 80) return false;
-                       const float by = __uint_as_float((uint32_t)(127 + max(exp_now[m] - e, -126)) << 23);
-#pragma unroll
-                       for (int n = 0; n < P::AN; ++n)
-#pragma unroll
-                           for (int r = 0; r < 16; ++r) {
-                               big[m][n][r] *= by;
-                               small[m][n][r] *= by;
-                           }
-                       exp_now[m] = e;
+                       csum_s[tid] = s;
+                   } else {
+                       csum_s[tid] = 0.f;
                    }
-               }
-               return true;
-           });
-    const int lane1 = (int)lane_here(), cl = lane1 & 31, hl = lane1 >> 5;
-    // the self rows' own scales leave the sums
+               },
+               [&](int slab) __attribute__((always_inline)) {
+                   if (slab && !(slab & 63)) load_exps(slab);
+                   const int word = __builtin_amdgcn_readlane(exp_reg, slab & 63);
+                   if (MAIN && word == now) return true;  // the rule
+                   if (!alive || word >= kNoExponent) {
+                       if (MAIN && alive && word == kDirect) todo |= kDirectPass;
+                       return false;
+                   }
+                   int e = word & ~3;
+                   if (first == kNone) first = e;
+                   const int here = kMainPass + ((e - first + 32) >> 6), of_small = kSmallPass + ((e - kSmallShift - first + 32) >> 6);
+                   if (MAIN) {
+                       if (word & 1) todo |= 1u << of_small;
+                       if (here != kMainPass) {
+                           todo |= 1u << here;
+                           return false;
+                       }
+                   } else {
+                       if (pass < 16 ? pass != here : !(word & 1) || pass != of_small) return false;
+                       if (pass >= 16) e -= kSmallShift;
+                   }
+                   if (now != kNone) {
+                       const float by = __uint_as_float((uint32_t)(127 + now - e) << 23);
 #pragma unroll
-    for (int m = 0; m < P::AM; ++m) {
-        const float scale = exp_now[m] == kNoExponent ? 1.f : __uint_as_float((uint32_t)(127 + exp_now[m]) << 23);
+                       for (int r = 0; r < 16; ++r) {
+                           big[0][0][r] *= by;
+                           small[0][0][r] *= by;
+                       }
+                   }
+                   now = e;
+                   return true;
+               });
+        const bool any = MAIN && __syncthreads_or(todo != 0u);  // (here: behind the results' stores it would wait for those)
+        const int lane1 = (int)lane_here(), cl = lane1 & 31, hl = lane1 >> 5;
+        // the self rows' own scales leave the sums
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float up = pow2_inverse(scale_s[wm + 32 * m + 8 * (r >> 2) + 4 * hl + (r & 3)]);
+        for (int r = 0; r < 16; ++r)
+            big[0][0][r] = ldexpf(fmaf(small[0][0][r], kHalfStep, big[0][0][r]),
+                                  (now == kNone ? 0 : now) - exp_s[wm + 8 * (r >> 2) + 4 * hl + (r & 3)]);
+        const char* const self = p.rows.halves + (int64_t)(self0 + i0) * pitch;
+        // neighbouring lanes swap values: a lane stores two columns of one row
+        const bool odd = lane1 & 1;
+        float* const out = p.grad + (size_t)(self0 + i0) * Dp;
+        const int k = kt0 + wn + (cl & ~1);
+        if (k >= Dp) return any;
+        // (a row: the wave's part, in scalars, and the lane's, in one offset for all of them)
+        const uint32_t in_off = (uint32_t)((4 * hl + odd) * pitch + (k >> 5) * kHalfBytes + (k & 31) * 2);
+        const uint32_t lost_off = (uint32_t)((4 * hl + odd) * (Kp >> 5) + (k >> 5)) * 4;
+        const uint32_t out_off = (uint32_t)((4 * hl + odd) * Dp + k) * 4;
+        auto wave_row = [&](int i) __attribute__((always_inline)) { return wm + 8 * (i >> 1) + 2 * (i & 1); };
+        constexpr bool kSelf = MAIN && DIST == DIST_L2;
+        uint32_t w[kSelf ? 8 : 1][3];
+        if (kSelf)
 #pragma unroll
-            for (int n = 0; n < P::AN; ++n) big[m][n][r] = fmaf(small[m][n][r], kHalfStep, big[m][n][r]) * scale * up;
-        }
-    }
-    const char* const self = p.rows.halves + (int64_t)(self0 + i0) * pitch;
-    // neighbouring lanes swap values: a lane stores two columns of one row
-    const bool odd = lane1 & 1;
-    float* const out = p.grad + (size_t)(self0 + i0) * Dp;
+            for (int i = 0; i < 8; ++i) {  // all loads before any use, rows past the last among them
+                const char* const row = self + (int64_t)wave_row(i) * pitch;
 #pragma unroll
-    for (int mi = 0; mi < P::AM; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < P::AN; ++ni) {
-            const int k = kt0 + wn + 32 * ni + (cl & ~1);
-            if (k >= Dp) continue;
-            // (a row: the wave's part, in scalars, and the lane's, in one offset for all of them)
-            const uint32_t in_off = (uint32_t)((4 * hl + odd) * pitch + (k >> 5) * kHalfBytes + (k & 31) * 2);
-            const uint32_t lost_off = (uint32_t)((4 * hl + odd) * (Kp >> 5) + (k >> 5)) * 4;
-            const uint32_t out_off = (uint32_t)((4 * hl + odd) * Dp + k) * 4;
-            auto wave_row = [&](int i) __attribute__((always_inline)) { return wm + 32 * mi + 8 * (i >> 1) + 2 * (i & 1); };
-            uint32_t w[DIST == DIST_L2 ? 8 : 1][3];
-            if (DIST == DIST_L2)
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {  // all loads before any use, rows past the last among them
-                    const char* const row = self + (int64_t)wave_row(i) * pitch;
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) w[i][q] = *reinterpret_cast<const uint32_t*>(row + in_off + 64 * q);
-                    w[i][2] = *reinterpret_cast<const uint32_t*>((const char*)(p.rows.lost + (int64_t)(self0 + i0 + wave_row(i)) * (Kp >> 5)) + lost_off);
-                }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float got = swap1(odd ? big[mi][ni][2 * i] : big[mi][ni][2 * i + 1]);
-                float x = odd ? got : big[mi][ni][2 * i], y = odd ? big[mi][ni][2 * i + 1] : got;
-                const int row = wave_row(i) + 4 * hl + odd;
-                if (DIST == DIST_L2) {
-                    const f16x2 h = __builtin_bit_cast(f16x2, w[i][0]), l = __builtin_bit_cast(f16x2, w[i][1]);
-                    float sum = csum_s[row];
-#pragma unroll
-                    for (int q = 1; q < kSums; ++q) sum += csum_s[row + q * TM];
-                    sum *= scale_s[row];
-                    // (every bit of the self row: against this product the other one is small)
-                    const uint32_t lost = w[i][2] >> lost_at(k);
-                    x = join_lost(h.x, l.x, lost & 1u) * sum - x;
-                    y = join_lost(h.y, l.y, (lost >> 8) & 1u) * sum - y;
-                }
-                if (i0 + row < n_self) *reinterpret_cast<float2*>((char*)(out + (size_t)wave_row(i) * Dp) + out_off) = make_float2(x, y);
+                for (int q = 0; q < 2; ++q) w[i][q] = *reinterpret_cast<const uint32_t*>(row + in_off + 64 * q);
+                w[i][2] = *reinterpret_cast<const uint32_t*>((const char*)(p.rows.lost + (int64_t)(self0 + i0 + wave_row(i)) * (Kp >> 5)) + lost_off);
             }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float got = swap1(odd ? big[0][0][2 * i] : big[0][0][2 * i + 1]);
+            float x = odd ? got : big[0][0][2 * i], y = odd ? big[0][0][2 * i + 1] : got;
+            const int row = wave_row(i) + 4 * hl + odd;
+            if (kSelf) {
+                const f16x2 h = __builtin_bit_cast(f16x2, w[i][0]), l = __builtin_bit_cast(f16x2, w[i][1]);
+                float sum = csum_s[row];
+#pragma unroll
+                for (int q = 1; q < kSums; ++q) sum += csum_s[row + q * TM];
+                sum = ldexpf(sum, exp_s[row]);
+                // (every bit of the self row: against this product the other one is small)
+                const uint32_t lost = w[i][2] >> lost_at(k);
+                x = join_lost(h.x, l.x, lost & 1u) * sum - x;
+                y = join_lost(h.y, l.y, (lost >> 8) & 1u) * sum - y;
+            }
+            if (i0 + row >= n_self) continue;
+            float2* const at = reinterpret_cast<float2*>((char*)(out + (size_t)wave_row(i) * Dp) + out_off);
+            *at = MAIN ? make_float2(x, y) : DIST == DIST_L2 ? make_float2(at->x - x, at->y - y) : make_float2(at->x + x, at->y + y);
         }
-    if (DIST != DIST_L2 || !__syncthreads_or(seen)) return;
-    __syncthreads();
-    // sub-blocks in which some pair is nearly identical: c (self - other) directly, as the reference codelet
-    // does (their coefficients went into the product as zeros), added to what the workgroup has just
+        return any;
+    }
+
+    // the direct form: c (self - other), or c other, one pair after the other as the reference codelet does (sub-blocks in
+    // which some pair is nearly identical, or coefficients that halves do not hold), added to what the workgroup has
     // stored.  A wave takes four rows at a time, a lane a column.
-    static_assert(TN == 64, "a lane per column");
-    const float* const cf = p.coef + (size_t)d * B * T;
-    const int k = kt0 + (int)lane_here();
-    if (k >= Dp) return;
-    for (int i = i0 + 4 * wave; i < min(i0 + TM, n_self); i += 4 * WM * WN) {
-        float add[4] = {0.f, 0.f, 0.f, 0.f};
-        int row[4];
+    DEVINL void direct() const {
+        static_assert(TN == 64, "a lane per column");
+        const float* const cf = p.coef + (size_t)d * B * T;
+        const int k = kt0 + (int)lane_here();
+        if (k >= Dp) return;
+        for (int i = i0 + 4 * wave; i < min(i0 + TM, n_self); i += 4 * WM * WN) {
+            float add[4] = {0.f, 0.f, 0.f, 0.f};
+            int row[4];
 #pragma unroll
-        for (int x = 0; x < 4; ++x) row[x] = min(i + x, n_self - 1);
-        bool any = false;
-        for (int ot = 0; ot < n_slab; ++ot) {
-            if (nflag[SIDE_B ? (size_t)ot * NT + (i >> 5) : (size_t)(i >> 5) * NT + ot] == 0u) continue;
-            any = true;
-            float sv[4];
+            for (int x = 0; x < 4; ++x) row[x] = min(i + x, n_self - 1);
+            bool any = false;
+            for (int ot = 0; ot < n_slab; ++ot) {
+                if (exponent_of(i >> 5, ot) != kDirect) continue;
+                any = true;
+                float sv[4];
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                Row1 raw;
-                raw.load(p.rows, self0 + row[x], k);
-                sv[x] = raw.value(k);
-            }
-#pragma unroll 1
-            for (int j0 = 32 * ot; j0 < min(32 * ot + 32, n_other); j0 += 4) {
-                Row1 raw[4];
-                float c[4][4];
-#pragma unroll
-                for (int y = 0; y < 4; ++y) {
-                    const int j = min(j0 + y, n_other - 1);
-                    raw[y].load(p.rows, other0 + j, k);
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) c[y][x] = j0 + y < n_other ? (SIDE_B ? cf[(size_t)j * T + row[x]] : cf[(size_t)row[x] * T + j]) : 0.f;
+                for (int x = 0; x < 4; ++x) {
+                    Row1 raw;
+                    raw.load(p.rows, self0 + row[x], k);
+                    sv[x] = raw.value(k);
                 }
+#pragma unroll 1
+                for (int j0 = 32 * ot; j0 < min(32 * ot + 32, n_other); j0 += 2) {
+                    Row1 raw[2];
 #pragma unroll
-                for (int y = 0; y < 4; ++y)
+                    for (int y = 0; y < 2; ++y) raw[y].load(p.rows, other0 + min(j0 + y, n_other - 1), k);
 #pragma unroll
-                    for (int x = 0; x < 4; ++x) add[x] = fmaf(c[y][x], sv[x] - raw[y].value(k), add[x]);
+                    for (int y = 0; y < 2; ++y) {
+                        const int j = min(j0 + y, n_other - 1);
+                        const float other = raw[y].value(k);
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            const float c = j0 + y < n_other ? (SIDE_B ? cf[(size_t)j * T + row[x]] : cf[(size_t)row[x] * T + j]) : 0.f;
+                            add[x] = fmaf(c, DIST == DIST_L2 ? sv[x] - other : other, add[x]);
+                        }
+                    }
+                }
             }
-        }
-        if (!any) continue;
+            if (!any) continue;
 #pragma unroll
-        for (int x = 0; x < 4; ++x)
-            if (i + x < n_self) p.grad[(size_t)(self0 + i + x) * Dp + k] += add[x];
+            for (int x = 0; x < 4; ++x)
+                if (i + x < n_self) p.grad[(size_t)(self0 + i + x) * Dp + k] += add[x];
+        }
     }
-}
+};
 
 // Both sides in one launch: the side whose tiles loop over more rows comes first, for every block, so
 // that the long tiles do not start last.  A block's tiles of one side stay together on one XCD.
@@ -766,18 +838,51 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
     constexpr int TM = Tile::TM, TN = Tile::TN;
     using PA = SplitProduct<RowTile<TM, 2>, ColTile<TN, 2>, Tile>;
     __shared__ __attribute__((aligned(16))) char smem[PA::kLds];
-    __shared__ float csum_s[Tile::threads], scale_s[TM];
-    const int gx = (p.rows.Dp + TN - 1) / TN, ga = (p.B + TM - 1) / TM, gb = (p.T + TM - 1) / TM;
-    const bool heads_first = p.T >= p.B;
-    const int n_first = gx * (heads_first ? ga : gb) * p.S;
-    const int L = blockIdx.x;
-    if ((L < n_first) == heads_first) {
-        const TileId tile = xcd_tile(gx, ga, p.S, heads_first ? L : L - n_first);
-        split_bwd_tile<DIST, false, Tile>(p, tile.z, tile.x, tile.y, smem, csum_s, scale_s);
-    } else {
-        const TileId tile = xcd_tile(gx, gb, p.S, heads_first ? L - n_first : L);
-        split_bwd_tile<DIST, true, Tile>(p, tile.z, tile.x, tile.y, smem, csum_s, scale_s);
+    __shared__ float csum_s[Tile::threads];
+    __shared__ int exp_s[TM];
+    // tile L's work: with(its side, its place)
+    auto place = [](const SplitBwd& q, int L, auto&& with) __attribute__((always_inline)) {
+        const int gx = (q.rows.Dp + TN - 1) / TN, ga = (q.B + TM - 1) / TM, gb = (q.T + TM - 1) / TM;
+        const bool heads_first = q.T >= q.B;
+        const int n_first = gx * (heads_first ? ga : gb) * q.S;
+        if ((L < n_first) == heads_first) with(std::false_type{}, xcd_tile(gx, ga, q.S, heads_first ? L : L - n_first));
+        else with(std::true_type{}, xcd_tile(gx, gb, q.S, heads_first ? L - n_first : L));
+    };
+    uint32_t todo = 0u;
+    bool any = false;
+    place(p, blockIdx.x, [&](auto side_b, const TileId& t) __attribute__((always_inline)) {
+        const SplitBwdTile<DIST, decltype(side_b)::value, Tile> tile(p, smem, csum_s, exp_s, threadIdx.x, t.z, t.x, t.y);
+        if (tile.i0 < tile.n_self) any = tile.template sums<true>(kMainPass, todo);
+    });
+    if (__builtin_expect(!__builtin_amdgcn_readfirstlane((int)any), 1)) return;
+    // seldom.  Nothing that the main pass has computed is kept for this, nor from one pass for the next.
+    auto anew = [&](auto&& with) __attribute__((always_inline)) {
+        auto args = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
+        int L = blockIdx.x, tid = threadIdx.x;
+        asm volatile("" : "+s"(args), "+s"(L), "+v"(tid));
+        struct Words { uint32_t w[sizeof(SplitBwd) / 4]; } words;
+        static_assert(sizeof(Words) == sizeof(SplitBwd));
+#pragma unroll
+        for (size_t i = 0; i < sizeof(SplitBwd) / 4; ++i) words.w[i] = args[i];
+        const SplitBwd q = __builtin_bit_cast(SplitBwd, words);
+        place(q, L, [&](auto side_b, const TileId& t) __attribute__((always_inline)) {
+            with(SplitBwdTile<DIST, decltype(side_b)::value, Tile>(q, smem, csum_s, exp_s, tid, t.z, t.x, t.y));
+        });
+    };
+    __syncthreads();
+    uint32_t* const all = reinterpret_cast<uint32_t*>(csum_s);  // (no longer read)
+    if (threadIdx.x == 0) *all = 0u;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0 && todo) atomicOr(all, todo);
+    __syncthreads();
+    todo = (uint32_t)__builtin_amdgcn_readfirstlane((int)*all);
+#pragma unroll 1
+    for (; todo & ~kDirectPass; todo &= todo - 1u) {
+        uint32_t none = 0u;
+        anew([&](auto&& tile) __attribute__((always_inline)) { tile.template sums<false>(__ffs((int)todo) - 1, none); });
+        __syncthreads();  // (of the tiles in LDS, too)
     }
+    if (todo) anew([](auto&& tile) __attribute__((always_inline)) { tile.direct(); });
 }
 
 // --------------------------------------------------------------------------
@@ -814,12 +919,11 @@ void launch_split_fwd(const SplitFwd& p, bool fused_loss, hipStream_t stream) {
     else fused_loss ? split_fwd<DIST_DOT, 0>(p, stream) : split_fwd<DIST_DOT, 1>(p, stream);
 }
 
-void launch_coef_halves(const ScoreShape& sh, const float* coef, const uint32_t* nearflag, const SplitRows& rows,
-                        const SplitCoef& out, hipStream_t stream) {
+void launch_coef_halves(const ScoreShape& sh, const float* coef, const SplitRows& rows, const SplitCoef& out, hipStream_t stream) {
     const int n = sh.S * (out.Bp / 32) * (out.Tp / 32);
     const bool l2 = sh.dist_fn == DIST_L2 && sh.score_fn != SCORE_DISTMULT;
 #define KGE_COEF(D_) \
-    hipLaunchKernelGGL(k_coef_halves<D_>, dim3((n + 3) / 4), dim3(256), 0, stream, sh, coef, nearflag, rows.scale, rows.n_head, out)
+    hipLaunchKernelGGL(k_coef_halves<D_>, dim3((n + 3) / 4), dim3(256), 0, stream, sh, coef, rows.scale, rows.n_head, out)
     if (l2) KGE_COEF(DIST_L2);
     else KGE_COEF(DIST_DOT);
 #undef KGE_COEF
