@@ -64,10 +64,10 @@ constexpr float kHalfStep = 1.f / 2048.f;
 constexpr int kHalfBytes = 128;  // of 32 columns of a row
 
 // the scale for a largest magnitude (not negative; infinities and NaN take some scale, their halves say the rest).
-// Rows below 2^-40 share one, so that the product of two rows' scales stays a normal number.  Rows of zeros, which any scale
-// would do for, have an ordinary row's: their coefficients carry it and stand beside the other rows' in one block.
+// Rows below 2^-112 share one: it and its reciprocal are normal numbers.  Rows of zeros, which any scale would do for, have
+// an ordinary row's: their coefficients carry it and stand beside the other rows' in one block.
 DEVINL float half_scale(float largest) {
-    const int e = largest == 0.f ? 0 : min(max((int)(__float_as_uint(largest) >> 23) - 127, -40), 100);
+    const int e = largest == 0.f ? 0 : min(max((int)(__float_as_uint(largest) >> 23) - 127, -112), 127);
     return __uint_as_float((uint32_t)(e - 14 + 127) << 23);
 }
 // a power of two's exponent, its reciprocal

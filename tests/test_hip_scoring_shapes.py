@@ -307,6 +307,18 @@ def test_slabs_far_apart(oracle64, powers, side, loss_power):
     _assert_each_row(*_first_moments(c, state, batch, 2.0**loss_power, oracle64, **{"execution.merge_tails": False}))
 
 
+# The product of very long rows with very short ones is of an ordinary size
+@pytest.mark.parametrize("power", [-105, -90, -70, 70, 90, 105])
+def test_dot_of_long_and_short_rows(oracle64, power):
+    B, A, D = 70, 100, 64
+    c = K.cfg_dict(score_fn="DistMult", distance_fn="MatMul", n_shard=1, batch=B, a2a=A, dim=D, feature=0, n_entity=300,
+                   n_relation=B, gamma=4.0, shared_table=True)
+    rng = np.random.default_rng(7)
+    state = K.make_state(c, rng, warm=False, scale=0.25)
+    batch = _one_block(c, state, np.repeat([2.0**power, 2.0**-power], [B, A]), rng)
+    _assert_each_row(*_first_moments(c, state, batch, 1, oracle64))
+
+
 def _two_disjoint_blocks(kind, loss_fn, B, A, D, bad, merge):
     """One step of two blocks that share no row (entity or relation); `bad`: (role, value) of block 1's
     first head or tail, or None.  Returns the losses and block 0's rows afterwards."""

@@ -311,6 +311,41 @@ def test_predict_sweep_close_rows(dim, dtype, n_query, n_entity):
     assert np.all(np.sort(found.shard_idx[:, :, 1], axis=1) == np.arange(1, n_entity))
 
 
+@pytest.mark.parametrize("power", [-105, -90, 90, 105])
+@pytest.mark.parametrize("dim", [64, 250])
+def test_predict_sweep_of_long_and_short_rows(dim, power):
+    """Queries (ordinary heads with relations of 2^power) against rows of 2^-power: products of an ordinary size, each within
+    1e-6 of its two norms'."""
+    import poplar_kge as kge
+
+    settings = kge.Settings.create_demo()
+    m, ex = settings.model, settings.execution
+    m.score_fn, m.distance_fn = "DistMult", "MatMul"
+    m.n_shard, m.n_entity, m.embedding_size, m.entity_feature_size, m.n_relation_type = 1, 301, dim, 0, 4
+    settings.data.batch_size, settings.data.a2a_size, ex.rw_batch_size = 2, 2, 301
+    ex.predict_hr_batch_size, ex.predict_n_best = 40, 300
+    settings.prepare()
+    engine = kge.Engine(settings, np.array([300]))
+    rng = np.random.default_rng(8)
+    rows = np.zeros((1, 301, 3 * dim), np.float32)
+    rows[0, :, :dim] = rng.normal(size=(301, dim)) * np.where(np.arange(301) > 40, 2.0**-power, 1.0)[:, None]
+    relation = (rng.normal(size=(4, dim)) * 2.0**power).astype(np.float32)
+    for name in engine.uninitialized_variables.copy():
+        engine.write_variable(name, np.zeros(engine.variable_to_shape[name], engine.variable_to_dtype[name]))
+    engine.write_variable("relation_embedding", relation)
+    engine.write_entity_raw(0, rows)
+    queries = np.stack([np.zeros(40), 1 + np.arange(40), np.arange(40) % 4], axis=1).astype(np.uint32)
+    found = engine.predict(queries)
+    query = rows[0, queries[:, 1], :dim].astype(np.float64) * relation[queries[:, 2]]
+    for i in range(40):
+        of_size = found.shard_idx[i, :, 1] > 40
+        index = found.shard_idx[i, of_size, 1]
+        tails = rows[0, index, :dim].astype(np.float64)
+        bound = 1e-6 * np.linalg.norm(query[i]) * np.linalg.norm(tails, axis=1)
+        assert np.all(np.abs(found.score[i, of_size] - tails @ query[i]) <= bound)
+        np.testing.assert_array_equal(np.sort(index), np.arange(41, 301))
+
+
 @pytest.mark.parametrize("score_fn", ["TransE", "DistMult"])
 @pytest.mark.parametrize("dim,dtype", [(30, "float32"), (64, "float16"), (100, "float32"), (130, "float16"), (256, "float32"),
                                        (320, "float32"), (300, "float16")])
