@@ -166,34 +166,25 @@ struct SplitTile { static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, 
 using TileSmall = SplitTile<64, 64, 2, 2, 4>;
 using TileLarge = SplitTile<128, 64, 4, 2, 6>;
 
-// The product loop of a tile: n_slab slabs of 32 contraction steps, three tile copies in LDS
-// (two fill while the third is multiplied, one barrier per slab).  TA, TB: RowTile / ColTile;
-// a_step, b_step: bytes from slab to slab.  Waves as WM x WN, each (TM/WM) x (TN/WN) in 32 x 32
-// accumulators: `big` the products of first halves, `small` the cross products.
+// The product loop of a tile: n_slab slabs of 32 contraction steps, two tile copies in LDS
+// (one fills while the other is multiplied, one barrier per slab).  TA, TB: RowTile / ColTile;
+// a_step, b_step: bytes from slab to slab.  Each wave's 32 x 32 of the tile in two accumulators:
+// `big` the products of first halves, `small` the cross products.
 // b_rows: rows of `b` along the contraction where it lies across it (ColTile).  The last slab's rows past them
 // repeat the last one: their coefficients are zero, but what lies behind a block's rows are other
 // blocks', and zero times a neighbour's infinity or NaN would be this block's NaN.
 template <class TA, class TB, class Tile>
 struct SplitProduct {
-    static constexpr int kStages = 2;
-    static constexpr int NW = Tile::WM * Tile::WN, AM = Tile::TM / Tile::WM / 32, AN = Tile::TN / Tile::WN / 32;
-    static constexpr int kStage = TA::kBytes + TB::kBytes, kLds = kStages * kStage;
+    static constexpr int NW = Tile::WM * Tile::WN, kCopy = TA::kBytes + TB::kBytes, kLds = 2 * kCopy;
+    static_assert(Tile::TM == 32 * Tile::WM && Tile::TN == 32 * Tile::WN, "one 32 x 32 block to a wave");
     static constexpr int kCopies = TA::kCopies + TB::kCopies, kEach = kCopies / NW;
     static_assert(kCopies % NW == 0, "every wave issues the same number of copies");
 
-    static DEVINL void products(const floatx4 (&fa)[2], const floatx4 (&fb)[2], floatx16& big, floatx16& small) {
-        auto one = [&](int qa, int qb, floatx16& acc) __attribute__((always_inline)) {
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fa[qa]), __builtin_bit_cast(f16x8, fb[qb]), acc, 0, 0, 0);
-        };
-        one(0, 0, big);
-        one(0, 1, small);
-        one(1, 0, small);
-    }
     // meanwhile(): what the caller has to fetch for itself, under the first slab's way from memory;
     // before(slab): ahead of the slab's products, whether to form them
     template <class Meanwhile, class Before>
     static DEVINL void run(char* smem, const char* a, int a_pitch, size_t a_step, const char* b, int b_pitch, size_t b_step,
-                           int n_slab, int b_rows, floatx16 (&big)[AM][AN], floatx16 (&small)[AM][AN], int lane, int wave,
+                           int n_slab, int b_rows, floatx16& big, floatx16& small, int lane, int wave,
                            Meanwhile&& meanwhile, Before&& before) {
         uint32_t off[kEach];
 #pragma unroll
@@ -205,7 +196,7 @@ struct SplitProduct {
         auto fill = [&](int slab) __attribute__((always_inline)) {
             const char* as = a + slab * a_step;
             const char* bs = b + slab * b_step;
-            const uint32_t to = lds0 + slab % kStages * kStage;
+            const uint32_t to = lds0 + (slab & 1) * kCopy;
             if constexpr (!std::is_same_v<TB, RowTile<Tile::TN, 2>>) {
                 const int last = b_rows - 32 * slab - 1;
                 if (last < 31)  // the last slab's offsets take the others' place
@@ -222,39 +213,32 @@ struct SplitProduct {
             }
         };
         fill(0);
-        if (kStages > 2 && n_slab > 1) fill(1);
         meanwhile();
 #pragma unroll
-        for (int m = 0; m < AM; ++m)
-#pragma unroll
-            for (int n = 0; n < AN; ++n)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) big[m][n][r] = small[m][n][r] = 0.f;
-        const int wm = (wave / Tile::WN) * (Tile::TM / Tile::WM), wn = (wave % Tile::WN) * (Tile::TN / Tile::WN);
+        for (int r = 0; r < 16; ++r) big[r] = small[r] = 0.f;
+        const int wm = 32 * (wave / Tile::WN), wn = 32 * (wave % Tile::WN);
         for (int slab = 0; slab < n_slab; ++slab) {
-            // (a wave's copies arrive in order: all but the next slab's are there)
-            if (kStages > 2 && slab + 1 < n_slab) wait_copies_and_barrier<kEach>();
-            else wait_copies_and_barrier<0>();
+            wait_copies_and_barrier<0>();
             const bool count = before(slab);  // (ahead of the copies: behind them, its wait for
             // exponents that it may have loaded was one for the next slab, 55 -> 44 us of 16 blocks of 256 x 1536)
-            if (slab + kStages - 1 < n_slab) fill(slab + kStages - 1);
+            if (slab + 1 < n_slab) fill(slab + 1);
             if (!count) continue;
-            const char* ta = smem + slab % kStages * kStage;
+            const char* ta = smem + (slab & 1) * kCopy;
             const char* tb = ta + TA::kBytes;
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
-                floatx4 fa[AM][2], fb[AN][2];
+                floatx4 fa[2], fb[2];
 #pragma unroll
                 for (int q = 0; q < 2; ++q) {
-#pragma unroll
-                    for (int m = 0; m < AM; ++m) fa[m][q] = TA::fragment(ta, q, wm + 32 * m, ks, lane);
-#pragma unroll
-                    for (int n = 0; n < AN; ++n) fb[n][q] = TB::fragment(tb, q, wn + 32 * n, ks, lane);
+                    fa[q] = TA::fragment(ta, q, wm, ks, lane);
+                    fb[q] = TB::fragment(tb, q, wn, ks, lane);
                 }
-#pragma unroll
-                for (int m = 0; m < AM; ++m)
-#pragma unroll
-                    for (int n = 0; n < AN; ++n) products(fa[m], fb[n], big[m][n], small[m][n]);
+                auto product = [&](int qa, int qb, floatx16& acc) __attribute__((always_inline)) {
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fa[qa]), __builtin_bit_cast(f16x8, fb[qb]), acc, 0, 0, 0);
+                };
+                product(0, 0, big);
+                product(0, 1, small);
+                product(1, 0, small);
             }
         }
     }
@@ -433,7 +417,7 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
     const int pitch = half_pitch(Kp);
     const char* a = p.rows.halves + (int64_t)(a_row + m0) * pitch;
     const char* b = p.rows.halves + (int64_t)(b_row + n0) * pitch;
-    floatx16 big[P::AM][P::AN], small[P::AM][P::AN];
+    floatx16 big, small;
     P::run(smem, a, pitch, kHalfBytes, b, pitch, kHalfBytes, Kp / 32, 0, big, small, lane, wave, [&]() __attribute__((always_inline)) {
         for (int i = tid; i < TM; i += Tile::threads) {
             if (DIST == DIST_L2) na_s[i] = p.rows.norm[a_row + m0 + i];
@@ -448,7 +432,7 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
     }, [](int) { return true; });
 
     // epilogue.  Register r of lane l holds row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
-    const int wm = (wave / WN) * (TM / WM), wn = (wave % WN) * (TN / WN);
+    const int mb = 32 * (wave / WN), nbk = 32 * (wave % WN);  // the wave's block's corner in the tile
     const int lane1 = (int)lane_here(), tid1 = 64 * wave + lane1, cl = lane1 & 31, hl = lane1 >> 5;
     const float Tn = (float)T;
     const float w_pos = uniform_f32(0.5f * Tn), w_neg = uniform_f32((0.5f * Tn) / (float)(T - 1));
@@ -459,157 +443,150 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
     const float coef_scale = uniform_f32(inv_norm * sh.loss_scale * score_sign);
     const int Bp = p.out.Bp, Tp = p.out.Tp, MT = Bp >> 5, NT = Tp >> 5;
     float loss_acc = 0.f;
+    const int n = n0 + nbk + cl;
+    // columns behind a block's distinct tails repeat its first row, the most popular one more
+    // often than not: no pair of theirs is worth a second look
+    const bool col_counts = n < n_live;
+    const float sb = sb_s[nbk + cl];
+    float val[16];
+    const float* const sa = sa_s + mb + 4 * hl;
+    auto scale_a = [&](int r) __attribute__((always_inline)) { return sa[8 * (r >> 2) + (r & 3)]; };
+    const float nb = DIST == DIST_L2 ? nb_s[nbk + cl] : 0.f;
+    const float* const na = na_s + mb + 4 * hl;
+    auto norms = [&](int r) __attribute__((always_inline)) { return na[8 * (r >> 2) + (r & 3)] + nb; };
+    uint64_t redo = 0u;
 #pragma unroll
-    for (int mi = 0; mi < P::AM; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < P::AN; ++ni) {
-            const int mb = wm + 32 * mi, nbk = wn + 32 * ni;  // the sub-block's corner in the tile
-            const int n = n0 + nbk + cl;
-            // columns behind a block's distinct tails repeat its first row, the most popular one more
-            // often than not: no pair of theirs is worth a second look
-            const bool col_counts = n < n_live;
-            const float sb = sb_s[nbk + cl];
-            float val[16];
-            const float* const sa = sa_s + mb + 4 * hl;
-            auto scale_a = [&](int r) __attribute__((always_inline)) { return sa[8 * (r >> 2) + (r & 3)]; };
-            const float nb = DIST == DIST_L2 ? nb_s[nbk + cl] : 0.f;
-            const float* const na = na_s + mb + 4 * hl;
-            auto norms = [&](int r) __attribute__((always_inline)) { return na[8 * (r >> 2) + (r & 3)] + nb; };
-            uint64_t redo = 0u;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float product = fmaf(small[mi][ni][r], kHalfStep, big[mi][ni][r]);
-                if (DIST == DIST_L2) {
-                    const float ns = norms(r);
-                    val[r] = fmaf(product, -2.f * sb * scale_a(r), ns);
-                    redo |= __ballot(!(val[r] > kCancelRatio * ns));
-                } else {
-                    val[r] = product * scale_a(r) * sb;
-                    redo |= __ballot(!(fabsf(val[r]) < INFINITY));
-                }
-            }
-            bool flagged = false;
-            // rare: pairs are recomputed directly, half a wave to a pair, by all of the workgroup (a popular row's
-            // come together in one wave's block): those that cancelled, and those that are not finite (an infinity's
-            // second half is NaN).  Pairs that do not count, a NaN among them, get any finite value.
-            static_assert(P::AM == 1 && P::AN == 1, "one block to a wave");
-            if (__syncthreads_or(redo != 0u)) {
-                float* const result = reinterpret_cast<float*>(smem);  // [TM][TN]; the tiles are no longer needed
-                uint16_t* const list = reinterpret_cast<uint16_t*>(smem + TM * TN * 4);
-                static_assert(TM * TN * 6 <= P::kLds, "the tile's pairs as a list and as results");
-                if (tid1 == 0) n_redo = 0;
-                __syncthreads();
-                uint32_t cancel = 0u, near = 0u;
-                const int at = (mb + 4 * hl) * TN + nbk + cl;  // of register 0
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const bool live = col_counts && scale_a(r) != 0.f;
-                    if (!live) val[r] = 0.f;
-                    else if (DIST == DIST_L2 ? !(val[r] > kCancelRatio * norms(r)) : !(fabsf(val[r]) < INFINITY)) cancel |= 1u << r;
-                    result[at + (8 * (r >> 2) + (r & 3)) * TN] = val[r];  // (their registers are wanted meanwhile)
-                }
-                for (uint32_t left = cancel; left; left &= left - 1) {
-                    const int r = __ffs((int)left) - 1;
-                    list[atomicAdd(&n_redo, 1)] = (uint16_t)(at + (8 * (r >> 2) + (r & 3)) * TN);
-                }
-                __syncthreads();
-#pragma unroll 1
-                for (int q = tid1 >> 5; q < n_redo; q += Tile::threads / 32) {
-                    const int pos = list[q];
-                    float part = 0.f;
-#pragma unroll 1
-                    for (int k = (lane1 & 31) * 8; k < Kp; k += 256) {
-                        Row8 x, y;
-                        x.load(p.rows, a_row + m0 + pos / TN, k);
-                        y.load(p.rows, b_row + n0 + pos % TN, k);
-                        static_for<8>([&](auto I) {
-                            const float u = x.template value<I>(), v = y.template value<I>();
-                            part = DIST == DIST_L2 ? fmaf(u - v, u - v, part) : fmaf(u, v, part);
-                        });
-                    }
-                    part += swap1(part);
-                    part += swap2(part);
-                    part += mirror8(part);
-                    part += mirror16(part);
-                    part += __shfl_xor(part, 16, 64);
-                    if ((lane1 & 31) == 0) result[pos] = part;
-                }
-                __syncthreads();
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    val[r] = result[at + (8 * (r >> 2) + (r & 3)) * TN];
-                    if (DIST == DIST_L2 && ((cancel >> r) & 1u) && val[r] < kNearRatio * norms(r)) near |= 1u << r;
-                }
-                flagged = DIST == DIST_L2 && __ballot(near != 0u) != 0;
-                if (OM == 0)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) loss_acc += val[r] - val[r];  // a pair that is not finite shows in the loss
-            }
-            if (OM != 0) {  // raw scores (and distances), and which blocks the direct form is to take
-                if (DIST == DIST_L2 && lane1 == 0 && m0 + mb < Bp && n0 + nbk < Tp)
-                    p.out.exponent[((size_t)d * MT + ((m0 + mb) >> 5)) * NT + ((n0 + nbk) >> 5)] = flagged ? kDirect : kNoExponent;
-                float* const out = p.coef + (size_t)d * B * T;
-                float* const out_d = (DIST == DIST_L2 && p.dist) ? p.dist + (size_t)d * B * T : nullptr;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + mb + 8 * (r >> 2) + 4 * hl + (r & 3);
-                    const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[r]) : val[r];  // (never negative; a NaN stays one)
-                    if (m < B && n < T) {
-                        out[(size_t)m * T + n] = score_is_distance_value(sh.score_fn) ? dist : sh.gamma - dist;
-                        if (out_d) out_d[(size_t)m * T + n] = dist;
-                    }
-                }
-                continue;
-            }
-            // a column's negatives: mult of them, or one less where one is the row's label (src/poplar_kge.cpp:615-636)
-            const float mult = mult_s[nbk + cl], w_all = mult * w_neg, w_less = (mult - 1.f) * w_neg;
-            const bool whole = m0 + mb + 32 <= B && n0 + nbk + 32 <= T;
-            float c[16];
-            asm volatile("" ::: "memory");  // what stands in LDS is read again, not kept in registers
-#pragma unroll
-            for (int g = 0; g < 16; g += 4) {  // four rows at a time: their chains of dependent instructions side by side
-                const uint4 label4 = *reinterpret_cast<const uint4*>(&label_s[mb + 4 * hl + 2 * g]);
-                const uint32_t label[4] = {label4.x, label4.y, label4.z, label4.w};
-                float dist[4], term[4], ds[4];
-                LogSigmoid z[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    dist[r] = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[g + r]) : val[g + r];  // (never negative; a NaN stays one)
-                    z[r] = LogSigmoid(fmaf(dist[r], score_sign, score_base));
-                    const float w = (uint32_t)n == label[r] ? w_less : w_all;
-                    term[r] = -(w * z[r].minus_value());
-                    ds[r] = w * z[r].minus_grad();
-                }
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const bool pos = (uint32_t)n == label[r];
-                    if (__ballot(pos)) {  // one pair of a positive's row
-                        term[r] -= pos ? w_pos * z[r].plus_value() : 0.f;
-                        ds[r] -= pos ? w_pos * z[r].plus_grad() : 0.f;
-                    }
-                }
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float v = ds[r] * coef_scale;
-                    if (DIST == DIST_L2) v = dist[r] != 0.f ? v * __builtin_amdgcn_rcpf(dist[r]) : 0.f;
-                    if (!whole && !(scale_a(g + r) != 0.f && sb != 0.f)) term[r] = v = 0.f;
-                    loss_acc += term[r];
-                    c[g + r] = v;
-                }
-                __builtin_amdgcn_sched_barrier(0);  // no more rows' intermediate values at once
-            }
-            asm volatile("" ::: "memory");
-            const int word = flagged ? kDirect : coef_block_exponent(c, scale_a, sb, lane1);
-            if (word == kDirect) {  // the backward takes this block in the direct form, from the coefficients as they are
-                char* const out = (char*)(p.coef + ((size_t)d * B + m0 + mb) * T + n0 + nbk);
-                const uint32_t off = (uint32_t)(4 * hl * T + cl) * 4;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    if (scale_a(r) != 0.f && sb != 0.f) *reinterpret_cast<float*>(out + (size_t)(8 * (r >> 2) + (r & 3)) * T * 4 + off) = c[r];
-                }
-            }
-            store_coef_block<DIST>(c, scale_a, sb, word, p.out, d, m0 + mb, n0 + nbk, lane1);
+    for (int r = 0; r < 16; ++r) {
+        const float product = fmaf(small[r], kHalfStep, big[r]);
+        if (DIST == DIST_L2) {
+            const float ns = norms(r);
+            val[r] = fmaf(product, -2.f * sb * scale_a(r), ns);
+            redo |= __ballot(!(val[r] > kCancelRatio * ns));
+        } else {
+            val[r] = product * scale_a(r) * sb;
+            redo |= __ballot(!(fabsf(val[r]) < INFINITY));
         }
+    }
+    bool flagged = false;
+    // rare: pairs are recomputed directly, half a wave to a pair, by all of the workgroup (a popular row's
+    // come together in one wave's block): those that cancelled, and those that are not finite (an infinity's
+    // second half is NaN).  Pairs that do not count, a NaN among them, get any finite value.
+    if (__syncthreads_or(redo != 0u)) {
+        float* const result = reinterpret_cast<float*>(smem);  // [TM][TN]; the tiles are no longer needed
+        uint16_t* const list = reinterpret_cast<uint16_t*>(smem + TM * TN * 4);
+        static_assert(TM * TN * 6 <= P::kLds, "the tile's pairs as a list and as results");
+        if (tid1 == 0) n_redo = 0;
+        __syncthreads();
+        uint32_t cancel = 0u, near = 0u;
+        const int at = (mb + 4 * hl) * TN + nbk + cl;  // of register 0
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const bool live = col_counts && scale_a(r) != 0.f;
+            if (!live) val[r] = 0.f;
+            else if (DIST == DIST_L2 ? !(val[r] > kCancelRatio * norms(r)) : !(fabsf(val[r]) < INFINITY)) cancel |= 1u << r;
+            result[at + (8 * (r >> 2) + (r & 3)) * TN] = val[r];  // (their registers are wanted meanwhile)
+        }
+        for (uint32_t left = cancel; left; left &= left - 1) {
+            const int r = __ffs((int)left) - 1;
+            list[atomicAdd(&n_redo, 1)] = (uint16_t)(at + (8 * (r >> 2) + (r & 3)) * TN);
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int q = tid1 >> 5; q < n_redo; q += Tile::threads / 32) {
+            const int pos = list[q];
+            float part = 0.f;
+#pragma unroll 1
+            for (int k = (lane1 & 31) * 8; k < Kp; k += 256) {
+                Row8 x, y;
+                x.load(p.rows, a_row + m0 + pos / TN, k);
+                y.load(p.rows, b_row + n0 + pos % TN, k);
+                static_for<8>([&](auto I) {
+                    const float u = x.template value<I>(), v = y.template value<I>();
+                    part = DIST == DIST_L2 ? fmaf(u - v, u - v, part) : fmaf(u, v, part);
+                });
+            }
+            part += swap1(part);
+            part += swap2(part);
+            part += mirror8(part);
+            part += mirror16(part);
+            part += __shfl_xor(part, 16, 64);
+            if ((lane1 & 31) == 0) result[pos] = part;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            val[r] = result[at + (8 * (r >> 2) + (r & 3)) * TN];
+            if (DIST == DIST_L2 && ((cancel >> r) & 1u) && val[r] < kNearRatio * norms(r)) near |= 1u << r;
+        }
+        flagged = DIST == DIST_L2 && __ballot(near != 0u) != 0;
+        if (OM == 0)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) loss_acc += val[r] - val[r];  // a pair that is not finite shows in the loss
+    }
+    if (OM != 0) {  // raw scores (and distances), and which blocks the direct form is to take
+        if (DIST == DIST_L2 && lane1 == 0 && m0 + mb < Bp && n0 + nbk < Tp)
+            p.out.exponent[((size_t)d * MT + ((m0 + mb) >> 5)) * NT + ((n0 + nbk) >> 5)] = flagged ? kDirect : kNoExponent;
+        float* const out = p.coef + (size_t)d * B * T;
+        float* const out_d = (DIST == DIST_L2 && p.dist) ? p.dist + (size_t)d * B * T : nullptr;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = m0 + mb + 8 * (r >> 2) + 4 * hl + (r & 3);
+            const float dist = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[r]) : val[r];  // (never negative; a NaN stays one)
+            if (m < B && n < T) {
+                out[(size_t)m * T + n] = score_is_distance_value(sh.score_fn) ? dist : sh.gamma - dist;
+                if (out_d) out_d[(size_t)m * T + n] = dist;
+            }
+        }
+        return;
+    }
+    // a column's negatives: mult of them, or one less where one is the row's label (src/poplar_kge.cpp:615-636)
+    const float mult = mult_s[nbk + cl], w_all = mult * w_neg, w_less = (mult - 1.f) * w_neg;
+    const bool whole = m0 + mb + 32 <= B && n0 + nbk + 32 <= T;
+    float c[16];
+    asm volatile("" ::: "memory");  // what stands in LDS is read again, not kept in registers
+#pragma unroll
+    for (int g = 0; g < 16; g += 4) {  // four rows at a time: their chains of dependent instructions side by side
+        const uint4 label4 = *reinterpret_cast<const uint4*>(&label_s[mb + 4 * hl + 2 * g]);
+        const uint32_t label[4] = {label4.x, label4.y, label4.z, label4.w};
+        float dist[4], term[4], ds[4];
+        LogSigmoid z[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            dist[r] = DIST == DIST_L2 ? __builtin_amdgcn_sqrtf(val[g + r]) : val[g + r];  // (never negative; a NaN stays one)
+            z[r] = LogSigmoid(fmaf(dist[r], score_sign, score_base));
+            const float w = (uint32_t)n == label[r] ? w_less : w_all;
+            term[r] = -(w * z[r].minus_value());
+            ds[r] = w * z[r].minus_grad();
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const bool pos = (uint32_t)n == label[r];
+            if (__ballot(pos)) {  // one pair of a positive's row
+                term[r] -= pos ? w_pos * z[r].plus_value() : 0.f;
+                ds[r] -= pos ? w_pos * z[r].plus_grad() : 0.f;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float v = ds[r] * coef_scale;
+            if (DIST == DIST_L2) v = dist[r] != 0.f ? v * __builtin_amdgcn_rcpf(dist[r]) : 0.f;
+            if (!whole && !(scale_a(g + r) != 0.f && sb != 0.f)) term[r] = v = 0.f;
+            loss_acc += term[r];
+            c[g + r] = v;
+        }
+        __builtin_amdgcn_sched_barrier(0);  // no more rows' intermediate values at once
+    }
+    asm volatile("" ::: "memory");
+    const int word = flagged ? kDirect : coef_block_exponent(c, scale_a, sb, lane1);
+    if (word == kDirect) {  // the backward takes this block in the direct form, from the coefficients as they are
+        char* const out = (char*)(p.coef + ((size_t)d * B + m0 + mb) * T + n0 + nbk);
+        const uint32_t off = (uint32_t)(4 * hl * T + cl) * 4;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            if (scale_a(r) != 0.f && sb != 0.f) *reinterpret_cast<float*>(out + (size_t)(8 * (r >> 2) + (r & 3)) * T * 4 + off) = c[r];
+        }
+    }
+    store_coef_block<DIST>(c, scale_a, sb, word, p.out, d, m0 + mb, n0 + nbk, lane1);
     if (OM == 0) {
         loss_acc = wave_sum(loss_acc);
         if (lane1 == 0) red[wave] = loss_acc;
@@ -642,7 +619,6 @@ struct SplitBwdTile {
     static constexpr int TM = Tile::TM, TN = Tile::TN, WM = Tile::WM, WN = Tile::WN, kSums = Tile::threads / TM;
     using TA = std::conditional_t<SIDE_B, ColTile<TM, 2>, RowTile<TM, 2>>;
     using P = SplitProduct<TA, ColTile<TN, 2>, Tile>;
-    static_assert(P::AM == 1 && P::AN == 1, "one sub-block to a wave and slab");
     const SplitBwd& p;
     char* const smem;
     float* const csum_s;
@@ -674,7 +650,7 @@ struct SplitBwdTile {
         auto load_exps = [&](int slab0) __attribute__((always_inline)) { exp_reg = exponent_of(st0, min(slab0 + lane, n_slab - 1)); };
         constexpr int kNone = kDirect + 4;
         int first = kNone, now = kNone;  // the wave's first slab's exponent; what the sums are in
-        floatx16 big[1][1], small[1][1];
+        floatx16 big, small;
         P::run(smem, a, coef_pitch, SIDE_B ? (size_t)32 * coef_pitch : kHalfBytes, b, pitch, (size_t)32 * pitch, n_slab, n_other, big, small, lane, wave,
                [&]() __attribute__((always_inline)) {
                    load_exps(0);
@@ -724,8 +700,8 @@ struct SplitBwdTile {
                        const float by = __uint_as_float((uint32_t)(127 + now - e) << 23);
 #pragma unroll
                        for (int r = 0; r < 16; ++r) {
-                           big[0][0][r] *= by;
-                           small[0][0][r] *= by;
+                           big[r] *= by;
+                           small[r] *= by;
                        }
                    }
                    now = e;
@@ -736,7 +712,7 @@ struct SplitBwdTile {
         // the self rows' own scales leave the sums
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-            big[0][0][r] = ldexpf(fmaf(small[0][0][r], kHalfStep, big[0][0][r]),
+            big[r] = ldexpf(fmaf(small[r], kHalfStep, big[r]),
                                   (now == kNone ? 0 : now) - exp_s[wm + 8 * (r >> 2) + 4 * hl + (r & 3)]);
         const char* const self = p.rows.halves + (int64_t)(self0 + i0) * pitch;
         // neighbouring lanes swap values: a lane stores two columns of one row
@@ -761,8 +737,8 @@ struct SplitBwdTile {
             }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float got = swap1(odd ? big[0][0][2 * i] : big[0][0][2 * i + 1]);
-            float x = odd ? got : big[0][0][2 * i], y = odd ? big[0][0][2 * i + 1] : got;
+            const float got = swap1(odd ? big[2 * i] : big[2 * i + 1]);
+            float x = odd ? got : big[2 * i], y = odd ? big[2 * i + 1] : got;
             const int row = wave_row(i) + 4 * hl + odd;
             if (kSelf) {
                 const f16x2 h = __builtin_bit_cast(f16x2, w[i][0]), l = __builtin_bit_cast(f16x2, w[i][1]);
