@@ -247,13 +247,11 @@ inline size_t nearflag_words(const ScoreShape& sh) {
 int score_fwd_parts(const ScoreShape& sh, const RowSource& ent);  // n_part of such a launch (of `sh.tcount`, only whether it is there counts)
 
 // ---- scoring on float16 halves (kge_split.hip; L2 and dot, any shape) ----
-// Matrices of halves hold every float32 value as two scaled float16 numbers, rows of half_pitch(cols) bytes (columns
-// filled up to a multiple of 32 with zeros).  The product kernels read whole tiles: kSplitSpareRows
-// rows behind a matrix's last must be readable.
+// Matrices of halves hold every float32 value as two scaled float16 numbers, rows as long as float32's (columns filled up
+// to a multiple of 32 with zeros).  The product kernels read whole tiles: kSplitSpareRows rows behind a
+// matrix's last must be readable.
 constexpr int kSplitSpareRows = 128;
-// The workgroups on an XCD read the same 128 bytes of many rows at about the same time: a pitch that is an odd
-// number of 128-byte lines spreads those over the L2's channels, a power of two does not.
-inline __host__ __device__ int half_pitch(int cols) { return (cols / 32 | 1) * 128; }
+inline __host__ __device__ int half_pitch(int cols) { return cols / 32 * 128; }
 inline size_t half_bytes(size_t rows, size_t cols) { return (rows + kSplitSpareRows) * half_pitch((int)cols) + 128 * 4; }
 // bytes of a matrix of three bfloat16 pieces
 inline size_t split_bytes(size_t rows, size_t cols) {

@@ -38,7 +38,8 @@ DEVINL uint32_t wave_max_bits(float v) {
 // --------------------------------------------------------------------------
 // operand gather: RPW contributions per wave, their entity (or hidden) rows with the relation
 // applied for the heads, as halves; and the rows' scales and squared norms.  Workgroup (d, y, z): a lot of
-// block d's B heads and then T tails (z: a grid's y ends at 65535), which finds its XCD (d % 8) where the block's tiles will run.
+// block d's B heads and then T tails (z: a grid's y ends at 65535).  Where S is a multiple of 8, that runs on the XCD (d % 8) of the
+// block's tiles.
 // ET: the rows' element type, or -1: as `ent` says, the complex product and the rotation among the
 // relations; ONE: rows of at most 256 columns, which stay in their registers between the largest value and the halves.
 template <int RPW, int ET, bool ONE>
