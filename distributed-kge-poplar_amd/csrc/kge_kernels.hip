@@ -619,7 +619,7 @@ __global__ __launch_bounds__(NW * 64) void k_score_fwd_mfma(FwdParams p) {
         if (ALIGNED || decltype(set)::value * BKT < Dp) prefetch(set, decltype(set)::value * BKT);
     });
     if constexpr (SPLIT) {
-        static_assert(BKT == 32 && PF % 2 == 0 && ALIGNED, "the three-piece path: aligned shapes, slabs of 32");
+        static_assert(BKT == 32 && PF % 2 == 0 && ALIGNED && OM == 1, "the three-piece path: raw scores of aligned shapes, slabs of 32");
         const int hl = lane >> 5, cl = lane & 31;
         // writes one register set (a slab) into tile copy `buf`, as pieces; `live` = 0 for the
         // slab past the end (its squares must not count)
@@ -1000,9 +1000,9 @@ static void launch_fwd(const FwdParams& p, hipStream_t stream) {
         const bool aligned = choice.dense && p.sh.B % FM_TM == 0 && p.sh.T % FM_TN == 0;
 #define KGE_FWD_OM(D_, OM_)                                                                                  \
     do {                                                                                                     \
-        if (aligned && p.sh.Dp % 64 == 0 && p.sh.use_mfma == 2) {                                            \
-            hipLaunchKernelGGL((k_score_fwd_mfma<D_, 32, true, 8, OM_, true, 2>), grid, dim3(512), 0, stream, p); \
-        }                                                                                                    \
+        /* on pieces: raw scores (a step with the loss fused takes split_scoring's kernels under use_mfma == 2) */ \
+        if (OM_ == 1 && aligned && p.sh.Dp % 64 == 0 && p.sh.use_mfma == 2)                                  \
+            hipLaunchKernelGGL((k_score_fwd_mfma<D_, 32, true, 8, 1, true, 2>), grid, dim3(512), 0, stream, p); \
         else if (aligned && p.sh.Dp % 32 == 0) /* eight waves: two per SIMD hide each other's latencies */ \
             hipLaunchKernelGGL((k_score_fwd_mfma<D_, 32, true, 8, OM_>), grid, dim3(512), 0, stream, p);      \
         else hipLaunchKernelGGL((k_score_fwd_mfma<D_, 32, false, 4, OM_>), grid, dim3(256), 0, stream, p);    \
