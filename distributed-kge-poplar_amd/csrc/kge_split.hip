@@ -276,9 +276,10 @@ DEVINL float block_rows(Value&& value, int lane, Op&& op) {
     return op(v, __shfl_xor(v, 16, 64));
 }
 
-// What stands for a block among the exponents.  sa[r], sb: the scales of the rows and of the column.
+// What stands for a block among the exponents.  scale_of_row, sb: the scales of the rows and of the column; live: the column is
+// one of the block's (others' coefficients are zeros, and no reason to look twice).
 template <class Scales>
-DEVINL int coef_block_exponent(const float (&c)[16], Scales&& scale_of_row, float sb, int lane) {
+DEVINL int coef_block_exponent(const float (&c)[16], Scales&& scale_of_row, float sb, bool live, int lane) {
     constexpr float kTiny = 0x1p-100f;
     float top = 0.f, least = INFINITY;
 #pragma unroll
@@ -291,8 +292,8 @@ DEVINL int coef_block_exponent(const float (&c)[16], Scales&& scale_of_row, floa
     const uint32_t bits = wave_max_bits(ldexpf(top, col));
     const int e = ((int)(bits >> 23) - 127 - 14 + 3) & ~3;
     const bool fits = bits >= __float_as_uint(kTiny) && bits < __float_as_uint(0x1p100f);
-    if (fits && !__ballot(least < kTiny || ldexpf(least, col - e) < kSmallCoef)) return e;
-    // seldom (zeros among them: columns behind a block's last tail)
+    if (__builtin_expect(fits && !__ballot(live && (least < kTiny || ldexpf(least, col - e) < kSmallCoef)), 1)) return e;
+    // seldom (zeros among them: rows behind a block's last head)
     asm volatile("" ::: "memory");  // (scales that stand in LDS are read again, not kept)
     uint64_t gone = 0u;  // a coefficient that is not zero, but is with its scales, or nearly
     float most = 0.f;
@@ -355,7 +356,7 @@ DEVINL void store_coef_block(float (&c)[16], Scales&& scale_of_row, float sb, in
     };
     auto scaled = [&](int r) __attribute__((always_inline)) { return ldexpf(c[r] * scale_of_row(r), shift); };
     pack(p.coefp + corner, std::false_type{}, scaled);
-    if (!(word & 1)) return;
+    if (__builtin_expect(!(word & 1), 1)) return;
     // seldom: once more, in two parts (and from the coefficients, instead of what would have to be kept for it)
     auto apart = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -388,7 +389,7 @@ __global__ __launch_bounds__(256) void k_coef_halves(ScoreShape sh, const float*
         c[r] = m < sh.B && n < sh.T ? src[(size_t)m * sh.T + n] : 0.f;
     }
     auto scale_a = [&](int r) __attribute__((always_inline)) { return sa[r]; };
-    store_coef_block<DIST>(c, scale_a, sb, near ? kDirect : coef_block_exponent(c, scale_a, sb, lane), p, d, 32 * mt, 32 * nt, lane);
+    store_coef_block<DIST>(c, scale_a, sb, near ? kDirect : coef_block_exponent(c, scale_a, sb, !sh.tcount || n < (int)sh.tcount[d], lane), p, d, 32 * mt, 32 * nt, lane);
 }
 
 // --------------------------------------------------------------------------
@@ -578,7 +579,7 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
         __builtin_amdgcn_sched_barrier(0);  // no more rows' intermediate values at once
     }
     asm volatile("" ::: "memory");
-    const int word = flagged ? kDirect : coef_block_exponent(c, scale_a, sb, lane1);
+    const int word = flagged ? kDirect : coef_block_exponent(c, scale_a, sb, col_counts, lane1);
     if (word == kDirect) {  // the backward takes this block in the direct form, from the coefficients as they are
         char* const out = (char*)(p.coef + ((size_t)d * B + m0 + mb) * T + n0 + nbk);
         const uint32_t off = (uint32_t)(4 * hl * T + cl) * 4;
