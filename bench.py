@@ -48,8 +48,9 @@ PEAK_FP32_TFLOPS = 157.3
 PEAK_BF16_TFLOPS = 2500.0
 
 # kernels of the step by the names the profiler summaries list them under
-KERNEL_SYMBOLS = {"gather_operands": "k_gather_operands", "score_fwd": "k_score_fwd", "score_bwd": "k_score_bwd",
-                  "reduce_entity": "k_reduce_chunks", "adam_entity": "k_adam_rows", "loss_rows": "k_loss_rows"}
+KERNEL_SYMBOLS = {"gather_operands": ("k_gather_operands", "k_gather_halves"), "score_fwd": ("k_score_fwd", "k_split_fwd"),
+                  "score_bwd": ("k_score_bwd", "k_split_bwd"), "reduce_entity": ("k_reduce_chunks",),
+                  "adam_entity": ("k_adam_rows",), "loss_rows": ("k_loss_rows",)}
 
 
 def measured_traffic(workload):
@@ -70,8 +71,8 @@ def measured_traffic(workload):
             except ValueError:
                 pass
     out = {}
-    for name, symbol in KERNEL_SYMBOLS.items():
-        hits = [v for k, v in table.items() if symbol in k]
+    for name, symbols in KERNEL_SYMBOLS.items():
+        hits = [v for k, v in table.items() if any(symbol in k for symbol in symbols)]
         if hits:
             out[name] = max(hits)[1]  # variants of one kernel (with and without hot rows): the one launched most
     return out, f"profiles/{path.name}"
