@@ -54,7 +54,9 @@ DEVINL void store_pieces4(char* row, int k, float4 v) {
 // each, the rounding of h0 to either side worth one more, so the sum differs from x by at most one unit in its
 // 24th bit, and for three values of four by nothing.  The scale s is a power of two that brings the largest of a
 // row (or of a block of coefficients) to 2^14; with the second half 2^11 times as large as it counts, both are
-// normal float16 numbers down to 2^-28 of that largest value, and what is smaller is off by 2^-49 of it at most.
+// normal float16 numbers down to 2^-28 of that largest value, and what is smaller is off by 2^-49 of it at most.  Where a
+// column is that small in one row after the other, and so in every gradient, they are wide ones: their places hold them as
+// float32, their scales are NaN, and their pairs and sub-blocks are taken in the direct forms.
 //   a b = sa sb (a0 b0 + (a0 b1 + a1 b0) / 2048 + O(2^-24 |a0 b0|)):
 // three matrix instructions where three bfloat16 pieces take six, two fragments of an operand where they take
 // three, and a row of halves is as long as the float32 row.  The cross products have an accumulator of their own.
@@ -73,6 +75,13 @@ DEVINL float half_scale(float largest) {
 // a power of two's exponent, its reciprocal
 DEVINL int pow2_exponent(float s) { return (int)(__float_as_uint(s) >> 23) - 127; }
 DEVINL float pow2_inverse(float s) { return __uint_as_float(0x7f000000u - __float_as_uint(s)); }
+// The scale of a wide row, among the exponents of scales, and where its columns k .. k + 3 (k % 4 == 0) lie: eight columns are
+// the sixteen bytes of their first halves and then those of the second ones.
+constexpr float kLeastHalf = 0x1p-14f;
+constexpr int kWideExponent = 128;
+DEVINL float wide_scale() { return __uint_as_float(0x7fc00000u); }
+DEVINL bool is_wide(float scale) { return scale != scale; }
+DEVINL size_t wide_at(int k) { return (size_t)(k >> 5) * kHalfBytes + (k & 4) * 16 + ((k & 31) >> 3) * 16; }
 // Coefficients are halves with a scale per block, whose largest comes to 2^11 .. 2^15; those below kSmallCoef can go to a
 // matrix of their own, 2^kSmallShift times as large.
 constexpr float kSmallCoef = 0x1p-13f;
@@ -105,7 +114,7 @@ DEVINL void store_halves4(char* row, int k, float4 v, bool live, uint64_t (&lost
 #pragma unroll
     for (int q = 0; q < 2; ++q) *reinterpret_cast<uint2*>(p + 64 * q) = make_uint2(w[q][0], w[q][1]);
 }
-// The rows of a gather as they were (values below 2^-28 of their row's largest to 2^-49 of that).
+// The rows of a gather as they were.
 DEVINL float join_lost(_Float16 h, _Float16 l, uint32_t bit) {  // (of a finite value, without its scale)
     return fmaf(__uint_as_float(__float_as_uint((float)l) + (bit << 12)), kHalfStep, (float)h);
 }
@@ -125,26 +134,31 @@ struct Row8 {
         lost = s.lost[(size_t)c * (s.Kp >> 5) + (k >> 5)] >> ((k & 31) >> 2);
         scale = s.scale[c];
     }
-    template <int I>
+    template <int I, bool WIDE>  // (WIDE: it may be a wide row)
     DEVINL float value() const {
         constexpr int W = I >> 1;
+        if (WIDE && is_wide(scale)) {
+            const uint4 four = I < 4 ? h : l;
+            return __uint_as_float((I & 3) == 0 ? four.x : (I & 3) == 1 ? four.y : (I & 3) == 2 ? four.z : four.w);
+        }
         const f16x2 hw = __builtin_bit_cast(f16x2, W == 0 ? h.x : W == 1 ? h.y : W == 2 ? h.z : h.w);
         const f16x2 lw = __builtin_bit_cast(f16x2, W == 0 ? l.x : W == 1 ? l.y : W == 2 ? l.z : l.w);
         return with_lost(I & 1 ? hw.y : hw.x, I & 1 ? lw.y : lw.x, (lost >> lost_at(I)) & 1u, scale);
     }
 };
-struct Row1 {  // one column
-    _Float16 h, l;
-    uint32_t lost;
-    float scale;
-    DEVINL void load(const SplitRows& s, int c, int k) {
-        const char* p = s.halves + (size_t)c * half_pitch(s.Kp) + (size_t)(k >> 5) * kHalfBytes + (k & 31) * 2;
-        h = *reinterpret_cast<const _Float16*>(p);
-        l = *reinterpret_cast<const _Float16*>(p + 64);
+struct Row1 {  // one column of a row whose scale is known
+    uint32_t h, l, lost;
+    DEVINL void load(const SplitRows& s, int c, int k, float scale) {
+        const char* const row = s.halves + (size_t)c * half_pitch(s.Kp);
+        const uint32_t at = is_wide(scale) ? (uint32_t)wide_at(k) + (k & 3) * 4 : (uint32_t)((k >> 5) * kHalfBytes + (k & 31) * 2);
+        h = *reinterpret_cast<const uint16_t*>(row + at);
+        l = *reinterpret_cast<const uint16_t*>(row + at + (is_wide(scale) ? 2 : 64));  // (a wide row's: the upper half of the value)
         lost = s.lost[(size_t)c * (s.Kp >> 5) + (k >> 5)];
-        scale = s.scale[c];
     }
-    DEVINL float value(int k) const { return with_lost(h, l, (lost >> lost_at(k)) & 1u, scale); }
+    DEVINL float value(int k, float scale) const {
+        if (is_wide(scale)) return __uint_as_float(h | l << 16);
+        return with_lost(__builtin_bit_cast(_Float16, (uint16_t)h), __builtin_bit_cast(_Float16, (uint16_t)l), (lost >> lost_at(k)) & 1u, scale);
+    }
 };
 
 // --------------------------------------------------------------------------

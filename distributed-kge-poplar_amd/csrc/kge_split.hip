@@ -43,7 +43,7 @@ DEVINL uint32_t wave_max_bits(float v) {
 // ET: the rows' element type, or -1: as `ent` says, the complex product and the rotation among the
 // relations; ONE: rows of at most 256 columns, which stay in their registers between the largest value and the halves.
 template <int RPW, int ET, bool ONE>
-__global__ __launch_bounds__(256) void k_gather_halves(RowSource ent, const float* __restrict__ rel, const uint32_t* __restrict__ crel,
+__global__ __launch_bounds__(256, 8) void k_gather_halves(RowSource ent, const float* __restrict__ rel, const uint32_t* __restrict__ crel,
                                                        int rel_mode, int half, SplitRows s, const uint32_t* __restrict__ tcount,
                                                        int B, int T, int tpad) {
     constexpr bool XF = ET < 0;
@@ -67,12 +67,13 @@ __global__ __launch_bounds__(256) void k_gather_halves(RowSource ent, const floa
     if (i0 >= end) return;
     const char* row[RPW];
     const float* rrow[RPW];
-    float sq[RPW], top[RPW];
+    float sq[RPW], top[RPW], least[RPW];
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
         row[r] = ent.base + (int64_t)key[r] * ent.pitch;
         rrow[r] = (i0 + r < B && rel_mode) ? rel + (size_t)rkey[r] * s.Dp : nullptr;
         sq[r] = top[r] = 0.f;
+        least[r] = INFINITY;
     }
     float4 v[RPW];
     auto fetch = [&](int k) __attribute__((always_inline)) {
@@ -99,23 +100,78 @@ __global__ __launch_bounds__(256) void k_gather_halves(RowSource ent, const floa
         for (int r = 0; r < RPW; ++r) {
             sq[r] += v[r].x * v[r].x + v[r].y * v[r].y + v[r].z * v[r].z + v[r].w * v[r].w;
             top[r] = fmaxf(fmaxf(top[r], fmaxf(fabsf(v[r].x), fabsf(v[r].y))), fmaxf(fabsf(v[r].z), fabsf(v[r].w)));
+            if (k < s.Dp) least[r] = fminf(fminf(least[r], fminf(fabsf(v[r].x), fabsf(v[r].y))), fminf(fabsf(v[r].z), fabsf(v[r].w)));
         }
     }
-    float up[RPW];
+    // Seldom (or where there are zeros): whether some element of row i is too small for halves, and not zero, and the next
+    // three rows' of its column are too.  Of ordinary rows' elements one in 10^8 is so small by chance, and then the others make up its
+    // column of every gradient.  (With a row in the direct form for each of those, a step of 64 blocks of 256 x 512 took 2 us
+    // more on average, one of 16 blocks of 256 x 1536 7.)
+    auto small_column = [&](int i) __attribute__((always_inline)) {
+        const int first = i < B ? 0 : B, n = i < B ? B : end - B;
+        auto row4 = [&](int x, int k) __attribute__((always_inline)) {
+            if (k >= s.Dp) return make_float4(0.f, 0.f, 0.f, 0.f);
+            const int at = first + (i - first + x) % n, c = at < B ? d * B + at : s.n_head + d * T + at - B;
+            const char* const row = ent.base + (int64_t)(ent.index ? ent.index[c] : (uint32_t)c) * ent.pitch;
+            const float4 v = XF ? load4(row, k, ent) : load4(row, k, ET);
+            if (at >= B || !rel_mode) return v;
+            const float* const rrow = rel + (size_t)crel[c] * s.Dp;
+            if (XF && rel_mode >= 3) return relation_xf(v, row, ent.etype, rrow, k, half, rel_mode);
+            const float4 w = *reinterpret_cast<const float4*>(rrow + k);
+            return rel_mode == 1 ? f4add(v, w) : f4mul(v, w);
+        };
+#pragma unroll 1
+        for (int k0 = 0; k0 < k_end; k0 += 256) {  // for each of the rows its largest element, then the lane's four of these columns
+            int is = 15;
+            float limit = 0.f;
+#pragma unroll 1
+            for (int t = 0; t < 8 && __ballot(is); ++t) {
+                const bool look = t & 1;
+                float most = 0.f;
+#pragma unroll 1
+                for (int q = look ? k0 : 0; q < (look ? k0 + 1 : k_end); q += 256) {
+                    const float4 a = row4(t >> 1, q + 4 * lane);
+                    most = fmaxf(fmaxf(most, fmaxf(fabsf(a.x), fabsf(a.y))), fmaxf(fabsf(a.z), fabsf(a.w)));
+                    if (!look) continue;
+                    is &= (fabsf(a.x) < limit) | (fabsf(a.y) < limit) << 1 | (fabsf(a.z) < limit) << 2 | (fabsf(a.w) < limit) << 3;
+                    if (t == 1) is &= (a.x != 0.f) | (a.y != 0.f) << 1 | (a.z != 0.f) << 2 | (a.w != 0.f) << 3;
+                }
+                if (!look) limit = kLeastHalf * half_scale(__uint_as_float(wave_max_bits(most)));
+            }
+            if (__ballot(is)) return true;
+        }
+        return false;
+    };
+    float up[RPW], sum[RPW];
+    uint32_t look = 0u, wide = 0u;  // rows' bits
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
-        const float sum = wave_reduce63(sq[r], [](float a, float b) { return a + b; });
-        const float scale = half_scale(__uint_as_float(wave_max_bits(top[r])));
-        up[r] = pow2_inverse(scale);
-        if (lane == 63 && i0 + r < end) {
-            s.norm[c[r]] = sum;
-            s.scale[c[r]] = scale;
-        }
+        sum[r] = wave_reduce63(sq[r], [](float a, float b) { return a + b; });
+        const float most = __uint_as_float(wave_max_bits(top[r]));
+        up[r] = pow2_inverse(half_scale(most));
+        if (__ballot(least[r] * up[r] < kLeastHalf) && most < INFINITY && i0 + r < end) look |= 1u << r;
     }
+    if (__builtin_expect(look != 0u, 0)) {
+#pragma unroll 1
+        for (; look; look &= look - 1u)
+            if (small_column(i0 + __ffs((int)look) - 1)) wide |= look & (0u - look);
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): without it, the waits for these loads come behind the stores below, and for those
+    }
+#pragma unroll
+    for (int r = 0; r < RPW; ++r)
+        if (lane == 63 && i0 + r < end) {
+            s.norm[c[r]] = sum[r];
+            s.scale[c[r]] = (wide >> r) & 1u ? wide_scale() : pow2_inverse(up[r]);
+        }
     for (int k = lane * 4; k < k_end; k += 256) {
         if (!ONE) fetch(k);
 #pragma unroll
         for (int r = 0; r < RPW; ++r) {
+            if (__builtin_expect((wide >> r) & 1u, 0)) {
+                if (i0 + r < end && k < s.Kp)
+                    *reinterpret_cast<float4*>(s.halves + (size_t)c[r] * half_pitch(s.Kp) + wide_at(k)) = v[r];
+                continue;
+            }
             uint64_t lost[4];
             store_halves4(s.halves + (size_t)c[r] * half_pitch(s.Kp), k,
                           make_float4(v[r].x * up[r], v[r].y * up[r], v[r].z * up[r], v[r].w * up[r]), i0 + r < end && k < s.Kp, lost);
@@ -378,14 +434,14 @@ __global__ __launch_bounds__(256) void k_coef_halves(ScoreShape sh, const float*
     const int d = g / (MT * NT), mt = (g - d * MT * NT) / NT, nt = g % NT;
     if (d >= sh.S || 32 * nt >= tail_limit(sh.tcount, d, sh.T, sh.tpad)) return;
     const float* src = coef + (size_t)d * sh.B * sh.T;
-    const bool near = DIST == DIST_L2 && p.exponent[((size_t)d * MT + mt) * NT + nt] == kDirect;  // as the forward left it
+    const bool near = p.exponent[((size_t)d * MT + mt) * NT + nt] == kDirect;  // as the forward left it
     const int n = 32 * nt + (lane & 31);
     const float sb = scale[n_head + d * sh.T + n];
     float c[16], sa[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int m = 32 * mt + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        sa[r] = scale[d * sh.B + m];
+        sa[r] = m < sh.B ? scale[d * sh.B + m] : 0.f;  // (another block's may be NaN)
         c[r] = m < sh.B && n < sh.T ? src[(size_t)m * sh.T + n] : 0.f;
     }
     auto scale_a = [&](int r) __attribute__((always_inline)) { return sa[r]; };
@@ -472,7 +528,7 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
     bool flagged = false;
     // rare: pairs are recomputed directly, half a wave to a pair, by all of the workgroup (a popular row's
     // come together in one wave's block): those that cancelled, and those that are not finite (an infinity's
-    // second half is NaN).  Pairs that do not count, a NaN among them, get any finite value.
+    // second half is NaN; a wide row's scale is).  Pairs that do not count, a NaN among them, get any finite value.
     if (__syncthreads_or(redo != 0u)) {
         float* const result = reinterpret_cast<float*>(smem);  // [TM][TN]; the tiles are no longer needed
         uint16_t* const list = reinterpret_cast<uint16_t*>(smem + TM * TN * 4);
@@ -502,10 +558,14 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
                 Row8 x, y;
                 x.load(p.rows, a_row + m0 + pos / TN, k);
                 y.load(p.rows, b_row + n0 + pos % TN, k);
-                static_for<8>([&](auto I) {
-                    const float u = x.template value<I>(), v = y.template value<I>();
-                    part = DIST == DIST_L2 ? fmaf(u - v, u - v, part) : fmaf(u, v, part);
-                });
+                auto add = [&](auto wide) __attribute__((always_inline)) {
+                    static_for<8>([&](auto I) {
+                        const float u = x.template value<I, decltype(wide)::value>(), v = y.template value<I, decltype(wide)::value>();
+                        part = DIST == DIST_L2 ? fmaf(u - v, u - v, part) : fmaf(u, v, part);
+                    });
+                };
+                if (__builtin_expect(__ballot(is_wide(x.scale) || is_wide(y.scale)) != 0u, 0)) add(std::true_type{});
+                else add(std::false_type{});
             }
             part += swap1(part);
             part += swap2(part);
@@ -520,13 +580,17 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
             val[r] = result[at + (8 * (r >> 2) + (r & 3)) * TN];
             if (DIST == DIST_L2 && ((cancel >> r) & 1u) && val[r] < kNearRatio * norms(r)) near |= 1u << r;
         }
-        flagged = DIST == DIST_L2 && __ballot(near != 0u) != 0;
+        for (uint32_t left = cancel; left; left &= left - 1) {  // (a wide row's pairs)
+            const int r = __ffs((int)left) - 1;
+            if (is_wide(sa[8 * (r >> 2) + (r & 3)]) || is_wide(sb)) near |= 1u << r;
+        }
+        flagged = __ballot(near != 0u) != 0;
         if (OM == 0)
 #pragma unroll
             for (int r = 0; r < 16; ++r) loss_acc += val[r] - val[r];  // a pair that is not finite shows in the loss
     }
     if (OM != 0) {  // raw scores (and distances), and which blocks the direct form is to take
-        if (DIST == DIST_L2 && lane1 == 0 && m0 + mb < Bp && n0 + nbk < Tp)
+        if (lane1 == 0 && m0 + mb < Bp && n0 + nbk < Tp)
             p.out.exponent[((size_t)d * MT + ((m0 + mb) >> 5)) * NT + ((n0 + nbk) >> 5)] = flagged ? kDirect : kNoExponent;
         float* const out = p.coef + (size_t)d * B * T;
         float* const out_d = (DIST == DIST_L2 && p.dist) ? p.dist + (size_t)d * B * T : nullptr;
@@ -752,6 +816,7 @@ struct SplitBwdTile {
                 const uint32_t lost = w[i][2] >> lost_at(k);
                 x = join_lost(h.x, l.x, lost & 1u) * sum - x;
                 y = join_lost(h.y, l.y, (lost >> 8) & 1u) * sum - y;
+                if (exp_s[row] == kWideExponent) x = y = 0.f;  // (all of it by the direct form)
             }
             if (i0 + row >= n_self) continue;
             float2* const at = reinterpret_cast<float2*>((char*)(out + (size_t)wave_row(i) * Dp) + out_off);
@@ -766,8 +831,8 @@ struct SplitBwdTile {
     DEVINL void direct() const {
         static_assert(TN == 64, "a lane per column");
         const float* const cf = p.coef + (size_t)d * B * T;
-        const int k = kt0 + (int)lane_here();
-        if (k >= Dp) return;
+        const int lane1 = (int)lane_here(), k = min(kt0 + lane1, Dp - 1);
+        auto lane_value = [&](float v, int l) __attribute__((always_inline)) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
         for (int i = i0 + 4 * wave; i < min(i0 + TM, n_self); i += 4 * WM * WN) {
             float add[4] = {0.f, 0.f, 0.f, 0.f};
             int row[4];
@@ -777,31 +842,34 @@ struct SplitBwdTile {
             for (int ot = 0; ot < n_slab; ++ot) {
                 if (exponent_of(i >> 5, ot) != kDirect) continue;
                 any = true;
+                // the slab's scales, and behind them those of the self rows
+                const float scales = p.rows.scale[lane1 < 32 ? other0 + min(32 * ot + lane1, n_other - 1) : self0 + min(i + (lane1 & 3), n_self - 1)];
                 float sv[4];
+                Row1 raw_self[4];
 #pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    Row1 raw;
-                    raw.load(p.rows, self0 + row[x], k);
-                    sv[x] = raw.value(k);
-                }
+                for (int x = 0; x < 4; ++x) raw_self[x].load(p.rows, self0 + row[x], k, lane_value(scales, 32 + x));
+#pragma unroll
+                for (int x = 0; x < 4; ++x) sv[x] = raw_self[x].value(k, lane_value(scales, 32 + x));
+                const int n = min(32, n_other - 32 * ot);
 #pragma unroll 1
-                for (int j0 = 32 * ot; j0 < min(32 * ot + 32, n_other); j0 += 2) {
+                for (int j0 = 0; j0 < n; j0 += 2) {
                     Row1 raw[2];
+                    const int js[2] = {j0, min(j0 + 1, n - 1)};
 #pragma unroll
-                    for (int y = 0; y < 2; ++y) raw[y].load(p.rows, other0 + min(j0 + y, n_other - 1), k);
+                    for (int y = 0; y < 2; ++y) raw[y].load(p.rows, other0 + 32 * ot + js[y], k, lane_value(scales, js[y]));
 #pragma unroll
                     for (int y = 0; y < 2; ++y) {
-                        const int j = min(j0 + y, n_other - 1);
-                        const float other = raw[y].value(k);
+                        const int j = 32 * ot + js[y];
+                        const float other = raw[y].value(k, lane_value(scales, js[y]));
 #pragma unroll
                         for (int x = 0; x < 4; ++x) {
-                            const float c = j0 + y < n_other ? (SIDE_B ? cf[(size_t)j * T + row[x]] : cf[(size_t)row[x] * T + j]) : 0.f;
+                            const float c = j0 + y < n ? (SIDE_B ? cf[(size_t)j * T + row[x]] : cf[(size_t)row[x] * T + j]) : 0.f;
                             add[x] = fmaf(c, DIST == DIST_L2 ? sv[x] - other : other, add[x]);
                         }
                     }
                 }
             }
-            if (!any) continue;
+            if (!any || kt0 + lane1 >= Dp) continue;
 #pragma unroll
             for (int x = 0; x < 4; ++x)
                 if (i + x < n_self) p.grad[(size_t)(self0 + i + x) * Dp + k] += add[x];

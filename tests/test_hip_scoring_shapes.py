@@ -319,6 +319,29 @@ def test_dot_of_long_and_short_rows(oracle64, power):
     _assert_each_row(*_first_moments(c, state, batch, 1, oracle64))
 
 
+# Columns much smaller than their rows' largest element, in every row or in one head and one tail: the gradients of such
+# columns by their own norm, as the rows' above
+@pytest.mark.parametrize("score_fn,distance_fn,loss_fn", [("TransE", "L2", "logsigmoid"), ("TransE", "L2", "softmax"),
+                                                          ("DistMult", "MatMul", "logsigmoid"), ("DistMult", "MatMul", "softmax")])
+@pytest.mark.parametrize("power", [-24, -30, -40, -60])
+@pytest.mark.parametrize("every", [True, False])
+@pytest.mark.parametrize("B,A,D", [(70, 100, 62), (200, 1024, 260)])
+def test_columns_of_other_sizes(oracle64, score_fn, distance_fn, loss_fn, power, every, B, A, D):
+    c = K.cfg_dict(score_fn=score_fn, distance_fn=distance_fn, loss_fn=loss_fn, n_shard=1, batch=B, a2a=A, dim=D, feature=0,
+                   n_entity=2000, n_relation=B, gamma=4.0, shared_table=True)
+    rng = np.random.default_rng(7)
+    state = K.make_state(c, rng, warm=False, scale=0.25)
+    batch = _one_block(c, state, np.full(B + A, 0.25), rng)
+    columns = [1, 34, D - 1]
+    rows = 1 + np.arange(B + A) if every else np.array([1 + 3, 1 + B + 37])
+    state["entity_data"][rows[:, None], columns] *= 2.0**power
+    if score_fn == "TransE":
+        state["relation_embedding"][(np.arange(B) if every else np.array([3]))[:, None], columns] *= 2.0**power
+    got, want = _first_moments(c, state, batch, B * A, oracle64)
+    _assert_each_row(got, want)
+    _assert_each_row(*[(l, e[:, columns].T, r[:, columns].T) for l, e, r in (got, want)])
+
+
 def _two_disjoint_blocks(kind, loss_fn, B, A, D, bad, merge):
     """One step of two blocks that share no row (entity or relation); `bad`: (role, value) of block 1's
     first head or tail, or None.  Returns the losses and block 0's rows afterwards."""
