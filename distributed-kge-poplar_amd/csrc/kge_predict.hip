@@ -48,6 +48,11 @@ DEVINL float4 raw4_f32(const Raw4<ET>& r) {
         return load4(reinterpret_cast<const char*>(r.v), 0, ET);
 }
 
+// Dot products below this, of rows whose largest elements are 2^14, are computed directly: the elements below 2^-28 of their
+// row's largest are off by 2^-50 of it, and where the large ones meet only such ones, they are the product.  (Of ordinary rows'
+// one in 10^6 is.)  Rows of zeros have a scale of 0, and no such product.
+constexpr float kLeastProduct = 0x1p10f;
+
 template <int DIST, int ET, int NS>  // ET: the rows' element type, NS: slabs of 32 columns
 __global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(PredictArgs p) {
     using Tile = RowTile<PT_ROWS, 2>;
@@ -121,7 +126,7 @@ __global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(Predict
                 }
                 if (c4 == 0) {
                     nb_s[buf][s_row] = sq;
-                    sb_s[buf][s_row] = scale;
+                    sb_s[buf][s_row] = DIST == DIST_L2 || top != 0.f ? scale : 0.f;  // (dot: the products of zeros are right)
                 }
                 // barrier i: tile i is in LDS; the other waves then multiply it while tile i + 1 is staged into
                 // the copy that they left before barrier i
@@ -155,7 +160,7 @@ __global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(Predict
     const float scale_a = half_scale(top), up_a = pow2_inverse(scale_a);
     if (lane < 32) {  // (read by this wave alone)
         na_s[32 * wave + lane] = na;
-        sa_s[32 * wave + lane] = DIST == DIST_L2 ? -2.f * scale_a : scale_a;
+        sa_s[32 * wave + lane] = DIST == DIST_L2 ? -2.f * scale_a : top != 0.f ? scale_a : 0.f;
     }
     asm volatile("" ::: "memory");  // (the rows are read again, not kept)
 #pragma unroll
@@ -209,6 +214,7 @@ __global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(Predict
         };
         float val[16];
         uint64_t bad = 0u;
+        float least = INFINITY;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int m = 8 * (r >> 2) + 4 * hl + (r & 3);
@@ -220,8 +226,10 @@ __global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(Predict
             } else {
                 val[r] = product * scale * sb;
                 bad |= __ballot(!(fabsf(val[r]) < INFINITY));
+                least = fminf(least, fabsf(product));
             }
         }
+        if (DIST != DIST_L2) bad |= __ballot(least < kLeastProduct);
         if (!bad && q0 + 32 <= p.n_query && (tile + 1) * PT_ROWS <= p.n_row) {  // the rule: all of them, without a look at any
             float* const out = p.scores + (size_t)q0 * p.ldc + tile * PT_ROWS;
             const uint32_t off = (uint32_t)(4 * hl * p.ldc + (lane & 31));
@@ -232,17 +240,26 @@ __global__ __launch_bounds__(2 * PT_WAVES * 64, 1) void k_predict_scores(Predict
             }
             continue;
         }
+        if (!bad) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int q = q0 + 8 * (r >> 2) + 4 * hl + (r & 3);
+                if (n < p.n_row && q < p.n_query) put(q, n, val[r]);
+            }
+            continue;
+        }
         uint32_t again = 0u;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int m = 8 * (r >> 2) + 4 * hl + (r & 3);
-            const bool good = DIST == DIST_L2 ? val[r] >= kCancelRatio * (na_s[32 * wave + m] + nb) : fabsf(val[r]) < INFINITY;
+            const bool good = DIST == DIST_L2 ? val[r] >= kCancelRatio * (na_s[32 * wave + m] + nb)
+                                              : fabsf(val[r]) < INFINITY && fabsf(val[r]) >= kLeastProduct * sa_s[32 * wave + m] * sb;
             if (n < p.n_row && q0 + m < p.n_query) {
                 if (good) put(q0 + m, n, val[r]); else again |= 1u << r;
             }
         }
         // rare: the wave computes pairs directly, eight at a time, eight lanes to a pair (two pairs of each
-        // of four lanes; fewer lanes: the last one's again): those that cancelled, and those that are not
+        // of four lanes; fewer lanes: the last one's again): those that cancelled, the smallest products, and those that are not
         // finite (an infinity's halves are infinity and NaN; from the values themselves its distance is
         // infinite and its row comes last, a NaN's score is NaN and the merge takes none).  Each round is a
         // ballot, a shuffle and trips to L2, one after the other, which four waves to a CU do not hide: at two

@@ -346,6 +346,40 @@ def test_predict_sweep_of_long_and_short_rows(dim, power):
         np.testing.assert_array_equal(np.sort(index), np.arange(41, 301))
 
 
+@pytest.mark.parametrize("power", [-20, -30, -45])
+@pytest.mark.parametrize("dim", [64, 250])
+def test_predict_sweep_of_large_against_small_elements(dim, power):
+    """The queries' large elements meet the rows' small ones (2^power of them) and the other way round, a row and a query of zeros
+    among them: products within 1e-6 of the sum of their terms' magnitudes."""
+    import poplar_kge as kge
+
+    settings = kge.Settings.create_demo()
+    m, ex = settings.model, settings.execution
+    m.score_fn, m.distance_fn, m.gamma = "DistMult", "MatMul", 0.0
+    m.n_shard, m.n_entity, m.embedding_size, m.entity_feature_size, m.n_relation_type = 1, 301, dim, 0, 4
+    settings.data.batch_size, settings.data.a2a_size, ex.rw_batch_size = 2, 2, 301
+    ex.predict_hr_batch_size, ex.predict_n_best = 40, 300
+    settings.prepare()
+    engine = kge.Engine(settings, np.array([300]))
+    rng = np.random.default_rng(8)
+    rows = np.zeros((1, 301, 3 * dim), np.float32)
+    even = np.arange(dim) % 2 == 0
+    rows[0, :, :dim] = rng.normal(size=(301, dim)) * np.where((np.arange(301)[:, None] > 40) == even, 2.0**power, 1.0)
+    rows[0, [7, 77]] = 0.0
+    for name in engine.uninitialized_variables.copy():
+        engine.write_variable(name, np.zeros(engine.variable_to_shape[name], engine.variable_to_dtype[name]))
+    engine.write_variable("relation_embedding", np.ones((4, dim), np.float32))
+    engine.write_entity_raw(0, rows)
+    queries = np.stack([np.zeros(40), 1 + np.arange(40), np.arange(40) % 4], axis=1).astype(np.uint32)
+    found = engine.predict(queries)
+    entity = rows[0, :, :dim].astype(np.float64)
+    for i in range(40):
+        index = found.shard_idx[i, :, 1]
+        np.testing.assert_array_equal(np.sort(index), np.arange(1, 301))
+        query = entity[1 + i]
+        assert np.all(np.abs(np.abs(found.score[i]) - np.abs(entity[index] @ query)) <= 1e-6 * (np.abs(entity[index]) @ np.abs(query)))
+
+
 @pytest.mark.parametrize("score_fn", ["TransE", "DistMult"])
 @pytest.mark.parametrize("dim,dtype", [(30, "float32"), (64, "float16"), (100, "float32"), (130, "float16"), (256, "float32"),
                                        (320, "float32"), (300, "float16")])
