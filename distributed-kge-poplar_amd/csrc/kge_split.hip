@@ -934,9 +934,15 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
 // --------------------------------------------------------------------------
 // launches
 
-// Which tiles.  128 x 64 read a third less, 64 x 64 are twice as many.  Forward, us, 64 x 64 and 128 x 64: 64 blocks of 256 x 512
-// (1024 large tiles) 33.4, 28.7; 32 of 256 x 256 (256) 13.5, 14.2; 4 of 200 x 268, D = 100 (40) 6.3, 6.8; one of 256 x 64,
-// D = 64 (2) 8.8, 9.9.  Backward: 45.2, 42.6; 16.5, 16.0 (512); 8.3, 8.5; 9.2, 9.2.
+// Which tiles.  128 x 64 read a third less, 64 x 64 are twice as many.  Large tiles are counted as if all tails were distinct (how many
+// are, only the device knows).  Launches, us, 64 x 64 and 128 x 64, D = 256, all tails distinct, behind each the large tiles:
+// Forward: 32 blocks of 256 x 256 14.6, 15.3 (256); 40 of 256 x 240 17.4, 19.2 (320); 48 18.5, 20.5 (384); 64 of 256 x 256 21.9, 23.6,
+// 32 of 256 x 512 21.3, 22.0, 8 of 1024 x 512 20.7, 20.7 (512); 40 of 256 x 480 27.8, 26.1 (640); 16 of 256 x 1536 32.1, 27.8 (768);
+// 64 of 256 x 512, 331 distinct, 31.1, 26.9 (1024); 4 of 200 x 268, D = 100, 11.6, 13.1 (40); one of 256 x 64, D = 64, 9.1, 10.1 (2).
+// Heads that fill half of their large tiles: 48 of 129 x 672, D = 100, 27.0, 30.6 (1056).
+// Backward: 6 of 1024 x 510 27.5, 31.4 (288); 8 of 1024 x 512 25.4, 28.4 (384); 32 of 256 x 256 18.3, 17.4 (512); 32 of 256 x 512
+// 32.6, 27.1 (768); 64 of 256 x 256 32.3, 31.1 (1024); 64 of 256 x 512, 331 distinct, 39.8, 40.4 (1536); 4 of 200 x 268 9.8, 11.1 (40).
+// Where the contraction is long on one side only, the small ones would be the faster: 16 of 256 x 1536 38.5, 44.0 (896).
 static bool large_tiles(const ScoreShape& sh) {
     return (int64_t)sh.S * ((sh.B + 127) / 128) * ((sh.T + 63) / 64) >= 512;
 }
