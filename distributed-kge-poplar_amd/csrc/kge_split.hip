@@ -61,7 +61,8 @@ __global__ __launch_bounds__(256, 8) void k_gather_halves(RowSource ent, const f
         key[r] = ent.index ? ent.index[c[r]] : (uint32_t)c[r];
         rkey[r] = (i < B && rel_mode) ? crel[c[r]] : 0u;
     }
-    const int end = B + tail_limit(tcount, d, T, tpad);
+    // (rows behind a block's distinct tails repeat its first one, and what they hold meets coefficients of zero: halves, always)
+    const int end = B + tail_limit(tcount, d, T, tpad), live = B + (tcount ? (int)tcount[d] : T);
 #pragma unroll
     for (int r = 0; r < RPW; ++r) asm volatile("" : "+s"(key[r]), "+s"(rkey[r]));
     if (i0 >= end) return;
@@ -108,7 +109,7 @@ __global__ __launch_bounds__(256, 8) void k_gather_halves(RowSource ent, const f
     // column of every gradient.  (With a row in the direct form for each of those, a step of 64 blocks of 256 x 512 took 2 us
     // more on average, one of 16 blocks of 256 x 1536 7.)
     auto small_column = [&](int i) __attribute__((always_inline)) {
-        const int first = i < B ? 0 : B, n = i < B ? B : end - B;
+        const int first = i < B ? 0 : B, n = i < B ? B : live - B;
         auto row4 = [&](int x, int k) __attribute__((always_inline)) {
             if (k >= s.Dp) return make_float4(0.f, 0.f, 0.f, 0.f);
             const int at = first + (i - first + x) % n, c = at < B ? d * B + at : s.n_head + d * T + at - B;
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(256, 8) void k_gather_halves(RowSource ent, const f
         sum[r] = wave_reduce63(sq[r], [](float a, float b) { return a + b; });
         const float most = __uint_as_float(wave_max_bits(top[r]));
         up[r] = pow2_inverse(half_scale(most));
-        if (__ballot(least[r] * up[r] < kLeastHalf) && most < INFINITY && i0 + r < end) look |= 1u << r;
+        if (__ballot(least[r] * up[r] < kLeastHalf) && most < INFINITY && i0 + r < live) look |= 1u << r;
     }
     if (__builtin_expect(look != 0u, 0)) {
 #pragma unroll 1

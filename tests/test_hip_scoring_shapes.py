@@ -342,6 +342,24 @@ def test_columns_of_other_sizes(oracle64, score_fn, distance_fn, loss_fn, power,
     _assert_each_row(*[(l, e[:, columns].T, r[:, columns].T) for l, e, r in (got, want)])
 
 
+# Merged tails: the slots behind a block's distinct ones repeat its first row.  That one has a column far below its largest
+# element, the last distinct ones have none: what the repeated slots hold is multiplied by zeros
+@pytest.mark.parametrize("score_fn,distance_fn,loss_fn", [("TransE", "L2", "logsigmoid"), ("TransE", "L2", "softmax"),
+                                                          ("DistMult", "MatMul", "logsigmoid"), ("DistMult", "MatMul", "softmax")])
+@pytest.mark.parametrize("live", [33, 71, 127])
+def test_repeated_tails_behind_small_columns(oracle64, score_fn, distance_fn, loss_fn, live):
+    B, A, D = 70, 300, 64
+    c = K.cfg_dict(score_fn=score_fn, distance_fn=distance_fn, loss_fn=loss_fn, n_shard=1, batch=B, a2a=A, dim=D, feature=0,
+                   n_entity=2000, n_relation=B, gamma=4.0, shared_table=True)
+    rng = np.random.default_rng(7)
+    state = K.make_state(c, rng, warm=False, scale=0.25)
+    batch = _one_block(c, state, np.full(B + A, 0.25), rng)
+    batch["a2a"][:] = B + np.arange(A, dtype=np.uint32) % live
+    state["entity_data"][1 + B:1 + B + 32, 1] *= 2.0**-40
+    state["entity_data"][1 + B:1 + B + 32, 34] *= 2.0**-40
+    _assert_each_row(*_first_moments(c, state, batch, B * A, oracle64))
+
+
 def _two_disjoint_blocks(kind, loss_fn, B, A, D, bad, merge):
     """One step of two blocks that share no row (entity or relation); `bad`: (role, value) of block 1's
     first head or tail, or None.  Returns the losses and block 0's rows afterwards."""
