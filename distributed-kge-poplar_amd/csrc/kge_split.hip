@@ -434,19 +434,26 @@ __global__ __launch_bounds__(256) void k_coef_halves(ScoreShape sh, const float*
     const int g = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int d = g / (MT * NT), mt = (g - d * MT * NT) / NT, nt = g % NT;
     if (d >= sh.S || 32 * nt >= tail_limit(sh.tcount, d, sh.T, sh.tpad)) return;
+    const int n_live = sh.tcount ? (int)sh.tcount[d] : sh.T;
     const float* src = coef + (size_t)d * sh.B * sh.T;
     const bool near = p.exponent[((size_t)d * MT + mt) * NT + nt] == kDirect;  // as the forward left it
     const int n = 32 * nt + (lane & 31);
-    const float sb = scale[n_head + d * sh.T + n];
+    const float sb = scale[n_head + d * sh.T + min(n, sh.T - 1)];
     float c[16], sa[16];
+    auto row = [&](int r) __attribute__((always_inline)) { return 32 * mt + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); };
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {  // all loads in one go: past the last row and column those of the last
+        const int m = min(row(r), sh.B - 1);
+        sa[r] = scale[d * sh.B + m];
+        c[r] = src[(size_t)m * sh.T + min(n, sh.T - 1)];
+    }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-        const int m = 32 * mt + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        sa[r] = m < sh.B ? scale[d * sh.B + m] : 0.f;  // (another block's may be NaN)
-        c[r] = m < sh.B && n < sh.T ? src[(size_t)m * sh.T + n] : 0.f;
+        if (row(r) >= sh.B) sa[r] = 0.f;
+        if (row(r) >= sh.B || n >= sh.T) c[r] = 0.f;
     }
     auto scale_a = [&](int r) __attribute__((always_inline)) { return sa[r]; };
-    store_coef_block<DIST>(c, scale_a, sb, near ? kDirect : coef_block_exponent(c, scale_a, sb, !sh.tcount || n < (int)sh.tcount[d], lane), p, d, 32 * mt, 32 * nt, lane);
+    store_coef_block<DIST>(c, scale_a, sb, near ? kDirect : coef_block_exponent(c, scale_a, sb, n < n_live, lane), p, d, 32 * mt, 32 * nt, lane);
 }
 
 // --------------------------------------------------------------------------
