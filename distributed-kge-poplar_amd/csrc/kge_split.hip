@@ -537,7 +537,7 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
     // rare: pairs are recomputed directly, half a wave to a pair, by all of the workgroup (a popular row's
     // come together in one wave's block): those that cancelled, and those that are not finite (an infinity's
     // second half is NaN; a wide row's scale is).  Pairs that do not count, a NaN among them, get any finite value.
-    if (__syncthreads_or(redo != 0u)) {
+    if (__builtin_expect(__syncthreads_or(redo != 0u), 0)) {
         float* const result = reinterpret_cast<float*>(smem);  // [TM][TN]; the tiles are no longer needed
         uint16_t* const list = reinterpret_cast<uint16_t*>(smem + TM * TN * 4);
         static_assert(TM * TN * 6 <= P::kLds, "the tile's pairs as a list and as results");
@@ -572,8 +572,10 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
                         part = DIST == DIST_L2 ? fmaf(u - v, u - v, part) : fmaf(u, v, part);
                     });
                 };
-                if (__builtin_expect(__ballot(is_wide(x.scale) || is_wide(y.scale)) != 0u, 0)) add(std::true_type{});
-                else add(std::false_type{});
+                // (L2 recomputes pairs every day, and without the look 16 blocks of 256 x 1536 take 34.3 us instead of 33.4; dot does not, and the
+                // second copy's code costs it 0.7 of 7.0, 4 blocks of 200 x 268, D = 100)
+                if (DIST == DIST_L2 && __builtin_expect(!__ballot(is_wide(x.scale) || is_wide(y.scale)), 1)) add(std::false_type{});
+                else add(std::true_type{});
             }
             part += swap1(part);
             part += swap2(part);
