@@ -840,6 +840,7 @@ struct SplitBwdTile {
     // stored.  A wave takes four rows at a time, a lane a column.
     DEVINL void direct() const {
         static_assert(TN == 64, "a lane per column");
+        constexpr int kRows = 4;  // of a slab under way (a divisor of 32)
         const float* const cf = p.coef + (size_t)d * B * T;
         const int lane1 = (int)lane_here(), k = min(kt0 + lane1, Dp - 1);
         auto lane_value = [&](float v, int l) __attribute__((always_inline)) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
@@ -861,21 +862,28 @@ struct SplitBwdTile {
 #pragma unroll
                 for (int x = 0; x < 4; ++x) sv[x] = raw_self[x].value(k, lane_value(scales, 32 + x));
                 const int n = min(32, n_other - 32 * ot);
+                float c[4];  // of the slab's row `lane`, zero past the last
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const int j = 32 * ot + min(lane1, n - 1);
+                    c[x] = SIDE_B ? cf[(size_t)j * T + row[x]] : cf[(size_t)row[x] * T + j];
+                }
+#pragma unroll
+                for (int x = 0; x < 4; ++x) c[x] = lane1 < n ? c[x] : 0.f;
 #pragma unroll 1
-                for (int j0 = 0; j0 < n; j0 += 2) {
-                    Row1 raw[2];
-                    const int js[2] = {j0, min(j0 + 1, n - 1)};
+                for (int j0 = 0; j0 < n; j0 += kRows) {
+                    Row1 raw[kRows];
+                    int j[kRows];
 #pragma unroll
-                    for (int y = 0; y < 2; ++y) raw[y].load(p.rows, other0 + 32 * ot + js[y], k, lane_value(scales, js[y]));
+                    for (int y = 0; y < kRows; ++y) {
+                        j[y] = min(j0 + y, n - 1);
+                        raw[y].load(p.rows, other0 + 32 * ot + j[y], k, lane_value(scales, j[y]));
+                    }
 #pragma unroll
-                    for (int y = 0; y < 2; ++y) {
-                        const int j = 32 * ot + js[y];
-                        const float other = raw[y].value(k, lane_value(scales, js[y]));
+                    for (int y = 0; y < kRows; ++y) {
+                        const float other = raw[y].value(k, lane_value(scales, j[y]));
 #pragma unroll
-                        for (int x = 0; x < 4; ++x) {
-                            const float c = j0 + y < n ? (SIDE_B ? cf[(size_t)j * T + row[x]] : cf[(size_t)row[x] * T + j]) : 0.f;
-                            add[x] = fmaf(c, DIST == DIST_L2 ? sv[x] - other : other, add[x]);
-                        }
+                        for (int x = 0; x < 4; ++x) add[x] = fmaf(lane_value(c[x], j0 + y), DIST == DIST_L2 ? sv[x] - other : other, add[x]);
                     }
                 }
             }
