@@ -714,9 +714,9 @@ struct SplitBwdTile {
     // a sub-block's exponent: of the self rows' group st and of slab ot
     DEVINL int exponent_of(int st, int ot) const { return p.in.exponent[(size_t)d * MT * NT + (SIDE_B ? (size_t)ot * NT + st : (size_t)st * NT + ot)]; }
 
-    // MAIN: the main pass, what this wave leaves to `todo`, whether any of the workgroup's does; or pass `pass`, added to the results
+    // MAIN: the main pass, what this wave leaves to `todo`; or pass `pass`, added to the results
     template <bool MAIN>
-    DEVINL bool sums(int pass, uint32_t& todo) const {
+    DEVINL void sums(int pass, uint32_t& todo) const {
         const size_t corner = (size_t)d * Bp * coef_pitch + (SIDE_B ? (size_t)(i0 >> 5) * kHalfBytes : (size_t)i0 * coef_pitch);
         const char* const a = (MAIN || pass < 16 ? p.in.coefp : p.in.small) + corner;
         const char* const b = p.rows.halves + (int64_t)other0 * pitch + (size_t)(kt0 >> 5) * kHalfBytes;
@@ -783,7 +783,6 @@ struct SplitBwdTile {
                    now = e;
                    return true;
                });
-        const bool any = MAIN && __syncthreads_or(todo != 0u);  // (here: behind the results' stores it would wait for those)
         const int lane1 = (int)lane_here(), cl = lane1 & 31, hl = lane1 >> 5;
         // the self rows' own scales leave the sums
 #pragma unroll
@@ -795,7 +794,7 @@ struct SplitBwdTile {
         const bool odd = lane1 & 1;
         float* const out = p.grad + (size_t)(self0 + i0) * Dp;
         const int k = kt0 + wn + (cl & ~1);
-        if (k >= Dp) return any;
+        if (k >= Dp) return;
         // (a row: the wave's part, in scalars, and the lane's, in one offset for all of them)
         const uint32_t in_off = (uint32_t)((4 * hl + odd) * pitch + (k >> 5) * kHalfBytes + (k & 31) * 2);
         const uint32_t lost_off = (uint32_t)((4 * hl + odd) * (Kp >> 5) + (k >> 5)) * 4;
@@ -832,7 +831,6 @@ struct SplitBwdTile {
             float2* const at = reinterpret_cast<float2*>((char*)(out + (size_t)wave_row(i) * Dp) + out_off);
             *at = MAIN ? make_float2(x, y) : DIST == DIST_L2 ? make_float2(at->x - x, at->y - y) : make_float2(at->x + x, at->y + y);
         }
-        return any;
     }
 
     // the direct form: c (self - other), or c other, one pair after the other as the reference codelet does (sub-blocks in
@@ -904,6 +902,7 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
     __shared__ __attribute__((aligned(16))) char smem[PA::kLds];
     __shared__ float csum_s[Tile::threads];
     __shared__ int exp_s[TM];
+    __shared__ uint32_t todo_s;
     // tile L's work: with(its side, its place)
     auto place = [](const SplitBwd& q, int L, auto&& with) __attribute__((always_inline)) {
         const int gx = (q.rows.Dp + TN - 1) / TN, ga = (q.B + TM - 1) / TM, gb = (q.T + TM - 1) / TM;
@@ -913,12 +912,18 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
         else with(std::true_type{}, xcd_tile(gx, gb, q.S, heads_first ? L - n_first : L));
     };
     uint32_t todo = 0u;
-    bool any = false;
+    if (threadIdx.x == 0) todo_s = 0u;  // (the loop's barriers stand between this and what follows it)
+    bool ran = false;
     place(p, blockIdx.x, [&](auto side_b, const TileId& t) __attribute__((always_inline)) {
         const SplitBwdTile<DIST, decltype(side_b)::value, Tile> tile(p, smem, csum_s, exp_s, threadIdx.x, t.z, t.x, t.y);
-        if (tile.i0 < tile.n_self) any = tile.template sums<true>(kMainPass, todo);
+        ran = tile.i0 < tile.n_self;
+        if (ran) tile.template sums<true>(kMainPass, todo);
     });
-    if (__builtin_expect(!__builtin_amdgcn_readfirstlane((int)any), 1)) return;
+    if (!ran) return;
+    if (todo && (threadIdx.x & 63) == 0) atomicOr(&todo_s, todo);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (not __syncthreads: the results' stores are no reason to wait)
+    todo = (uint32_t)__builtin_amdgcn_readfirstlane((int)todo_s);
+    if (__builtin_expect(!todo, 1)) return;
     // seldom.  Nothing that the main pass has computed is kept for this, nor from one pass for the next.
     auto anew = [&](auto&& with) __attribute__((always_inline)) {
         auto args = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
@@ -934,12 +939,6 @@ __global__ __launch_bounds__(Tile::threads) __attribute__((amdgpu_waves_per_eu(T
         });
     };
     __syncthreads();
-    uint32_t* const all = reinterpret_cast<uint32_t*>(csum_s);  // (no longer read)
-    if (threadIdx.x == 0) *all = 0u;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0 && todo) atomicOr(all, todo);
-    __syncthreads();
-    todo = (uint32_t)__builtin_amdgcn_readfirstlane((int)*all);
 #pragma unroll 1
     for (; todo & ~kDirectPass; todo &= todo - 1u) {
         uint32_t none = 0u;
